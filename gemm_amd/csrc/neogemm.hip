@@ -361,7 +361,12 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
   constexpr int CH = WTN / 8;        // 16-byte chunks per staged row
   constexpr int RPI = 64 / CH;       // rows one store instruction covers
   constexpr bool CAN_STAGE = (size_t)NW * WTM * WTN * 2 <= (size_t)LDS_BYTES && CH >= 4 && CH <= 64;
-  const bool stage = CAN_STAGE && p.ksplit == 1 && p.beta == 0.f && (((uintptr_t)gC | (uintptr_t)(p.ldc * 2)) & 15) == 0;
+  const bool aligned_c = (((uintptr_t)gC | (uintptr_t)(p.ldc * 2)) & 15) == 0;
+  const bool stage = CAN_STAGE && p.ksplit == 1 && p.beta == 0.f && aligned_c;
+  // beta != 0: staged as fp32 (the sum is rounded once), row tiles of the wave tile at a time, as many as the LDS holds
+  constexpr int ST = TM % 4 == 0 && NW * 4 * 16 * WTN * 4 <= (int)LDS_BYTES ? 4 : TM % 2 == 0 && NW * 2 * 16 * WTN * 4 <= (int)LDS_BYTES ? 2 : 1;
+  constexpr bool CAN_STAGE_F32 = CAN_STAGE && (CH & (CH - 1)) == 0 && NW * ST * 16 * WTN * 4 <= (int)LDS_BYTES && ST * 16 % RPI == 0;
+  const bool stage_add = CAN_STAGE_F32 && p.ksplit == 1 && p.beta != 0.f && aligned_c;
   if (stage) {
     if constexpr (CAN_STAGE) {
       // every wave is done with the slab images (its LDS reads have returned: the MFMAs that used them
@@ -413,6 +418,67 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
 #pragma unroll
               for (int e = 0; e < 8; ++e)
                 if (col + e < p.N) ((__bf16*)dst)[e] = v[e];
+            }
+          }
+        }
+      }
+    }
+  } else if (stage_add) {
+    if constexpr (CAN_STAGE_F32) {
+      // C = alpha * acc + beta * C, the sum in fp32: the accumulators are parked as they are, ST row tiles at a time, and
+      // come back row-wise, eight columns a lane, beside the 16 bytes of C that they are added to.  All of C's old values
+      // are requested before the first of them is needed (up to 32 loads of a wave in flight; the fragments' registers are free).
+      // The branch below, which reads C two bytes at a time in the accumulators' layout, took 134 us at 4096^3 where the plain
+      // product takes 94; this one takes 98 (C read: 34 MB).
+      constexpr int CH4 = WTN / 4;  // 16-byte chunks per parked fp32 row
+      constexpr int NLD = WTM / RPI;
+      const int colc = lane % CH, col = map.col(colc * 8);
+      const bool whole_cols = col + 7 < p.N;
+      i32x4 old[NLD];
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // nothing of the main loop is on its way into LDS any more
+#pragma unroll
+      for (int st = 0; st < NLD; ++st) {
+        const int grow = map.row(st * RPI + lane / CH);
+        if (grow < p.M && whole_cols) old[st] = *(const i32x4*)(gC + ((size_t)grow * p.ldc + col) * 2);
+      }
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const uint32_t region = lds0 + (uint32_t)wave * (ST * 16 * WTN * 4);
+#pragma unroll
+      for (int i0 = 0; i0 < TM; i0 += ST) {
+#pragma unroll
+        for (int i = i0; i < i0 + ST; ++i) {
+          const uint32_t row = (i - i0) * 16 + row_l;
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            f32x4 v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = acc_get(acc[i][j][r]);
+            const uint32_t c = 4 * j + (lane >> 4);
+            *((NEOGEMM_AS3 f32x4*)(uintptr_t)(region + row * (WTN * 4) + ((c ^ (row & (CH4 - 1))) << 4))) = v;
+          }
+        }
+#pragma unroll
+        for (int st = 0; st < ST * 16 / RPI; ++st) {
+          const uint32_t row = st * RPI + lane / CH;
+          f32x4 v[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            v[h] = *((NEOGEMM_AS3 f32x4*)(uintptr_t)(region + row * (WTN * 4) + (((2u * colc + h) ^ (row & (CH4 - 1))) << 4)));
+          const int grow = map.row(i0 * 16 + (int)row);
+          if (grow < p.M) {
+            char* dst = gC + ((size_t)grow * p.ldc + col) * 2;
+            if (whole_cols) {
+              const bf16x8 c = __builtin_bit_cast(bf16x8, old[i0 * 16 / RPI + st]);
+              bf16x8 o;
+#pragma unroll
+              for (int e = 0; e < 8; ++e) o[e] = (__bf16)__builtin_fmaf(p.beta, (float)c[e], v[e >> 2][e & 3] * p.alpha);
+              __builtin_nontemporal_store(o, (bf16x8*)dst);
+            } else {
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                if (col + e < p.N)
+                  ((__bf16*)dst)[e] = (__bf16)__builtin_fmaf(p.beta, (float)((const __bf16*)dst)[e], v[e >> 2][e & 3] * p.alpha);
             }
           }
         }
