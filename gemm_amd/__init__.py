@@ -11,7 +11,7 @@ Nothing here computes: without libneogemm.so and a GPU every call raises.
 import torch
 
 from . import _abi
-from ._abi import (B_KN, B_NK, C_COL, C_ROW, NeoGemmError, VARIANT_AUTO, VARIANT_GENERIC, VARIANT_NAMES,  # noqa: F401
+from ._abi import (A_KM, A_MK, B_KN, B_NK, C_COL, C_ROW, NeoGemmError, VARIANT_AUTO, VARIANT_GENERIC, VARIANT_NAMES,  # noqa: F401
                    VARIANT_SKINNY16, VARIANT_SKINNY32, VARIANT_SKINNY64, VARIANT_SKINNY128, VARIANT_STRIP, VARIANT_T192x256_W4, VARIANT_T96x128_W4, VARIANT_T64x64_W4, VARIANT_C256x256_W4,
                    VARIANT_T128x128_W4, VARIANT_T128x256_W4, VARIANT_T256x128_W4, VARIANT_T256x256_W4,
                    VARIANT_T64x128_W4, plan, strerror, version, workspace_bytes)
@@ -52,8 +52,21 @@ def _workspace(device, nbytes):
 
 
 def gemm_into(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, variant=None, split_k=0, group_m=0, alpha=1.0,
-              beta=0.0):
+              beta=0.0, a_layout=A_MK):
     """Call the C ABI on torch's current stream; A, B, C are torch tensors used as device buffers."""
+    if a_layout != A_MK:
+        if variant is not None:
+            raise ValueError("a transposed A goes through neogemm_bf16_general, which chooses the kernel itself")
+        lib = _abi.load()
+        need = int(lib.neogemm_bf16_general_workspace_bytes(M, N, K, a_layout, b_layout, c_layout, 1))
+        ws_ptr = _workspace(C.device, need).data_ptr() if need else 0
+        with torch.cuda.device(C.device):
+            stream = torch.cuda.current_stream().cuda_stream
+            st = lib.neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, a_layout, b_layout,
+                                          c_layout, alpha, beta, 0, 0, 0, 1, ws_ptr or None, need, stream or None)
+        if st != _abi.OK:
+            raise NeoGemmError(st, f"M={M} N={N} K={K} a_layout={a_layout} b_layout={b_layout} c_layout={c_layout}")
+        return
     need = workspace_bytes(M, N, K)
     if variant is not None and split_k > 1:
         need = max(need, split_k * M * N * 4)
@@ -68,6 +81,27 @@ def gemm_into(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, variant=None,
         raise NeoGemmError(st, f"M={M} N={N} K={K} b_layout={b_layout} c_layout={c_layout} variant={variant}")
 
 
+def _describe(A, B, transposed_a=True):
+    """How A [M,K] and B [K,N] lie in memory: (A, B, lda, ldb, a_layout, b_layout); what no layout describes is made
+    contiguous.  A transposed A is read in place where the tile kernels take it: whole 16-byte chunks, and more rows than
+    the decode kernels, which want K-contiguous rows, would serve."""
+    M, K = A.shape
+    N = B.shape[1]
+    if B.stride(1) == 1 or N <= 1:
+        b_layout, ldb = B_KN, (B.stride(0) if K > 1 else max(N, 1))
+    elif B.stride(0) == 1:
+        b_layout, ldb = B_NK, (B.stride(1) if N > 1 else max(K, 1))
+    else:
+        B = B.contiguous()
+        b_layout, ldb = B_KN, max(N, 1)
+    if A.stride(1) == 1 or K <= 1:
+        return A, B, (A.stride(0) if M > 1 else max(K, 1)), ldb, A_MK, b_layout
+    if (transposed_a and A.stride(0) == 1 and A.stride(1) >= M > 128 and M % 8 == 0 and N % 8 == 0 and A.stride(1) % 8 == 0 and
+            ldb % 8 == 0 and A.data_ptr() % 16 == 0 and B.data_ptr() % 16 == 0 and (b_layout == B_KN or K % 8 == 0)):
+        return A, B, A.stride(1), ldb, A_KM, b_layout
+    return A.contiguous(), B, max(K, 1), ldb, A_MK, b_layout
+
+
 def gemm(A, B, variant=None, split_k=0, group_m=0):
     """C[M,N] = A[M,K] @ B[K,N]; bf16 in, fp32 accumulate, bf16 out (new tensor)."""
     _check(A, "A")
@@ -76,21 +110,13 @@ def gemm(A, B, variant=None, split_k=0, group_m=0):
         raise ValueError(f"inner dimensions differ: A is {tuple(A.shape)}, B is {tuple(B.shape)}")
     if A.device != B.device:
         raise ValueError("A and B must be on the same device")
-    if A.stride(1) != 1 and A.shape[1] > 1:
-        A = A.contiguous()
     M, K = A.shape
     N = B.shape[1]
-    lda = A.stride(0) if M > 1 else max(K, 1)
-    if B.stride(1) == 1 or N <= 1:
-        b_layout, ldb = B_KN, (B.stride(0) if K > 1 else max(N, 1))
-    elif B.stride(0) == 1:
-        b_layout, ldb = B_NK, (B.stride(1) if N > 1 else max(K, 1))
-    else:
-        B = B.contiguous()
-        b_layout, ldb = B_KN, max(N, 1)
+    A, B, lda, ldb, a_layout, b_layout = _describe(A, B, variant is None)
     C = torch.empty((M, N), dtype=torch.bfloat16, device=A.device)
     if M and N:
-        gemm_into(A, B, C, M, N, K, lda, ldb, max(N, 1), b_layout, C_ROW, variant, split_k, group_m)
+        gemm_into(A, B, C, M, N, K, lda, ldb, max(N, 1), b_layout, C_ROW, variant, split_k, group_m,
+                  a_layout=a_layout)
     return C
 
 
@@ -122,20 +148,12 @@ def gemm_scaled(A, B, C, alpha=1.0, beta=0.0):
     _check(C, "C")
     if A.shape[1] != B.shape[0] or C.shape != (A.shape[0], B.shape[1]) or not C.is_contiguous():
         raise ValueError(f"shapes: A {tuple(A.shape)}, B {tuple(B.shape)}, C {tuple(C.shape)} (contiguous [M,N])")
-    if A.stride(1) != 1 and A.shape[1] > 1:
-        A = A.contiguous()
     M, K = A.shape
     N = B.shape[1]
-    lda = A.stride(0) if M > 1 else max(K, 1)
-    if B.stride(1) == 1 or N <= 1:
-        b_layout, ldb = B_KN, (B.stride(0) if K > 1 else max(N, 1))
-    elif B.stride(0) == 1:
-        b_layout, ldb = B_NK, (B.stride(1) if N > 1 else max(K, 1))
-    else:
-        B = B.contiguous()
-        b_layout, ldb = B_KN, max(N, 1)
+    A, B, lda, ldb, a_layout, b_layout = _describe(A, B)
     if M and N:
-        gemm_into(A, B, C, M, N, K, lda, ldb, max(N, 1), b_layout, C_ROW, alpha=float(alpha), beta=float(beta))
+        gemm_into(A, B, C, M, N, K, lda, ldb, max(N, 1), b_layout, C_ROW, alpha=float(alpha), beta=float(beta),
+                  a_layout=a_layout)
     return C
 
 

@@ -11,6 +11,7 @@ LIB_PATH = os.path.join(_HERE, "libneogemm.so")
 
 OK, ERR_BAD_ARG, ERR_WORKSPACE, ERR_UNSUPPORTED, ERR_LAUNCH, ERR_SCRATCH_LIMIT = 0, -1, -2, -3, -4, -5
 NOALLOC_SCRATCH_BYTES = 32 * 1024 * 1024
+A_MK, A_KM = 0, 1
 B_KN, B_NK = 0, 1
 C_ROW, C_COL = 0, 1
 VARIANT_AUTO, VARIANT_GENERIC = 0, 1
@@ -38,6 +39,9 @@ PROTOTYPES = {
     "neogemm_bf16_batched": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int,
                                     _vp, _sz, _vp]),
     "neogemm_bf16_batched_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "neogemm_bf16_general": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, ctypes.c_float,
+                                    ctypes.c_float, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
+    "neogemm_bf16_general_workspace_bytes": (_sz, [_i64, _i64, _i64, _int, _int, _int, _i64]),
     "neogemm_bf16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "neogemm_bf16_variant": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _sz, _vp,
                                     _int, _int, _int]),

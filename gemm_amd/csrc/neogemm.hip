@@ -552,7 +552,6 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_tile_kernel(TileArgs p) {
   constexpr int WTM = BM / WGM, WTN = BN / WGN;
   constexpr int TM = WTM / 16, TN = WTN / 16;
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be a multiple of the 16x16 MFMA tile");
-  static_assert(AK || BK, "at least one operand is K-major");
   // images per operand: four 32-deep slabs if MN-major; three 64-deep tiles if K-major, except that
   // B gets by with NB_KK = two when both are K-major and the tile is large (160 KiB of LDS for a 256x256 tile either way)
   using OpA = Operand<BM, AK, NW, AK ? 3 : 4>;
@@ -611,7 +610,8 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_tile_kernel(TileArgs p) {
   // Which of this wave's loads go under which half of a slab step.  The schedule has a period of two
   // slabs (four halves P0..P3, starting with an odd slab):
   //   next to an MN-major operand, a K-major one loads a 64-deep tile in P0 and P1, the MN-major one a
-  //   slab in P2 and one in P3; if both are K-major, B loads its tile in P0 and A over P1..P3.
+  //   slab in P2 and one in P3; if both are K-major, B loads its tile in P0 and A over P1..P3; if both are
+  //   MN-major, a slab of A and the same slab of B per iteration.
   // Segment = loads [lo, hi) of operand A (op 1) or B (op 2); a half carries up to two segments.
   struct Seg { int op, lo, hi; };
   auto plan = [](int phase, int which) constexpr -> Seg {
@@ -625,6 +625,9 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_tile_kernel(TileArgs p) {
       if (phase == 0) return Seg{1, 0, IA / 2};
       if (phase == 1) return Seg{1, IA / 2, IA};
       return Seg{2, 0, IB};
+    } else if (!BK) {
+      if (which == 1) return Seg{0, 0, 0};
+      return phase & 1 ? Seg{2, 0, IB} : Seg{1, 0, IA};
     } else {
       if (which == 1) return Seg{0, 0, 0};
       if (phase == 0) return Seg{2, 0, IB / 2};
@@ -781,19 +784,26 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_tile_kernel(TileArgs p) {
   //     the sync before P0 needs A tile t+1 and B tile t+1: all but A tile t+2
   //   (B three images: P0: B tile t+3; the sync before P0 keeps B tile t+2 and A tile t+2 in flight)
   //     no loads land between the sync before P0 and the reads of slab 2t+3: no second sync
-  constexpr int KEEP_ODD = (AK && BK) ? IA + (NB_KK == 3 ? IB : 0) : (IA + IB + (AK ? IB : IA));
-  constexpr int KEEP_EVEN = (AK && BK) ? -1 : IA + IB;
+  //   both MN-major (four images each; the product of a weight gradient dY^T * X, which used to wait for a copy of dY: 68 us
+  //     at 4096 x 4096, where the product takes 95): P0, P1: slab 2t+5 of A, of B; P2, P3: slab 2t+6 of A, of B
+  //     the sync before iteration j needs slab j+1 of both: all but slabs j+2 and j+3
+  constexpr bool MN_MN = !AK && !BK;
+  constexpr int KEEP_ODD = (AK && BK) ? IA + (NB_KK == 3 ? IB : 0) : MN_MN ? 2 * (IA + IB) : (IA + IB + (AK ? IB : IA));
+  constexpr int KEEP_EVEN = (AK && BK) ? -1 : MN_MN ? 2 * (IA + IB) : IA + IB;
 
   // prologue: every image of both operands is requested, what slabs 0 and 1 need first, and only that
   // is waited for (units past K are requested too, fully masked: the counts below hold for any K).
   //   K-major A next to MN-major B: A0 B0 B1 | A1 B2 B3 A2      (mirrored if B is the K-major one)
   //   both K-major:                 A0 B0 | A1 B1 A2 (B2)
+  //   both MN-major:                A0 B0 A1 B1 | A2 B2 A3 B3
   constexpr int KEEP_PRO = (AK && BK) ? 2 * IA + IB + (NB_KK == 3 ? IB : 0) : 2 * IA + 2 * IB;
   if constexpr (AK && BK) {
     burst_a(0); burst_b(0); burst_a(1); burst_b(1); burst_a(2);
     if constexpr (NB_KK == 3) burst_b(2);
   } else if constexpr (AK) {
     burst_a(0); burst_b(0); burst_b(1); burst_a(1); burst_b(2); burst_b(3); burst_a(2);
+  } else if constexpr (MN_MN) {
+    burst_a(0); burst_b(0); burst_a(1); burst_b(1); burst_a(2); burst_b(2); burst_a(3); burst_b(3);
   } else {
     burst_b(0); burst_a(0); burst_a(1); burst_b(1); burst_a(2); burst_a(3); burst_b(2);
   }
@@ -848,8 +858,8 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_tile_kernel(TileArgs p) {
       slab_step(P1{}, T{}, jo + 1, ra0, rb0, std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, da0, db0,
                 da0, db0);
       if constexpr (KEEP_EVEN >= 0) sync(std::integral_constant<int, KEEP_EVEN>{});
-      slab_step(P0{}, T{}, jo + 2, ra1, rb1, std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{}, da0, db0,
-                da1, db1);
+      slab_step(P0{}, T{}, jo + 2, ra1, rb1, std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{},
+                MN_MN ? da1 : da0, MN_MN ? db1 : db0, da1, db1);
       x_ld = x_rd;
       x_rd = x_rd + 1 == 3 ? 0 : x_rd + 1;
     }
@@ -955,6 +965,10 @@ hipError_t launch_tile(const TileArgs& a, bool ak, bool bk, hipStream_t st) {
   }
   if (!ak && bk) {
     if constexpr (BM >= 128 && (BM & (BM - 1)) == 0) return go(gemm_tile_kernel<BM, BN, WGM, WGN, false, true>);
+  }
+  if (!ak && !bk) {
+    if constexpr (BM >= 128 && (BM & (BM - 1)) == 0 && BN >= 128 && (BN & (BN - 1)) == 0)
+      return go(gemm_tile_kernel<BM, BN, WGM, WGN, false, false>);
   }
   return hipErrorInvalidValue;
 }
@@ -1825,9 +1839,11 @@ static const VariantInfo kVariants[NEOGEMM_VARIANT_COUNT] = {
 // a shape against the kernels above in any sweep; their numbers stay reserved and a call that names one is refused.
 static bool variant_retired(int v) { return v == NEOGEMM_VARIANT_RETIRED_2 || v == NEOGEMM_VARIANT_RETIRED_8; }
 
-static bool is_aligned(const void* A, const void* B, const void* C, int64_t K, int64_t lda, int64_t ldb,
-                       int64_t ldc) {
-  return (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && ((uintptr_t)C & 7) == 0 && (K & 7) == 0 && (lda & 7) == 0 &&
+// What the MFMA kernels with direct-to-LDS loads assume: 16-byte chunks that start on 16-byte addresses and, where an
+// operand has K-contiguous rows, do not straddle the end of K.
+static bool is_aligned(const void* A, const void* B, const void* C, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
+                       bool any_kmajor) {
+  return (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && ((uintptr_t)C & 7) == 0 && ((K & 7) == 0 || !any_kmajor) && (lda & 7) == 0 &&
          (ldb & 7) == 0 && (ldc & 3) == 0;
 }
 
@@ -1868,13 +1884,16 @@ static int planning_cus() {
   return cus;
 }
 static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
-                       int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int ncus = 256) {
+                       int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int ncus = 256, int a_layout = NEOGEMM_A_MK) {
   if (!aligned || K == 0) {
     *variant = NEOGEMM_VARIANT_GENERIC;
     *split_k = 1;
     return;
   }
   const int64_t rows = c_layout == NEOGEMM_C_ROW ? M : N, cols = c_layout == NEOGEMM_C_ROW ? N : M;
+  const bool both_k = a_layout == NEOGEMM_A_MK && b_layout == NEOGEMM_B_NK;
+  // the operand that supplies the kernel's rows has them contiguous (an MN-major image: tiles of 128 or 256 rows only)
+  const bool rows_mn = c_layout == NEOGEMM_C_ROW ? a_layout == NEOGEMM_A_KM : b_layout == NEOGEMM_B_KN;
   const int64_t ktiles = ceil_div(K, KTILE);
   const double cus = (double)ncus;
   const double bytes = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch;
@@ -1886,12 +1905,11 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
     // the 64x128 tile has too little in flight to stream from HBM: only for problems that stay in cache
     if (c.variant == NEOGEMM_VARIANT_T64x128_W4 && bytes > 32e6) continue;
     // 192 rows only of a K-major operand (an MN-major image needs a power of two)
-    if ((c.variant == NEOGEMM_VARIANT_T192x256_W4 || c.variant == NEOGEMM_VARIANT_T96x128_W4) && c_layout == NEOGEMM_C_COL &&
-        b_layout != NEOGEMM_B_NK)
-      continue;
+    if ((c.variant == NEOGEMM_VARIANT_T192x256_W4 || c.variant == NEOGEMM_VARIANT_T96x128_W4) && rows_mn) continue;
+    if (c.variant == NEOGEMM_VARIANT_T64x128_W4 && rows_mn && a_layout == NEOGEMM_A_KM) continue;
     // the small tiles have too little in flight to stream from HBM; 64x64 takes K-major operands only
     if ((c.variant == NEOGEMM_VARIANT_T96x128_W4 || c.variant == NEOGEMM_VARIANT_T64x64_W4) && bytes > 32e6) continue;
-    if (c.variant == NEOGEMM_VARIANT_T64x64_W4 && b_layout != NEOGEMM_B_NK) continue;
+    if (c.variant == NEOGEMM_VARIANT_T64x64_W4 && !both_k) continue;
     const double tiles = (double)ceil_div(rows, kVariants[c.variant].bm) * (double)ceil_div(cols, kVariants[c.variant].bn);
     for (int sp : kSplits) {
       if (sp > 1 && ktiles / sp < 2) break;  // at least 128 deep per split
@@ -1906,14 +1924,14 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
       const double rounds = rounds_of(wgs / (cus * c.per_cu));
       double t = per_cu_wgs * ktps * c.ktile_us;
       // both operands K-major: the tall tile runs a little ahead of the wide one (2560^3: 33.8 against 35.0 us)
-      if (c.variant == NEOGEMM_VARIANT_T128x256_W4 && b_layout == NEOGEMM_B_NK) t *= 1.02;
+      if (c.variant == NEOGEMM_VARIANT_T128x256_W4 && both_k) t *= 1.02;
       // latency knows no discount, and two latency-bound workgroups on one CU were measured to take turns
       // (with both operands K-major the 128x128 tile has three tiles of each in flight when it streams: 256 x 14336 x 4096
       // unsplit, 224 workgroups, runs its 64 K tiles in 32.3 us; with far fewer workgroups than CUs a K tile takes longer,
       // and with more than CUs the second workgroup of a CU goes at the pace of the first: 128 x 5120 x 27648 with split 6,
       // 240 workgroups, 69 us; split 8, 320 of them, 98; split 12, 480, 76)
       const double lat_v =
-          c.variant == NEOGEMM_VARIANT_T128x128_W4 && bytes > 32e6 && b_layout == NEOGEMM_B_NK && wgs >= 0.6 * cus && wgs <= cus ? 0.46 : lat_us;
+          c.variant == NEOGEMM_VARIANT_T128x128_W4 && bytes > 32e6 && both_k && wgs >= 0.6 * cus && wgs <= cus ? 0.46 : lat_us;
       const double lat_floor = __builtin_ceil(wgs / cus) * ktps * lat_v;
       if (t < lat_floor) t = lat_floor;
       t += rounds * (c.fixed_us + (sp > 1 ? c.split_fixed_us : 0.0));
@@ -1947,7 +1965,7 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
   // onto a few memory channels (128 x 8192 x 8192 streams at 3.6 TB/s where 128 x 4096 x 14336 reaches 4.4), which the
   // estimates above do not know; the strip kernels start every strip at another depth for this reason.  So against them
   // the tiles' estimate counts for a fifth more there.
-  const double best_tile = best * (b_layout == NEOGEMM_B_NK && K % 8192 == 0 && bytes > 32e6 ? 1.2 : 1.0);
+  const double best_tile = best * (both_k && K % 8192 == 0 && bytes > 32e6 ? 1.2 : 1.0);
   // The strip kernel with K split over s workgroups per strip, for few strips and deep K (128 x 8192 x 8192: 128 strips,
   // two splits, 38.0 us against 44.0 for split-K tiles; 112 x 4096 x 16384: four, 37 against 47): the unsplit kernel's
   // estimate with a workgroup's bytes divided by s, plus the reduction as for the tiles; 1024 to 8192 deep per split
@@ -1976,7 +1994,9 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
     return split_best;
   };
   const bool skinny_m = M <= 64, skinny_n = !skinny_m && N <= 64 && b_layout == NEOGEMM_B_NK;
-  if ((skinny_m || skinny_n) && batch == 1 && K >= 4 * KTILE) {
+  // (the skinny and strip kernels read the short operand as K-contiguous rows)
+  const bool skinny_ok = batch == 1 && a_layout == NEOGEMM_A_MK;
+  if ((skinny_m || skinny_n) && skinny_ok && K >= 4 * KTILE) {
     const int64_t rows = skinny_m ? M : N, cols = skinny_m ? N : M;  // the kernel's own terms, whatever the layout of C
     double t;
     if (b_layout == NEOGEMM_B_NK) {
@@ -2044,7 +2064,7 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
   // the factor.
   const bool wide_m = !skinny_m && !skinny_n && M <= 128;
   const bool wide_n = !skinny_m && !skinny_n && !wide_m && N <= 128 && b_layout == NEOGEMM_B_NK;
-  if ((wide_m || wide_n) && batch == 1 && K >= 2048) {
+  if ((wide_m || wide_n) && skinny_ok && K >= 2048) {
     const int64_t rows = wide_m ? M : N, cols = wide_m ? N : M;
     const bool strip_kernel = b_layout == NEOGEMM_B_NK && rows > 96;
     int w = 64;  // strip width: see launch_strip
@@ -2092,8 +2112,7 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
   }
   // the 256x256 tile unsplit, K in whole periods of 128, rows from a K-major operand: the kernel that accumulates twice
   // in a row into each tile does the same work on less power (8192^3 +1.3 %, 4096^3 +1.2 %, bit-identical results)
-  if (bv == NEOGEMM_VARIANT_T256x256_W4 && bs == 1 && K % (2 * KTILE) == 0 &&
-      (c_layout == NEOGEMM_C_ROW || b_layout == NEOGEMM_B_NK))
+  if (bv == NEOGEMM_VARIANT_T256x256_W4 && bs == 1 && K % (2 * KTILE) == 0 && !rows_mn)
     bv = NEOGEMM_VARIANT_C256x256_W4;
   *variant = bv;
   *split_k = bs;
@@ -2147,29 +2166,29 @@ static const std::vector<PlanEntry>& plan_table() {
   return table;
 }
 static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
-                          int64_t batch, int b_layout, int ncus);
+                          int64_t batch, int b_layout, int ncus, int a_layout);
 // The cost model walks every (tile, split) candidate: a few microseconds on the host, as long as a small GEMM takes
 // on the GPU.  A caller in a loop repeats a handful of shapes, so each thread remembers its last few answers.
 static void plan(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
-                 int64_t batch = 1, int b_layout = NEOGEMM_B_KN) {
+                 int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int a_layout = NEOGEMM_A_MK) {
   struct Memo {
     int64_t M = -1, N = -1, K = -1, batch = -1;
-    int b_layout = -1, c_layout = -1, aligned = -1, ncus = -1, variant = 0, split_k = 0;
+    int a_layout = -1, b_layout = -1, c_layout = -1, aligned = -1, ncus = -1, variant = 0, split_k = 0;
   };
   static thread_local Memo memo[32];  // the workspace query alone asks for four layouts of a shape
   static thread_local unsigned next = 0;
   const int ncus = planning_cus();
   for (const Memo& m : memo)
     if (m.M == M && m.N == N && m.K == K && m.batch == batch && m.b_layout == b_layout && m.c_layout == c_layout &&
-        m.aligned == (int)aligned && m.ncus == ncus) {
+        m.aligned == (int)aligned && m.ncus == ncus && m.a_layout == a_layout) {
       *variant = m.variant;
       *split_k = m.split_k;
       return;
     }
-  plan_uncached(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus);
+  plan_uncached(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout);
   Memo& m = memo[next++ & 31];
   m.M = M, m.N = N, m.K = K, m.batch = batch, m.b_layout = b_layout, m.c_layout = c_layout, m.aligned = (int)aligned;
-  m.ncus = ncus;
+  m.ncus = ncus, m.a_layout = a_layout;
   m.variant = *variant, m.split_k = *split_k;
 }
 // Tuned choices that ship with the library: shapes of a sweep (gemm_amd/tune.py over M in 256 .. 8192 x the (N, K) pairs of
@@ -2181,8 +2200,8 @@ static const PlanEntry kDefaultPlan[] = {
 #include "neogemm_default_plan.inc"
 };
 static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
-                          int64_t batch, int b_layout, int ncus) {
-  if (aligned && K > 0 && batch == 1) {
+                          int64_t batch, int b_layout, int ncus, int a_layout) {
+  if (aligned && K > 0 && batch == 1 && a_layout == NEOGEMM_A_MK) {
     auto match = [&](const PlanEntry& e) {
       return e.M == M && e.N == N && e.K == K && e.c_layout == c_layout && e.b_layout == b_layout;
     };
@@ -2200,7 +2219,7 @@ static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_l
           return;
         }
   }
-  plan_model(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus);
+  plan_model(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout);
 }
 
 // The largest split-K factor plan() returns for this shape over the four (b_layout, c_layout) combinations a call can
@@ -2311,9 +2330,11 @@ static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream
   return NEOGEMM_OK;
 }
 
-// A batch of `count` problems of one shape; strides in elements between consecutive problems (0: shared operand).
+// A batch of `count` problems of one shape; strides in elements between consecutive problems (0: shared operand); and how
+// A is laid out, which only the general entry point lets a caller choose.
 struct BatchArgs {
   int64_t count = 1, sa = 0, sb = 0, sc = 0;
+  int a_layout = NEOGEMM_A_MK;
 };
 
 static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
@@ -2327,37 +2348,40 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     const int64_t c_extent = c_layout == NEOGEMM_C_ROW ? (M - 1) * ldc + N : (N - 1) * ldc + M;
     if (bt.sc < c_extent) return NEOGEMM_ERR_BAD_ARG;
   }
-  if ((b_layout != NEOGEMM_B_KN && b_layout != NEOGEMM_B_NK) || (c_layout != NEOGEMM_C_ROW && c_layout != NEOGEMM_C_COL))
+  if ((b_layout != NEOGEMM_B_KN && b_layout != NEOGEMM_B_NK) || (c_layout != NEOGEMM_C_ROW && c_layout != NEOGEMM_C_COL) ||
+      (bt.a_layout != NEOGEMM_A_MK && bt.a_layout != NEOGEMM_A_KM))
     return NEOGEMM_ERR_BAD_ARG;
+  const bool a_mk = bt.a_layout == NEOGEMM_A_MK;
   if (variant < 0 || variant >= NEOGEMM_VARIANT_COUNT || split_k < 0 || group_m < 0) return NEOGEMM_ERR_BAD_ARG;
   if (variant_retired(variant)) return NEOGEMM_ERR_UNSUPPORTED;
   if (M == 0 || N == 0) return NEOGEMM_OK;
   if (!C || (K > 0 && (!A || !B))) return NEOGEMM_ERR_BAD_ARG;
-  if (lda < K || ldb < (b_layout == NEOGEMM_B_KN ? N : K) || ldc < (c_layout == NEOGEMM_C_ROW ? N : M))
+  if (lda < (a_mk ? K : M) || ldb < (b_layout == NEOGEMM_B_KN ? N : K) || ldc < (c_layout == NEOGEMM_C_ROW ? N : M))
     return NEOGEMM_ERR_BAD_ARG;
   if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return NEOGEMM_ERR_BAD_ARG;
   hipStream_t st = (hipStream_t)hip_stream;
 
   // ld limits keep every in-tile byte offset below 2^31 (the buffer range check uses 32-bit offsets)
-  const bool aligned = is_aligned(A, B, C, K, lda, ldb, ldc) && lda < (1 << 21) && ldb < (1 << 21) && K > 0 &&
+  const bool aligned = is_aligned(A, B, C, K, lda, ldb, ldc, a_mk || b_layout == NEOGEMM_B_NK) && lda < (1 << 21) && ldb < (1 << 21) && K > 0 &&
                        (bt.sa & 7) == 0 && (bt.sb & 7) == 0 && (bt.sc & 3) == 0;
   int v = variant, s = split_k;
   if (v == NEOGEMM_VARIANT_AUTO) {
     int pv, ps;
-    plan(M, N, K, aligned, c_layout, &pv, &ps, bt.count, b_layout);
+    plan(M, N, K, aligned, c_layout, &pv, &ps, bt.count, b_layout, bt.a_layout);
     v = pv;
     if (s == 0) s = ps;
   }
   if (s == 0) s = 1;
 
   if (v == NEOGEMM_VARIANT_GENERIC) {
+    const long sam = a_mk ? lda : 1, sak = a_mk ? 1 : lda;
     const long sbk = b_layout == NEOGEMM_B_KN ? ldb : 1, sbn = b_layout == NEOGEMM_B_KN ? 1 : ldb;
     const long scm = c_layout == NEOGEMM_C_ROW ? ldc : 1, scn = c_layout == NEOGEMM_C_ROW ? 1 : ldc;
     const int64_t nbx = ceil_div(N, 16), nblocks = nbx * ceil_div(M, 16);
     if (nblocks > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;
     dim3 grid((unsigned)nblocks, 1, (unsigned)bt.count);
     gemm_generic_kernel<<<grid, 256, 0, st>>>((const __bf16*)A, (const __bf16*)B, (__bf16*)C, (int)M, (int)N, (int)K,
-                                              lda, 1, sbk, sbn, scm, scn, alpha, beta, bt.sa, bt.sb, bt.sc,
+                                              sam, sak, sbk, sbn, scm, scn, alpha, beta, bt.sa, bt.sb, bt.sc,
                                               (unsigned)nbx);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -2375,7 +2399,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     // one problem.  If M is too large but N fits and B is [N,K], it runs the transposed problem
     // C^T = B * A^T: its small operand is B then, its wide one A, and the layout of C flips.
     const bool swap = M > kVariants[v].bm && N <= kVariants[v].bm && b_layout == NEOGEMM_B_NK;
-    const bool ok = bt.count == 1 && (M <= kVariants[v].bm || swap) &&
+    const bool ok = bt.count == 1 && a_mk && (M <= kVariants[v].bm || swap) &&
                     (b_layout == NEOGEMM_B_NK || (N & 7) == 0) &&
                     (split_k <= 1 || variant == NEOGEMM_VARIANT_AUTO || v == NEOGEMM_VARIANT_STRIP) && !prof;
     if (!ok) {
@@ -2460,11 +2484,11 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   TileArgs a;
   bool ak, bk;
   if (c_layout == NEOGEMM_C_ROW) {
-    a.A = (const char*)A; a.lda = lda; ak = true; a.M = (int)M; a.bsa = bt.sa;
+    a.A = (const char*)A; a.lda = lda; ak = a_mk; a.M = (int)M; a.bsa = bt.sa;
     a.B = (const char*)B; a.ldb = ldb; bk = (b_layout == NEOGEMM_B_NK); a.N = (int)N; a.bsb = bt.sb;
   } else {
     a.A = (const char*)B; a.lda = ldb; ak = (b_layout == NEOGEMM_B_NK); a.M = (int)N; a.bsa = bt.sb;
-    a.B = (const char*)A; a.ldb = lda; bk = true; a.N = (int)M; a.bsb = bt.sa;
+    a.B = (const char*)A; a.ldb = lda; bk = a_mk; a.N = (int)M; a.bsb = bt.sa;
   }
   a.C = (char*)C;
   a.ldc = ldc;
@@ -2612,6 +2636,30 @@ int neogemm_bf16_batched(const void* A, const void* B, void* C, int64_t M, int64
   bt.sc = stride_c;
   return neogemm::run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
                       NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, 1.f, 0.f, bt);
+}
+
+int neogemm_bf16_general(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                         int64_t ldc, int a_layout, int b_layout, int c_layout, float alpha, float beta, int64_t stride_a,
+                         int64_t stride_b, int64_t stride_c, int64_t batch, void* workspace, size_t workspace_bytes,
+                         void* hip_stream) {
+  if (!(alpha == alpha) || !(beta == beta)) return NEOGEMM_ERR_BAD_ARG;  // NaN scale factors
+  if (batch == 0) return (M < 0 || N < 0 || K < 0) ? NEOGEMM_ERR_BAD_ARG : NEOGEMM_OK;
+  neogemm::BatchArgs bt;
+  bt.count = batch;
+  bt.sa = stride_a;
+  bt.sb = stride_b;
+  bt.sc = stride_c;
+  bt.a_layout = a_layout;
+  return neogemm::run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
+                      NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, alpha, beta, bt);
+}
+
+size_t neogemm_bf16_general_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_layout, int b_layout, int c_layout,
+                                            int64_t batch) {
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
+  int v, s;
+  neogemm::plan(M, N, K, true, c_layout, &v, &s, batch, b_layout, a_layout);
+  return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)batch : 0;
 }
 
 size_t neogemm_bf16_batched_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch) {

@@ -73,9 +73,19 @@ torch::Tensor& workspace_for(const torch::Tensor& like, hipStream_t stream, size
 }
 
 void run(const torch::Tensor& A, const torch::Tensor& B, torch::Tensor& C, int64_t M, int64_t N, int64_t K,
-         int64_t lda, int64_t ldb, int64_t ldc, int b_layout, int c_layout, float alpha = 1.f, float beta = 0.f) {
+         int64_t lda, int64_t ldb, int64_t ldc, int b_layout, int c_layout, float alpha = 1.f, float beta = 0.f,
+         int a_layout = NEOGEMM_A_MK) {
   // PyTorch-ROCm names its HIP devices "cuda"; these are the guard and stream accessors for that naming
   c10::hip::HIPGuardMasqueradingAsCUDA guard(A.device());
+  if (a_layout == NEOGEMM_A_KM) {
+    const size_t need = neogemm_bf16_general_workspace_bytes(M, N, K, a_layout, b_layout, c_layout, 1);
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A.get_device()).stream();
+    void* ws = need ? workspace_for(A, stream, need).data_ptr() : nullptr;
+    const int st = neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, a_layout, b_layout,
+                                        c_layout, alpha, beta, 0, 0, 0, 1, ws, need, (void*)stream);
+    TORCH_CHECK(st == NEOGEMM_OK, "neogemm_bf16_general failed: ", neogemm_strerror(st));
+    return;
+  }
   const size_t need = neogemm_bf16_workspace_bytes(M, N, K);
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A.get_device()).stream();
   void* ws = nullptr;
@@ -88,29 +98,56 @@ void run(const torch::Tensor& A, const torch::Tensor& B, torch::Tensor& C, int64
   TORCH_CHECK(st == NEOGEMM_OK, "neogemm_bf16 failed: ", neogemm_strerror(st));
 }
 
+// How the two operands of a product lie in memory; a tensor that no layout describes is made contiguous.
+struct Operands {
+  torch::Tensor A, B;
+  int a_layout = NEOGEMM_A_MK, b_layout = NEOGEMM_B_KN;
+  int64_t lda, ldb;
+};
+Operands describe(torch::Tensor A, torch::Tensor B) {
+  Operands o;
+  if (row_major(B)) {
+    o.ldb = row_ld(B);
+  } else if (B.stride(0) == 1) {  // B = W.t() with W [N,K] row-major
+    o.b_layout = NEOGEMM_B_NK;
+    o.ldb = B.size(1) <= 1 ? std::max<int64_t>(B.size(0), 1) : B.stride(1);
+  } else {
+    B = B.contiguous();
+    o.ldb = row_ld(B);
+  }
+  // A = X.t() with X [K,M] row-major, as in a weight gradient dY.t() * X, is read in place where the tile kernels take it:
+  // whole 16-byte chunks, and more rows than the decode kernels, which want K-contiguous rows, would serve.  The copy
+  // took 68 us for 4096 x 4096 where the product itself takes 98.
+  auto chunks = [](const torch::Tensor& t, int64_t ld) { return ((uintptr_t)t.data_ptr() & 15) == 0 && ld % 8 == 0; };
+  const int64_t M = A.size(0), N = B.size(1), K = A.size(1);
+  o.lda = row_ld(A);
+  if (!row_major(A)) {
+    if (A.stride(0) == 1 && A.stride(1) >= M && M > 128 && M % 8 == 0 && chunks(A, A.stride(1)) && chunks(B, o.ldb) && N % 8 == 0 &&
+        (o.b_layout == NEOGEMM_B_KN || K % 8 == 0)) {
+      o.a_layout = NEOGEMM_A_KM;
+      o.lda = A.stride(1);
+    } else {
+      A = A.contiguous();
+      o.lda = row_ld(A);
+    }
+  }
+  o.A = A;
+  o.B = B;
+  return o;
+}
+
 // C = gemm(A, B): A [M,K], B [K,N] -> new C [M,N], all bf16.  A transposed view of a contiguous
-// [N,K] tensor is taken as is (that is the reference's own B layout), anything else is made contiguous.
+// tensor is taken as is where the kernels can read it (for B that is the reference's own layout).
 torch::Tensor gemm(torch::Tensor A, torch::Tensor B) {
   check_operand(A, "A");
   check_operand(B, "B");
   TORCH_CHECK(A.device() == B.device(), "A and B must be on the same device");
   TORCH_CHECK(A.size(1) == B.size(0), "inner dimensions differ: A is ", A.sizes(), ", B is ", B.sizes());
-  if (!row_major(A)) A = A.contiguous();
-  int b_layout = NEOGEMM_B_KN;
-  int64_t ldb;
-  if (row_major(B)) {
-    ldb = row_ld(B);
-  } else if (B.stride(0) == 1) {  // B = W.t() with W [N,K] row-major
-    b_layout = NEOGEMM_B_NK;
-    ldb = B.size(1) <= 1 ? std::max<int64_t>(B.size(0), 1) : B.stride(1);
-  } else {
-    B = B.contiguous();
-    ldb = row_ld(B);
-  }
   const int64_t M = A.size(0), K = A.size(1), N = B.size(1);
   torch::Tensor C = torch::empty({M, N}, A.options());
   if (M == 0 || N == 0) return C;
-  run(A, B, C, M, N, K, row_ld(A), ldb, std::max<int64_t>(N, 1), b_layout, NEOGEMM_C_ROW);
+  const Operands o = describe(std::move(A), std::move(B));
+  run(o.A, o.B, C, M, N, K, o.lda, o.ldb, std::max<int64_t>(N, 1), o.b_layout, NEOGEMM_C_ROW, 1.f, 0.f, o.a_layout);
   return C;
 }
 
@@ -123,21 +160,10 @@ void gemm_scaled(torch::Tensor A, torch::Tensor B, torch::Tensor C, double alpha
   TORCH_CHECK(A.device() == B.device() && A.device() == C.device(), "A, B and C must be on the same device");
   TORCH_CHECK(A.size(1) == B.size(0), "inner dimensions differ: A is ", A.sizes(), ", B is ", B.sizes());
   TORCH_CHECK(C.size(0) == A.size(0) && C.size(1) == B.size(1) && C.is_contiguous(), "C must be a contiguous [M,N]");
-  if (!row_major(A)) A = A.contiguous();
-  int b_layout = NEOGEMM_B_KN;
-  int64_t ldb;
-  if (row_major(B)) {
-    ldb = row_ld(B);
-  } else if (B.stride(0) == 1) {
-    b_layout = NEOGEMM_B_NK;
-    ldb = B.size(1) <= 1 ? std::max<int64_t>(B.size(0), 1) : B.stride(1);
-  } else {
-    B = B.contiguous();
-    ldb = row_ld(B);
-  }
   const int64_t M = A.size(0), K = A.size(1), N = B.size(1);
   if (M == 0 || N == 0) return;
-  run(A, B, C, M, N, K, row_ld(A), ldb, std::max<int64_t>(N, 1), b_layout, NEOGEMM_C_ROW, (float)alpha, (float)beta);
+  const Operands o = describe(std::move(A), std::move(B));
+  run(o.A, o.B, C, M, N, K, o.lda, o.ldb, std::max<int64_t>(N, 1), o.b_layout, NEOGEMM_C_ROW, (float)alpha, (float)beta, o.a_layout);
 }
 
 // bmm(A, B): A [b,M,K], B [b,K,N] or [K,N] (shared) -> new C [b,M,N]; one launch (neogemm_bf16_batched).

@@ -36,6 +36,9 @@ extern "C" {
 #define NEOGEMM_B_KN 0 /* B is [K,N] row-major (N contiguous): the layout `C = gemm(A, B)` is quoted on */
 #define NEOGEMM_B_NK 1 /* B is [N,K] row-major (K contiguous): the reference's layout, N = B.size(0)
                           (nemgemmV03.cu:346), C = A * B^T (v01.cu:232-235) */
+/* a_layout values (neogemm_bf16_general; every other entry point takes A as NEOGEMM_A_MK) */
+#define NEOGEMM_A_MK 0 /* A is [M,K] row-major (K contiguous) */
+#define NEOGEMM_A_KM 1 /* A is [K,M] row-major (M contiguous): a transposed view, as dY in a weight gradient dY^T * X */
 /* c_layout values */
 #define NEOGEMM_C_ROW 0 /* C(i,j) at C[i*ldc + j] */
 #define NEOGEMM_C_COL 1 /* C(i,j) at C[j*ldc + i]: what the reference's epilogue writes (v01.cu:246,252) */
@@ -128,6 +131,19 @@ int neogemm_bf16_batched(const void* A, const void* B, void* C, int64_t M, int64
                          int64_t batch, int b_layout, int c_layout, void* workspace, size_t workspace_bytes,
                          void* hip_stream);
 size_t neogemm_bf16_batched_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch);
+
+/*
+ * Every choice the calls above leave open in one: C = alpha * op(A) * op(B) + beta * C for `batch` problems, op(A) from
+ * a_layout (lda >= K, or >= M for NEOGEMM_A_KM).  The wrappers use it for operands that are transposed views, which the
+ * kernels read in place instead of a copy.  neogemm_bf16_general_workspace_bytes is what this call may use for these
+ * layouts.  The reference takes both operands K-contiguous only (v01.cu:232-235).
+ */
+int neogemm_bf16_general(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
+                         int64_t ldb, int64_t ldc, int a_layout, int b_layout, int c_layout, float alpha, float beta,
+                         int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t batch, void* workspace,
+                         size_t workspace_bytes, void* hip_stream);
+size_t neogemm_bf16_general_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_layout, int b_layout, int c_layout,
+                                            int64_t batch);
 
 /*
  * neogemm_bf16 for callers that cannot allocate device memory (code under HIP graph capture, tight serving
