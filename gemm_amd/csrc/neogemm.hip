@@ -44,6 +44,11 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 typedef __attribute__((ext_vector_type(4))) short i16x4;
 typedef __attribute__((ext_vector_type(8))) short i16x8;
+// C and the split-K partials may begin at any element: the same one load or store per lane, without the alignment
+typedef __attribute__((ext_vector_type(8), aligned(2))) __bf16 bf16x8_u;
+typedef __attribute__((ext_vector_type(4), aligned(2))) __bf16 bf16x4_u;
+typedef __attribute__((ext_vector_type(4), aligned(2))) int i32x4_u;
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_u;
 
 #define NEOGEMM_AS3 __attribute__((address_space(3)))
 
@@ -361,12 +366,13 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
   constexpr int CH = WTN / 8;        // 16-byte chunks per staged row
   constexpr int RPI = 64 / CH;       // rows one store instruction covers
   constexpr bool CAN_STAGE = (size_t)NW * WTM * WTN * 2 <= (size_t)LDS_BYTES && CH >= 4 && CH <= 64;
-  const bool aligned_c = (((uintptr_t)gC | (uintptr_t)(p.ldc * 2)) & 15) == 0;
-  const bool stage = CAN_STAGE && p.ksplit == 1 && p.beta == 0.f && aligned_c;
+  // C may start at any element and have any leading dimension: a 16-byte store takes a two-byte address, at little cost (512 x 10001
+  // x 1024 17.8 us, 512 x 10000 x 1024 17.7; 4096 x 4095 x 4096 94.7 us, 4096^3 91.3; the generic kernel took 767 and 9137)
+  const bool stage = CAN_STAGE && p.ksplit == 1 && p.beta == 0.f;
   // beta != 0: staged as fp32 (the sum is rounded once), row tiles of the wave tile at a time, as many as the LDS holds
   constexpr int ST = TM % 4 == 0 && NW * 4 * 16 * WTN * 4 <= (int)LDS_BYTES ? 4 : TM % 2 == 0 && NW * 2 * 16 * WTN * 4 <= (int)LDS_BYTES ? 2 : 1;
   constexpr bool CAN_STAGE_F32 = CAN_STAGE && (CH & (CH - 1)) == 0 && NW * ST * 16 * WTN * 4 <= (int)LDS_BYTES && ST * 16 % RPI == 0;
-  const bool stage_add = CAN_STAGE_F32 && p.ksplit == 1 && p.beta != 0.f && aligned_c;
+  const bool stage_add = CAN_STAGE_F32 && p.ksplit == 1 && p.beta != 0.f;
   if (stage) {
     if constexpr (CAN_STAGE) {
       // every wave is done with the slab images (its LDS reads have returned: the MFMAs that used them
@@ -413,7 +419,7 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
             char* dst = gC + ((size_t)grow * p.ldc + col) * 2;
             if (col + 7 < p.N) {
               // C is written once and not read again here: streaming stores leave the L2 to A and B
-              __builtin_nontemporal_store(v, (bf16x8*)dst);
+              __builtin_nontemporal_store((bf16x8_u)v, (bf16x8_u*)dst);
             } else {
 #pragma unroll
               for (int e = 0; e < 8; ++e)
@@ -439,7 +445,7 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
 #pragma unroll
       for (int st = 0; st < NLD; ++st) {
         const int grow = map.row(st * RPI + lane / CH);
-        if (grow < p.M && whole_cols) old[st] = *(const i32x4*)(gC + ((size_t)grow * p.ldc + col) * 2);
+        if (grow < p.M && whole_cols) old[st] = *(const i32x4_u*)(gC + ((size_t)grow * p.ldc + col) * 2);
       }
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
@@ -473,7 +479,7 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
               bf16x8 o;
 #pragma unroll
               for (int e = 0; e < 8; ++e) o[e] = (__bf16)__builtin_fmaf(p.beta, (float)c[e], v[e >> 2][e & 3] * p.alpha);
-              __builtin_nontemporal_store(o, (bf16x8*)dst);
+              __builtin_nontemporal_store((bf16x8_u)o, (bf16x8_u*)dst);
             } else {
 #pragma unroll
               for (int e = 0; e < 8; ++e)
@@ -503,7 +509,7 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
         }
         const bf16x4 o = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
         if (col + 3 < p.N) {
-          __builtin_nontemporal_store(o, (bf16x4*)(crow + (size_t)col * 2));
+          __builtin_nontemporal_store((bf16x4_u)o, (bf16x4_u*)(crow + (size_t)col * 2));
         } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r)
@@ -513,7 +519,6 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
     }
   } else {
     float* wsz = p.ws + ((size_t)blockIdx.z * p.ksplit + kz) * p.M * p.N;
-    const bool vec = (p.N & 3) == 0;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int row = map.row(i * 16 + row_l);
@@ -525,8 +530,8 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
         f32x4 o;
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = acc_get(acc[i][j][r]);
-        if (vec && col + 3 < p.N) {
-          *(f32x4*)(wrow + col) = o;
+        if (col + 3 < p.N) {
+          *(f32x4_u*)(wrow + col) = o;
         } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r)
@@ -1285,10 +1290,10 @@ __device__ __forceinline__ void skinny_store_partial(f32x4 sum, int t, int f, co
   const int col = CCOL ? n0 + 16 * f + (int)frow : n0 + 16 * f + 4 * (int)fq;
   const int col_end = n0 + p.strip < p.N ? n0 + p.strip : p.N;
   if (row >= p.M || col >= col_end) return;
-  const int fast = CCOL ? row : col, fast_end = CCOL ? p.M : col_end, ld = CCOL ? p.M : p.N;
+  const int fast = CCOL ? row : col, fast_end = CCOL ? p.M : col_end;
   float* wp = part + (CCOL ? (size_t)col * p.M + row : (size_t)row * p.N + col);
-  if (fast + 3 < fast_end && (ld & 3) == 0) {
-    *(f32x4*)wp = sum;
+  if (fast + 3 < fast_end) {
+    *(f32x4_u*)wp = sum;
   } else {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -1315,7 +1320,7 @@ __device__ __forceinline__ void skinny_store_frag(f32x4 sum, int t, int f, const
   }
   const bf16x4 o = {(__bf16)sum[0], (__bf16)sum[1], (__bf16)sum[2], (__bf16)sum[3]};
   if (fast + 3 < fast_end) {
-    *(bf16x4*)cp = o;
+    *(bf16x4_u*)cp = o;
   } else {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -1751,42 +1756,51 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   C += (size_t)blockIdx.y * bsc * 2;
   const size_t idx = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (idx >= MN) return;
-  if ((N & 3) == 0) {
-    // up to four splits are fetched at a time (the loads of one trip are independent; one at a time the
-    // kernel would spend a memory latency per split) and added in split order
-    f32x4 s = *(const f32x4*)(ws + idx);
-    for (int z = 1; z < ksplit; z += 4) {
-      f32x4 t[4];
+  // the four elements from idx on, which may belong to two rows and end past the matrix; the partials of a split start
+  // at any multiple of four bytes
+  const bool whole = idx + 3 < MN;
+  auto partial = [&](int z) -> f32x4 {
+    const float* src = ws + (size_t)z * MN + idx;
+    if (whole) return *(const f32x4_u*)src;
+    f32x4 t = {0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 4 && idx + e < MN; ++e) t[e] = src[e];
+    return t;
+  };
+  // up to four splits are fetched at a time (the loads of one trip are independent; one at a time the
+  // kernel would spend a memory latency per split) and added in split order
+  f32x4 s = partial(0);
+  for (int z = 1; z < ksplit; z += 4) {
+    f32x4 t[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (z + k < ksplit) t[k] = *(const f32x4*)(ws + (size_t)(z + k) * MN + idx);
+    for (int k = 0; k < 4; ++k)
+      if (z + k < ksplit) t[k] = partial(z + k);
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (z + k < ksplit) {
+    for (int k = 0; k < 4; ++k)
+      if (z + k < ksplit) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s[e] += t[k][e];
-        }
-    }
-    const size_t row = idx / N, col = idx - row * N;
-    bf16x4* dst = (bf16x4*)(C + (row * ldc + col) * 2);
+        for (int e = 0; e < 4; ++e) s[e] += t[k][e];
+      }
+  }
+  size_t row = idx / N, col = idx - row * N;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] *= alpha;
+  for (int e = 0; e < 4; ++e) s[e] *= alpha;
+  if (whole && col + 3 < (size_t)N) {
+    bf16x4_u* dst = (bf16x4_u*)(C + (row * ldc + col) * 2);
     if (beta != 0.f) {
       const bf16x4 c = *dst;
 #pragma unroll
       for (int e = 0; e < 4; ++e) s[e] = __builtin_fmaf(beta, (float)c[e], s[e]);
     }
-    bf16x4 o = {(__bf16)s[0], (__bf16)s[1], (__bf16)s[2], (__bf16)s[3]};
+    const bf16x4 o = {(__bf16)s[0], (__bf16)s[1], (__bf16)s[2], (__bf16)s[3]};
     *dst = o;
   } else {
     for (int e = 0; e < 4 && idx + e < MN; ++e) {
-      float s = ws[idx + e];
-      for (int z = 1; z < ksplit; ++z) s += ws[z * MN + idx + e];
-      const size_t row = (idx + e) / N, col = (idx + e) - row * N;
       __bf16* dst = (__bf16*)(C + (row * ldc + col) * 2);
-      s *= alpha;
-      if (beta != 0.f) s = __builtin_fmaf(beta, (float)*dst, s);
-      *dst = (__bf16)s;
+      *dst = (__bf16)(beta != 0.f ? __builtin_fmaf(beta, (float)*dst, s[e]) : s[e]);
+      if (++col == (size_t)N) {
+        col = 0;
+        ++row;
+      }
     }
   }
 }
@@ -1840,11 +1854,9 @@ static const VariantInfo kVariants[NEOGEMM_VARIANT_COUNT] = {
 static bool variant_retired(int v) { return v == NEOGEMM_VARIANT_RETIRED_2 || v == NEOGEMM_VARIANT_RETIRED_8; }
 
 // What the MFMA kernels with direct-to-LDS loads assume: 16-byte chunks that start on 16-byte addresses and, where an
-// operand has K-contiguous rows, do not straddle the end of K.
-static bool is_aligned(const void* A, const void* B, const void* C, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
-                       bool any_kmajor) {
-  return (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && ((uintptr_t)C & 7) == 0 && ((K & 7) == 0 || !any_kmajor) && (lda & 7) == 0 &&
-         (ldb & 7) == 0 && (ldc & 3) == 0;
+// operand has K-contiguous rows, do not straddle the end of K.  C may lie anywhere.
+static bool is_aligned(const void* A, const void* B, int64_t K, int64_t lda, int64_t ldb, bool any_kmajor) {
+  return (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && ((K & 7) == 0 || !any_kmajor) && (lda & 7) == 0 && (ldb & 7) == 0;
 }
 
 static int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
@@ -2362,14 +2374,20 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   hipStream_t st = (hipStream_t)hip_stream;
 
   // ld limits keep every in-tile byte offset below 2^31 (the buffer range check uses 32-bit offsets)
-  const bool aligned = is_aligned(A, B, C, K, lda, ldb, ldc, a_mk || b_layout == NEOGEMM_B_NK) && lda < (1 << 21) && ldb < (1 << 21) && K > 0 &&
-                       (bt.sa & 7) == 0 && (bt.sb & 7) == 0 && (bt.sc & 3) == 0;
+  const bool aligned = is_aligned(A, B, K, lda, ldb, a_mk || b_layout == NEOGEMM_B_NK) && lda < (1 << 21) && ldb < (1 << 21) && K > 0 &&
+                       (bt.sa & 7) == 0 && (bt.sb & 7) == 0;
   int v = variant, s = split_k;
   if (v == NEOGEMM_VARIANT_AUTO) {
     int pv, ps;
     plan(M, N, K, aligned, c_layout, &pv, &ps, bt.count, b_layout, bt.a_layout);
     v = pv;
     if (s == 0) s = ps;
+    // a C that is not on 8-byte addresses ran without a workspace before the MFMA kernels took it: it still does
+    if (s > 1 && ((((uintptr_t)C | (uintptr_t)(ldc * 2)) & 7) != 0) &&
+        (!workspace || workspace_bytes < (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count)) {
+      v = NEOGEMM_VARIANT_T128x128_W4;
+      s = 1;
+    }
   }
   if (s == 0) s = 1;
 

@@ -32,3 +32,42 @@ def test_accumulating_epilogue(M, N, K, pad, variant, c_layout):
     want[:, :cols] = (0.5 * (prod if c_layout == g.C_ROW else prod.t()) - 3.0 * buf[:, :cols].float()).to(torch.bfloat16)
     g.gemm_into(A, B, buf, M, N, K, K, K, cols + pad, g.B_NK, c_layout, alpha=0.5, beta=-3.0)
     assert torch.equal(buf, want)   # the padding between rows included
+
+
+# C at any element and with any leading dimension: staged stores of the tile kernels, strips, the skinny kernel, the fp32 partials
+# of a split and their reduction (rows of partials that straddle a lane's four elements), each to the edge of an odd N
+@pytest.mark.parametrize("M,N,K", [(300, 521, 200), (5128, 5125, 256), (1000, 1027, 512), (16, 1001, 4096), (3, 4099, 1024), (128, 4097, 16384),
+                                   (120, 14339, 2048), (256, 261, 8192), (257, 131, 16384)])
+@pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
+@pytest.mark.parametrize("shift", [1, 2])
+def test_c_at_any_address(M, N, K, c_layout, shift):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A, B = small_ints(gen, M, K, top=1), small_ints(gen, N, K, top=1)
+    rows, cols = (M, N) if c_layout == g.C_ROW else (N, M)
+    ldc = cols + shift
+    flat = small_ints(gen, rows * ldc + shift, top=8)
+    want = flat.clone()
+    prod = A.float() @ B.float().t()
+    prod = prod if c_layout == g.C_ROW else prod.t()
+    view = want[shift:].view(rows, ldc)[:, :cols]
+    old = view.clone()
+    view.copy_(prod.to(torch.bfloat16))
+    C = flat.clone()
+    g.gemm_into(A, B, C[shift:], M, N, K, K, K, ldc, g.B_NK, c_layout)
+    assert torch.equal(C, want)   # what lies between the rows included
+    C = flat.clone()
+    view.copy_((2.0 * prod + old.float()).to(torch.bfloat16))
+    g.gemm_into(A, B, C[shift:], M, N, K, K, K, ldc, g.B_NK, c_layout, alpha=2.0, beta=1.0)
+    assert torch.equal(C, want)
+
+
+def test_odd_c_without_a_workspace():
+    """A shape whose plan splits K, into a C on odd addresses, with no workspace: unsplit, as such a C always ran."""
+    from gemm_amd import _abi
+    M, N, K = 256, 261, 8192
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    A, B = small_ints(gen, M, K, top=1), small_ints(gen, N, K, top=1)
+    C = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    assert g.plan(M, N, K, g.B_NK)[1] > 1
+    st = _abi.gemm_raw(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, K, K, N, g.B_NK, g.C_ROW, 0, 0, torch.cuda.current_stream().cuda_stream)
+    assert st == _abi.OK and torch.equal(C, (A.float() @ B.float().t()).to(torch.bfloat16))
