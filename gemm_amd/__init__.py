@@ -54,11 +54,9 @@ def _workspace(device, nbytes):
 def gemm_into(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, variant=None, split_k=0, group_m=0, alpha=1.0,
               beta=0.0, a_layout=A_MK):
     """Call the C ABI on torch's current stream; A, B, C are torch tensors used as device buffers."""
-    if a_layout != A_MK:
-        if variant is not None:
-            raise ValueError("a transposed A goes through neogemm_bf16_general, which chooses the kernel itself")
+    if variant is None:
         lib = _abi.load()
-        need = int(lib.neogemm_bf16_general_workspace_bytes(M, N, K, a_layout, b_layout, c_layout, 1))
+        need = int(lib.neogemm_bf16_call_workspace_bytes(A.data_ptr(), B.data_ptr(), M, N, K, lda, ldb, a_layout, b_layout, c_layout, 0, 0, 1))
         ws_ptr = _workspace(C.device, need).data_ptr() if need else 0
         with torch.cuda.device(C.device):
             stream = torch.cuda.current_stream().cuda_stream
@@ -67,6 +65,8 @@ def gemm_into(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, variant=None,
         if st != _abi.OK:
             raise NeoGemmError(st, f"M={M} N={N} K={K} a_layout={a_layout} b_layout={b_layout} c_layout={c_layout}")
         return
+    if a_layout != A_MK:
+        raise ValueError("a transposed A goes through neogemm_bf16_general, which chooses the kernel itself")
     need = workspace_bytes(M, N, K)
     if variant is not None and split_k > 1:
         need = max(need, split_k * M * N * 4)
@@ -83,8 +83,7 @@ def gemm_into(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, variant=None,
 
 def _describe(A, B, transposed_a=True):
     """How A [M,K] and B [K,N] lie in memory: (A, B, lda, ldb, a_layout, b_layout); what no layout describes is made
-    contiguous.  A transposed A is read in place where the tile kernels take it: whole 16-byte chunks, and more rows than
-    the decode kernels, which want K-contiguous rows, would serve."""
+    contiguous.  A transposed A is read in place, but for the few rows of the decode kernels, which want them K-contiguous."""
     M, K = A.shape
     N = B.shape[1]
     if B.stride(1) == 1 or N <= 1:
@@ -96,8 +95,8 @@ def _describe(A, B, transposed_a=True):
         b_layout, ldb = B_KN, max(N, 1)
     if A.stride(1) == 1 or K <= 1:
         return A, B, (A.stride(0) if M > 1 else max(K, 1)), ldb, A_MK, b_layout
-    if (transposed_a and A.stride(0) == 1 and A.stride(1) >= M > 128 and M % 8 == 0 and N % 8 == 0 and A.stride(1) % 8 == 0 and
-            ldb % 8 == 0 and A.data_ptr() % 16 == 0 and B.data_ptr() % 16 == 0 and (b_layout == B_KN or K % 8 == 0)):
+    decode = M <= 128 and K % 8 == 0 and ldb % 8 == 0 and B.data_ptr() % 16 == 0 and (b_layout == B_NK or N % 8 == 0)
+    if transposed_a and A.stride(0) == 1 and A.stride(1) >= M and not decode:
         return A, B, A.stride(1), ldb, A_KM, b_layout
     return A.contiguous(), B, max(K, 1), ldb, A_MK, b_layout
 

@@ -42,6 +42,7 @@ PROTOTYPES = {
     "neogemm_bf16_general": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, ctypes.c_float,
                                     ctypes.c_float, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
     "neogemm_bf16_general_workspace_bytes": (_sz, [_i64, _i64, _i64, _int, _int, _int, _i64]),
+    "neogemm_bf16_call_workspace_bytes": (_sz, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _i64, _i64, _i64]),
     "neogemm_bf16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "neogemm_bf16_variant": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _sz, _vp,
                                     _int, _int, _int]),

@@ -27,13 +27,13 @@
 // Split build: compiling this one file takes minutes because of the many instances of the tile kernel, so setup.py
 // compiles it NEOGEMM_PARTS times in parallel with -DNEOGEMM_PART=0..NEOGEMM_PARTS-1 and links the objects.  Part 0
 // holds everything but the tile kernels; part k > 0 instantiates its share of launch_tile<> (listed behind
-// launch_tile) or, the last one, launch_chain, and nothing else.  Without NEOGEMM_PART the file is one self-contained translation unit.
+// launch_tile) or, the last two, launch_chain and launch_ragged, and nothing else.  Without NEOGEMM_PART the file is one self-contained translation unit.
 #ifdef NEOGEMM_PART
 #define NEOGEMM_HAS_PART(p) (NEOGEMM_PART == (p))
 #else
 #define NEOGEMM_HAS_PART(p) 1
 #endif
-#define NEOGEMM_PARTS 9
+#define NEOGEMM_PARTS 10
 
 namespace neogemm {
 
@@ -132,6 +132,18 @@ __device__ __forceinline__ void static_for_impl(Fn&& fn, std::integer_sequence<i
 template <int N, class Fn>
 __device__ __forceinline__ void static_for(Fn&& fn) {
   static_for_impl<N>(fn, std::make_integer_sequence<int, N>{});
+}
+
+__device__ __forceinline__ uint32_t swz_mn64(uint32_t kk) {
+  // k-row kk (0..31 within a slab) of a 64-column MN-major image: even values 0..6 XOR-ed into the 16-byte chunk
+  // index, chosen so that the sixteen 32-byte pieces of one transposing read spread over the banks
+  return ((((kk >> 3) & 3u) ^ (((kk >> 1) & 1u) << 1)) << 1);
+}
+// the swizzle of an MN-major slab image of ROWS columns
+template <int ROWS>
+__device__ __forceinline__ uint32_t swz_mn_rows(uint32_t krow) {
+  if constexpr (ROWS == 64) return swz_mn64(krow);
+  else return swz_mn(krow);
 }
 
 struct TileArgs {
@@ -297,7 +309,7 @@ struct FragReader {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         uint32_t chunk = (uint32_t)(wrow0 >> 3) + 2 * t + (tr_c >> 1);
-        lane_off[t] = region + krow * ROWB + ((chunk ^ swz_mn(krow)) << 4) + ((tr_c & 1) << 3);
+        lane_off[t] = region + krow * ROWB + ((chunk ^ swz_mn_rows<ROWS>(krow)) << 4) + ((tr_c & 1) << 3);
       }
     }
   }
@@ -345,7 +357,8 @@ struct BlockMap {  // one block
 // Epilogue of the tile kernels: the TM x TN accumulator tiles of a wave (NW waves per workgroup, LDS_BYTES of LDS
 // that the main loop is done with) go to C as bf16, or to the split-K partials as fp32.
 // STAGE_TM: row tiles of the wave tile that go through LDS at a time (TM: all of it at once).
-template <int TM, int TN, int NW, uint32_t LDS_BYTES, int STAGE_TM = TM, class Map>
+// IN_AGPRS: the accumulators are pinned there (mfma_16x16x32); false: where the compiler put them.
+template <int TM, int TN, int NW, uint32_t LDS_BYTES, int STAGE_TM = TM, bool IN_AGPRS = true, class Map>
 __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const TileArgs& p, char* gC, int kz, int lane,
                                                 int wave, uint32_t lds0, const Map map) {
   constexpr int WTM = TM * 16, WTN = TN * 16;
@@ -355,8 +368,8 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
   // An accumulator element is read out of its AGPR where it is used: left to itself the compiler copies
   // all 256 accumulators to VGPRs ahead of the three epilogue variants below, and spills.
   auto acc_get = [](float a) -> float {
-    float v;
-    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
+    float v = a;
+    if constexpr (IN_AGPRS) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
     return v;
   };
   // Coalesced path: the wave parks its bf16 tile in LDS (the slab ring is dead by now) and reads it back
@@ -1191,6 +1204,217 @@ hipError_t launch_chain(const TileArgs& a, bool bk, hipStream_t st) {
 }
 #endif
 
+// ---------------------------------------------------------------------------------------------
+// Operands at any address and with any leading dimension (an odd K or N, a view that starts in the middle of a row), which
+// gemm_generic_kernel computed at 14 TFLOP/s: 1023 x 2047 x 1535 416 us, 21 with this kernel (1024 x 2048 x 1536 by the tile
+// kernels: 11); 512 x 1024 x 10001 767 us, 29.  The direct-to-LDS loads of the kernels above want 16-byte addresses; here a
+// chunk of eight elements is fetched into registers, which takes a two-byte address, and written to the same swizzled LDS
+// images.  The loads of tile t+3 are requested while tile t is computed (two register sets, two LDS images per operand), so that
+// a workgroup has 2.5 tiles on the way.  What bounds it is the vector memory path into the CU: 16-byte loads run at 43 B/clk
+// and CU from addresses that are a multiple of four, at 23 where every other row begins between two dwords, at 15 where all
+// do.  (Reading the dwords from the one a chunk begins in, with the fifth one by a load of its own, and shifting them together took 24 us.)
+// What does not belong to the product: rows past the end of the output take the last row's place and columns past it
+// whatever lies there, in bounds, since they only reach elements that are not stored; what lies past the end of K is
+// zeroed on its way into LDS.  A chunk may reach past the end of its row, but past the end of the matrix only near its
+// last K rows or columns: there ("careful" tiles) the address is held back and the register shifted.
+// ---------------------------------------------------------------------------------------------
+template <int ROWS, bool KMAJOR>
+struct RaggedOperand {
+  static constexpr int NCH = ROWS * 8 / 256;     // 16-byte chunks of a 64-deep tile per thread
+  static constexpr uint32_t IMG = ROWS * 128;    // K-major: one 64-deep image; MN-major: two 32-deep slab images
+  static constexpr uint32_t SLAB = KMAJOR ? 0 : ROWS * 64;
+  static constexpr int CPR = ROWS / 8;           // chunks per k-row (MN-major)
+  uint32_t voff[NCH], loff[NCH];
+  const char* base0;   // first element of tile 0
+  const char* last;    // the last 16 bytes of the matrix
+  uint64_t kadv;
+
+  __device__ __forceinline__ void init(const char* ptr, long ld, int rows_total, int r0, int K, int k_begin, int tid) {
+    base0 = ptr + (KMAJOR ? (size_t)r0 * ld + k_begin : (size_t)k_begin * ld + r0) * 2;
+    last = ptr + ((KMAJOR ? (size_t)(rows_total - 1) * ld + K : (size_t)(K - 1) * ld + rows_total) - 8) * 2;
+    kadv = (KMAJOR ? (uint64_t)KTILE : (uint64_t)KTILE * ld) * 2;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      const uint32_t q = j * 256 + tid;
+      if constexpr (KMAJOR) {
+        const uint32_t row = q >> 3, c = q & 7, left = rows_total - 1 - r0;
+        voff[j] = (row < left ? row : left) * (uint32_t)ld * 2 + c * 16;
+        loff[j] = row * 128 + ((c ^ swz_k(row)) << 4);
+      } else {
+        const uint32_t krow = q / CPR, c = q % CPR, left = rows_total - 1 - r0;
+        voff[j] = krow * (uint32_t)ld * 2 + (c * 8 < left ? c * 8 : left) * 2;
+        loff[j] = (krow >> 5) * SLAB + (krow & 31) * (ROWS * 2) + ((c ^ swz_mn_rows<ROWS>(krow & 31)) << 4);
+      }
+    }
+  }
+  // A tile none of whose chunks reaches past the end of K or of the matrix ...
+  __device__ __forceinline__ void load(i32x4 (&r)[NCH], int t) const {
+    const char* base = base0 + (uint64_t)t * kadv;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) r[j] = *(const i32x4_u*)(base + voff[j]);
+  }
+  __device__ __forceinline__ void store(const i32x4 (&r)[NCH], uint32_t img) const {
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) *((NEOGEMM_AS3 i32x4*)(uintptr_t)(img + loff[j])) = r[j];
+  }
+  // ... and any tile (live: it exists; one past the end is requested all the same, at `last`: the count of loads in flight
+  // does not depend on K).  krem: depth left from the tile's first element on.
+  __device__ __forceinline__ void load_careful(i32x4 (&r)[NCH], int t, bool live) const {
+    const char* base = base0 + (uint64_t)t * kadv;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      const char* a = base + voff[j];
+      r[j] = *(const i32x4_u*)(live && a < last ? a : last);
+    }
+  }
+  __device__ __forceinline__ void store_careful(const i32x4 (&r)[NCH], uint32_t img, int t, int krem, int tid) const {
+    const char* base = base0 + (uint64_t)t * kadv;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      const uint32_t q = j * 256 + tid;
+      const char* a = base + voff[j];
+      int valid = KMAJOR ? krem - (int)(q & 7) * 8 : (int)(q / CPR) < krem ? 8 : 0;  // elements of the chunk inside K
+      valid = valid < 0 ? 0 : valid > 8 ? 8 : valid;
+      const uint32_t held = a > last ? (uint32_t)(a - last) * 8 : 0, h = held & 63;  // bits the load was held back by (from 128 on nothing is valid)
+      uint64_t lo = (uint32_t)r[j][0] | (uint64_t)(uint32_t)r[j][1] << 32, hi = (uint32_t)r[j][2] | (uint64_t)(uint32_t)r[j][3] << 32;
+      lo = lo >> h | hi << 1 << (63 - h);
+      hi >>= h;
+      lo = held >= 64 ? hi : lo;
+      hi = held >= 64 ? 0 : hi;
+      lo = valid >= 4 ? lo : lo & ((1ull << (16 * valid)) - 1);
+      hi = valid >= 8 ? hi : valid > 4 ? hi & ((1ull << (16 * (valid - 4))) - 1) : 0;
+      const i32x4 v = {(int)(uint32_t)lo, (int)(lo >> 32), (int)(uint32_t)hi, (int)(hi >> 32)};
+      *((NEOGEMM_AS3 i32x4*)(uintptr_t)(img + loff[j])) = v;
+    }
+  }
+};
+
+template <int BM, int BN, bool AK, bool BK>
+__global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(TileArgs p) {
+  constexpr int NW = 4, WTM = BM / 2, WTN = BN / 2, TM = WTM / 16, TN = WTN / 16;
+  using OpA = RaggedOperand<BM, AK>;
+  using OpB = RaggedOperand<BN, BK>;
+  constexpr uint32_t STAGE = OpA::IMG + OpB::IMG, LDS_BYTES = 2 * STAGE;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(NEOGEMM_AS3 char*)smem;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+
+  int m0, n0, kz;
+  tile_of_workgroup<BM, BN>(p, m0, n0, kz);
+  const int k_begin = kz * p.ktiles_per_split * KTILE;
+  int k_end = k_begin + p.ktiles_per_split * KTILE;
+  if (k_end > p.K) k_end = p.K;
+  const int ntile = (k_end - k_begin + KTILE - 1) / KTILE;
+  // tiles before this one need no care: a chunk of a K-major row ends inside K, one of an MN-major k-row less than eight k-rows on
+  const int nplain = (p.K - 8 - k_begin) / KTILE;
+
+  OpA opa;
+  OpB opb;
+  opa.init(p.A + (size_t)blockIdx.z * p.bsa * 2, p.lda, p.M, m0, p.K, k_begin, tid);
+  opb.init(p.B + (size_t)blockIdx.z * p.bsb * 2, p.ldb, p.N, n0, p.K, k_begin, tid);
+  char* gC = p.C + (size_t)blockIdx.z * p.bsc * 2;
+  FragReader<BM, AK, TM> fa;
+  FragReader<BN, BK, TN> fb;
+  fa.init(lds0, wm * WTM, lane);
+  fb.init(lds0 + OpA::IMG, wn * WTN, lane);
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  i32x4 ra[2][OpA::NCH], rb[2][OpB::NCH];
+  using T = std::true_type;
+  using F = std::false_type;
+  auto load = [&](auto set, auto plain, int t) {
+    constexpr int S = decltype(set)::value;
+    if constexpr (decltype(plain)::value) {
+      opa.load(ra[S], t);
+      opb.load(rb[S], t);
+    } else {
+      opa.load_careful(ra[S], t, t < ntile);
+      opb.load_careful(rb[S], t, t < ntile);
+    }
+  };
+  auto store = [&](auto set, auto plain, int t) {
+    constexpr int S = decltype(set)::value;
+    if constexpr (decltype(plain)::value) {
+      opa.store(ra[S], lds0 + S * STAGE);
+      opb.store(rb[S], lds0 + S * STAGE + OpA::IMG);
+    } else {
+      const int krem = p.K - (k_begin + t * KTILE);
+      opa.store_careful(ra[S], lds0 + S * STAGE, t, krem, tid);
+      opb.store_careful(rb[S], lds0 + S * STAGE + OpA::IMG, t, krem, tid);
+    }
+  };
+  auto meet = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  load(S0{}, F{}, 0);
+  load(S1{}, F{}, 1);
+  store(S0{}, F{}, 0);
+  load(S0{}, F{}, 2);
+  meet();
+  auto step = [&](auto set, auto other, auto plain, int t) {
+    constexpr int S = decltype(set)::value;
+#pragma unroll
+    for (int sl = 0; sl < 2; ++sl) {
+      bf16x8 a[TM], b[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[i] = fa.read(S * STAGE + sl * OpA::SLAB, i, sl);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[j] = fb.read(S * STAGE + sl * OpB::SLAB, j, sl);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+    }
+    // the other image was read during step t - 1, before the barrier at its end
+    store(other, plain, t + 1);
+    load(other, plain, t + 3);
+    meet();
+  };
+  int t = 0;
+  for (; t + 4 < (nplain < ntile ? nplain : ntile); t += 2) {
+    step(S0{}, S1{}, T{}, t);
+    step(S1{}, S0{}, T{}, t + 1);
+  }
+  for (; t < ntile; t += 2) {
+    step(S0{}, S1{}, F{}, t);
+    if (t + 1 < ntile) step(S1{}, S0{}, F{}, t + 1);
+  }
+  store_wave_tile<TM, TN, NW, LDS_BYTES, TM, false>(acc, p, gC, kz, lane, wave, lds0, BlockMap{m0 + wm * WTM, n0 + wn * WTN});
+}
+
+// tile: 64 or 128 (square)
+hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int tile, hipStream_t st);
+#if NEOGEMM_HAS_PART(9)
+hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int tile, hipStream_t st) {
+  const size_t lds = (size_t)tile * 512;
+  dim3 grid(a.ntm * a.ntn * a.ksplit, 1, a.batch), block(256);
+  auto go = [&](auto kern) -> hipError_t {
+    if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
+    kern<<<grid, block, lds, st>>>(a);
+    return hipGetLastError();
+  };
+  auto pick = [&](auto tc) -> hipError_t {
+    constexpr int T = decltype(tc)::value;
+    if (ak) return bk ? go(gemm_ragged_kernel<T, T, true, true>) : go(gemm_ragged_kernel<T, T, true, false>);
+    return bk ? go(gemm_ragged_kernel<T, T, false, true>) : go(gemm_ragged_kernel<T, T, false, false>);
+  };
+  if (tile == 64) return pick(std::integral_constant<int, 64>{});
+  if (tile == 128) return pick(std::integral_constant<int, 128>{});
+  return hipErrorInvalidValue;
+}
+#endif
+
 // The tile kernels are instantiated through launch_tile.  In a split build each part instantiates its share and
 // the others only declare it.
 #ifdef NEOGEMM_PART
@@ -1260,11 +1484,6 @@ namespace neogemm {
 // (Fetching the fragments straight into registers instead, which would hold three steps of both, was slower by 40 %:
 // a fragment load touches 16 rows x 64 bytes, half a line each, and the vector L1 charges by the line.)
 // ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t swz_mn64(uint32_t kk) {
-  // k-row kk (0..31 within a slab) of a 64-column MN-major image: even values 0..6 XOR-ed into the 16-byte chunk
-  // index, chosen so that the sixteen 32-byte pieces of one transposing read spread over the banks
-  return ((((kk >> 3) & 3u) ^ (((kk >> 1) & 1u) << 1)) << 1);
-}
 struct SkinnyArgs {
   const char* A;
   const char* B;
@@ -2347,7 +2566,93 @@ static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream
 struct BatchArgs {
   int64_t count = 1, sa = 0, sb = 0, sc = 0;
   int a_layout = NEOGEMM_A_MK;
+  bool split_ragged = false;  // operands off the 16-byte grid may split K over the workspace (see neogemm_bf16_call_workspace_bytes)
 };
+
+// ld limits keep every in-tile byte offset below 2^31 (the buffer range check uses 32-bit offsets)
+static bool mfma_aligned(const void* A, const void* B, int64_t K, int64_t lda, int64_t ldb, int b_layout, const BatchArgs& bt) {
+  return is_aligned(A, B, K, lda, ldb, bt.a_layout == NEOGEMM_A_MK || b_layout == NEOGEMM_B_NK) && lda < (1 << 21) && ldb < (1 << 21) &&
+         K > 0 && (bt.sa & 7) == 0 && (bt.sb & 7) == 0;
+}
+
+// What gemm_ragged_kernel assumes: matrices of eight elements at least (a chunk is held back to the last eight), in-tile offsets
+// below 2^31, two-byte addresses.
+static bool ragged_takes(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int b_layout,
+                         const BatchArgs& bt) {
+  const int64_t ext_a = bt.a_layout == NEOGEMM_A_MK ? (M - 1) * lda + K : (K - 1) * lda + M;
+  const int64_t ext_b = b_layout == NEOGEMM_B_KN ? (K - 1) * ldb + N : (N - 1) * ldb + K;
+  return K > 0 && ext_a >= 8 && ext_b >= 8 && lda < (1 << 21) && ldb < (1 << 21) && (((uintptr_t)A | (uintptr_t)B) & 1) == 0;
+}
+// Tile (64 or 128) and split of K of gemm_ragged_kernel, by the time of its K tiles: a workgroup of the 64x64 tile takes 0.40 us
+// per K tile where several share a CU (the loads at two-byte addresses bound it: 1023 x 2047 x 1535, 512 of them, 21 us), 0.29
+// alone on one (64 x 256 x 20001 in 16 splits, 14.5 us; the same in 4, 26); one of the 128x128 tile, four times the work, 0.95
+// (1500 x 1501 x 1401: 25.3 us for 144 of them, 28.3 for 576 small ones; 1023 x 2047 x 1535: 28 for 128).  A split costs the
+// second launch and the partials (512 x 1024 x 10001 in 64x64 tiles: 29 us with two, 47 unsplit).
+static void ragged_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, int* tile, int* split) {
+  const int64_t ktiles = ceil_div(K, KTILE);
+  double best = 1e300;
+  for (int t : {64, 128})
+    for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      if (sp > 1 && ktiles / sp < 4) break;
+      const double wgs = (double)ceil_div(M, t) * ceil_div(N, t) * (double)batch * sp, per_cu = __builtin_ceil(wgs / cus);
+      double us = per_cu * ceil_div(ktiles, sp) * (t == 128 ? 0.95 : per_cu > 1 ? 0.40 : 0.29) + (t == 128 ? 4.0 : 3.0);
+      if (sp > 1) us += 5.0 + (4.0 * sp + 2.0) * (double)M * (double)N * (double)batch / 4.0e6;
+      if (us < best) {
+        best = us;
+        *tile = t;
+        *split = sp;
+      }
+    }
+}
+// Operands at any address: gemm_ragged_kernel, and the reduction where K is split.  NEOGEMM_ERR_UNSUPPORTED: not launched.
+static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                            int64_t ldc, int b_layout, int c_layout, void* ws, size_t ws_bytes, hipStream_t st, float alpha, float beta,
+                            const BatchArgs& bt) {
+  if (!ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt)) return NEOGEMM_ERR_UNSUPPORTED;
+  int tile = 128, split = 1;
+  ragged_plan(M, N, K, bt.count, planning_cus(), &tile, &split);
+  TileArgs a{};
+  const bool a_mk = bt.a_layout == NEOGEMM_A_MK, b_nk = b_layout == NEOGEMM_B_NK;
+  bool ak = a_mk, bk = b_nk;
+  a.A = (const char*)A; a.lda = lda; a.M = (int)M; a.bsa = bt.sa;
+  a.B = (const char*)B; a.ldb = ldb; a.N = (int)N; a.bsb = bt.sb;
+  if (c_layout == NEOGEMM_C_COL) {  // the row-major transpose: the operands change roles
+    std::swap(a.A, a.B);
+    std::swap(a.lda, a.ldb);
+    std::swap(a.M, a.N);
+    std::swap(a.bsa, a.bsb);
+    ak = b_nk;
+    bk = a_mk;
+  }
+  a.C = (char*)C; a.ldc = ldc; a.bsc = bt.sc;
+  a.K = (int)K;
+  a.batch = (int)bt.count;
+  a.alpha = alpha; a.beta = beta;
+  a.ntm = ceil_div(a.M, tile);
+  a.ntn = ceil_div(a.N, tile);
+  a.group_m = 8;
+  const int ktiles = ceil_div(K, KTILE);
+  if (!bt.split_ragged || !ws || ((uintptr_t)ws & 15) != 0 || ws_bytes < (size_t)split * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count)
+    split = 1;
+  a.ktiles_per_split = ceil_div(ktiles, split);
+  a.ksplit = ceil_div(ktiles, a.ktiles_per_split);  // no empty split
+  if ((int64_t)a.ntm * a.ntn * a.ksplit > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;
+  a.ws = (float*)ws;
+  if (hipError_t e = launch_ragged(a, ak, bk, tile, st); e != hipSuccess) {
+    fprintf(stderr, "neogemm: ragged kernel launch failed: %s\n", hipGetErrorString(e));
+    return NEOGEMM_ERR_LAUNCH;
+  }
+  if (a.ksplit > 1) {
+    const size_t MN = (size_t)a.M * a.N;
+    splitk_reduce_kernel<<<dim3((unsigned)((MN + 1023) / 1024), (unsigned)bt.count), 256, 0, st>>>(a.ws, a.C, a.M, a.N, a.ldc, a.ksplit, alpha,
+                                                                                                   beta, a.bsc);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) {
+      fprintf(stderr, "neogemm: split-K reduce launch failed: %s\n", hipGetErrorString(e));
+      return NEOGEMM_ERR_LAUNCH;
+    }
+  }
+  return NEOGEMM_OK;
+}
 
 static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                int64_t ldc, int b_layout, int c_layout, void* workspace, size_t workspace_bytes, void* hip_stream,
@@ -2373,11 +2678,16 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return NEOGEMM_ERR_BAD_ARG;
   hipStream_t st = (hipStream_t)hip_stream;
 
-  // ld limits keep every in-tile byte offset below 2^31 (the buffer range check uses 32-bit offsets)
-  const bool aligned = is_aligned(A, B, K, lda, ldb, a_mk || b_layout == NEOGEMM_B_NK) && lda < (1 << 21) && ldb < (1 << 21) && K > 0 &&
-                       (bt.sa & 7) == 0 && (bt.sb & 7) == 0;
+  const bool aligned = mfma_aligned(A, B, K, lda, ldb, b_layout, bt);
+  auto unaligned = [&]() -> int {
+    const int r = launch_unaligned(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, st, alpha, beta, bt);
+    return r != NEOGEMM_ERR_UNSUPPORTED ? r
+                                        : run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
+                                              NEOGEMM_VARIANT_GENERIC, 1, 0, nullptr, alpha, beta, bt);
+  };
   int v = variant, s = split_k;
   if (v == NEOGEMM_VARIANT_AUTO) {
+    if (!aligned) return unaligned();
     int pv, ps;
     plan(M, N, K, aligned, c_layout, &pv, &ps, bt.count, b_layout, bt.a_layout);
     v = pv;
@@ -2422,13 +2732,10 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                     (split_k <= 1 || variant == NEOGEMM_VARIANT_AUTO || v == NEOGEMM_VARIANT_STRIP) && !prof;
     if (!ok) {
       if (variant != NEOGEMM_VARIANT_AUTO) return NEOGEMM_ERR_UNSUPPORTED;
-      // the 128x128 tile needs the least of the tile kernels, then the generic kernel
+      // the 128x128 tile needs the least of the tile kernels
       int st2 = run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
                     NEOGEMM_VARIANT_T128x128_W4, 1, 0, nullptr, alpha, beta, bt);
-      if (st2 == NEOGEMM_ERR_UNSUPPORTED)
-        st2 = run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
-                  NEOGEMM_VARIANT_GENERIC, 1, 0, nullptr, alpha, beta, bt);
-      return st2;
+      return st2 == NEOGEMM_ERR_UNSUPPORTED ? unaligned() : st2;
     }
     SkinnyArgs sa{(const char*)A, (const char*)B, (char*)C, (int)M, (int)N, (int)K, (long)lda, (long)ldb, (long)ldc, alpha, beta, 0, 64};
     bool bkm = b_layout == NEOGEMM_B_NK, ccol = c_layout == NEOGEMM_C_COL;
@@ -2523,14 +2830,11 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                     (v != NEOGEMM_VARIANT_C256x256_W4 || (ak && K % (2 * KTILE) == 0 && s <= 1));
   if (!fits) {
     if (variant != NEOGEMM_VARIANT_AUTO) return NEOGEMM_ERR_UNSUPPORTED;
-    // the planned tile is too wide for an MN-major operand: the 128x128 tile needs the least, then generic
-    const int next = v != NEOGEMM_VARIANT_T128x128_W4 ? NEOGEMM_VARIANT_T128x128_W4 : NEOGEMM_VARIANT_GENERIC;
-    int st = run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream, next,
-                 next == NEOGEMM_VARIANT_GENERIC ? 1 : s, 0, nullptr, alpha, beta, bt);
-    if (st == NEOGEMM_ERR_UNSUPPORTED && next != NEOGEMM_VARIANT_GENERIC)
-      st = run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
-               NEOGEMM_VARIANT_GENERIC, 1, 0, nullptr, alpha, beta, bt);
-    return st;
+    // the planned tile is too wide for an MN-major operand: the 128x128 tile needs the least
+    if (v == NEOGEMM_VARIANT_T128x128_W4) return unaligned();
+    const int r = run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
+                      NEOGEMM_VARIANT_T128x128_W4, s, 0, nullptr, alpha, beta, bt);
+    return r == NEOGEMM_ERR_UNSUPPORTED ? unaligned() : r;
   }
   a.ntm = ceil_div(a.M, vi.bm);
   a.ntn = ceil_div(a.N, vi.bn);
@@ -2668,6 +2972,7 @@ int neogemm_bf16_general(const void* A, const void* B, void* C, int64_t M, int64
   bt.sb = stride_b;
   bt.sc = stride_c;
   bt.a_layout = a_layout;
+  bt.split_ragged = true;
   return neogemm::run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
                       NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, alpha, beta, bt);
 }
@@ -2677,6 +2982,23 @@ size_t neogemm_bf16_general_workspace_bytes(int64_t M, int64_t N, int64_t K, int
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
   int v, s;
   neogemm::plan(M, N, K, true, c_layout, &v, &s, batch, b_layout, a_layout);
+  return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)batch : 0;
+}
+
+size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                         int a_layout, int b_layout, int c_layout, int64_t stride_a, int64_t stride_b, int64_t batch) {
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
+  neogemm::BatchArgs bt;
+  bt.count = batch;
+  bt.sa = stride_a;
+  bt.sb = stride_b;
+  bt.a_layout = a_layout;
+  int v, s = 1;
+  // (an MN-major operand whose rows do not end on a chunk goes the same way as one off the 16-byte grid)
+  if (neogemm::mfma_aligned(A, B, K, lda, ldb, b_layout, bt) && (a_layout == NEOGEMM_A_MK || M % 8 == 0) && (b_layout == NEOGEMM_B_NK || N % 8 == 0))
+    neogemm::plan(M, N, K, true, c_layout, &v, &s, batch, b_layout, a_layout);
+  else if (neogemm::ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt))
+    neogemm::ragged_plan(M, N, K, batch, neogemm::planning_cus(), &v, &s);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)batch : 0;
 }
 

@@ -72,29 +72,21 @@ torch::Tensor& workspace_for(const torch::Tensor& like, hipStream_t stream, size
   return t;
 }
 
+// How many problems of one shape a call holds and how far apart they lie, in elements.
+struct Batch {
+  int64_t count = 1, sa = 0, sb = 0, sc = 0;
+};
 void run(const torch::Tensor& A, const torch::Tensor& B, torch::Tensor& C, int64_t M, int64_t N, int64_t K,
-         int64_t lda, int64_t ldb, int64_t ldc, int b_layout, int c_layout, float alpha = 1.f, float beta = 0.f,
-         int a_layout = NEOGEMM_A_MK) {
+         int64_t lda, int64_t ldb, int64_t ldc, int a_layout, int b_layout, int c_layout, float alpha = 1.f, float beta = 0.f,
+         const Batch& bt = Batch()) {
   // PyTorch-ROCm names its HIP devices "cuda"; these are the guard and stream accessors for that naming
   c10::hip::HIPGuardMasqueradingAsCUDA guard(A.device());
-  if (a_layout == NEOGEMM_A_KM) {
-    const size_t need = neogemm_bf16_general_workspace_bytes(M, N, K, a_layout, b_layout, c_layout, 1);
-    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A.get_device()).stream();
-    void* ws = need ? workspace_for(A, stream, need).data_ptr() : nullptr;
-    const int st = neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, a_layout, b_layout,
-                                        c_layout, alpha, beta, 0, 0, 0, 1, ws, need, (void*)stream);
-    TORCH_CHECK(st == NEOGEMM_OK, "neogemm_bf16_general failed: ", neogemm_strerror(st));
-    return;
-  }
-  const size_t need = neogemm_bf16_workspace_bytes(M, N, K);
+  const size_t need = neogemm_bf16_call_workspace_bytes(A.data_ptr(), B.data_ptr(), M, N, K, lda, ldb, a_layout, b_layout, c_layout, bt.sa,
+                                                        bt.sb, bt.count);
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A.get_device()).stream();
-  void* ws = nullptr;
-  if (need) ws = workspace_for(A, stream, need).data_ptr();
-  const int st = (alpha == 1.f && beta == 0.f)
-                     ? neogemm_bf16(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, b_layout,
-                                    c_layout, ws, need, (void*)stream)
-                     : neogemm_bf16_scaled(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, b_layout,
-                                           c_layout, alpha, beta, ws, need, (void*)stream);
+  void* ws = need ? workspace_for(A, stream, need).data_ptr() : nullptr;
+  const int st = neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, a_layout, b_layout, c_layout,
+                                      alpha, beta, bt.sa, bt.sb, bt.sc, bt.count, ws, need, (void*)stream);
   TORCH_CHECK(st == NEOGEMM_OK, "neogemm_bf16 failed: ", neogemm_strerror(st));
 }
 
@@ -115,15 +107,16 @@ Operands describe(torch::Tensor A, torch::Tensor B) {
     B = B.contiguous();
     o.ldb = row_ld(B);
   }
-  // A = X.t() with X [K,M] row-major, as in a weight gradient dY.t() * X, is read in place where the tile kernels take it:
-  // whole 16-byte chunks, and more rows than the decode kernels, which want K-contiguous rows, would serve.  The copy
-  // took 68 us for 4096 x 4096 where the product itself takes 98.
+  // A = X.t() with X [K,M] row-major, as in a weight gradient dY.t() * X, is read in place: by the tile kernels where it comes in
+  // whole 16-byte chunks (a copy took 68 us for 4096 x 4096 where the product itself takes 98), by the kernel for operands at any
+  // address where not.  A copy is made for the decode kernels, which want K-contiguous rows and few of them.
   auto chunks = [](const torch::Tensor& t, int64_t ld) { return ((uintptr_t)t.data_ptr() & 15) == 0 && ld % 8 == 0; };
   const int64_t M = A.size(0), N = B.size(1), K = A.size(1);
   o.lda = row_ld(A);
   if (!row_major(A)) {
-    if (A.stride(0) == 1 && A.stride(1) >= M && M > 128 && M % 8 == 0 && chunks(A, A.stride(1)) && chunks(B, o.ldb) && N % 8 == 0 &&
-        (o.b_layout == NEOGEMM_B_KN || K % 8 == 0)) {
+    const bool b_whole = chunks(B, o.ldb) && (o.b_layout == NEOGEMM_B_NK || N % 8 == 0);
+    const bool decode = M <= 128 && K % 8 == 0 && b_whole;
+    if (A.stride(0) == 1 && A.stride(1) >= M && !decode) {
       o.a_layout = NEOGEMM_A_KM;
       o.lda = A.stride(1);
     } else {
@@ -147,7 +140,7 @@ torch::Tensor gemm(torch::Tensor A, torch::Tensor B) {
   torch::Tensor C = torch::empty({M, N}, A.options());
   if (M == 0 || N == 0) return C;
   const Operands o = describe(std::move(A), std::move(B));
-  run(o.A, o.B, C, M, N, K, o.lda, o.ldb, std::max<int64_t>(N, 1), o.b_layout, NEOGEMM_C_ROW, 1.f, 0.f, o.a_layout);
+  run(o.A, o.B, C, M, N, K, o.lda, o.ldb, std::max<int64_t>(N, 1), o.a_layout, o.b_layout, NEOGEMM_C_ROW);
   return C;
 }
 
@@ -163,10 +156,12 @@ void gemm_scaled(torch::Tensor A, torch::Tensor B, torch::Tensor C, double alpha
   const int64_t M = A.size(0), K = A.size(1), N = B.size(1);
   if (M == 0 || N == 0) return;
   const Operands o = describe(std::move(A), std::move(B));
-  run(o.A, o.B, C, M, N, K, o.lda, o.ldb, std::max<int64_t>(N, 1), o.b_layout, NEOGEMM_C_ROW, (float)alpha, (float)beta, o.a_layout);
+  run(o.A, o.B, C, M, N, K, o.lda, o.ldb, std::max<int64_t>(N, 1), o.a_layout, o.b_layout, NEOGEMM_C_ROW, (float)alpha, (float)beta);
 }
 
-// bmm(A, B): A [b,M,K], B [b,K,N] or [K,N] (shared) -> new C [b,M,N]; one launch (neogemm_bf16_batched).
+// bmm(A, B): A [b,M,K], B [b,K,N] or [K,N] (shared) -> new C [b,M,N]; one launch (neogemm_bf16_general).  Either operand may be
+// a transposed view (the k^T of attention scores) or a slice of a larger tensor: it is read in place unless only a copy of it would
+// lie on the 16-byte grid.
 torch::Tensor bmm(torch::Tensor A, torch::Tensor B) {
   TORCH_CHECK(A.is_cuda() && B.is_cuda(), "A and B must be GPU tensors (there is no CPU path)");
   TORCH_CHECK(A.scalar_type() == torch::kBFloat16 && B.scalar_type() == torch::kBFloat16, "A and B must be bfloat16");
@@ -174,20 +169,42 @@ torch::Tensor bmm(torch::Tensor A, torch::Tensor B) {
   TORCH_CHECK(A.device() == B.device(), "A and B must be on the same device");
   TORCH_CHECK(A.size(2) == B.size(B.dim() - 2) && (B.dim() == 2 || B.size(0) == A.size(0)), "shapes do not match: A ",
               A.sizes(), ", B ", B.sizes());
-  A = A.contiguous();
-  B = B.contiguous();
   const int64_t batch = A.size(0), M = A.size(1), K = A.size(2), N = B.size(B.dim() - 1);
   torch::Tensor C = torch::empty({batch, M, N}, A.options());
   if (batch == 0 || M == 0 || N == 0) return C;
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(A.device());
-  const size_t need = neogemm_bf16_batched_workspace_bytes(M, N, K, batch);
-  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A.get_device()).stream();
-  void* ws = nullptr;
-  if (need) ws = workspace_for(A, stream, need).data_ptr();
-  const int st = neogemm_bf16_batched(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, std::max<int64_t>(K, 1),
-                                      std::max<int64_t>(N, 1), std::max<int64_t>(N, 1), M * K, B.dim() == 3 ? K * N : 0,
-                                      M * N, batch, NEOGEMM_B_KN, NEOGEMM_C_ROW, ws, need, (void*)stream);
-  TORCH_CHECK(st == NEOGEMM_OK, "neogemm_bf16_batched failed: ", neogemm_strerror(st));
+  // rows x cols matrices of a 3-D tensor: row-major or its transpose, and the leading dimension
+  struct View {
+    bool ok, transposed;
+    int64_t ld, stride;
+    bool whole;  // on the 16-byte grid
+  };
+  auto view = [](const torch::Tensor& t) -> View {
+    const int d = t.dim() - 2;
+    const int64_t rows = t.size(d), cols = t.size(d + 1), sr = t.stride(d), sc = t.stride(d + 1);
+    View v{true, false, std::max<int64_t>(cols, 1), d && t.size(0) > 1 ? t.stride(0) : 0, false};
+    if (cols <= 1 || sc == 1) {
+      if (rows > 1) v.ld = sr;
+      v.ok = v.ld >= cols;
+    } else if (rows <= 1 || sr == 1) {
+      v.transposed = true;
+      v.ld = sc;
+      v.ok = sc >= rows;
+    } else {
+      v.ok = false;
+    }
+    v.whole = ((uintptr_t)t.data_ptr() & 15) == 0 && v.ld % 8 == 0 && v.ld < (1 << 21) && v.stride % 8 == 0 && (v.transposed ? rows : cols) % 8 == 0;
+    return v;
+  };
+  auto settle = [&](torch::Tensor& t) -> View {
+    View v = view(t);
+    if (t.is_contiguous() || (v.ok && (v.whole || t.size(t.dim() - 1) % 8 != 0))) return v;
+    t = t.contiguous();
+    return view(t);
+  };
+  if (batch == 1 && M <= 128 && A.stride(2) != 1) A = A.contiguous();  // the decode kernels want K-contiguous rows
+  const View va = settle(A), vb = settle(B);
+  run(A, B, C, M, N, K, va.ld, vb.ld, std::max<int64_t>(N, 1), va.transposed ? NEOGEMM_A_KM : NEOGEMM_A_MK,
+      vb.transposed ? NEOGEMM_B_NK : NEOGEMM_B_KN, NEOGEMM_C_ROW, 1.f, 0.f, Batch{batch, va.stride, vb.stride, M * N});
   return C;
 }
 
@@ -204,7 +221,7 @@ void neoGemmV1(torch::Tensor A, torch::Tensor B, torch::Tensor C) {
   const int64_t M = A.size(0), K = A.size(1), N = B.size(0);
   TORCH_CHECK(C.numel() == M * N, "C must hold M*N = ", M * N, " elements, has ", C.numel());
   if (M == 0 || N == 0) return;
-  run(A, B, C, M, N, K, std::max<int64_t>(K, 1), std::max<int64_t>(K, 1), M, NEOGEMM_B_NK, NEOGEMM_C_COL);
+  run(A, B, C, M, N, K, std::max<int64_t>(K, 1), std::max<int64_t>(K, 1), M, NEOGEMM_A_MK, NEOGEMM_B_NK, NEOGEMM_C_COL);
 }
 
 }  // namespace

@@ -144,6 +144,12 @@ int neogemm_bf16_general(const void* A, const void* B, void* C, int64_t M, int64
                          size_t workspace_bytes, void* hip_stream);
 size_t neogemm_bf16_general_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_layout, int b_layout, int c_layout,
                                             int64_t batch);
+/*
+ * What neogemm_bf16_general uses for exactly these operands.  Those that lie off the 16-byte grid (any pointer, leading
+ * dimension, batch stride or K that is no multiple of 8 elements) run with less, or none, as well: K is then not split.
+ */
+size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                         int a_layout, int b_layout, int c_layout, int64_t stride_a, int64_t stride_b, int64_t batch);
 
 /*
  * neogemm_bf16 for callers that cannot allocate device memory (code under HIP graph capture, tight serving

@@ -1,0 +1,90 @@
+"""Operands at any address and with any leading dimension (gemm_ragged_kernel): small integers between NaNs, so that every order
+of summation gives the same bits and an element that does not belong to the product shows."""
+import pytest
+import torch
+
+import gemm_amd as g
+import neoGEMM
+from gemm_amd import _abi
+
+pytestmark = pytest.mark.gpu
+
+
+def between_nans(gen, rows, cols, pad, shift):
+    """A rows x cols matrix of small integers, its rows cols + pad apart, `shift` elements into a buffer that is NaN elsewhere."""
+    ld = cols + pad
+    flat = torch.full((rows * ld + shift + 3,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    m = flat[shift:shift + rows * ld].view(rows, ld)[:, :cols]
+    m.copy_(torch.randint(-2, 3, (rows, cols), generator=gen, device="cuda"))
+    return m
+
+
+# K: one element, less than a chunk, around one, two, three and five tiles of 64 (prologue, plain loop, careful tail), deep enough to
+# be split; M, N: one row, less than a chunk, edges of the 64 and 128 tiles, enough tiles for the 128 one
+SIZES = [(9, 9, 1), (1, 9, 13), (17, 1, 9), (64, 65, 7), (63, 129, 64), (65, 64, 71), (130, 127, 129), (129, 257, 193), (65, 191, 322), (200, 77, 447),
+         (1, 1001, 1537), (127, 131, 4099), (2500, 2501, 137), (3001, 2999, 520)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("a_layout", [g.A_MK, g.A_KM])
+@pytest.mark.parametrize("b_layout", [g.B_KN, g.B_NK])
+@pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
+def test_operands_at_any_address(M, N, K, a_layout, b_layout, c_layout):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    for pad_a, pad_b, shift in ((0, 1, 1), (3, 0, 2)):
+        A = between_nans(gen, *((M, K) if a_layout == g.A_MK else (K, M)), pad_a, shift)
+        B = between_nans(gen, *((K, N) if b_layout == g.B_KN else (N, K)), pad_b, shift + 1)
+        At, Bkn = A if a_layout == g.A_MK else A.t(), B if b_layout == g.B_KN else B.t()
+        want = At.float() @ Bkn.float()
+        C = torch.full((M, N) if c_layout == g.C_ROW else (N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
+        g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout)
+        got = C if c_layout == g.C_ROW else C.t()
+        assert torch.equal(got, want.to(torch.bfloat16))
+        old = got.clone()
+        g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout, alpha=0.5, beta=-1.0)
+        assert torch.equal(got, (0.5 * want - old.float()).to(torch.bfloat16))
+
+
+def test_the_last_bytes_of_an_allocation():
+    """Operands that end where their buffer of a few elements ends."""
+    for M, N, K in ((1, 1, 8), (2, 3, 5), (3, 2, 7), (1, 8, 1), (8, 1, 1)):
+        A, B = torch.ones(M, K, dtype=torch.bfloat16, device="cuda"), torch.ones(K, N, dtype=torch.bfloat16, device="cuda")
+        assert torch.equal(neoGEMM.gemm(A, B), torch.full((M, N), float(K), dtype=torch.bfloat16, device="cuda"))
+
+
+def test_split_needs_the_general_call_and_its_workspace():
+    """K is split over the workspace the query asks for; with less, and through the calls that never took one, it is not."""
+    M, N, K = 127, 131, 8191
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    A, B = between_nans(gen, M, K, 0, 1), between_nans(gen, K, N, 0, 1)
+    want = (A.float() @ B.float()).to(torch.bfloat16)
+    lib = _abi.load()
+    need = int(lib.neogemm_bf16_call_workspace_bytes(A.data_ptr(), B.data_ptr(), M, N, K, K, N, g.A_MK, g.B_KN, g.C_ROW, 0, 0, 1))
+    assert need >= 2 * M * N * 4
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream or None
+    for size in (need, need - 1, 0):
+        C = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert lib.neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, K, N, N, g.A_MK, g.B_KN, g.C_ROW, 1.0, 0.0, 0, 0, 0, 1,
+                                        ws.data_ptr(), size, st) == _abi.OK
+        assert torch.equal(C, want)
+    C = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert lib.neogemm_bf16(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, K, N, N, g.B_KN, g.C_ROW, None, 0, st) == _abi.OK
+    assert torch.equal(C, want)
+
+
+# batches: transposed views, slices of a larger tensor, a shared operand, odd sizes; K of one and two tiles
+@pytest.mark.parametrize("b,M,N,K", [(3, 200, 136, 64), (2, 264, 392, 128), (5, 77, 77, 96), (3, 100, 64, 101), (1, 96, 520, 72), (4, 1, 9, 200), (2, 9, 1, 5)])
+def test_batches_of_views(b, M, N, K):
+    gen = torch.Generator(device="cuda").manual_seed(b + M)
+
+    def ints(*shape):
+        return torch.randint(-2, 3, shape, generator=gen, device="cuda").to(torch.bfloat16)
+
+    As = [ints(b, M, K), ints(b, K, M).transpose(1, 2), ints(b, M, K + 5)[:, :, 3:K + 3], ints(M, b, K).transpose(0, 1), ints(1, M, K).expand(b, M, K),
+          ints(K, b, M).permute(1, 2, 0)]
+    Bs = [ints(b, K, N), ints(b, N, K).transpose(1, 2), ints(K, N), ints(N, K).t(), ints(b, K + 1, N)[:, 1:], ints(K, N, b).permute(2, 0, 1)]
+    for A in As:
+        for B in Bs:
+            want = torch.stack([A[i].float() @ (B[i] if B.dim() == 3 else B).float() for i in range(b)])
+            assert torch.equal(neoGEMM.bmm(A, B), want.to(torch.bfloat16))
