@@ -1393,24 +1393,27 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(TileArgs p) {
   store_wave_tile<TM, TN, NW, LDS_BYTES, TM, false>(acc, p, gC, kz, lane, wave, lds0, BlockMap{m0 + wm * WTM, n0 + wn * WTN});
 }
 
-// tile: 64 or 128 (square)
-hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int tile, hipStream_t st);
+// bm x bn: 64x64, 128x64 or 128x128
+hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int bm, int bn, hipStream_t st);
 #if NEOGEMM_HAS_PART(9)
-hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int tile, hipStream_t st) {
-  const size_t lds = (size_t)tile * 512;
+hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int bm, int bn, hipStream_t st) {
+  const size_t lds = (size_t)(bm + bn) * 256;
   dim3 grid(a.ntm * a.ntn * a.ksplit, 1, a.batch), block(256);
   auto go = [&](auto kern) -> hipError_t {
     if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
     kern<<<grid, block, lds, st>>>(a);
     return hipGetLastError();
   };
-  auto pick = [&](auto tc) -> hipError_t {
-    constexpr int T = decltype(tc)::value;
-    if (ak) return bk ? go(gemm_ragged_kernel<T, T, true, true>) : go(gemm_ragged_kernel<T, T, true, false>);
-    return bk ? go(gemm_ragged_kernel<T, T, false, true>) : go(gemm_ragged_kernel<T, T, false, false>);
+  auto pick = [&](auto mc, auto nc) -> hipError_t {
+    constexpr int BM = decltype(mc)::value, BN = decltype(nc)::value;
+    if (ak) return bk ? go(gemm_ragged_kernel<BM, BN, true, true>) : go(gemm_ragged_kernel<BM, BN, true, false>);
+    return bk ? go(gemm_ragged_kernel<BM, BN, false, true>) : go(gemm_ragged_kernel<BM, BN, false, false>);
   };
-  if (tile == 64) return pick(std::integral_constant<int, 64>{});
-  if (tile == 128) return pick(std::integral_constant<int, 128>{});
+  using I64 = std::integral_constant<int, 64>;
+  using I128 = std::integral_constant<int, 128>;
+  if (bm == 64 && bn == 64) return pick(I64{}, I64{});
+  if (bm == 128 && bn == 64) return pick(I128{}, I64{});
+  if (bm == 128 && bn == 128) return pick(I128{}, I128{});
   return hipErrorInvalidValue;
 }
 #endif
@@ -2046,6 +2049,33 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   }
 }
 
+// An operand onto the 16-byte grid: `rows` x `cols` as it lies in memory, rows ld elements apart from any address on, to rows of
+// cpr chunks of eight elements, the last one filled up with zeros.  One chunk per thread; A's workgroups, then B's.
+struct PackArgs {
+  const char* src;
+  char* dst;
+  long ld, bs;              // elements between rows and between the problems of a batch (0: one matrix for all of them)
+  unsigned rows, cols, cpr, blocks;
+};
+__global__ __launch_bounds__(256) void pack_kernel(PackArgs a, PackArgs b) {
+  const bool first = blockIdx.x < a.blocks;
+  const PackArgs& p = first ? a : b;
+  if (blockIdx.z > 0 && p.bs == 0) return;
+  const unsigned q = (blockIdx.x - (first ? 0 : a.blocks)) * 256 + threadIdx.x, row = q / p.cpr, c = (q - row * p.cpr) * 8;
+  if (row >= p.rows) return;
+  const __bf16* src = (const __bf16*)p.src + (size_t)blockIdx.z * p.bs + (size_t)row * p.ld + c;
+  i32x4 v;
+  if (c + 8 <= p.cols) {
+    v = *(const i32x4_u*)src;
+  } else {
+    bf16x8 t;
+#pragma unroll
+    for (unsigned e = 0; e < 8; ++e) t[e] = c + e < p.cols ? src[e] : (__bf16)0.f;
+    v = __builtin_bit_cast(i32x4, t);
+  }
+  *(i32x4*)(p.dst + ((size_t)blockIdx.z * p.rows * p.cpr + q) * 16) = v;
+}
+
 // Fallback for anything the tile kernels do not take: arbitrary element strides, no alignment needs.
 // One thread per output element, 16x16 outputs per workgroup, K walked 16 at a time through LDS.
 __global__ __launch_bounds__(256) void gemm_generic_kernel(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
@@ -2137,7 +2167,8 @@ static int planning_cus() {
   return cus;
 }
 static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
-                       int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int ncus = 256, int a_layout = NEOGEMM_A_MK) {
+                       int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int ncus = 256, int a_layout = NEOGEMM_A_MK,
+                       double* estimate_us = nullptr) {
   if (!aligned || K == 0) {
     *variant = NEOGEMM_VARIANT_GENERIC;
     *split_k = 1;
@@ -2369,6 +2400,7 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
     bv = NEOGEMM_VARIANT_C256x256_W4;
   *variant = bv;
   *split_k = bs;
+  if (estimate_us) *estimate_us = best;
 }
 
 // Tuned choices override the model: the file named by the environment variable NEOGEMM_PLAN_TABLE, read
@@ -2588,12 +2620,13 @@ static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream
 struct BatchArgs {
   int64_t count = 1, sa = 0, sb = 0, sc = 0;
   int a_layout = NEOGEMM_A_MK;
-  bool split_ragged = false;  // operands off the 16-byte grid may split K over the workspace (see neogemm_bf16_call_workspace_bytes)
+  bool scratch_unaligned = false;  // operands off the 16-byte grid may use the workspace (see neogemm_bf16_call_workspace_bytes)
+  bool padded = false;             // rows of both operands end on whole chunks in memory, zeros behind K (pack_kernel)
 };
 
 // ld limits keep every in-tile byte offset below 2^31 (the buffer range check uses 32-bit offsets)
 static bool mfma_aligned(const void* A, const void* B, int64_t K, int64_t lda, int64_t ldb, int b_layout, const BatchArgs& bt) {
-  return is_aligned(A, B, K, lda, ldb, bt.a_layout == NEOGEMM_A_MK || b_layout == NEOGEMM_B_NK) && lda < (1 << 21) && ldb < (1 << 21) &&
+  return is_aligned(A, B, K, lda, ldb, !bt.padded && (bt.a_layout == NEOGEMM_A_MK || b_layout == NEOGEMM_B_NK)) && lda < (1 << 21) && ldb < (1 << 21) &&
          K > 0 && (bt.sa & 7) == 0 && (bt.sb & 7) == 0;
 }
 
@@ -2605,40 +2638,137 @@ static bool ragged_takes(const void* A, const void* B, int64_t M, int64_t N, int
   const int64_t ext_b = b_layout == NEOGEMM_B_KN ? (K - 1) * ldb + N : (N - 1) * ldb + K;
   return K > 0 && ext_a >= 8 && ext_b >= 8 && lda < (1 << 21) && ldb < (1 << 21) && (((uintptr_t)A | (uintptr_t)B) & 1) == 0;
 }
-// Tile (64 or 128) and split of K of gemm_ragged_kernel, by the time of its K tiles: a workgroup of the 64x64 tile takes 0.40 us
-// per K tile where several share a CU (the loads at two-byte addresses bound it: 1023 x 2047 x 1535, 512 of them, 21 us), 0.29
-// alone on one (64 x 256 x 20001 in 16 splits, 14.5 us; the same in 4, 26); one of the 128x128 tile, four times the work, 0.95
-// (1500 x 1501 x 1401: 25.3 us for 144 of them, 28.3 for 576 small ones; 1023 x 2047 x 1535: 28 for 128).  A split costs the
-// second launch and the partials (512 x 1024 x 10001 in 64x64 tiles: 29 us with two, 47 unsplit).
-static void ragged_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, int* tile, int* split) {
+// Tile (bm x bn of the output as it lies in memory, rows x cols) and split of K of gemm_ragged_kernel, by the time of its K tiles;
+// returns the estimate.  A workgroup of the 64x64 tile takes 0.40 us per K tile where several share a CU (the loads at two-byte
+// addresses bound it: 1023 x 2047 x 1535, 512 of them, 21 us), 0.29 alone on one (64 x 256 x 20001 in 16 splits, 14.5 us; the same
+// in 4, 26); one of the 128x128 tile, four times the work, 0.95 (1500 x 1501 x 1401: 25.3 us for 144 of them, 28.3 for 576 small
+// ones; 1023 x 2047 x 1535: 28 for 128).  A split costs the second launch and the partials (512 x 1024 x 10001 in 64x64 tiles:
+// 29 us with two, 47 unsplit).
+static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, int cus, int* bm, int* bn, int* split) {
+  struct Tile {
+    int bm, bn;
+    double alone_us, shared_us, fixed_us;  // per K tile of a workgroup that has its CU to itself / shares it
+  };
+  static const Tile kTiles[] = {{64, 64, 0.29, 0.40, 3.0}, {128, 64, 0.56, 0.56, 3.5}, {128, 128, 0.95, 0.95, 4.0}};
   const int64_t ktiles = ceil_div(K, KTILE);
   double best = 1e300;
-  for (int t : {64, 128})
+  for (const Tile& t : kTiles)
     for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
       if (sp > 1 && ktiles / sp < 4) break;
-      const double wgs = (double)ceil_div(M, t) * ceil_div(N, t) * (double)batch * sp, per_cu = __builtin_ceil(wgs / cus);
-      double us = per_cu * ceil_div(ktiles, sp) * (t == 128 ? 0.95 : per_cu > 1 ? 0.40 : 0.29) + (t == 128 ? 4.0 : 3.0);
-      if (sp > 1) us += 5.0 + (4.0 * sp + 2.0) * (double)M * (double)N * (double)batch / 4.0e6;
+      const double wgs = (double)ceil_div(rows, t.bm) * ceil_div(cols, t.bn) * (double)batch * sp, per_cu = __builtin_ceil(wgs / cus);
+      double us = per_cu * ceil_div(ktiles, sp) * (per_cu > 1 ? t.shared_us : t.alone_us) + t.fixed_us;
+      if (sp > 1) us += 5.0 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 4.0e6;
       if (us < best) {
         best = us;
-        *tile = t;
+        *bm = t.bm;
+        *bn = t.bn;
         *split = sp;
       }
     }
+  return best;
+}
+// Copies of the operands that are off the 16-byte grid (pack_kernel), and the product by the kernels for aligned ones.
+struct PackPlan {
+  bool a = false, b = false;                 // which operand is copied
+  int64_t ldpa = 0, ldpb = 0;                // leading dimensions of the copies
+  size_t partials = 0, bytes_a = 0, bytes_b = 0;  // what the workspace holds, in this order, each from a multiple of 256 on
+  size_t total() const { return partials + bytes_a + bytes_b; }
+};
+static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int b_layout, int c_layout,
+                      const BatchArgs& bt, PackPlan* out) {
+  const bool a_mk = bt.a_layout == NEOGEMM_A_MK, b_nk = b_layout == NEOGEMM_B_NK;
+  const int64_t rows_a = a_mk ? M : K, cols_a = a_mk ? K : M, rows_b = b_nk ? N : K, cols_b = b_nk ? K : N;
+  auto off_grid = [](const void* ptr, int64_t ld, int64_t bs, int64_t cols) {
+    return ((uintptr_t)ptr & 15) != 0 || (ld & 7) != 0 || ld >= (1 << 21) || (bs & 7) != 0 || (cols & 7) != 0;
+  };
+  PackPlan p;
+  p.a = off_grid(A, lda, bt.sa, cols_a);
+  p.b = off_grid(B, ldb, bt.sb, cols_b);
+  p.ldpa = (cols_a + 7) / 8 * 8;
+  p.ldpb = (cols_b + 7) / 8 * 8;
+  if ((!p.a && !p.b) || p.ldpa >= (1 << 21) || p.ldpb >= (1 << 21) || K < 1) return false;
+  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+  if (p.a) p.bytes_a = up((size_t)rows_a * p.ldpa * 2 * (bt.sa ? bt.count : 1));
+  if (p.b) p.bytes_b = up((size_t)rows_b * p.ldpb * 2 * (bt.sb ? bt.count : 1));
+  const size_t most = (size_t)1 << 30;  // of memory that a caller's workspace would keep for it
+  if (p.bytes_a + p.bytes_b > most) return false;
+  struct Memo {
+    int64_t M = -1, N = -1, K = -1, count = -1;
+    size_t bytes = 0;
+    int a_layout = -1, b_layout = -1, c_layout = -1, cus = -1, split = 1;
+    bool pays = false;
+  };
+  static thread_local Memo memo[32];
+  static thread_local unsigned next = 0;
+  const int cus = planning_cus();
+  const Memo* m = nullptr;
+  for (const Memo& e : memo)
+    if (e.M == M && e.N == N && e.K == K && e.count == bt.count && e.bytes == p.bytes_a + p.bytes_b && e.a_layout == bt.a_layout &&
+        e.b_layout == b_layout && e.c_layout == c_layout && e.cus == cus)
+      m = &e;
+  if (!m) {
+    Memo& e = memo[next++ & 31];
+    e = Memo{M, N, K, bt.count, p.bytes_a + p.bytes_b, bt.a_layout, b_layout, c_layout, cus, 1, false};
+    int v, bm, bn, sp;
+    double aligned_us = 0;
+    plan_model(M, N, K, true, c_layout, &v, &sp, bt.count, b_layout, cus, bt.a_layout, &aligned_us);
+    const bool row = c_layout == NEOGEMM_C_ROW;
+    const double ragged_us = ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, &bm, &bn, &sp);
+    // (10001 x 1024 x 512 with a transposed A takes a sixth more than the estimate)
+    // the copy and the product that waits for it: 6.5 us and 3 MB per us (1500 x 1501 x 1401 26.1 -> 23.0 us, 1000 x 2048 x 5001 47.0 ->
+    // 39.1, 4001^3 202 -> 120; below the line 700^3 9.0 against 14.9, 100 x 2999 x 2999 16.3 against 26.1)
+    e.pays = aligned_us + 6.5 + (double)e.bytes / 3.0e6 < ragged_us * (bt.a_layout == NEOGEMM_A_KM ? 1.15 : 1.0);
+    plan(M, N, K, true, c_layout, &v, &sp, bt.count, b_layout, bt.a_layout);
+    e.split = sp;
+    m = &e;
+  }
+  if (!m->pays) return false;
+  if (m->split > 1) p.partials = up((size_t)m->split * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count);
+  *out = p;
+  return true;
+}
+static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+               int64_t ldc, int b_layout, int c_layout, void* workspace, size_t workspace_bytes, void* hip_stream,
+               int variant, int split_k, int group_m, unsigned long long* prof = nullptr, float alpha = 1.f,
+               float beta = 0.f, const BatchArgs& bt = BatchArgs());
+static int launch_packed(const PackPlan& p, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                         int64_t ldc, int b_layout, int c_layout, void* ws, hipStream_t st, float alpha, float beta, const BatchArgs& bt) {
+  const bool a_mk = bt.a_layout == NEOGEMM_A_MK, b_nk = b_layout == NEOGEMM_B_NK;
+  char* at_a = (char*)ws + p.partials;
+  char* at_b = at_a + p.bytes_a;
+  auto args = [&](const void* src, char* dst, int64_t ld, int64_t bs, int64_t rows, int64_t cols, bool used) {
+    PackArgs r{(const char*)src, dst, (long)ld, bt.count > 1 ? (long)bs : 0, (unsigned)rows, (unsigned)cols, (unsigned)((cols + 7) / 8), 0};
+    if (used) r.blocks = (unsigned)(((uint64_t)r.rows * r.cpr + 255) / 256);
+    return r;
+  };
+  const PackArgs pa = args(A, at_a, lda, bt.sa, a_mk ? M : K, a_mk ? K : M, p.a), pb = args(B, at_b, ldb, bt.sb, b_nk ? N : K, b_nk ? K : N, p.b);
+  const bool one = (!p.a || pa.bs == 0) && (!p.b || pb.bs == 0);  // nothing that differs between the problems of the batch is copied
+  pack_kernel<<<dim3(pa.blocks + pb.blocks, 1, one ? 1u : (unsigned)bt.count), 256, 0, st>>>(pa, pb);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) {
+    fprintf(stderr, "neogemm: pack kernel launch failed: %s\n", hipGetErrorString(e));
+    return NEOGEMM_ERR_LAUNCH;
+  }
+  BatchArgs to = bt;
+  to.padded = true;
+  if (p.a) to.sa = pa.bs ? (int64_t)pa.rows * p.ldpa : 0;
+  if (p.b) to.sb = pb.bs ? (int64_t)pb.rows * p.ldpb : 0;
+  return run(p.a ? at_a : A, p.b ? at_b : B, C, M, N, K, p.a ? p.ldpa : lda, p.b ? p.ldpb : ldb, ldc, b_layout, c_layout, ws, p.partials,
+             (void*)st, NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, alpha, beta, to);
 }
 // Operands at any address: gemm_ragged_kernel, and the reduction where K is split.  NEOGEMM_ERR_UNSUPPORTED: not launched.
 static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                             int64_t ldc, int b_layout, int c_layout, void* ws, size_t ws_bytes, hipStream_t st, float alpha, float beta,
                             const BatchArgs& bt) {
   if (!ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt)) return NEOGEMM_ERR_UNSUPPORTED;
-  int tile = 128, split = 1;
-  ragged_plan(M, N, K, bt.count, planning_cus(), &tile, &split);
+  int bm = 128, bn = 128, split = 1;
+  const bool row = c_layout == NEOGEMM_C_ROW;
+  ragged_plan(row ? M : N, row ? N : M, K, bt.count, planning_cus(), &bm, &bn, &split);
   TileArgs a{};
   const bool a_mk = bt.a_layout == NEOGEMM_A_MK, b_nk = b_layout == NEOGEMM_B_NK;
   bool ak = a_mk, bk = b_nk;
   a.A = (const char*)A; a.lda = lda; a.M = (int)M; a.bsa = bt.sa;
   a.B = (const char*)B; a.ldb = ldb; a.N = (int)N; a.bsb = bt.sb;
-  if (c_layout == NEOGEMM_C_COL) {  // the row-major transpose: the operands change roles
+  if (!row) {  // the row-major transpose: the operands change roles
     std::swap(a.A, a.B);
     std::swap(a.lda, a.ldb);
     std::swap(a.M, a.N);
@@ -2650,17 +2780,17 @@ static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, in
   a.K = (int)K;
   a.batch = (int)bt.count;
   a.alpha = alpha; a.beta = beta;
-  a.ntm = ceil_div(a.M, tile);
-  a.ntn = ceil_div(a.N, tile);
+  a.ntm = ceil_div(a.M, bm);
+  a.ntn = ceil_div(a.N, bn);
   a.group_m = 8;
   const int ktiles = ceil_div(K, KTILE);
-  if (!bt.split_ragged || !ws || ((uintptr_t)ws & 15) != 0 || ws_bytes < (size_t)split * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count)
+  if (!bt.scratch_unaligned || !ws || ((uintptr_t)ws & 15) != 0 || ws_bytes < (size_t)split * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count)
     split = 1;
   a.ktiles_per_split = ceil_div(ktiles, split);
   a.ksplit = ceil_div(ktiles, a.ktiles_per_split);  // no empty split
   if ((int64_t)a.ntm * a.ntn * a.ksplit > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;
   a.ws = (float*)ws;
-  if (hipError_t e = launch_ragged(a, ak, bk, tile, st); e != hipSuccess) {
+  if (hipError_t e = launch_ragged(a, ak, bk, bm, bn, st); e != hipSuccess) {
     fprintf(stderr, "neogemm: ragged kernel launch failed: %s\n", hipGetErrorString(e));
     return NEOGEMM_ERR_LAUNCH;
   }
@@ -2678,8 +2808,7 @@ static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, in
 
 static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                int64_t ldc, int b_layout, int c_layout, void* workspace, size_t workspace_bytes, void* hip_stream,
-               int variant, int split_k, int group_m, unsigned long long* prof = nullptr, float alpha = 1.f,
-               float beta = 0.f, const BatchArgs& bt = BatchArgs()) {
+               int variant, int split_k, int group_m, unsigned long long* prof, float alpha, float beta, const BatchArgs& bt) {
   if (M < 0 || N < 0 || K < 0) return NEOGEMM_ERR_BAD_ARG;
   if (bt.count < 1 || bt.count > 65535 || bt.sa < 0 || bt.sb < 0 || bt.sc < 0) return NEOGEMM_ERR_BAD_ARG;
   if (bt.count > 1 && M > 0 && N > 0) {
@@ -2702,6 +2831,10 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
 
   const bool aligned = mfma_aligned(A, B, K, lda, ldb, b_layout, bt);
   auto unaligned = [&]() -> int {
+    PackPlan pp;
+    if (bt.scratch_unaligned && !bt.padded && workspace && ((uintptr_t)workspace & 15) == 0 &&
+        pack_plan(A, B, M, N, K, lda, ldb, b_layout, c_layout, bt, &pp) && workspace_bytes >= pp.total())
+      return launch_packed(pp, A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, st, alpha, beta, bt);
     const int r = launch_unaligned(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, st, alpha, beta, bt);
     return r != NEOGEMM_ERR_UNSUPPORTED ? r
                                         : run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
@@ -2750,7 +2883,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     // C^T = B * A^T: its small operand is B then, its wide one A, and the layout of C flips.
     const bool swap = M > kVariants[v].bm && N <= kVariants[v].bm && b_layout == NEOGEMM_B_NK;
     const bool ok = bt.count == 1 && a_mk && (M <= kVariants[v].bm || swap) &&
-                    (b_layout == NEOGEMM_B_NK || (N & 7) == 0) &&
+                    (b_layout == NEOGEMM_B_NK || (N & 7) == 0 || bt.padded) &&
                     (split_k <= 1 || variant == NEOGEMM_VARIANT_AUTO || v == NEOGEMM_VARIANT_STRIP) && !prof;
     if (!ok) {
       if (variant != NEOGEMM_VARIANT_AUTO) return NEOGEMM_ERR_UNSUPPORTED;
@@ -2846,7 +2979,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   // What the tile kernels assume about an MN-major operand (see Operand::init): a tile of >= 128 rows, a power
   // of two, for its swizzle and a row count that is a multiple of 8 (16-byte chunks must not straddle the
   // matrix edge).
-  auto mn_ok = [](int tile, int rows) { return tile >= 128 && (tile & (tile - 1)) == 0 && (rows & 7) == 0; };
+  auto mn_ok = [&](int tile, int rows) { return tile >= 128 && (tile & (tile - 1)) == 0 && ((rows & 7) == 0 || bt.padded); };
   // (the chained 256x256 kernel takes its rows from a K-major operand only, K in whole periods of 128 and no split)
   const bool fits = (ak || mn_ok(vi.bm, a.M)) && (bk || mn_ok(vi.bn, a.N)) &&
                     (v != NEOGEMM_VARIANT_C256x256_W4 || (ak && K % (2 * KTILE) == 0 && s <= 1));
@@ -2994,7 +3127,7 @@ int neogemm_bf16_general(const void* A, const void* B, void* C, int64_t M, int64
   bt.sb = stride_b;
   bt.sc = stride_c;
   bt.a_layout = a_layout;
-  bt.split_ragged = true;
+  bt.scratch_unaligned = true;
   return neogemm::run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
                       NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, alpha, beta, bt);
 }
@@ -3015,12 +3148,16 @@ size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M
   bt.sa = stride_a;
   bt.sb = stride_b;
   bt.a_layout = a_layout;
-  int v, s = 1;
+  int v, w, s = 1;
+  const bool row = c_layout == NEOGEMM_C_ROW;
+  neogemm::PackPlan pp;
   // (an MN-major operand whose rows do not end on a chunk goes the same way as one off the 16-byte grid)
   if (neogemm::mfma_aligned(A, B, K, lda, ldb, b_layout, bt) && (a_layout == NEOGEMM_A_MK || M % 8 == 0) && (b_layout == NEOGEMM_B_NK || N % 8 == 0))
     neogemm::plan(M, N, K, true, c_layout, &v, &s, batch, b_layout, a_layout);
+  else if (neogemm::pack_plan(A, B, M, N, K, lda, ldb, b_layout, c_layout, bt, &pp))
+    return pp.total();
   else if (neogemm::ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt))
-    neogemm::ragged_plan(M, N, K, batch, neogemm::planning_cus(), &v, &s);
+    neogemm::ragged_plan(row ? M : N, row ? N : M, K, batch, neogemm::planning_cus(), &v, &w, &s);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)batch : 0;
 }
 

@@ -88,3 +88,31 @@ def test_batches_of_views(b, M, N, K):
         for B in Bs:
             want = torch.stack([A[i].float() @ (B[i] if B.dim() == 3 else B).float() for i in range(b)])
             assert torch.equal(neoGEMM.bmm(A, B), want.to(torch.bfloat16))
+
+
+# large enough that copies on the 16-byte grid pay: K a part of a chunk past a tile, MN-major rows that end inside a chunk, one operand
+# on the grid already, K split, few rows (the decode kernels), a batch with a shared and with a strided operand
+@pytest.mark.parametrize("b,M,N,K", [(1, 1023, 2047, 1535), (1, 512, 1024, 10001), (1, 2049, 1032, 1001), (1, 2501, 1001, 1000), (1, 16, 4097, 4097),
+                                     (1, 128, 4097, 4096), (3, 1001, 1003, 1005)])
+def test_copies_on_the_grid(b, M, N, K):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    lib = _abi.load()
+    st = torch.cuda.current_stream().cuda_stream or None
+    for a_layout in (g.A_MK, g.A_KM):
+        for b_layout in (g.B_KN, g.B_NK):
+            for c_layout in (g.C_ROW, g.C_COL):
+                A = between_nans(gen, *((b * M, K) if a_layout == g.A_MK else (b * K, M)), 0, 1)
+                B = between_nans(gen, *((K, N) if b_layout == g.B_KN else (N, K)), 0, 8)
+                A3 = A.view(b, -1, A.shape[1])
+                want = (A3 if a_layout == g.A_MK else A3.transpose(1, 2)).float() @ (B if b_layout == g.B_KN else B.t()).float()
+                old = torch.randint(-8, 9, (b, M, N) if c_layout == g.C_ROW else (b, N, M), generator=gen, device="cuda").to(torch.bfloat16)
+                C = old.clone()
+                lda, ldb, sa = A.stride(0), B.stride(0), A3.stride(0) if b > 1 else 0
+                need = int(lib.neogemm_bf16_call_workspace_bytes(A.data_ptr(), B.data_ptr(), M, N, K, lda, ldb, a_layout, b_layout, c_layout, sa, 0, b))
+                ws = torch.full((need // 4 + 4,), float("nan"), device="cuda")
+                for size in (need, 0):   # with the copies, and by the kernel that reads in place
+                    C.copy_(old)
+                    assert lib.neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, C.stride(1), a_layout, b_layout, c_layout,
+                                                    1.0, 1.0, sa, 0, M * N, b, ws.data_ptr(), size, st) == _abi.OK
+                    got, add = (C, old) if c_layout == g.C_ROW else (C.transpose(1, 2), old.transpose(1, 2))
+                    assert torch.equal(got, (want + add.float()).to(torch.bfloat16))
