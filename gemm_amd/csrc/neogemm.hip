@@ -1418,6 +1418,164 @@ hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int bm, int bn, hi
 }
 #endif
 
+// ---------------------------------------------------------------------------------------------
+// Short K (at most 128), both operands K-major: attention scores q k^T.  Bound by writing C (32 heads x 1024 x 1024 with K = 128:
+// 67 MB of the 84 MB it moves), which a tile kernel does in one burst after its loads and products, two workgroups of a CU taking
+// turns at best: 30.3 us as 128x128 tiles, 27.7 as 256x256, 19.1 by this kernel (4.4 TB/s; a large copy runs at 5.25); with K = 64
+// 21.4 -> 15.6, 4 x 2048 x 2048 x 128 12.9 -> 11.8, 13 x 777 x 777 x 128 15.3 -> 12.9, 8192 x 4096 x 64 19.4 -> 15.7.
+// Here a wave keeps its 32 rows of A in registers and walks along the columns, 64 at a time: B's next tile is on its way into the
+// other LDS image and the last tile's stores are on their way out while this one is computed; two workgroups (128 rows each) share
+// a CU (with runs for three of them the first shape takes 24.7 us).  Stores and loads are counted together: what is older than the four stores of the tile before has landed.
+// ---------------------------------------------------------------------------------------------
+template <int NU>  // 64-deep units of K
+__global__ __launch_bounds__(256, 3) void gemm_shortk_kernel(TileArgs p) {
+  constexpr int BM = 128, BN = 64, TM = 2, TN = 4, NS = 2 * NU;
+  constexpr uint32_t UNIT = BN * 128, IMG = NU * UNIT;  // B: one K-major 64-deep image per unit
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(NEOGEMM_AS3 char*)smem;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // workgroup -> rows, run of column tiles (group_m of them)
+  const int parts = (p.ntn + p.group_m - 1) / p.group_m;
+  const int m0 = (int)(blockIdx.x / parts) * BM, first = (int)(blockIdx.x % parts) * p.group_m;
+  const int count = p.ntn - first < p.group_m ? p.ntn - first : p.group_m;
+  const char* gA = p.A + (size_t)blockIdx.z * p.bsa * 2;
+  const char* gB = p.B + (size_t)blockIdx.z * p.bsb * 2;
+  char* gC = p.C + (size_t)blockIdx.z * p.bsc * 2;
+
+  // fragments of A (see FragReader): rows past the end take the last row's place, what lies past K is zero
+  bf16x8 af[TM][NS];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int r = m0 + wave * 32 + i * 16 + (lane & 15), row = r < p.M ? r : p.M - 1;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int k = s * 32 + (lane >> 4) * 8;
+      i32x4 v = *(const i32x4*)(gA + ((size_t)row * p.lda + (k < p.K ? k : 0)) * 2);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = k < p.K ? v[e] : 0;
+      af[i][s] = __builtin_bit_cast(bf16x8, v);
+    }
+  }
+  // this wave's loads of a unit of B: two of 1 KiB, eight columns each (see Operand::init)
+  uint32_t vo[2], brow[2], bk[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    brow[j] = (wave * 2 + j) * 8 + (lane >> 3);
+    const uint32_t c = (lane & 7) ^ swz_k(brow[j]);
+    bk[j] = c * 8;
+    vo[j] = brow[j] * (uint32_t)p.ldb * 2 + c * 16 + VOFF_BIAS - j * 1024;
+  }
+  auto load_b = [&](int tile, uint32_t img) {
+    const int n0 = tile * BN;
+    static_for<NU>([&](auto uc) {
+      constexpr int u = decltype(uc)::value;
+      const uint64_t b = (uint64_t)gB + ((uint64_t)n0 * p.ldb + u * KTILE) * 2 - VOFF_BIAS;
+      const i32x4 rs = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), (int)0x80000000u, 0x00020000};
+      dma_set_m0(lds0 + img + u * UNIT + wave * 2048);
+      static_for<2>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const bool in = n0 + (int)brow[j] < p.N && u * KTILE + (int)bk[j] < p.K;
+        dma16<j * 1024>(rs, in ? vo[j] : OOB_OFFSET);
+      });
+    });
+  };
+  FragReader<BN, true, TN> fb;
+  fb.init(lds0, 0, lane);
+  const uint32_t region = lds0 + 2 * IMG + (uint32_t)wave * (32 * BN * 2);  // this wave's rows on their way to C
+  const bool whole_rows = m0 + BM <= p.M;
+  const int row_l = lane & 15;
+
+  load_b(first, 0);
+  // A's fragments are waited for here and not in the loop, where the compiler, which does not see B's loads, would wait for those as well
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(af[i][s]));
+  for (int t = 0; t < count; ++t) {
+    // B's tile has landed: all but the four stores behind it, which are that many only where no row is left out
+    if (t > 0 && whole_rows) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint32_t img = (t & 1) * IMG;
+    if (t + 1 < count) load_b(first + t + 1, IMG - img);
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const uint32_t b = fb.base(img + (s >> 1) * UNIT, s);
+      bf16x8 bf[TN];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bf[j] = fb.read_at(b, j);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i][s], acc[i][j], 0, 0, 0);
+    }
+    // through LDS into whole rows of 128 bytes, as in store_wave_tile
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        bf16x4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = (__bf16)(acc[i][j][r] * p.alpha);
+        const uint32_t row = i * 16 + row_l, c = 2 * j + (lane >> 5);
+        *((NEOGEMM_AS3 bf16x4*)(uintptr_t)(region + row * 128 + ((c ^ (row & 7)) << 4) + (((lane >> 4) & 1) << 3))) = o;
+      }
+    const int col = (first + t) * BN + (lane & 7) * 8;
+    const bool whole_cols = (first + t + 1) * BN <= p.N;  // (else the last tile of the run: nothing counts its stores)
+    auto staged = [&](int st) -> bf16x8 {
+      const uint32_t row = st * 8 + (lane >> 3);
+      return *((NEOGEMM_AS3 bf16x8*)(uintptr_t)(region + row * 128 + (((lane & 7) ^ (row & 7)) << 4)));
+    };
+    char* dst = gC + ((size_t)(m0 + wave * 32 + (lane >> 3)) * p.ldc + col) * 2;
+    if (whole_rows && whole_cols) {
+      bf16x8 v[4];
+#pragma unroll
+      for (int st = 0; st < 4; ++st) v[st] = staged(st);
+#pragma unroll
+      for (int st = 0; st < 4; ++st) __builtin_nontemporal_store((bf16x8_u)v[st], (bf16x8_u*)(dst + (size_t)st * 16 * p.ldc));
+    } else {
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const bf16x8 v = staged(st);
+        char* d = dst + (size_t)st * 16 * p.ldc;
+        if (m0 + wave * 32 + st * 8 + (lane >> 3) < p.M) {
+          if (col + 7 < p.N) {
+            __builtin_nontemporal_store((bf16x8_u)v, (bf16x8_u*)d);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (col + e < p.N) ((__bf16*)d)[e] = v[e];
+          }
+        }
+      }
+    }
+  }
+}
+
+hipError_t launch_shortk(TileArgs a, int run, hipStream_t st);
+#if NEOGEMM_HAS_PART(9)
+hipError_t launch_shortk(TileArgs a, int run, hipStream_t st) {
+  a.ntm = (a.M + 127) / 128;
+  a.ntn = (a.N + 63) / 64;
+  a.group_m = run;
+  const int nu = a.K > KTILE ? 2 : 1;
+  const size_t lds = (size_t)nu * 2 * 8192 + 16384;
+  auto go = [&](auto kern) -> hipError_t {
+    if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
+    kern<<<dim3(a.ntm * ((a.ntn + run - 1) / run), 1, a.batch), 256, lds, st>>>(a);
+    return hipGetLastError();
+  };
+  return nu == 2 ? go(gemm_shortk_kernel<2>) : go(gemm_shortk_kernel<1>);
+}
+#endif
+
 // The tile kernels are instantiated through launch_tile.  In a split build each part instantiates its share and
 // the others only declare it.
 #ifdef NEOGEMM_PART
@@ -3004,6 +3162,17 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   a.alpha = alpha;
   a.early_stores = 0;
   a.beta = beta;
+  if (variant == NEOGEMM_VARIANT_AUTO && ak && bk && K <= 2 * KTILE && beta == 0.f && a.ksplit == 1) {
+    // at least two column tiles for each of two workgroups per CU (16 x 512 x 512 x 96, one each: level with the tile kernels)
+    const int64_t tiles = (int64_t)ceil_div(a.M, 128) * ceil_div(a.N, 64) * bt.count, slots = 2 * (int64_t)planning_cus();
+    if (tiles >= 2 * slots) {
+      const int64_t per_row = ceil_div(slots, (int64_t)ceil_div(a.M, 128) * bt.count);  // workgroups that share a block of rows
+      const hipError_t e = launch_shortk(a, ceil_div(ceil_div(a.N, 64), per_row), st);
+      if (e == hipSuccess) return NEOGEMM_OK;
+      fprintf(stderr, "neogemm: short-K kernel launch failed: %s\n", hipGetErrorString(e));
+      return NEOGEMM_ERR_LAUNCH;
+    }
+  }
   if (prof && (bt.count > 1 || a.ksplit > 1 || vi.bm != 256 || vi.bn != 256 || !ak || v == NEOGEMM_VARIANT_C256x256_W4))
     return NEOGEMM_ERR_UNSUPPORTED;
   if (a.ksplit > 1) {

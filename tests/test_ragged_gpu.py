@@ -116,3 +116,23 @@ def test_copies_on_the_grid(b, M, N, K):
                                                     1.0, 1.0, sa, 0, M * N, b, ws.data_ptr(), size, st) == _abi.OK
                     got, add = (C, old) if c_layout == g.C_ROW else (C.transpose(1, 2), old.transpose(1, 2))
                     assert torch.equal(got, (want + add.float()).to(torch.bfloat16))
+
+
+# K of at most 128 with both operands K-major and enough tiles: one and two 64-deep units, whole and partial; rows and columns that end
+# inside a block, a run of column tiles per workgroup that does not divide them, C at odd addresses, alpha
+@pytest.mark.parametrize("b,M,N,K", [(32, 1024, 1024, 128), (40, 517, 801, 96), (1, 4100, 3001, 64), (7, 2048, 1000, 8), (300, 129, 129, 72), (1, 130, 60000, 104),
+                                     (1, 60000, 70, 120)])
+@pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
+def test_short_k(b, M, N, K, c_layout):
+    gen = torch.Generator(device="cuda").manual_seed(b + M + N + K)
+
+    def ints(*shape):
+        return torch.randint(-2, 3, shape, generator=gen, device="cuda").to(torch.bfloat16)
+
+    A, B = ints(b, M, K + 8), ints(b, N, K)
+    want = 0.5 * (A[:, :, :K].float() @ B.transpose(1, 2).float())
+    A[:, :, K:] = float("nan")
+    C = torch.full((b, M, N) if c_layout == g.C_ROW else (b, N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert _abi.load().neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, K + 8, K, C.stride(1), g.A_MK, g.B_NK, c_layout, 0.5, 0.0,
+                                            M * (K + 8), N * K, M * N, b, None, 0, torch.cuda.current_stream().cuda_stream or None) == _abi.OK
+    assert torch.equal(C if c_layout == g.C_ROW else C.transpose(1, 2), want.to(torch.bfloat16))
