@@ -27,7 +27,7 @@
 // Split build: compiling this one file takes minutes because of the many instances of the tile kernel, so setup.py
 // compiles it NEOGEMM_PARTS times in parallel with -DNEOGEMM_PART=0..NEOGEMM_PARTS-1 and links the objects.  Part 0
 // holds everything but the tile kernels; part k > 0 instantiates its share of launch_tile<> (listed behind
-// launch_tile) or, the last two, launch_chain and launch_ragged, and nothing else.  Without NEOGEMM_PART the file is one self-contained translation unit.
+// launch_tile) or, the last two, launch_chain and the launches of the other kernels that have many instances, and nothing else.  Without NEOGEMM_PART the file is one self-contained translation unit.
 #ifdef NEOGEMM_PART
 #define NEOGEMM_HAS_PART(p) (NEOGEMM_PART == (p))
 #else
@@ -1573,6 +1573,119 @@ hipError_t launch_shortk(TileArgs a, int run, hipStream_t st) {
     return hipGetLastError();
   };
   return nu == 2 ? go(gemm_shortk_kernel<2>) : go(gemm_shortk_kernel<1>);
+}
+#endif
+
+// ---------------------------------------------------------------------------------------------
+// Small problems: a 64x64 tile of operands in either order.  What counts is the way to the first product and from the last one to C,
+// and how many CUs take part: gemm_tile_kernel takes B [K,N] in tiles of 128 columns at least, asks for three K tiles of each operand
+// before the first product, and leaves its main loop up to six K tiles before the end, to wait for every one of those with nothing
+// behind it.  704^3 with B [K,N] 10.4 -> 6.0 us, with B [N,K] 7.8 -> 5.6; 1024^3 10.3 -> 7.6 and 7.8 -> 7.0; 512^3 with B [K,N] 5.6 ->
+// 5.2; 512 x 512 x 2048 in four splits 10.4 -> 9.3; 400 x 744 x 904 12.0 -> 7.7.  Two stages are on the way while one is computed;
+// four or seven only make the start longer (1024^3 with B [N,K]: 7.0, 7.2 and 7.9 us).
+// R stages of 16 KiB (a 64-deep K tile of A and of B each, K-major or 64 k-rows of 64 columns, swizzled as in FragReader), one barrier
+// per stage: behind it stage t has landed and everyone is past stage t - 1, whose place takes stage t + R - 1.
+// ---------------------------------------------------------------------------------------------
+template <bool AK, bool BK>
+__global__ __launch_bounds__(256) void gemm_small_kernel(TileArgs p) {
+  constexpr int R = 3, BM = 64, BN = 64, NW = 4, TM = 2, TN = 2;
+  constexpr uint32_t HALF = 8192, STAGE = 2 * HALF, LDS_BYTES = R * STAGE;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(NEOGEMM_AS3 char*)smem;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  int m0, n0, kz;
+  tile_of_workgroup<BM, BN>(p, m0, n0, kz);
+  const int k_begin = kz * p.ktiles_per_split * KTILE;
+  int k_end = k_begin + p.ktiles_per_split * KTILE;
+  if (k_end > p.K) k_end = p.K;
+  const int klen = k_end - k_begin, nst = (klen + KTILE - 1) / KTILE;
+
+  // this wave's loads of a stage: two of 1 KiB per operand, eight rows or k-rows each (see Operand::init); `key`: depth of the chunk
+  uint32_t voa[2], vob[2];
+  int keya[2], keyb[2];
+  auto offsets = [&](auto kmaj, uint32_t (&vo)[2], int (&key)[2], long ld, int rows_left) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t r = (wave * 2 + j) * 8 + (lane >> 3);
+      constexpr bool KM = decltype(kmaj)::value;
+      const uint32_t c = (lane & 7) ^ (KM ? swz_k(r) : swz_mn64(r & 31));
+      vo[j] = r * (uint32_t)ld * 2 + c * 16 + VOFF_BIAS - j * 1024;
+      if ((KM ? (int)r : (int)c * 8) >= rows_left) vo[j] = OOB_OFFSET;
+      key[j] = KM ? (int)c * 8 : (int)r;
+    }
+  };
+  offsets(std::integral_constant<bool, AK>{}, voa, keya, p.lda, p.M - m0);
+  offsets(std::integral_constant<bool, BK>{}, vob, keyb, p.ldb, p.N - n0);
+  const uint64_t baseA = (uint64_t)p.A + ((uint64_t)blockIdx.z * p.bsa + (AK ? (uint64_t)m0 * p.lda + k_begin : (uint64_t)k_begin * p.lda + m0)) * 2 - VOFF_BIAS;
+  const uint64_t baseB = (uint64_t)p.B + ((uint64_t)blockIdx.z * p.bsb + (BK ? (uint64_t)n0 * p.ldb + k_begin : (uint64_t)k_begin * p.ldb + n0)) * 2 - VOFF_BIAS;
+  const uint64_t advA = (AK ? (uint64_t)KTILE : (uint64_t)KTILE * p.lda) * 2, advB = (BK ? (uint64_t)KTILE : (uint64_t)KTILE * p.ldb) * 2;
+  auto issue = [&](int t, uint32_t slot) {
+    const int krem = klen - t * KTILE;
+    auto load = [&](uint64_t b, const uint32_t (&vo)[2], const int (&key)[2], uint32_t dst) {
+      const i32x4 rs = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), (int)0x80000000u, 0x00020000};
+      dma_set_m0(dst + wave * 2048);
+      static_for<2>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        dma16<j * 1024>(rs, key[j] < krem ? vo[j] : OOB_OFFSET);
+      });
+    };
+    load(baseA + (uint64_t)t * advA, voa, keya, lds0 + slot * STAGE);
+    load(baseB + (uint64_t)t * advB, vob, keyb, lds0 + slot * STAGE + HALF);
+  };
+  FragReader<BM, AK, TM> fa;
+  FragReader<BN, BK, TN> fb;
+  fa.init(lds0, wm * 32, lane);
+  fb.init(lds0 + HALF, wn * 32, lane);
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  for (int t = 0; t < R - 1 && t < nst; ++t) issue(t, t);
+  uint32_t slot = 0, slot_ld = R - 1;
+  for (int t = 0; t < nst; ++t) {
+    if (t + 1 < nst) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");  // all but the stage behind it
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of stage t - 1 have returned
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + R - 1 < nst) issue(t + R - 1, slot_ld);
+    const uint32_t img = slot * STAGE;
+    bf16x8 a[2][TM], b[2][TN];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[s][i] = fa.read(img + (AK ? 0 : s * 4096), i, s);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[s][j] = fb.read(img + (BK ? 0 : s * 4096), j, s);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][j], a[s][i], acc[i][j], 0, 0, 0);
+    slot = slot + 1 == R ? 0 : slot + 1;
+    slot_ld = slot_ld + 1 == R ? 0 : slot_ld + 1;
+  }
+  store_wave_tile<TM, TN, NW, LDS_BYTES, TM, false>(acc, p, p.C + (size_t)blockIdx.z * p.bsc * 2, kz, lane, wave, lds0, BlockMap{m0 + wm * 32, n0 + wn * 32});
+}
+
+hipError_t launch_small(const TileArgs& a, bool ak, bool bk, hipStream_t st);
+#if NEOGEMM_HAS_PART(9)
+hipError_t launch_small(const TileArgs& a, bool ak, bool bk, hipStream_t st) {
+  const size_t lds = 3 * 16384;
+  dim3 grid(a.ntm * a.ntn * a.ksplit, 1, a.batch), block(256);
+  auto go = [&](auto kern) -> hipError_t {
+    if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
+    kern<<<grid, block, lds, st>>>(a);
+    return hipGetLastError();
+  };
+  if (ak) return bk ? go(gemm_small_kernel<true, true>) : go(gemm_small_kernel<true, false>);
+  return bk ? go(gemm_small_kernel<false, true>) : go(gemm_small_kernel<false, false>);
 }
 #endif
 
@@ -3141,7 +3254,20 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   // (the chained 256x256 kernel takes its rows from a K-major operand only, K in whole periods of 128 and no split)
   const bool fits = (ak || mn_ok(vi.bm, a.M)) && (bk || mn_ok(vi.bn, a.N)) &&
                     (v != NEOGEMM_VARIANT_C256x256_W4 || (ak && K % (2 * KTILE) == 0 && s <= 1));
-  if (!fits) {
+  // Where the plan says 64 rows per tile, gemm_small_kernel takes over, in either order of the operands (an MN-major one on the
+  // rows went to the 128x128 tile: 512^3 with a transposed A 6.8 us, 5.1 now), as long as the 64x64 tiles fit the CUs one and a half
+  // times (B [N,K]: 1152^3, 324 of them, 10.6 -> 9.0 us, 1280^3, 400, level, 1024 x 2048 x 1536, 512, 11.8 and 12.4) or twice
+  // (B [K,N]: 13.7 and 12.5 for that last one).  Few workgroups with whole trips of the tile kernel's main loop stay there: 256 x 1024 x
+  // 1024, 64 of them, 5.9 us and 6.7 with B [N,K], 7.1 and 7.3 with B [K,N]; 200 x 1000 x 1000 with B [K,N] 9.3 and 7.6.
+  bool small = false;
+  if (variant == NEOGEMM_VARIANT_AUTO && (v == NEOGEMM_VARIANT_T64x64_W4 || v == NEOGEMM_VARIANT_T64x128_W4) &&
+      (ak || (a.M & 7) == 0 || bt.padded) && (bk || (a.N & 7) == 0 || bt.padded)) {
+    const int64_t cus = planning_cus(), wgs = (int64_t)ceil_div(a.M, 64) * ceil_div(a.N, 64) * s * bt.count;
+    const int kt = ceil_div(K, KTILE);
+    if (ak && bk) small = 2 * wgs <= 3 * cus && !(wgs <= 64 && s == 1 && kt >= 8 && kt % 4 == 0);
+    else small = wgs <= 2 * cus && !(fits && wgs <= 64 && s == 1 && K >= 1024 && K % 256 == 0);
+  }
+  if (!fits && !small) {
     if (variant != NEOGEMM_VARIANT_AUTO) return NEOGEMM_ERR_UNSUPPORTED;
     // the planned tile is too wide for an MN-major operand: the 128x128 tile needs the least
     if (v == NEOGEMM_VARIANT_T128x128_W4) return unaligned();
@@ -3149,9 +3275,10 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                       NEOGEMM_VARIANT_T128x128_W4, s, 0, nullptr, alpha, beta, bt);
     return r == NEOGEMM_ERR_UNSUPPORTED ? unaligned() : r;
   }
-  a.ntm = ceil_div(a.M, vi.bm);
-  a.ntn = ceil_div(a.N, vi.bn);
-  a.group_m = group_m > 0 ? group_m : 8;
+  a.ntm = ceil_div(a.M, small ? 64 : vi.bm);
+  a.ntn = ceil_div(a.N, small ? 64 : vi.bn);
+  // (the few 64x64 tiles: an XCD's share of eight lies closer to a square, 512 x 512 x 1024 7.5 -> 5.9 us, 1024 x 200 x 1024 8.1 -> 6.4)
+  a.group_m = group_m > 0 ? group_m : v == NEOGEMM_VARIANT_T64x64_W4 && (int64_t)a.ntm * a.ntn * s <= 64 ? 2 : 8;
   const int ktiles = ceil_div(K, KTILE);
   if (s > ktiles) s = ktiles;
   a.ktiles_per_split = ceil_div(ktiles, s);
@@ -3183,7 +3310,8 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   }
 
   hipError_t e;
-  switch (v) {
+  if (small) e = launch_small(a, ak, bk, st);
+  else switch (v) {
     case NEOGEMM_VARIANT_T256x256_W4: e = launch_tile<256, 256, 2, 2>(a, ak, bk, st); break;
     case NEOGEMM_VARIANT_T128x128_W4: e = launch_tile<128, 128, 2, 2>(a, ak, bk, st); break;
     case NEOGEMM_VARIANT_T256x128_W4: e = launch_tile<256, 128, 2, 2>(a, ak, bk, st); break;

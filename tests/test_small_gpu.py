@@ -1,0 +1,33 @@
+"""Small problems (gemm_small_kernel): small integers, so that every order of summation gives the same bits."""
+import pytest
+import torch
+
+import gemm_amd as g
+
+pytestmark = pytest.mark.gpu
+
+
+# K: part of a stage, one, two, three (the ring's depth), four, a partial last one, split; M, N: edges of the 64 tile, one column of chunks,
+# up to the most workgroups that the rule sends here
+@pytest.mark.parametrize("M,N,K", [(136, 136, 8), (136, 8, 64), (264, 200, 72), (328, 448, 128), (448, 448, 184), (192, 520, 256), (640, 640, 640), (1024, 1024, 1024),
+                                   (1152, 1152, 320), (1024, 2048, 264), (264, 264, 4104), (256, 256, 8192), (256, 1024, 1024)])
+@pytest.mark.parametrize("a_layout", [g.A_MK, g.A_KM])
+@pytest.mark.parametrize("b_layout", [g.B_KN, g.B_NK])
+@pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
+def test_small(M, N, K, a_layout, b_layout, c_layout):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+
+    def ints(rows, cols, pad):   # NaN between the rows
+        m = torch.full((rows, cols + pad), float("nan"), dtype=torch.bfloat16, device="cuda")
+        m[:, :cols] = torch.randint(-2, 3, (rows, cols), generator=gen, device="cuda")
+        return m[:, :cols]
+
+    A, B = ints(*((M, K) if a_layout == g.A_MK else (K, M)), 8), ints(*((K, N) if b_layout == g.B_KN else (N, K)), 16)
+    want = (A if a_layout == g.A_MK else A.t()).float() @ (B if b_layout == g.B_KN else B.t()).float()
+    C = torch.full((M, N) if c_layout == g.C_ROW else (N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
+    got = C if c_layout == g.C_ROW else C.t()
+    g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout)
+    assert torch.equal(got, want.to(torch.bfloat16))
+    old = got.clone()
+    g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout, alpha=0.5, beta=-1.0)
+    assert torch.equal(got, (0.5 * want - old.float()).to(torch.bfloat16))
