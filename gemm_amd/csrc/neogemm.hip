@@ -1397,10 +1397,9 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(TileArgs p) {
 hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int bm, int bn, hipStream_t st);
 #if NEOGEMM_HAS_PART(9)
 hipError_t launch_ragged(const TileArgs& a, bool ak, bool bk, int bm, int bn, hipStream_t st) {
-  const size_t lds = (size_t)(bm + bn) * 256;
+  const size_t lds = (size_t)(bm + bn) * 256;  // 64 KiB at most: no limit to raise, and so nothing that a capturing stream would mind
   dim3 grid(a.ntm * a.ntn * a.ksplit, 1, a.batch), block(256);
   auto go = [&](auto kern) -> hipError_t {
-    if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
     kern<<<grid, block, lds, st>>>(a);
     return hipGetLastError();
   };
@@ -1568,7 +1567,6 @@ hipError_t launch_shortk(TileArgs a, int run, hipStream_t st) {
   const int nu = a.K > KTILE ? 2 : 1;
   const size_t lds = (size_t)nu * 2 * 8192 + 16384;
   auto go = [&](auto kern) -> hipError_t {
-    if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
     kern<<<dim3(a.ntm * ((a.ntn + run - 1) / run), 1, a.batch), 256, lds, st>>>(a);
     return hipGetLastError();
   };
@@ -1680,7 +1678,6 @@ hipError_t launch_small(const TileArgs& a, bool ak, bool bk, hipStream_t st) {
   const size_t lds = 3 * 16384;
   dim3 grid(a.ntm * a.ntn * a.ksplit, 1, a.batch), block(256);
   auto go = [&](auto kern) -> hipError_t {
-    if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
     kern<<<grid, block, lds, st>>>(a);
     return hipGetLastError();
   };
