@@ -2958,7 +2958,7 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
   if (p.a) p.bytes_a = up((size_t)rows_a * p.ldpa * 2 * (bt.sa ? bt.count : 1));
   if (p.b) p.bytes_b = up((size_t)rows_b * p.ldpb * 2 * (bt.sb ? bt.count : 1));
-  const size_t most = (size_t)1 << 30;  // of memory that a caller's workspace would keep for it
+  const size_t most = (size_t)1 << 28;  // bytes that a workspace would keep for it: two operands of 8191 x 8191
   if (p.bytes_a + p.bytes_b > most) return false;
   struct Memo {
     int64_t M = -1, N = -1, K = -1, count = -1;

@@ -12,7 +12,7 @@
 //  * the launch goes to torch's current stream, not the legacy default stream (nemgemmV03.cu:383);
 //  * no state tied to a tensor is cached between calls (the reference caches TMA descriptors keyed on shape
 //    only, nemgemmV03.cu:27-30,359-371, which goes stale when another tensor of the same shape is passed); the
-//    only state kept is a split-K scratch buffer per (device, stream).
+//    only state kept is a scratch buffer per (device, stream), for split-K partials and copies onto the 16-byte grid.
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/extension.h>
@@ -35,7 +35,7 @@ void check_operand(const torch::Tensor& t, const char* name) {
 bool row_major(const torch::Tensor& t) { return t.size(1) <= 1 || t.stride(1) == 1; }
 int64_t row_ld(const torch::Tensor& t) { return t.size(0) <= 1 ? std::max<int64_t>(t.size(1), 1) : t.stride(0); }
 
-// Split-K scratch, one buffer per (device, stream): two GEMMs on two streams of one device must not share their
+// Scratch of a call (split-K partials, copies of operands), one buffer per (device, stream): two GEMMs on two streams of one device must not share their
 // partials, and a buffer is only ever used on the stream that was current when the caching allocator handed it out,
 // which is the stream whose order the allocator follows when the block is reused.  So dropping a buffer that has
 // become too small is safe: its block goes back to that stream's pool and is handed out again only to work queued

@@ -45,7 +45,7 @@ extern "C" {
 
 /* Kernel variants for neogemm_bf16_variant(); 0 lets the library choose. */
 #define NEOGEMM_VARIANT_AUTO 0
-#define NEOGEMM_VARIANT_GENERIC 1   /* scalar-load fallback: any shape, stride, alignment */
+#define NEOGEMM_VARIANT_GENERIC 1   /* scalar loads: any shape, stride, alignment; what neogemm_bf16 runs where no MFMA kernel fits */
 /* Tile variants: BM x BN macro-tile per workgroup, K in steps of 64, 16x16x32 MFMA; (r x c) = wave grid. */
 #define NEOGEMM_VARIANT_RETIRED_2 2   /* was 256x256 with 8 wave64: never the fastest on any shape; calls naming it are refused */
 #define NEOGEMM_VARIANT_T256x256_W4 3 /* 256x256, 4 wave64 (2x2): the default for large shapes */
@@ -99,7 +99,7 @@ extern "C" {
  *              that function returns 0 for the shape.  Only split-K paths use it (fp32 partials).
  *
  * Unlike the reference (M,N,K % 64 == 0, nemgemmV03.cu:375) every M,N,K >= 0 is accepted; shapes or
- * pointers that the MFMA path cannot take (K % 8, ld % 8, 16-byte alignment) run the generic kernel.
+ * pointers off the 16-byte grid (K % 8, ld % 8, alignment) run an MFMA kernel that takes any two-byte address.
  * M == 0 or N == 0 is a no-op; K == 0 writes zeros.
  */
 int neogemm_bf16(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
@@ -191,7 +191,9 @@ int neogemm_bf16_variant(const void* A, const void* B, void* C, int64_t M, int64
 
 /*
  * What neogemm_bf16 would pick for this call: writes the variant id and split-K factor.  Host only.
- * `aligned` is nonzero when pointers and leading dimensions satisfy the MFMA path (16-byte / 8-element).
+ * `aligned` is nonzero when pointers and leading dimensions satisfy the MFMA path (16-byte / 8-element); without it the answer is
+ * NEOGEMM_VARIANT_GENERIC, which stands for every kernel outside the plan (operands at any address among them).  Where the answer has
+ * 64 rows per tile, or K is at most 128, a call may run a kernel of its own for small problems or short K instead, in the same order of sums.
  * The choice comes from a cost model over the tile variants; if the environment variable
  * NEOGEMM_PLAN_TABLE names a JSON file of tuned choices (an array of objects with the integer fields
  * "M","N","K","b_layout","c_layout","variant","split_k"; the layouts default to 0; gemm_amd/tune.py writes one), an
