@@ -81,9 +81,17 @@ def gemm_into(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, variant=None,
         raise NeoGemmError(st, f"M={M} N={N} K={K} b_layout={b_layout} c_layout={c_layout} variant={variant}")
 
 
-def _describe(A, B, transposed_a=True):
+def _overlap(a, b):
+    """Whether the bytes from the first to the last element of a strided tensor meet those of another one."""
+    def end(t):
+        return t.data_ptr() + (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride()))) * t.element_size()
+    return a.numel() > 0 and b.numel() > 0 and a.data_ptr() < end(b) and b.data_ptr() < end(a)
+
+
+def _describe(A, B, transposed_a=True, out=None):
     """How A [M,K] and B [K,N] lie in memory: (A, B, lda, ldb, a_layout, b_layout); what no layout describes is made
-    contiguous.  A transposed A is read in place, but for the few rows of the decode kernels, which want them K-contiguous."""
+    contiguous.  A transposed A is read in place, but for the few rows of the decode kernels, which want them K-contiguous,
+    and for one whose memory `out`, which is written meanwhile, shares (C = C.t() @ X + C)."""
     M, K = A.shape
     N = B.shape[1]
     if B.stride(1) == 1 or N <= 1:
@@ -96,7 +104,7 @@ def _describe(A, B, transposed_a=True):
     if A.stride(1) == 1 or K <= 1:
         return A, B, (A.stride(0) if M > 1 else max(K, 1)), ldb, A_MK, b_layout
     decode = M <= 128 and K % 8 == 0 and ldb % 8 == 0 and B.data_ptr() % 16 == 0 and (b_layout == B_NK or N % 8 == 0)
-    if transposed_a and A.stride(0) == 1 and A.stride(1) >= M and not decode:
+    if transposed_a and A.stride(0) == 1 and A.stride(1) >= M and not decode and not (out is not None and _overlap(A, out)):
         return A, B, A.stride(1), ldb, A_KM, b_layout
     return A.contiguous(), B, max(K, 1), ldb, A_MK, b_layout
 
@@ -149,7 +157,7 @@ def gemm_scaled(A, B, C, alpha=1.0, beta=0.0):
         raise ValueError(f"shapes: A {tuple(A.shape)}, B {tuple(B.shape)}, C {tuple(C.shape)} (contiguous [M,N])")
     M, K = A.shape
     N = B.shape[1]
-    A, B, lda, ldb, a_layout, b_layout = _describe(A, B)
+    A, B, lda, ldb, a_layout, b_layout = _describe(A, B, out=C)
     if M and N:
         gemm_into(A, B, C, M, N, K, lda, ldb, max(N, 1), b_layout, C_ROW, alpha=float(alpha), beta=float(beta),
                   a_layout=a_layout)

@@ -96,7 +96,17 @@ struct Operands {
   int a_layout = NEOGEMM_A_MK, b_layout = NEOGEMM_B_KN;
   int64_t lda, ldb;
 };
-Operands describe(torch::Tensor A, torch::Tensor B) {
+// Whether the bytes from the first to the last element of a strided tensor meet those of another one.
+bool overlap(const torch::Tensor& a, const torch::Tensor& b) {
+  auto end = [](const torch::Tensor& t) {
+    int64_t n = 1;
+    for (int64_t d = 0; d < t.dim(); ++d) n += (t.size(d) - 1) * t.stride(d);
+    return (uintptr_t)t.data_ptr() + n * t.element_size();
+  };
+  return a.numel() > 0 && b.numel() > 0 && (uintptr_t)a.data_ptr() < end(b) && (uintptr_t)b.data_ptr() < end(a);
+}
+// out: the tensor that is written while A and B are read (none: a new one).
+Operands describe(torch::Tensor A, torch::Tensor B, const torch::Tensor* out = nullptr) {
   Operands o;
   if (row_major(B)) {
     o.ldb = row_ld(B);
@@ -109,14 +119,15 @@ Operands describe(torch::Tensor A, torch::Tensor B) {
   }
   // A = X.t() with X [K,M] row-major, as in a weight gradient dY.t() * X, is read in place: by the tile kernels where it comes in
   // whole 16-byte chunks (a copy took 68 us for 4096 x 4096 where the product itself takes 98), by the kernel for operands at any
-  // address where not.  A copy is made for the decode kernels, which want K-contiguous rows and few of them.
+  // address where not.  A copy is made for the decode kernels, which want K-contiguous rows and few of them, and where C lies in A's
+  // own memory (C = C.t() * X + C): a tile is read by workgroups that run after the one which has stored it.
   auto chunks = [](const torch::Tensor& t, int64_t ld) { return ((uintptr_t)t.data_ptr() & 15) == 0 && ld % 8 == 0; };
   const int64_t M = A.size(0), N = B.size(1), K = A.size(1);
   o.lda = row_ld(A);
   if (!row_major(A)) {
     const bool b_whole = chunks(B, o.ldb) && (o.b_layout == NEOGEMM_B_NK || N % 8 == 0);
     const bool decode = M <= 128 && K % 8 == 0 && b_whole;
-    if (A.stride(0) == 1 && A.stride(1) >= M && !decode) {
+    if (A.stride(0) == 1 && A.stride(1) >= M && !decode && !(out && overlap(A, *out))) {
       o.a_layout = NEOGEMM_A_KM;
       o.lda = A.stride(1);
     } else {
@@ -155,7 +166,7 @@ void gemm_scaled(torch::Tensor A, torch::Tensor B, torch::Tensor C, double alpha
   TORCH_CHECK(C.size(0) == A.size(0) && C.size(1) == B.size(1) && C.is_contiguous(), "C must be a contiguous [M,N]");
   const int64_t M = A.size(0), K = A.size(1), N = B.size(1);
   if (M == 0 || N == 0) return;
-  const Operands o = describe(std::move(A), std::move(B));
+  const Operands o = describe(std::move(A), std::move(B), &C);
   run(o.A, o.B, C, M, N, K, o.lda, o.ldb, std::max<int64_t>(N, 1), o.a_layout, o.b_layout, NEOGEMM_C_ROW, (float)alpha, (float)beta);
 }
 

@@ -47,3 +47,18 @@ def test_missing_library_is_an_error(monkeypatch):
 def test_error_class_carries_status():
     e = gemm_amd.NeoGemmError(-3, "shape")
     assert e.status == -3 and "variant" in str(e)
+
+
+def test_a_transposed_view_of_the_output_is_copied():
+    """gemm_scaled(C.t(), X, C): A is read while C is written, so a view of C's memory must not be read in place."""
+    C, X = torch.zeros(256, 256, dtype=torch.bfloat16), torch.zeros(256, 256, dtype=torch.bfloat16)
+    A, _, lda, _, a_layout, _ = gemm_amd._describe(C.t(), X, out=C)
+    assert a_layout == gemm_amd.A_MK and lda == 256 and A.data_ptr() != C.data_ptr()
+    # part of it shared: rows 100 .. 355 of a buffer whose rows 0 .. 255 are C
+    buf = torch.zeros(356, 256, dtype=torch.bfloat16)
+    A, _, _, _, a_layout, _ = gemm_amd._describe(buf[100:].t(), X, out=buf[:256])
+    assert a_layout == gemm_amd.A_MK and not gemm_amd._overlap(A, buf)
+    # neighbours share nothing and are read in place
+    both = torch.zeros(512, 256, dtype=torch.bfloat16)
+    A, _, lda, _, a_layout, _ = gemm_amd._describe(both[:256].t(), X, out=both[256:])
+    assert a_layout == gemm_amd.A_KM and A.data_ptr() == both.data_ptr()

@@ -66,3 +66,14 @@ def test_wrappers_on_transposed_views(mod):
     flat = small_ints(gen, 200 * 256 + 1)
     A, B = flat[1:].view(200, 256), small_ints(gen, 200, 256)
     assert torch.equal(mod.gemm(A.t(), B), (A.t().float() @ B.float()).to(torch.bfloat16))
+
+
+# several rounds of tiles, the kernels for operands at any address (odd n), copies of them on the 16-byte grid
+@pytest.mark.parametrize("n", [264, 515, 2501, 6144])
+@pytest.mark.parametrize("mod", [g, neoGEMM])
+def test_output_in_the_memory_of_a_transposed_a(mod, n):
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    C, X = small_ints(gen, n, n), small_ints(gen, n, n)
+    want = (C.t().float() @ X.float() + C.float()).to(torch.bfloat16)
+    mod.gemm_scaled(C.t(), X, C, 1.0, 1.0)
+    assert torch.equal(C, want)
