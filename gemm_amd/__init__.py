@@ -20,6 +20,7 @@ __all__ = ["gemm", "neoGemmV1", "neogemm", "gemm_into", "plan", "workspace_bytes
 
 _workspaces = {}        # (device index, stream) -> buffer, in order of last use
 _MAX_WORKSPACES = 16    # streams come and go: the least recently used buffer is dropped beyond this many
+_MAX_KEPT = 64 << 20    # bytes of one kept buffer
 
 
 def _check(t, name):
@@ -37,8 +38,12 @@ def _workspace(device, nbytes):
     """Split-K scratch for torch's current stream on `device`: one buffer per (device, stream), so that GEMMs on
     different streams never share partials.  A buffer is allocated while its stream is current and used on that
     stream only, so when a larger one replaces it, or it is dropped as the least recently used of too many, the
-    caching allocator reuses the block in that stream's order."""
+    caching allocator reuses the block in that stream's order.  A call that is captured into a graph gets a block of its own, from
+    the graph's own memory (a kept buffer that is outgrown later would be freed under the address that the graph replays), and
+    so does one that needs more than _MAX_KEPT; the caller holds it until the call is queued."""
     with torch.cuda.device(device):
+        if nbytes > _MAX_KEPT or torch.cuda.is_current_stream_capturing():
+            return torch.empty(nbytes, dtype=torch.uint8, device=device)
         key = (device.index if device.index is not None else torch.cuda.current_device(),
                torch.cuda.current_stream().cuda_stream)
         ws = _workspaces.pop(key, None)
@@ -57,7 +62,8 @@ def gemm_into(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, variant=None,
     if variant is None:
         lib = _abi.load()
         need = int(lib.neogemm_bf16_call_workspace_bytes(A.data_ptr(), B.data_ptr(), M, N, K, lda, ldb, a_layout, b_layout, c_layout, 0, 0, 1))
-        ws_ptr = _workspace(C.device, need).data_ptr() if need else 0
+        ws = _workspace(C.device, need) if need else None
+        ws_ptr = ws.data_ptr() if need else 0
         with torch.cuda.device(C.device):
             stream = torch.cuda.current_stream().cuda_stream
             st = lib.neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, a_layout, b_layout,
@@ -70,9 +76,8 @@ def gemm_into(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, variant=None,
     need = workspace_bytes(M, N, K)
     if variant is not None and split_k > 1:
         need = max(need, split_k * M * N * 4)
-    ws_ptr = 0
-    if need:
-        ws_ptr = _workspace(C.device, need).data_ptr()
+    ws = _workspace(C.device, need) if need else None
+    ws_ptr = ws.data_ptr() if need else 0
     with torch.cuda.device(C.device):
         stream = torch.cuda.current_stream().cuda_stream
         st = _abi.gemm_raw(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, b_layout, c_layout,
@@ -179,7 +184,8 @@ def gemm_batched(A, B):
         return C
     lib = _abi.load()
     need = int(lib.neogemm_bf16_batched_workspace_bytes(M, N, K, batch))
-    ws_ptr = _workspace(C.device, need).data_ptr() if need else 0
+    ws = _workspace(C.device, need) if need else None
+    ws_ptr = ws.data_ptr() if need else 0
     with torch.cuda.device(C.device):
         stream = torch.cuda.current_stream().cuda_stream
         st = lib.neogemm_bf16_batched(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, max(K, 1), max(N, 1), max(N, 1),

@@ -12,9 +12,10 @@
 //  * the launch goes to torch's current stream, not the legacy default stream (nemgemmV03.cu:383);
 //  * no state tied to a tensor is cached between calls (the reference caches TMA descriptors keyed on shape
 //    only, nemgemmV03.cu:27-30,359-371, which goes stale when another tensor of the same shape is passed); the
-//    only state kept is a scratch buffer per (device, stream), for split-K partials and copies onto the 16-byte grid.
+//    only state kept is a scratch buffer of at most 64 MiB per (device, stream), for split-K partials and copies onto the 16-byte grid.
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <torch/extension.h>
 
 #include <map>
@@ -35,11 +36,15 @@ void check_operand(const torch::Tensor& t, const char* name) {
 bool row_major(const torch::Tensor& t) { return t.size(1) <= 1 || t.stride(1) == 1; }
 int64_t row_ld(const torch::Tensor& t) { return t.size(0) <= 1 ? std::max<int64_t>(t.size(1), 1) : t.stride(0); }
 
-// Scratch of a call (split-K partials, copies of operands), one buffer per (device, stream): two GEMMs on two streams of one device must not share their
-// partials, and a buffer is only ever used on the stream that was current when the caching allocator handed it out,
+// Scratch of a call (split-K partials, copies of operands), one buffer per (device, stream): two GEMMs on two streams of one device
+// must not share their partials, and a buffer is only ever used on the stream that was current when the caching allocator handed it out,
 // which is the stream whose order the allocator follows when the block is reused.  So dropping a buffer that has
 // become too small is safe: its block goes back to that stream's pool and is handed out again only to work queued
 // on that same stream, behind the kernels that still use it.  The cache is per host thread.
+// Two kinds of call take a block of their own from the caching allocator instead, and give it back when they return:
+//  * one that is captured into a graph: the block comes from the graph's own memory then and stays valid for as long as the graph,
+//    while a kept buffer that is outgrown later would be freed under the address that the graph replays;
+//  * one that needs more than kMaxKept: it runs long enough not to notice, and nothing of that size stays behind it.
 struct WorkspaceKey {
   int device;
   hipStream_t stream;
@@ -48,11 +53,15 @@ struct WorkspaceKey {
 // At most kMaxWorkspaces buffers are kept: streams come and go, and a buffer whose stream is gone would otherwise stay
 // for the life of the thread.  The least recently used one is dropped (safe for the reason above).
 constexpr size_t kMaxWorkspaces = 16;
+constexpr size_t kMaxKept = (size_t)64 << 20;
 struct WorkspaceSlot {
   torch::Tensor buffer;
   uint64_t last_use = 0;
 };
-torch::Tensor& workspace_for(const torch::Tensor& like, hipStream_t stream, size_t bytes) {
+torch::Tensor workspace_for(const torch::Tensor& like, hipStream_t stream, size_t bytes) {
+  const auto options = like.options().dtype(torch::kUInt8);
+  if (bytes > kMaxKept || c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+    return torch::empty({(int64_t)bytes}, options);
   static thread_local std::map<WorkspaceKey, WorkspaceSlot> ws;
   static thread_local uint64_t clock = 0;
   const WorkspaceKey key{(int)like.get_device(), stream};
@@ -67,7 +76,7 @@ torch::Tensor& workspace_for(const torch::Tensor& like, hipStream_t stream, size
   torch::Tensor& t = slot.buffer;
   if (!t.defined() || (size_t)t.numel() < bytes) {
     t = torch::Tensor();  // give the old block back first
-    t = torch::empty({(int64_t)bytes}, like.options().dtype(torch::kUInt8));
+    t = torch::empty({(int64_t)bytes}, options);
   }
   return t;
 }
@@ -84,7 +93,8 @@ void run(const torch::Tensor& A, const torch::Tensor& B, torch::Tensor& C, int64
   const size_t need = neogemm_bf16_call_workspace_bytes(A.data_ptr(), B.data_ptr(), M, N, K, lda, ldb, a_layout, b_layout, c_layout, bt.sa,
                                                         bt.sb, bt.count);
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A.get_device()).stream();
-  void* ws = need ? workspace_for(A, stream, need).data_ptr() : nullptr;
+  const torch::Tensor scratch = need ? workspace_for(A, stream, need) : torch::Tensor();
+  void* ws = need ? scratch.data_ptr() : nullptr;
   const int st = neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, ldc, a_layout, b_layout, c_layout,
                                       alpha, beta, bt.sa, bt.sb, bt.sc, bt.count, ws, need, (void*)stream);
   TORCH_CHECK(st == NEOGEMM_OK, "neogemm_bf16 failed: ", neogemm_strerror(st));

@@ -62,3 +62,26 @@ def test_a_transposed_view_of_the_output_is_copied():
     both = torch.zeros(512, 256, dtype=torch.bfloat16)
     A, _, lda, _, a_layout, _ = gemm_amd._describe(both[:256].t(), X, out=both[256:])
     assert a_layout == gemm_amd.A_KM and A.data_ptr() == both.data_ptr()
+
+
+def test_scratch_of_captured_and_of_large_calls_is_not_kept(monkeypatch):
+    """A buffer whose address a graph replays must not be dropped when a later call outgrows it: captured calls take their own."""
+    import contextlib
+    import types
+
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: types.SimpleNamespace(cuda_stream=7))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(gemm_amd, "_workspaces", {})
+    monkeypatch.setattr(gemm_amd, "_MAX_KEPT", 4096, raising=False)
+    cpu = torch.device("cpu")
+    kept = gemm_amd._workspace(cpu, 1000)
+    assert gemm_amd._workspace(cpu, 500) is kept
+    capturing[0] = True
+    a, b = gemm_amd._workspace(cpu, 500), gemm_amd._workspace(cpu, 2000)
+    assert a is not kept and a.numel() >= 500 and b.numel() >= 2000
+    capturing[0] = False
+    assert gemm_amd._workspace(cpu, 500) is kept
+    assert gemm_amd._workspace(cpu, 4097).numel() >= 4097 and gemm_amd._workspace(cpu, 500) is kept
