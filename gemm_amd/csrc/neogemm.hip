@@ -3115,9 +3115,10 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     plan(M, N, K, aligned, c_layout, &pv, &ps, bt.count, b_layout, bt.a_layout);
     v = pv;
     if (s == 0) s = ps;
-    // a C that is not on 8-byte addresses ran without a workspace before the MFMA kernels took it: it still does
-    if (s > 1 && ((((uintptr_t)C | (uintptr_t)(ldc * 2)) & 7) != 0) &&
-        (!workspace || workspace_bytes < (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count)) {
+    // a C that is not on 8-byte addresses (bt.sc: any problem of a batch) needs no workspace: such calls always ran, unsplit, without one
+    const uintptr_t c_bytes = (uintptr_t)C | (uintptr_t)(ldc * 2) | (uintptr_t)(bt.sc * 2);
+    if (s > 1 && (c_bytes & 7) != 0 &&
+        (!workspace || ((uintptr_t)workspace & 15) != 0 || workspace_bytes < (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count)) {
       v = NEOGEMM_VARIANT_T128x128_W4;
       s = 1;
     }

@@ -71,3 +71,21 @@ def test_odd_c_without_a_workspace():
     assert g.plan(M, N, K, g.B_NK)[1] > 1
     st = _abi.gemm_raw(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, K, K, N, g.B_NK, g.C_ROW, 0, 0, torch.cuda.current_stream().cuda_stream)
     assert st == _abi.OK and torch.equal(C, (A.float() @ B.float().t()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
+def test_odd_c_stride_without_a_workspace(c_layout):
+    """The same for the problems of a batch, whose outputs lie an odd number of elements apart."""
+    from gemm_amd import _abi
+    b, M, N, K = 2, 64, 64, 8192
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    A, B = small_ints(gen, b, M, K, top=1), small_ints(gen, b, N, K, top=1)
+    lib = _abi.load()
+    assert lib.neogemm_bf16_batched_workspace_bytes(M, N, K, b) > 0
+    flat = torch.full((b * (M * N + 1),), 5.0, dtype=torch.bfloat16, device="cuda")
+    st = lib.neogemm_bf16_batched(A.data_ptr(), B.data_ptr(), flat.data_ptr(), M, N, K, K, K, N, M * K, N * K, M * N + 1, b, g.B_NK, c_layout,
+                                  None, 0, torch.cuda.current_stream().cuda_stream or None)
+    assert st == _abi.OK
+    want = torch.stack([A[i].float() @ B[i].float().t() for i in range(b)])
+    want = (want if c_layout == g.C_ROW else want.transpose(1, 2)).reshape(b, M * N).to(torch.bfloat16)
+    assert torch.equal(flat.view(b, M * N + 1)[:, :M * N], want) and bool((flat.view(b, M * N + 1)[:, M * N] == 5.0).all())
