@@ -1575,7 +1575,8 @@ hipError_t launch_shortk(TileArgs a, int run, hipStream_t st) {
 #endif
 
 // ---------------------------------------------------------------------------------------------
-// Small problems: a 64x64 tile of operands in either order.  What counts is the way to the first product and from the last one to C,
+// Small problems: a 64x64 tile, at most one of the operands MN-major (with both, and with a transposed A on the rows, the plan names no
+// tile of 64 rows).  What counts is the way to the first product and from the last one to C,
 // and how many CUs take part: gemm_tile_kernel takes B [K,N] in tiles of 128 columns at least, asks for three K tiles of each operand
 // before the first product, and leaves its main loop up to six K tiles before the end, to wait for every one of those with nothing
 // behind it.  704^3 with B [K,N] 10.4 -> 6.0 us, with B [N,K] 7.8 -> 5.6; 1024^3 10.3 -> 7.6 and 7.8 -> 7.0; 512^3 with B [K,N] 5.6 ->
@@ -1682,7 +1683,7 @@ hipError_t launch_small(const TileArgs& a, bool ak, bool bk, hipStream_t st) {
     return hipGetLastError();
   };
   if (ak) return bk ? go(gemm_small_kernel<true, true>) : go(gemm_small_kernel<true, false>);
-  return bk ? go(gemm_small_kernel<false, true>) : go(gemm_small_kernel<false, false>);
+  return bk ? go(gemm_small_kernel<false, true>) : hipErrorInvalidValue;
 }
 #endif
 
@@ -3252,14 +3253,13 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   // (the chained 256x256 kernel takes its rows from a K-major operand only, K in whole periods of 128 and no split)
   const bool fits = (ak || mn_ok(vi.bm, a.M)) && (bk || mn_ok(vi.bn, a.N)) &&
                     (v != NEOGEMM_VARIANT_C256x256_W4 || (ak && K % (2 * KTILE) == 0 && s <= 1));
-  // Where the plan says 64 rows per tile, gemm_small_kernel takes over, in either order of the operands (an MN-major one on the
-  // rows went to the 128x128 tile: 512^3 with a transposed A 6.8 us, 5.1 now), as long as the 64x64 tiles fit the CUs one and a half
-  // times (B [N,K]: 1152^3, 324 of them, 10.6 -> 9.0 us, 1280^3, 400, level, 1024 x 2048 x 1536, 512, 11.8 and 12.4) or twice
+  // Where the plan says 64 rows per tile, gemm_small_kernel takes over, with B [K,N] on the rows too (a column-major C; that went to the
+  // 128x128 tile), as long as the 64x64 tiles fit the CUs one and a half times (B [N,K]: 1152^3, 324 of them, 10.6 -> 9.0 us, 1280^3, 400, level, 1024 x 2048 x 1536, 512, 11.8 and 12.4) or twice
   // (B [K,N]: 13.7 and 12.5 for that last one).  Few workgroups with whole trips of the tile kernel's main loop stay there: 256 x 1024 x
   // 1024, 64 of them, 5.9 us and 6.7 with B [N,K], 7.1 and 7.3 with B [K,N]; 200 x 1000 x 1000 with B [K,N] 9.3 and 7.6.
   bool small = false;
   if (variant == NEOGEMM_VARIANT_AUTO && (v == NEOGEMM_VARIANT_T64x64_W4 || v == NEOGEMM_VARIANT_T64x128_W4) &&
-      (ak || (a.M & 7) == 0 || bt.padded) && (bk || (a.N & 7) == 0 || bt.padded)) {
+      (ak || bk) && (ak || (a.M & 7) == 0 || bt.padded) && (bk || (a.N & 7) == 0 || bt.padded)) {
     const int64_t cus = planning_cus(), wgs = (int64_t)ceil_div(a.M, 64) * ceil_div(a.N, 64) * s * bt.count;
     const int kt = ceil_div(K, KTILE);
     if (ak && bk) small = 2 * wgs <= 3 * cus && !(wgs <= 64 && s == 1 && kt >= 8 && kt % 4 == 0);
