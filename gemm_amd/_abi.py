@@ -43,6 +43,8 @@ PROTOTYPES = {
                                     ctypes.c_float, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
     "neogemm_bf16_general_workspace_bytes": (_sz, [_i64, _i64, _i64, _int, _int, _int, _i64]),
     "neogemm_bf16_call_workspace_bytes": (_sz, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _i64, _i64, _i64]),
+    "neogemm_bf16_call_kernel": (ctypes.c_char_p, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, ctypes.c_float,
+                                                   _i64, _i64, _i64, _i64, _sz]),
     "neogemm_bf16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "neogemm_bf16_variant": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _sz, _vp,
                                     _int, _int, _int]),
@@ -92,6 +94,20 @@ def version():
 
 def workspace_bytes(M, N, K):
     return int(load().neogemm_bf16_workspace_bytes(M, N, K))
+
+
+def call_workspace_bytes(A_ptr, B_ptr, M, N, K, lda, ldb, b_layout, c_layout, a_layout=A_MK, stride_a=0, stride_b=0, batch=1):
+    return int(load().neogemm_bf16_call_workspace_bytes(A_ptr, B_ptr, M, N, K, lda, ldb, a_layout, b_layout, c_layout, stride_a, stride_b, batch))
+
+
+def call_kernel(A_ptr, B_ptr, C_ptr, M, N, K, lda, ldb, ldc, b_layout, c_layout, a_layout=A_MK, beta=0.0, stride_a=0, stride_b=0,
+                stride_c=0, batch=1, ws_bytes=None):
+    """The kernel neogemm_bf16_general would run, with the workspace its query asks for or with ws_bytes; None: refused."""
+    if ws_bytes is None:
+        ws_bytes = call_workspace_bytes(A_ptr, B_ptr, M, N, K, lda, ldb, b_layout, c_layout, a_layout, stride_a, stride_b, batch)
+    name = load().neogemm_bf16_call_kernel(A_ptr, B_ptr, C_ptr, M, N, K, lda, ldb, ldc, a_layout, b_layout, c_layout, beta, stride_a, stride_b,
+                                           stride_c, batch, ws_bytes)
+    return name.decode() if name else None
 
 
 def plan(M, N, K, b_layout=B_KN, c_layout=C_ROW, aligned=True):

@@ -2884,6 +2884,8 @@ static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream
   return NEOGEMM_OK;
 }
 
+// The kernels that a call may end on, without the copies ahead of them and the reduction behind them.
+enum class Kernel { kNone, kGeneric, kRagged, kTile, kChain, kSkinny, kStrip, kSmall, kShortK };
 // A batch of `count` problems of one shape; strides in elements between consecutive problems (0: shared operand); and how
 // A is laid out, which only the general entry point lets a caller choose.
 struct BatchArgs {
@@ -2891,6 +2893,8 @@ struct BatchArgs {
   int a_layout = NEOGEMM_A_MK;
   bool scratch_unaligned = false;  // operands off the 16-byte grid may use the workspace (see neogemm_bf16_call_workspace_bytes)
   bool padded = false;             // rows of both operands end on whole chunks in memory, zeros behind K (pack_kernel)
+  Kernel* only_name = nullptr;     // nothing is launched; what would be is written here (neogemm_bf16_call_kernel) ...
+  bool* copies = nullptr;          // ... and here whether copies on the 16-byte grid come first
 };
 
 // ld limits keep every in-tile byte offset below 2^31 (the buffer range check uses 32-bit offsets)
@@ -3012,10 +3016,14 @@ static int launch_packed(const PackPlan& p, const void* A, const void* B, void* 
   };
   const PackArgs pa = args(A, at_a, lda, bt.sa, a_mk ? M : K, a_mk ? K : M, p.a), pb = args(B, at_b, ldb, bt.sb, b_nk ? N : K, b_nk ? K : N, p.b);
   const bool one = (!p.a || pa.bs == 0) && (!p.b || pb.bs == 0);  // nothing that differs between the problems of the batch is copied
-  pack_kernel<<<dim3(pa.blocks + pb.blocks, 1, one ? 1u : (unsigned)bt.count), 256, 0, st>>>(pa, pb);
-  if (hipError_t e = hipGetLastError(); e != hipSuccess) {
-    fprintf(stderr, "neogemm: pack kernel launch failed: %s\n", hipGetErrorString(e));
-    return NEOGEMM_ERR_LAUNCH;
+  if (bt.only_name) {
+    *bt.copies = true;
+  } else {
+    pack_kernel<<<dim3(pa.blocks + pb.blocks, 1, one ? 1u : (unsigned)bt.count), 256, 0, st>>>(pa, pb);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) {
+      fprintf(stderr, "neogemm: pack kernel launch failed: %s\n", hipGetErrorString(e));
+      return NEOGEMM_ERR_LAUNCH;
+    }
   }
   BatchArgs to = bt;
   to.padded = true;
@@ -3059,6 +3067,7 @@ static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, in
   a.ksplit = ceil_div(ktiles, a.ktiles_per_split);  // no empty split
   if ((int64_t)a.ntm * a.ntn * a.ksplit > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;
   a.ws = (float*)ws;
+  if (bt.only_name) return *bt.only_name = Kernel::kRagged, NEOGEMM_OK;
   if (hipError_t e = launch_ragged(a, ak, bk, bm, bn, st); e != hipSuccess) {
     fprintf(stderr, "neogemm: ragged kernel launch failed: %s\n", hipGetErrorString(e));
     return NEOGEMM_ERR_LAUNCH;
@@ -3132,6 +3141,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     const long scm = c_layout == NEOGEMM_C_ROW ? ldc : 1, scn = c_layout == NEOGEMM_C_ROW ? 1 : ldc;
     const int64_t nbx = ceil_div(N, 16), nblocks = nbx * ceil_div(M, 16);
     if (nblocks > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;
+    if (bt.only_name) return *bt.only_name = Kernel::kGeneric, NEOGEMM_OK;
     dim3 grid((unsigned)nblocks, 1, (unsigned)bt.count);
     gemm_generic_kernel<<<grid, 256, 0, st>>>((const __bf16*)A, (const __bf16*)B, (__bf16*)C, (int)M, (int)N, (int)K,
                                               sam, sak, sbk, sbn, scm, scn, alpha, beta, bt.sa, bt.sb, bt.sc,
@@ -3162,6 +3172,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                     NEOGEMM_VARIANT_T128x128_W4, 1, 0, nullptr, alpha, beta, bt);
       return st2 == NEOGEMM_ERR_UNSUPPORTED ? unaligned() : st2;
     }
+    if (bt.only_name) return *bt.only_name = v == NEOGEMM_VARIANT_STRIP ? Kernel::kStrip : Kernel::kSkinny, NEOGEMM_OK;
     SkinnyArgs sa{(const char*)A, (const char*)B, (char*)C, (int)M, (int)N, (int)K, (long)lda, (long)ldb, (long)ldc, alpha, beta, 0, 64};
     bool bkm = b_layout == NEOGEMM_B_NK, ccol = c_layout == NEOGEMM_C_COL;
     if (swap) {
@@ -3291,6 +3302,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     // at least two column tiles for each of two workgroups per CU (16 x 512 x 512 x 96, one each: level with the tile kernels)
     const int64_t tiles = (int64_t)ceil_div(a.M, 128) * ceil_div(a.N, 64) * bt.count, slots = 2 * (int64_t)planning_cus();
     if (tiles >= 2 * slots) {
+      if (bt.only_name) return *bt.only_name = Kernel::kShortK, NEOGEMM_OK;
       const int64_t per_row = ceil_div(slots, (int64_t)ceil_div(a.M, 128) * bt.count);  // workgroups that share a block of rows
       const hipError_t e = launch_shortk(a, ceil_div(ceil_div(a.N, 64), per_row), st);
       if (e == hipSuccess) return NEOGEMM_OK;
@@ -3307,6 +3319,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     a.ws = (float*)workspace;
   }
 
+  if (bt.only_name) return *bt.only_name = small ? Kernel::kSmall : v == NEOGEMM_VARIANT_C256x256_W4 ? Kernel::kChain : Kernel::kTile, NEOGEMM_OK;
   hipError_t e;
   if (small) e = launch_small(a, ak, bk, st);
   else switch (v) {
@@ -3454,6 +3467,30 @@ size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M
   else if (neogemm::ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt))
     neogemm::ragged_plan(row ? M : N, row ? N : M, K, batch, neogemm::planning_cus(), &v, &w, &s);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)batch : 0;
+}
+
+const char* neogemm_bf16_call_kernel(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                     int64_t ldc, int a_layout, int b_layout, int c_layout, float beta, int64_t stride_a, int64_t stride_b,
+                                     int64_t stride_c, int64_t batch, size_t workspace_bytes) {
+  static const char* const kNames[][2] = {{"none", "none"},         {"generic", "copy+generic"}, {"ragged", "copy+ragged"},
+                                          {"tile", "copy+tile"}, {"chain", "copy+chain"},    {"skinny", "copy+skinny"},
+                                          {"strip", "copy+strip"}, {"small", "copy+small"}, {"short K", "copy+short K"}};
+  neogemm::BatchArgs bt;
+  bt.count = batch;
+  bt.sa = stride_a;
+  bt.sb = stride_b;
+  bt.sc = stride_c;
+  bt.a_layout = a_layout;
+  bt.scratch_unaligned = true;
+  neogemm::Kernel kernel = neogemm::Kernel::kNone;
+  bool copies = false;
+  bt.only_name = &kernel;
+  bt.copies = &copies;
+  void* ws = workspace_bytes ? (void*)256 : nullptr;  // never read: nothing is launched
+  if (neogemm::run(A, B, const_cast<void*>(C), M, N, K, lda, ldb, ldc, b_layout, c_layout, ws, workspace_bytes, nullptr, NEOGEMM_VARIANT_AUTO, 0, 0,
+                   nullptr, 1.f, beta, bt) != NEOGEMM_OK)
+    return nullptr;
+  return kNames[(int)kernel][copies ? 1 : 0];
 }
 
 size_t neogemm_bf16_batched_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch) {

@@ -150,6 +150,15 @@ size_t neogemm_bf16_general_workspace_bytes(int64_t M, int64_t N, int64_t K, int
  */
 size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                          int a_layout, int b_layout, int c_layout, int64_t stride_a, int64_t stride_b, int64_t batch);
+/*
+ * Which kernel neogemm_bf16_general runs for exactly these operands, given that many bytes of workspace: "tile", "chain" (the 256x256
+ * tile that accumulates twice in a row), "small", "short K", "skinny", "strip", each with "copy+" in front where operands are first
+ * copied onto the 16-byte grid; "ragged" (operands at any address), "generic", "none" (an empty problem); NULL for a call that is
+ * refused.  Host only, for tests and tuning: the pointers are not read, their low bits are what counts.
+ */
+const char* neogemm_bf16_call_kernel(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                     int64_t ldc, int a_layout, int b_layout, int c_layout, float beta, int64_t stride_a, int64_t stride_b,
+                                     int64_t stride_c, int64_t batch, size_t workspace_bytes);
 
 /*
  * neogemm_bf16 for callers that cannot allocate device memory (code under HIP graph capture, tight serving

@@ -178,6 +178,25 @@ def test_argument_validation_returns_before_touching_the_gpu():
     assert _abi.gemm_raw(0, 0, 0, 4, 0, 4, 4, 4, 4, 0, 0) == _abi.OK
 
 
+def test_call_kernel_names_without_a_gpu():
+    """neogemm_bf16_call_kernel launches nothing: the same checks and the same choice as the call itself."""
+    p, q, c = 1 << 20, 1 << 40, 1 << 44
+    nk, col = _abi.B_NK, _abi.C_COL
+    assert _abi.call_kernel(p, q, c, 8192, 8192, 8192, 8192, 8192, 8192, 0, 0) == "chain"
+    assert _abi.call_kernel(p, q, c, 1024, 1024, 1024, 1024, 1024, 1024, nk, col) == "small"
+    assert _abi.call_kernel(p, q, c, 16, 14336, 4096, 4096, 14336, 14336, 0, 0) == "skinny"
+    assert _abi.call_kernel(p, q, c, 128, 14336, 4096, 4096, 4096, 14336, nk, 0) == "strip"
+    assert _abi.call_kernel(p, q, c, 100, 100, 101, 101, 100, 100, 0, 0) == "ragged"
+    assert _abi.call_kernel(p, q, c, 4001, 4001, 4001, 4001, 4001, 4001, 0, 0) == "copy+tile"
+    assert _abi.call_kernel(p, q, c, 4001, 4001, 4001, 4001, 4001, 4001, 0, 0, ws_bytes=0) == "ragged"
+    assert _abi.call_kernel(p, q, c, 1, 1, 7, 7, 1, 1, 0, 0) == "generic" and _abi.call_kernel(p, q, c, 8, 8, 0, 1, 8, 8, 0, 0) == "generic"
+    assert _abi.call_kernel(0, 0, 0, 0, 8, 8, 8, 8, 8, 0, 0) == "none"
+    # refused: the argument checks, and a split without its workspace
+    assert _abi.call_kernel(p, q, c, 8, 8, 8, 7, 8, 8, 0, 0) is None and _abi.call_kernel(0, q, c, 8, 8, 8, 8, 8, 8, 0, 0) is None
+    assert _abi.call_kernel(p, q, c, 1024, 1024, 32768, 32768, 1024, 1024, 0, 0) == "tile"
+    assert _abi.call_kernel(p, q, c, 1024, 1024, 32768, 32768, 1024, 1024, 0, 0, ws_bytes=0) is None
+
+
 def test_plan_rejects_null_outputs():
     lib = _abi.load()
     assert lib.neogemm_bf16_plan(4, 4, 4, 0, 0, 1, None, None) == _abi.ERR_BAD_ARG

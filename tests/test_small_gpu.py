@@ -3,12 +3,13 @@ import pytest
 import torch
 
 import gemm_amd as g
+from gemm_amd import _abi
 
 pytestmark = pytest.mark.gpu
 
 
 # K: part of a stage, one, two, three (the ring's depth), four, a partial last one, split; M, N: edges of the 64 tile, one column of chunks,
-# up to the most workgroups that the rule sends here
+# up to the most workgroups that the rule sends here, and what lies beyond it
 @pytest.mark.parametrize("M,N,K", [(136, 136, 8), (136, 8, 64), (264, 200, 72), (328, 448, 128), (448, 448, 184), (192, 520, 256), (640, 640, 640), (1024, 1024, 1024),
                                    (1152, 1152, 320), (1024, 2048, 264), (264, 264, 4104), (256, 256, 8192), (256, 1024, 1024)])
 @pytest.mark.parametrize("a_layout", [g.A_MK, g.A_KM])
@@ -24,8 +25,14 @@ def test_small(M, N, K, a_layout, b_layout, c_layout):
 
     A, B = ints(*((M, K) if a_layout == g.A_MK else (K, M)), 8), ints(*((K, N) if b_layout == g.B_KN else (N, K)), 16)
     want = (A if a_layout == g.A_MK else A.t()).float() @ (B if b_layout == g.B_KN else B.t()).float()
+    # with B [N,K] at most one and a half 64x64 tiles per CU; few tiles and whole trips of the tile kernel's main loop; a transposed A only
+    # where it supplies the columns of a product whose rows are K-major
+    stays = {(1024, 2048, 264): b_layout == g.B_NK, (256, 1024, 1024): (b_layout, c_layout) != (g.B_KN, g.C_COL)}.get((M, N, K), False)
+    here = not stays if a_layout == g.A_MK else (b_layout, c_layout) == (g.B_NK, g.C_COL) and (M, N, K) != (256, 1024, 1024)
     C = torch.full((M, N) if c_layout == g.C_ROW else (N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
     got = C if c_layout == g.C_ROW else C.t()
+    assert _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout,
+                            a_layout) == ("small" if here else "tile")
     g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout)
     assert torch.equal(got, want.to(torch.bfloat16))
     old = got.clone()
