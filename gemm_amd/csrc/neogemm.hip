@@ -2987,10 +2987,12 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
     plan_model(M, N, K, true, c_layout, &v, &sp, bt.count, b_layout, cus, bt.a_layout, &aligned_us);
     const bool row = c_layout == NEOGEMM_C_ROW;
     const double ragged_us = ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, &bm, &bn, &sp);
-    // (10001 x 1024 x 512 with a transposed A takes a sixth more than the estimate)
-    // the copy and the product that waits for it: 6.5 us and 3 MB per us (1500 x 1501 x 1401 26.1 -> 23.0 us, 1000 x 2048 x 5001 47.0 ->
-    // 39.1, 4001^3 202 -> 120; below the line 700^3 9.0 against 14.9, 100 x 2999 x 2999 16.3 against 26.1)
-    e.pays = aligned_us + 6.5 + (double)e.bytes / 3.0e6 < ragged_us * (bt.a_layout == NEOGEMM_A_KM ? 1.15 : 1.0);
+    // The copy and the product that waits for it: 6.5 us and 3 MB per us; in place: 3 us over ragged_plan's estimate, which compares its
+    // own tiles only.  Both ways measured at 68 sizes, one operand or both off the grid (us, copies / in place,
+    // A [M,K] and A [K,M]): 2001 x 2000 x 504 14.1 / 17.0 and 13.9 / 16.7, 10001 x 1024 x 512 26.0 / 38.3 and 27.2 / 34.7, 20001 x 2048 x
+    // 1024 104.5 / 157.6 and 105.5 / 149.9; below the line 1001 x 1024 x 1024 11.4 / 10.0 and 15.3 / 9.4, 1501 x 512 x 2048 19.5 / 14.7 and
+    // 24.8 / 16.2.  The choice costs 1.7 % over the better one on average (without the 3 us 4.2 %), 24 % at worst (201 x 4096 x 4096).
+    e.pays = aligned_us + 6.5 + (double)e.bytes / 3.0e6 < ragged_us + 3.0;
     plan(M, N, K, true, c_layout, &v, &sp, bt.count, b_layout, bt.a_layout);
     e.split = sp;
     m = &e;

@@ -197,6 +197,20 @@ def test_call_kernel_names_without_a_gpu():
     assert _abi.call_kernel(p, q, c, 1024, 1024, 32768, 32768, 1024, 1024, 0, 0, ws_bytes=0) is None
 
 
+def test_copies_are_made_where_they_pay():
+    """Shapes measured both ways, A one element off the grid ([M,K]) or with odd rows ([K,M]): us with copies / in place beside each."""
+    for (M, N, K), better in (((2001, 2000, 504), "copy+tile"),     # 14.1 / 17.0, transposed A 13.9 / 16.7
+                              ((10001, 1024, 512), "copy+tile"),    # 26.0 / 38.3, 27.2 / 34.7
+                              ((5001, 1024, 304), "copy+tile"),     # 14.5 / 20.2, 13.0 / 17.9
+                              ((1501, 1504, 1504), "copy+tile"),    # 20.0 / 30.9, 21.6 / 30.0
+                              ((1001, 1024, 1024), "ragged"),       # 11.4 / 10.0, 15.3 / 9.4
+                              ((1501, 512, 2048), "ragged"),        # 19.5 / 14.7, 24.8 / 16.2
+                              ((501, 256, 1024), "ragged")):        # 12.3 / 9.9, 14.2 / 9.1
+        for a, lda, off in ((_abi.A_MK, K, 2), (_abi.A_KM, M, 0)):
+            for b, ldb in ((_abi.B_KN, N), (_abi.B_NK, K)):
+                assert _abi.call_kernel((1 << 20) + off, 1 << 40, 1 << 44, M, N, K, lda, ldb, N, b, _abi.C_ROW, a) == better
+
+
 def test_plan_rejects_null_outputs():
     lib = _abi.load()
     assert lib.neogemm_bf16_plan(4, 4, 4, 0, 0, 1, None, None) == _abi.ERR_BAD_ARG
