@@ -14,6 +14,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -2940,66 +2941,108 @@ static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, 
     }
   return best;
 }
-// Copies of the operands that are off the 16-byte grid (pack_kernel), and the product by the kernels for aligned ones.
+// Copies of the operands that are off the 16-byte grid (pack_kernel), and the product by the kernels for aligned ones.  The copies take
+// kPackMost bytes at most (two operands of 8191 x 8191): beyond it, or where a copy's rows would be 2^21 elements long, the product is made
+// in passes over some of the problems of a batch and over panels of C, which copy what they need of the operands one after the other.
+// 50257 x 4096 x 4096 with a transposed A (412 MB of copies) 1470 us; in place, as such sizes ran without panels, 2264.
+static constexpr size_t kPackMost = (size_t)1 << 28;
 struct PackPlan {
-  bool a = false, b = false;                 // which operand is copied
-  int64_t ldpa = 0, ldpb = 0;                // leading dimensions of the copies
+  bool a = false, b = false;                      // which operand is copied
+  int64_t count = 1, rows = 0, cols = 0;          // problems, rows and columns of C per pass
   size_t partials = 0, bytes_a = 0, bytes_b = 0;  // what the workspace holds, in this order, each from a multiple of 256 on
   size_t total() const { return partials + bytes_a + bytes_b; }
 };
+static int64_t chunked(int64_t n) { return (n + 7) / 8 * 8; }
+// Problems, rows and columns per pass; false: no pass is small enough.
+static bool pack_passes(int64_t M, int64_t N, int64_t K, bool a_mk, bool b_nk, const BatchArgs& bt, PackPlan& p) {
+  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+  // (a panel of whole 256-wide tiles, or of 64-wide ones where K is very deep)
+  auto halve = [](int64_t& n) {
+    if (n <= 64) return false;
+    const int64_t step = n > 256 ? 256 : 64;
+    n = (n / 2 + step - 1) / step * step;
+    return true;
+  };
+  p.count = bt.count;
+  p.rows = M;
+  p.cols = N;
+  for (;;) {
+    const int64_t lda = chunked(a_mk ? K : p.rows), ldb = chunked(b_nk ? K : p.cols);
+    const bool wide_a = p.a && lda >= (1 << 21), wide_b = p.b && ldb >= (1 << 21);
+    p.bytes_a = p.a ? up((size_t)(a_mk ? p.rows : K) * lda * 2 * (bt.sa ? p.count : 1)) : 0;
+    p.bytes_b = p.b ? up((size_t)(b_nk ? p.cols : K) * ldb * 2 * (bt.sb ? p.count : 1)) : 0;
+    if (!wide_a && !wide_b && p.bytes_a + p.bytes_b <= kPackMost) return true;
+    if ((wide_a && a_mk) || (wide_b && b_nk)) return false;
+    if (wide_a) {
+      halve(p.rows);
+    } else if (wide_b) {
+      halve(p.cols);
+    } else if (p.count > 1) {
+      p.count = (p.count + 1) / 2;
+    } else if (p.bytes_a >= p.bytes_b ? !halve(p.rows) && (!p.b || !halve(p.cols)) : !halve(p.cols) && (!p.a || !halve(p.rows))) {
+      return false;
+    }
+  }
+}
 static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int b_layout, int c_layout,
                       const BatchArgs& bt, PackPlan* out) {
   const bool a_mk = bt.a_layout == NEOGEMM_A_MK, b_nk = b_layout == NEOGEMM_B_NK;
-  const int64_t rows_a = a_mk ? M : K, cols_a = a_mk ? K : M, rows_b = b_nk ? N : K, cols_b = b_nk ? K : N;
   auto off_grid = [](const void* ptr, int64_t ld, int64_t bs, int64_t cols) {
     return ((uintptr_t)ptr & 15) != 0 || (ld & 7) != 0 || ld >= (1 << 21) || (bs & 7) != 0 || (cols & 7) != 0;
   };
-  PackPlan p;
-  p.a = off_grid(A, lda, bt.sa, cols_a);
-  p.b = off_grid(B, ldb, bt.sb, cols_b);
-  p.ldpa = (cols_a + 7) / 8 * 8;
-  p.ldpb = (cols_b + 7) / 8 * 8;
-  if ((!p.a && !p.b) || p.ldpa >= (1 << 21) || p.ldpb >= (1 << 21) || K < 1) return false;
-  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
-  if (p.a) p.bytes_a = up((size_t)rows_a * p.ldpa * 2 * (bt.sa ? bt.count : 1));
-  if (p.b) p.bytes_b = up((size_t)rows_b * p.ldpb * 2 * (bt.sb ? bt.count : 1));
-  const size_t most = (size_t)1 << 28;  // bytes that a workspace would keep for it: two operands of 8191 x 8191
-  if (p.bytes_a + p.bytes_b > most) return false;
+  const bool a = off_grid(A, lda, bt.sa, a_mk ? K : M), b = off_grid(B, ldb, bt.sb, b_nk ? K : N);
+  if ((!a && !b) || K < 1) return false;
+  const int cus = planning_cus();
   struct Memo {
     int64_t M = -1, N = -1, K = -1, count = -1;
-    size_t bytes = 0;
-    int a_layout = -1, b_layout = -1, c_layout = -1, cus = -1, split = 1;
+    int a_layout = -1, b_layout = -1, c_layout = -1, cus = -1, what = -1;
     bool pays = false;
+    PackPlan plan;
   };
+  const int what = a | b << 1 | (bt.sa != 0) << 2 | (bt.sb != 0) << 3;
   static thread_local Memo memo[32];
   static thread_local unsigned next = 0;
-  const int cus = planning_cus();
   const Memo* m = nullptr;
   for (const Memo& e : memo)
-    if (e.M == M && e.N == N && e.K == K && e.count == bt.count && e.bytes == p.bytes_a + p.bytes_b && e.a_layout == bt.a_layout &&
-        e.b_layout == b_layout && e.c_layout == c_layout && e.cus == cus)
+    if (e.M == M && e.N == N && e.K == K && e.count == bt.count && e.a_layout == bt.a_layout && e.b_layout == b_layout &&
+        e.c_layout == c_layout && e.cus == cus && e.what == what)
       m = &e;
   if (!m) {
     Memo& e = memo[next++ & 31];
-    e = Memo{M, N, K, bt.count, p.bytes_a + p.bytes_b, bt.a_layout, b_layout, c_layout, cus, 1, false};
-    int v, bm, bn, sp;
-    double aligned_us = 0;
-    plan_model(M, N, K, true, c_layout, &v, &sp, bt.count, b_layout, cus, bt.a_layout, &aligned_us);
-    const bool row = c_layout == NEOGEMM_C_ROW;
-    const double ragged_us = ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, &bm, &bn, &sp);
-    // The copy and the product that waits for it: 6.5 us and 3 MB per us; in place: 3 us over ragged_plan's estimate, which compares its
-    // own tiles only.  Both ways measured at 68 sizes, one operand or both off the grid (us, copies / in place,
-    // A [M,K] and A [K,M]): 2001 x 2000 x 504 14.1 / 17.0 and 13.9 / 16.7, 10001 x 1024 x 512 26.0 / 38.3 and 27.2 / 34.7, 20001 x 2048 x
-    // 1024 104.5 / 157.6 and 105.5 / 149.9; below the line 1001 x 1024 x 1024 11.4 / 10.0 and 15.3 / 9.4, 1501 x 512 x 2048 19.5 / 14.7 and
-    // 24.8 / 16.2.  The choice costs 1.7 % over the better one on average (without the 3 us 4.2 %), 24 % at worst (201 x 4096 x 4096).
-    e.pays = aligned_us + 6.5 + (double)e.bytes / 3.0e6 < ragged_us + 3.0;
-    plan(M, N, K, true, c_layout, &v, &sp, bt.count, b_layout, bt.a_layout);
-    e.split = sp;
+    e = Memo{M, N, K, bt.count, bt.a_layout, b_layout, c_layout, cus, what, false, PackPlan()};
+    PackPlan& p = e.plan;
+    p.a = a;
+    p.b = b;
     m = &e;
+    if (pack_passes(M, N, K, a_mk, b_nk, bt, p)) {
+      int v, bm, bn, sp;
+      double aligned_us = 0;
+      plan_model(p.rows, p.cols, K, true, c_layout, &v, &sp, p.count, b_layout, cus, bt.a_layout, &aligned_us);
+      const bool row = c_layout == NEOGEMM_C_ROW;
+      const double other_us = ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, &bm, &bn, &sp) + 3.0;
+      // a panel's copy of A is made again for each panel of columns, and a shared operand's panels for each part of the batch
+      const int nb = ceil_div(bt.count, p.count), nr = ceil_div(M, p.rows), nc = ceil_div(N, p.cols);
+      const double moved = (double)p.bytes_a * nr * (bt.sa ? nb : nr > 1 ? nb : 1) * (nr > 1 ? nc : 1) +
+                           (double)p.bytes_b * nc * (bt.sb ? nb : nc > 1 ? nb : 1);
+      // The copy and the product that waits for it: 6.5 us and 3 MB per us; in place: 3 us over ragged_plan's estimate, which compares its
+      // own tiles only.  Both ways measured at 68 sizes, one operand or both off the grid (us, copies / in place,
+      // A [M,K] and A [K,M]): 2001 x 2000 x 504 14.1 / 17.0 and 13.9 / 16.7, 10001 x 1024 x 512 26.0 / 38.3 and 27.2 / 34.7, 20001 x 2048 x
+      // 1024 104.5 / 157.6 and 105.5 / 149.9; below the line 1001 x 1024 x 1024 11.4 / 10.0 and 15.3 / 9.4, 1501 x 512 x 2048 19.5 / 14.7 and
+      // 24.8 / 16.2.  The choice costs 1.7 % over the better one on average (without the 3 us 4.2 %), 24 % at worst (201 x 4096 x 4096).
+      e.pays = (double)nb * nr * nc * (aligned_us + 6.5) + moved / 3.0e6 < other_us;
+      // (the last problems, rows and columns may be fewer, and split otherwise)
+      for (const int64_t c : {p.count, bt.count % p.count})
+        for (const int64_t r : {p.rows, M % p.rows})
+          for (const int64_t n : {p.cols, N % p.cols}) {
+            if (!e.pays || c == 0 || r == 0 || n == 0) continue;
+            plan(r, n, K, true, c_layout, &v, &sp, c, b_layout, bt.a_layout);
+            const size_t bytes = sp > 1 ? ((size_t)sp * (size_t)r * (size_t)n * sizeof(float) * (size_t)c + 255) / 256 * 256 : 0;
+            if (bytes > p.partials) p.partials = bytes;
+          }
+    }
   }
   if (!m->pays) return false;
-  if (m->split > 1) p.partials = up((size_t)m->split * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count);
-  *out = p;
+  *out = m->plan;
   return true;
 }
 static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
@@ -3008,31 +3051,47 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                float beta = 0.f, const BatchArgs& bt = BatchArgs());
 static int launch_packed(const PackPlan& p, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                          int64_t ldc, int b_layout, int c_layout, void* ws, hipStream_t st, float alpha, float beta, const BatchArgs& bt) {
-  const bool a_mk = bt.a_layout == NEOGEMM_A_MK, b_nk = b_layout == NEOGEMM_B_NK;
-  char* at_a = (char*)ws + p.partials;
-  char* at_b = at_a + p.bytes_a;
-  auto args = [&](const void* src, char* dst, int64_t ld, int64_t bs, int64_t rows, int64_t cols, bool used) {
-    PackArgs r{(const char*)src, dst, (long)ld, bt.count > 1 ? (long)bs : 0, (unsigned)rows, (unsigned)cols, (unsigned)((cols + 7) / 8), 0};
-    if (used) r.blocks = (unsigned)(((uint64_t)r.rows * r.cpr + 255) / 256);
-    return r;
-  };
-  const PackArgs pa = args(A, at_a, lda, bt.sa, a_mk ? M : K, a_mk ? K : M, p.a), pb = args(B, at_b, ldb, bt.sb, b_nk ? N : K, b_nk ? K : N, p.b);
-  const bool one = (!p.a || pa.bs == 0) && (!p.b || pb.bs == 0);  // nothing that differs between the problems of the batch is copied
-  if (bt.only_name) {
-    *bt.copies = true;
-  } else {
-    pack_kernel<<<dim3(pa.blocks + pb.blocks, 1, one ? 1u : (unsigned)bt.count), 256, 0, st>>>(pa, pb);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) {
-      fprintf(stderr, "neogemm: pack kernel launch failed: %s\n", hipGetErrorString(e));
-      return NEOGEMM_ERR_LAUNCH;
-    }
-  }
-  BatchArgs to = bt;
-  to.padded = true;
-  if (p.a) to.sa = pa.bs ? (int64_t)pa.rows * p.ldpa : 0;
-  if (p.b) to.sb = pb.bs ? (int64_t)pb.rows * p.ldpb : 0;
-  return run(p.a ? at_a : A, p.b ? at_b : B, C, M, N, K, p.a ? p.ldpa : lda, p.b ? p.ldpb : ldb, ldc, b_layout, c_layout, ws, p.partials,
-             (void*)st, NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, alpha, beta, to);
+  const bool a_mk = bt.a_layout == NEOGEMM_A_MK, b_nk = b_layout == NEOGEMM_B_NK, row = c_layout == NEOGEMM_C_ROW;
+  char* const at_a = (char*)ws + p.partials;
+  char* const at_b = at_a + p.bytes_a;
+  const char* in_a = nullptr;  // what the copies hold: the stream's order keeps a copy until the products before it have read it
+  const char* in_b = nullptr;
+  for (int64_t b0 = 0; b0 < bt.count; b0 += p.count)
+    for (int64_t n0 = 0; n0 < N; n0 += p.cols)
+      for (int64_t m0 = 0; m0 < M; m0 += p.rows) {
+        const int64_t count = std::min(p.count, bt.count - b0), rows = std::min(p.rows, M - m0), cols = std::min(p.cols, N - n0);
+        const char* a = (const char*)A + (b0 * bt.sa + (a_mk ? m0 * lda : m0)) * 2;
+        const char* b = (const char*)B + (b0 * bt.sb + (b_nk ? n0 * ldb : n0)) * 2;
+        char* c = (char*)C + (b0 * bt.sc + (row ? m0 * ldc + n0 : n0 * ldc + m0)) * 2;
+        auto args = [&](const char* src, char* dst, int64_t ld, int64_t bs, int64_t rows, int64_t cols, bool copied, bool needed) {
+          PackArgs r{src, dst, (long)ld, count > 1 ? (long)bs : 0, (unsigned)rows, (unsigned)cols, (unsigned)((cols + 7) / 8), 0};
+          if (copied && needed) r.blocks = (unsigned)(((uint64_t)r.rows * r.cpr + 255) / 256);
+          return r;
+        };
+        const PackArgs pa = args(a, at_a, lda, bt.sa, a_mk ? rows : K, a_mk ? K : rows, p.a, a != in_a);
+        const PackArgs pb = args(b, at_b, ldb, bt.sb, b_nk ? cols : K, b_nk ? K : cols, p.b, b != in_b);
+        in_a = a;
+        in_b = b;
+        const bool one = (!pa.blocks || pa.bs == 0) && (!pb.blocks || pb.bs == 0);  // nothing that differs between the problems is copied
+        if (bt.only_name) {
+          *bt.copies = true;
+        } else if (pa.blocks + pb.blocks) {
+          pack_kernel<<<dim3(pa.blocks + pb.blocks, 1, one ? 1u : (unsigned)count), 256, 0, st>>>(pa, pb);
+          if (hipError_t e = hipGetLastError(); e != hipSuccess) {
+            fprintf(stderr, "neogemm: pack kernel launch failed: %s\n", hipGetErrorString(e));
+            return NEOGEMM_ERR_LAUNCH;
+          }
+        }
+        BatchArgs to = bt;
+        to.count = count;
+        to.padded = true;
+        if (p.a) to.sa = pa.bs ? (int64_t)pa.rows * pa.cpr * 8 : 0;
+        if (p.b) to.sb = pb.bs ? (int64_t)pb.rows * pb.cpr * 8 : 0;
+        const int r = run(p.a ? at_a : a, p.b ? at_b : b, c, rows, cols, K, p.a ? (int64_t)pa.cpr * 8 : lda, p.b ? (int64_t)pb.cpr * 8 : ldb, ldc,
+                          b_layout, c_layout, ws, p.partials, (void*)st, NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, alpha, beta, to);
+        if (r != NEOGEMM_OK || bt.only_name) return r;
+      }
+  return NEOGEMM_OK;
 }
 // Operands at any address: gemm_ragged_kernel, and the reduction where K is split.  NEOGEMM_ERR_UNSUPPORTED: not launched.
 static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,

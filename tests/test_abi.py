@@ -211,6 +211,29 @@ def test_copies_are_made_where_they_pay():
                 assert _abi.call_kernel((1 << 20) + off, 1 << 40, 1 << 44, M, N, K, lda, ldb, N, b, _abi.C_ROW, a) == better
 
 
+def test_copies_stay_bounded_and_are_made_above_the_bound():
+    """Operands of more than 256 MiB are copied panel by panel: scratch of at most that, and of the partials of a panel whose K is split."""
+    p, q, c = (1 << 20) + 2, 1 << 40, 1 << 44
+
+    def ask(M, N, K, a, b, lda=None, batch=1):
+        lda, ldb = lda or (K if a == _abi.A_MK else M), N if b == _abi.B_KN else K
+        strides = (M * K, N * K, M * N) if batch > 1 else (0, 0, 0)
+        need = _abi.call_workspace_bytes(p, q, M, N, K, lda, ldb, b, _abi.C_ROW, a, *strides[:2], batch)
+        return need, _abi.call_kernel(p, q, c, M, N, K, lda, ldb, N, b, _abi.C_ROW, a, 0.0, *strides, batch)
+
+    bound = (256 << 20) + 2 * 2048 * 4096 * 4
+    for (M, N, K, a, b) in ((50257, 4096, 4096, _abi.A_KM, _abi.B_KN),   # a weight gradient with an odd number of classes ...
+                            (4096, 4096, 50257, _abi.A_MK, _abi.B_KN),   # ... and the input gradient
+                            (8191, 8191, 8191, _abi.A_MK, _abi.B_KN), (8193, 8193, 8193, _abi.A_MK, _abi.B_KN), (40001, 40001, 8193, _abi.A_MK, _abi.B_NK),
+                            (4001, 4001, 40001, _abi.A_MK, _abi.B_KN)):
+        need, kernel = ask(M, N, K, a, b)
+        assert kernel in ("copy+tile", "copy+chain") and (1 << 24) < need <= bound, (M, N, K, need, kernel)
+    need, kernel = ask(1001, 1001, 1801, _abi.A_MK, _abi.B_KN, batch=60)
+    assert kernel == "copy+tile" and (1 << 24) < need <= bound
+    # rows of a copy of 2^21 elements and more
+    assert ask(64, 64, 3000001, _abi.A_MK, _abi.B_KN)[1] == "generic"
+
+
 def test_plan_rejects_null_outputs():
     lib = _abi.load()
     assert lib.neogemm_bf16_plan(4, 4, 4, 0, 0, 1, None, None) == _abi.ERR_BAD_ARG

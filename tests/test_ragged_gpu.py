@@ -122,6 +122,37 @@ def test_copies_on_the_grid(b, M, N, K):
                     assert torch.equal(got, (want + add.float()).to(torch.bfloat16))
 
 
+# copies of more than 256 MiB in panels: of the rows, of the columns, of both (a panel of A copied for each panel of columns), of the
+# problems of a batch; a last panel of one row, split otherwise than the others
+@pytest.mark.parametrize("b,M,N,K,a_layout,b_layout,c_layout", [
+    (1, 70001, 520, 2049, g.A_MK, g.B_KN, g.C_ROW), (1, 70001, 520, 2048, g.A_KM, g.B_KN, g.C_COL), (1, 513, 70003, 2049, g.A_MK, g.B_NK, g.C_ROW),
+    (1, 4001, 4001, 40001, g.A_MK, g.B_KN, g.C_COL), (1, 4001, 4003, 40001, g.A_KM, g.B_NK, g.C_ROW), (1, 257, 2056, 600001, g.A_MK, g.B_KN, g.C_ROW),
+    (41, 1001, 1003, 1801, g.A_MK, g.B_KN, g.C_ROW)])
+def test_copies_in_panels(b, M, N, K, a_layout, b_layout, c_layout):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+
+    def ints(*shape):
+        return torch.randint(-2, 3, shape, generator=gen, device="cuda", dtype=torch.int8).to(torch.bfloat16)
+
+    A, B = ints(b, *((M, K) if a_layout == g.A_MK else (K, M))), ints(b, *((K, N) if b_layout == g.B_KN else (N, K)))
+    C = ints(b, *((M, N) if c_layout == g.C_ROW else (N, M)))
+    old, got = C.clone(), C if c_layout == g.C_ROW else C.transpose(1, 2)
+    strides = (A.stride(0), B.stride(0)) if b > 1 else (0, 0)
+    need = _abi.call_workspace_bytes(A.data_ptr(), B.data_ptr(), M, N, K, A.stride(1), B.stride(1), b_layout, c_layout, a_layout, *strides, b)
+    ws = torch.full((need // 4 + 4,), float("nan"), device="cuda")
+    assert _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(1), B.stride(1), C.stride(1), b_layout, c_layout, a_layout, 1.0,
+                            *strides, M * N, b, need).startswith("copy+")
+    assert A.numel() * 2 + (B.numel() * 2 if B.stride(1) % 8 else 0) > 256 << 20
+    assert _abi.load().neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(1), B.stride(1), C.stride(1), a_layout, b_layout,
+                                            c_layout, 1.0, 1.0, *strides, M * N, b, ws.data_ptr(), need,
+                                            torch.cuda.current_stream().cuda_stream or None) == _abi.OK
+    assert bool(torch.isnan(ws[need // 4:]).all())
+    for i in range(b):
+        want = (A[i] if a_layout == g.A_MK else A[i].t()).float() @ (B[i] if b_layout == g.B_KN else B[i].t()).float()
+        want += (old[i] if c_layout == g.C_ROW else old[i].t()).float()
+        assert torch.equal(got[i], want.to(torch.bfloat16))
+
+
 # K of at most 128 with both operands K-major and enough tiles: one and two 64-deep units, whole and partial; rows and columns that end
 # inside a block, a run of column tiles per workgroup that does not divide them, C at odd addresses, alpha
 @pytest.mark.parametrize("b,M,N,K", [(32, 1024, 1024, 128), (40, 517, 801, 96), (1, 4100, 3001, 64), (7, 2048, 1000, 8), (300, 129, 129, 72), (1, 130, 60000, 104),
