@@ -2941,6 +2941,12 @@ static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, 
     }
   return best;
 }
+// What gemm_generic_kernel takes, which runs where nothing else does (a leading dimension of 2^21 or more): a round trip per 16 deep,
+// and 0.125 us for each 16x16 block of a CU (129 x 64 x 4096 118 us, 1024^3 148, 2048 x 2048 x 1024 527, 20000 x 64 x 128 24.8).
+static double generic_us(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
+  const double blocks = (double)ceil_div(M, 16) * ceil_div(N, 16) * (double)batch;
+  return 2.5 + ceil_div(K, 16) * (0.32 + 0.125 * __builtin_ceil(blocks / cus));
+}
 // Copies of the operands that are off the 16-byte grid (pack_kernel), and the product by the kernels for aligned ones.  The copies take
 // kPackMost bytes at most (two operands of 8191 x 8191): beyond it, or where a copy's rows would be 2^21 elements long, the product is made
 // in passes over some of the problems of a batch and over panels of C, which copy what they need of the operands one after the other.
@@ -2993,13 +2999,14 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
   const bool a = off_grid(A, lda, bt.sa, a_mk ? K : M), b = off_grid(B, ldb, bt.sb, b_nk ? K : N);
   if ((!a && !b) || K < 1) return false;
   const int cus = planning_cus();
+  const bool in_place = ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt);
   struct Memo {
     int64_t M = -1, N = -1, K = -1, count = -1;
     int a_layout = -1, b_layout = -1, c_layout = -1, cus = -1, what = -1;
     bool pays = false;
     PackPlan plan;
   };
-  const int what = a | b << 1 | (bt.sa != 0) << 2 | (bt.sb != 0) << 3;
+  const int what = a | b << 1 | (bt.sa != 0) << 2 | (bt.sb != 0) << 3 | in_place << 4;
   static thread_local Memo memo[32];
   static thread_local unsigned next = 0;
   const Memo* m = nullptr;
@@ -3019,7 +3026,8 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
       double aligned_us = 0;
       plan_model(p.rows, p.cols, K, true, c_layout, &v, &sp, p.count, b_layout, cus, bt.a_layout, &aligned_us);
       const bool row = c_layout == NEOGEMM_C_ROW;
-      const double other_us = ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, &bm, &bn, &sp) + 3.0;
+      const double other_us =
+          in_place ? ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, &bm, &bn, &sp) + 3.0 : generic_us(M, N, K, bt.count, cus);
       // a panel's copy of A is made again for each panel of columns, and a shared operand's panels for each part of the batch
       const int nb = ceil_div(bt.count, p.count), nr = ceil_div(M, p.rows), nc = ceil_div(N, p.cols);
       const double moved = (double)p.bytes_a * nr * (bt.sa ? nb : nr > 1 ? nb : 1) * (nr > 1 ? nc : 1) +

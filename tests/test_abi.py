@@ -234,6 +234,15 @@ def test_copies_stay_bounded_and_are_made_above_the_bound():
     assert ask(64, 64, 3000001, _abi.A_MK, _abi.B_KN)[1] == "generic"
 
 
+def test_long_rows_are_compared_with_the_kernel_that_would_run():
+    """No MFMA kernel reads rows 2^21 elements apart in place: copies against the scalar kernel (10007 us for the first shape on it)."""
+    p, q, c = 1 << 20, 1 << 40, 1 << 44
+    for (M, N, K, lda) in ((2097160, 256, 128, 2097160), (300, 264, 512, 1 << 21), (129, 64, 4096, (1 << 21) + 8)):
+        assert _abi.call_kernel(p, q, c, M, N, K, lda, N, N, _abi.B_KN, _abi.C_ROW, _abi.A_KM) in ("copy+tile", "copy+small")
+        assert _abi.call_workspace_bytes(p, q, M, N, K, lda, N, _abi.B_KN, _abi.C_ROW, _abi.A_KM) <= 256 << 20
+    assert _abi.call_kernel(p, q, c, 16, 16, 16, 1 << 21, 16, 16, _abi.B_KN, _abi.C_ROW, _abi.A_KM) == "generic"
+
+
 def test_plan_rejects_null_outputs():
     lib = _abi.load()
     assert lib.neogemm_bf16_plan(4, 4, 4, 0, 0, 1, None, None) == _abi.ERR_BAD_ARG

@@ -123,11 +123,11 @@ def test_copies_on_the_grid(b, M, N, K):
 
 
 # copies of more than 256 MiB in panels: of the rows, of the columns, of both (a panel of A copied for each panel of columns), of the
-# problems of a batch; a last panel of one row, split otherwise than the others
+# problems of a batch; a last panel of one row, split otherwise than the others; rows of A [K,M] 2^21 elements apart and more
 @pytest.mark.parametrize("b,M,N,K,a_layout,b_layout,c_layout", [
     (1, 70001, 520, 2049, g.A_MK, g.B_KN, g.C_ROW), (1, 70001, 520, 2048, g.A_KM, g.B_KN, g.C_COL), (1, 513, 70003, 2049, g.A_MK, g.B_NK, g.C_ROW),
     (1, 4001, 4001, 40001, g.A_MK, g.B_KN, g.C_COL), (1, 4001, 4003, 40001, g.A_KM, g.B_NK, g.C_ROW), (1, 257, 2056, 600001, g.A_MK, g.B_KN, g.C_ROW),
-    (41, 1001, 1003, 1801, g.A_MK, g.B_KN, g.C_ROW)])
+    (41, 1001, 1003, 1801, g.A_MK, g.B_KN, g.C_ROW), (1, 2097167, 264, 16, g.A_KM, g.B_KN, g.C_ROW)])
 def test_copies_in_panels(b, M, N, K, a_layout, b_layout, c_layout):
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
 
@@ -142,7 +142,7 @@ def test_copies_in_panels(b, M, N, K, a_layout, b_layout, c_layout):
     ws = torch.full((need // 4 + 4,), float("nan"), device="cuda")
     assert _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(1), B.stride(1), C.stride(1), b_layout, c_layout, a_layout, 1.0,
                             *strides, M * N, b, need).startswith("copy+")
-    assert A.numel() * 2 + (B.numel() * 2 if B.stride(1) % 8 else 0) > 256 << 20
+    assert A.numel() * 2 + (B.numel() * 2 if B.stride(1) % 8 else 0) > 256 << 20 or A.stride(1) >= 1 << 21
     assert _abi.load().neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(1), B.stride(1), C.stride(1), a_layout, b_layout,
                                             c_layout, 1.0, 1.0, *strides, M * N, b, ws.data_ptr(), need,
                                             torch.cuda.current_stream().cuda_stream or None) == _abi.OK
