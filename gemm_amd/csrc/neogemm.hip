@@ -2913,19 +2913,21 @@ static bool ragged_takes(const void* A, const void* B, int64_t M, int64_t N, int
   return K > 0 && ext_a >= 8 && ext_b >= 8 && lda < (1 << 21) && ldb < (1 << 21) && (((uintptr_t)A | (uintptr_t)B) & 1) == 0;
 }
 // Tile (bm x bn of the output as it lies in memory, rows x cols) and split of K of gemm_ragged_kernel, by the time of its K tiles;
-// returns the estimate.  A workgroup of the 64x64 tile takes 0.40 us per K tile where several share a CU (the loads at two-byte
+// returns the estimate for operands that come from HBM.  A workgroup of the 64x64 tile takes 0.40 us per K tile where several share a CU (the loads at two-byte
 // addresses bound it: 1023 x 2047 x 1535, 512 of them, 21 us), 0.29 alone on one (64 x 256 x 20001 in 16 splits, 14.5 us; the same
 // in 4, 26); one of the 128x128 tile, four times the work, 0.95 (1500 x 1501 x 1401: 25.3 us for 144 of them, 28.3 for 576 small
 // ones; 1023 x 2047 x 1535: 28 for 128).  A split costs the second launch and the partials (512 x 1024 x 10001 in 64x64 tiles:
-// 29 us with two, 47 unsplit).
-static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, int cus, int* bm, int* bn, int* split) {
+// 29 us with two, 47 unsplit).  From HBM a workgroup gains nothing by being alone on its CU unless K is in three parts or more
+// (1001 x 1024 x 4096 28 to 34 us, the estimate without this 21.6; 256 x 1024 x 8193 in four 22, 21.8), and a K tile takes 0.05 us more
+// with both operands MN-major (255 x 4096 x 4096, 256 workgroups: 35.8 us with both, 28.9 with B [N,K]).
+static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, int cus, bool both_mn, int* bm, int* bn, int* split) {
   struct Tile {
     int bm, bn;
     double alone_us, shared_us, fixed_us;  // per K tile of a workgroup that has its CU to itself / shares it
   };
   static const Tile kTiles[] = {{64, 64, 0.29, 0.40, 3.0}, {128, 64, 0.56, 0.56, 3.5}, {128, 128, 0.95, 0.95, 4.0}};
   const int64_t ktiles = ceil_div(K, KTILE);
-  double best = 1e300;
+  double best = 1e300, from_hbm = 0;
   for (const Tile& t : kTiles)
     for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
       if (sp > 1 && ktiles / sp < 4) break;
@@ -2934,12 +2936,13 @@ static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, 
       if (sp > 1) us += 5.0 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 4.0e6;
       if (us < best) {
         best = us;
+        from_hbm = us + per_cu * ceil_div(ktiles, sp) * ((per_cu > 1 || sp > 2 ? 0.0 : t.shared_us - t.alone_us) + (both_mn ? 0.05 : 0.0));
         *bm = t.bm;
         *bn = t.bn;
         *split = sp;
       }
     }
-  return best;
+  return from_hbm;
 }
 // What gemm_generic_kernel takes, which runs where nothing else does (a leading dimension of 2^21 or more): a round trip per 16 deep,
 // and 0.125 us for each 16x16 block of a CU (129 x 64 x 4096 118 us, 1024^3 148, 2048 x 2048 x 1024 527, 20000 x 64 x 128 24.8).
@@ -3027,16 +3030,17 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
       plan_model(p.rows, p.cols, K, true, c_layout, &v, &sp, p.count, b_layout, cus, bt.a_layout, &aligned_us);
       const bool row = c_layout == NEOGEMM_C_ROW;
       const double other_us =
-          in_place ? ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, &bm, &bn, &sp) + 3.0 : generic_us(M, N, K, bt.count, cus);
+          in_place ? ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, !a_mk && !b_nk, &bm, &bn, &sp) + 3.0 : generic_us(M, N, K, bt.count, cus);
       // a panel's copy of A is made again for each panel of columns, and a shared operand's panels for each part of the batch
       const int nb = ceil_div(bt.count, p.count), nr = ceil_div(M, p.rows), nc = ceil_div(N, p.cols);
       const double moved = (double)p.bytes_a * nr * (bt.sa ? nb : nr > 1 ? nb : 1) * (nr > 1 ? nc : 1) +
                            (double)p.bytes_b * nc * (bt.sb ? nb : nc > 1 ? nb : 1);
       // The copy and the product that waits for it: 6.5 us and 3 MB per us; in place: 3 us over ragged_plan's estimate, which compares its
-      // own tiles only.  Both ways measured at 68 sizes, one operand or both off the grid (us, copies / in place,
-      // A [M,K] and A [K,M]): 2001 x 2000 x 504 14.1 / 17.0 and 13.9 / 16.7, 10001 x 1024 x 512 26.0 / 38.3 and 27.2 / 34.7, 20001 x 2048 x
-      // 1024 104.5 / 157.6 and 105.5 / 149.9; below the line 1001 x 1024 x 1024 11.4 / 10.0 and 15.3 / 9.4, 1501 x 512 x 2048 19.5 / 14.7 and
-      // 24.8 / 16.2.  The choice costs 1.7 % over the better one on average (without the 3 us 4.2 %), 24 % at worst (201 x 4096 x 4096).
+      // own tiles only.  Both ways measured at 68 sizes with the operands in the caches and at 44 from HBM, one operand or both off the grid
+      // (us, copies / in place, A [M,K] and A [K,M]): 2001 x 2000 x 504 14.5 / 17.5 and 14.1 / 17.0, 201 x 4096 x 4096 26.7 / 31.3 and 26.7 /
+      // 36.9, 201 x 2048 x 8192 26.7 / 35.2 and 26.2 / 39.5, 10001 x 1024 x 512 26.0 / 38.3 and 27.2 / 34.7; below the line 777 x 784 x 776
+      // 11.6 / 11.8 and 16.9 / 11.3, 1501 x 512 x 2048 21.5 / 17.7 and 29.8 / 19.6.  The choice costs 1.7 % (1.8 % from HBM) over the better
+      // one on average, 43 % at worst (401 x 4096 x 4096, 0.4 us from the line); without the 3 us and the rates from HBM 4 % (8 %).
       e.pays = (double)nb * nr * nc * (aligned_us + 6.5) + moved / 3.0e6 < other_us;
       // (the last problems, rows and columns may be fewer, and split otherwise)
       for (const int64_t c : {p.count, bt.count % p.count})
@@ -3108,7 +3112,7 @@ static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, in
   if (!ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt)) return NEOGEMM_ERR_UNSUPPORTED;
   int bm = 128, bn = 128, split = 1;
   const bool row = c_layout == NEOGEMM_C_ROW;
-  ragged_plan(row ? M : N, row ? N : M, K, bt.count, planning_cus(), &bm, &bn, &split);
+  ragged_plan(row ? M : N, row ? N : M, K, bt.count, planning_cus(), false, &bm, &bn, &split);
   TileArgs a{};
   const bool a_mk = bt.a_layout == NEOGEMM_A_MK, b_nk = b_layout == NEOGEMM_B_NK;
   bool ak = a_mk, bk = b_nk;
@@ -3534,7 +3538,7 @@ size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M
   else if (neogemm::pack_plan(A, B, M, N, K, lda, ldb, b_layout, c_layout, bt, &pp))
     return pp.total();
   else if (neogemm::ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt))
-    neogemm::ragged_plan(row ? M : N, row ? N : M, K, batch, neogemm::planning_cus(), &v, &w, &s);
+    neogemm::ragged_plan(row ? M : N, row ? N : M, K, batch, neogemm::planning_cus(), false, &v, &w, &s);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)batch : 0;
 }
 

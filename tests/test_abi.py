@@ -203,12 +203,16 @@ def test_copies_are_made_where_they_pay():
                               ((10001, 1024, 512), "copy+tile"),    # 26.0 / 38.3, 27.2 / 34.7
                               ((5001, 1024, 304), "copy+tile"),     # 14.5 / 20.2, 13.0 / 17.9
                               ((1501, 1504, 1504), "copy+tile"),    # 20.0 / 30.9, 21.6 / 30.0
+                              ((201, 4096, 4096), "copy+tile"),     # 26.7 / 31.3, 26.7 / 36.9 (from HBM; a transposed A that torch copies: 31.4)
+                              ((255, 4096, 4096), None),            # 26.8 / 35.8 with both MN-major, where torch's copy makes it 32.5
                               ((1001, 1024, 1024), "ragged"),       # 11.4 / 10.0, 15.3 / 9.4
                               ((1501, 512, 2048), "ragged"),        # 19.5 / 14.7, 24.8 / 16.2
                               ((501, 256, 1024), "ragged")):        # 12.3 / 9.9, 14.2 / 9.1
         for a, lda, off in ((_abi.A_MK, K, 2), (_abi.A_KM, M, 0)):
             for b, ldb in ((_abi.B_KN, N), (_abi.B_NK, K)):
-                assert _abi.call_kernel((1 << 20) + off, 1 << 40, 1 << 44, M, N, K, lda, ldb, N, b, _abi.C_ROW, a) == better
+                want = better or ("copy+tile" if (a, b) == (_abi.A_KM, _abi.B_KN) else None)
+                got = _abi.call_kernel((1 << 20) + off, 1 << 40, 1 << 44, M, N, K, lda, ldb, N, b, _abi.C_ROW, a)
+                assert want in (None, got), (M, N, K, a, b)
 
 
 def test_copies_stay_bounded_and_are_made_above_the_bound():
