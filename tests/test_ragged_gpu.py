@@ -120,6 +120,28 @@ def test_copies_on_the_grid(b, M, N, K):
                     assert torch.equal(got, (want + add.float()).to(torch.bfloat16))
 
 
+# few rows of A off the grid beside a B on it: copies of A alone for the decode kernels, every number of row fragments, K whose last
+# chunk is part padding (B [K,N]; the k-rows behind K are NaN), K split
+@pytest.mark.parametrize("M,N,K,b_layout,kernel", [
+    (5, 2056, 1025, g.B_KN, "skinny"), (20, 4104, 1025, g.B_KN, "skinny"), (40, 12296, 4097, g.B_KN, "skinny"), (72, 12296, 3001, g.B_KN, "skinny"),
+    (96, 14344, 4097, g.B_KN, "skinny"), (40, 6152, 4097, g.B_KN, "strip"), (64, 6152, 6001, g.B_KN, "strip"), (16, 2056, 1024, g.B_NK, "skinny"),
+    (32, 2056, 1024, g.B_NK, "skinny"), (64, 2056, 1024, g.B_NK, "skinny"), (72, 12296, 3000, g.B_NK, "skinny"), (104, 4104, 3000, g.B_NK, "strip"),
+    (128, 4104, 4096, g.B_NK, "strip"), (72, 2056, 16384, g.B_NK, "strip")])
+@pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
+def test_copies_for_the_decode_kernels(M, N, K, b_layout, kernel, c_layout):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A, B = between_nans(gen, M, K, 0, 1), between_nans(gen, *((K, N) if b_layout == g.B_KN else (N, K)), 8, 8)
+    want = A.float() @ (B if b_layout == g.B_KN else B.t()).float()
+    C = torch.full((M, N) if c_layout == g.C_ROW else (N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
+    got = C if c_layout == g.C_ROW else C.t()
+    assert _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, K, B.stride(0), C.stride(0), b_layout, c_layout) == "copy+" + kernel
+    g.gemm_into(A, B, C, M, N, K, K, B.stride(0), C.stride(0), b_layout, c_layout)
+    assert torch.equal(got, want.to(torch.bfloat16))
+    old = got.clone()
+    g.gemm_into(A, B, C, M, N, K, K, B.stride(0), C.stride(0), b_layout, c_layout, alpha=0.5, beta=-1.0)
+    assert torch.equal(got, (0.5 * want - old.float()).to(torch.bfloat16))
+
+
 # copies of more than 256 MiB in panels: of the rows, of the columns, of both (a panel of A copied for each panel of columns), of the
 # problems of a batch; a last panel of one row, split otherwise than the others; rows of A [K,M] 2^21 elements apart and more
 @pytest.mark.parametrize("b,M,N,K,a_layout,b_layout,c_layout", [
