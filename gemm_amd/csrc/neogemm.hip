@@ -379,155 +379,122 @@ __device__ __forceinline__ void store_wave_tile(f32x4 (&acc)[TM][TN], const Tile
   // so that neither the 8-byte writes (16 rows per instruction) nor the 16-byte reads collide on banks.
   constexpr int CH = WTN / 8;        // 16-byte chunks per staged row
   constexpr int RPI = 64 / CH;       // rows one store instruction covers
-  constexpr bool CAN_STAGE = (size_t)NW * WTM * WTN * 2 <= (size_t)LDS_BYTES && CH >= 4 && CH <= 64;
-  // C may start at any element and have any leading dimension: a 16-byte store takes a two-byte address, at little cost (512 x 10001
-  // x 1024 17.8 us, 512 x 10000 x 1024 17.7; 4096 x 4095 x 4096 94.7 us, 4096^3 91.3; the generic kernel took 767 and 9137)
-  const bool stage = CAN_STAGE && p.ksplit == 1 && p.beta == 0.f;
+  static_assert((size_t)NW * WTM * WTN * 2 <= (size_t)LDS_BYTES && CH >= 4 && CH <= 64 && (CH & (CH - 1)) == 0, "the staged bf16 tiles of all waves fit the LDS");
   // beta != 0: staged as fp32 (the sum is rounded once), row tiles of the wave tile at a time, as many as the LDS holds
   constexpr int ST = TM % 4 == 0 && NW * 4 * 16 * WTN * 4 <= (int)LDS_BYTES ? 4 : TM % 2 == 0 && NW * 2 * 16 * WTN * 4 <= (int)LDS_BYTES ? 2 : 1;
-  constexpr bool CAN_STAGE_F32 = CAN_STAGE && (CH & (CH - 1)) == 0 && NW * ST * 16 * WTN * 4 <= (int)LDS_BYTES && ST * 16 % RPI == 0;
-  const bool stage_add = CAN_STAGE_F32 && p.ksplit == 1 && p.beta != 0.f;
-  if (stage) {
-    if constexpr (CAN_STAGE) {
-      // every wave is done with the slab images (its LDS reads have returned: the MFMAs that used them
-      // were issued; wait anyway) before any wave overwrites them; so are its direct-to-LDS loads (when K is
-      // short the prologue's fully masked zero fills of later images may still be in flight)
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      const uint32_t region = lds0 + (uint32_t)wave * (WTM * WTN * 2);
-      const int colc = lane % CH;
-      const int col = map.col(colc * 8);
+  static_assert(NW * ST * 16 * WTN * 4 <= (int)LDS_BYTES && ST * 16 % RPI == 0, "the staged fp32 row tiles of all waves fit the LDS");
+  // C may start at any element and have any leading dimension: a 16-byte store takes a two-byte address, at little cost (512 x 10001
+  // x 1024 17.8 us, 512 x 10000 x 1024 17.7; 4096 x 4095 x 4096 94.7 us, 4096^3 91.3; the generic kernel took 767 and 9137)
+  if (p.ksplit == 1 && p.beta == 0.f) {
+    // every wave is done with the slab images (its LDS reads have returned: the MFMAs that used them
+    // were issued; wait anyway) before any wave overwrites them; so are its direct-to-LDS loads (when K is
+    // short the prologue's fully masked zero fills of later images may still be in flight)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint32_t region = lds0 + (uint32_t)wave * (WTM * WTN * 2);
+    const int colc = lane % CH;
+    const int col = map.col(colc * 8);
 #pragma unroll
-      for (int i0 = 0; i0 < TM; i0 += STAGE_TM) {
-        // rows i0*16 .. of the wave tile are rows 0 .. of the staging region
-        auto park = [&](auto scaled) {
+    for (int i0 = 0; i0 < TM; i0 += STAGE_TM) {
+      // rows i0*16 .. of the wave tile are rows 0 .. of the staging region
+      auto park = [&](auto scaled) {
 #pragma unroll
-          for (int i = i0; i < i0 + STAGE_TM; ++i) {
-            const uint32_t row = (i - i0) * 16 + row_l;
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-              bf16x4 o;
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                float v = acc_get(acc[i][j][r]);
-                if constexpr (decltype(scaled)::value) v *= p.alpha;
-                o[r] = (__bf16)v;
-              }
-              const uint32_t c = 2 * j + (lane >> 5);
-              const uint32_t addr = region + row * (WTN * 2) + ((c ^ (row & (CH - 1))) << 4) + (((lane >> 4) & 1) << 3);
-              *((NEOGEMM_AS3 bf16x4*)(uintptr_t)addr) = o;
-            }
-          }
-        };
-        if (p.alpha == 1.f) park(std::false_type{});
-        else park(std::true_type{});
-        // same wave wrote and reads: LDS operations of a wave complete in order; the compiler orders them
-#pragma unroll
-        for (int st = 0; st < STAGE_TM * 16 / RPI; ++st) {
-          const uint32_t row = st * RPI + lane / CH;
-          const uint32_t addr = region + row * (WTN * 2) + (((uint32_t)colc ^ (row & (CH - 1))) << 4);
-          const bf16x8 v = *((NEOGEMM_AS3 bf16x8*)(uintptr_t)addr);
-          const int grow = map.row(i0 * 16 + (int)row);
-          if (grow < p.M) {
-            char* dst = gC + ((size_t)grow * p.ldc + col) * 2;
-            if (col + 7 < p.N) {
-              // C is written once and not read again here: streaming stores leave the L2 to A and B
-              __builtin_nontemporal_store((bf16x8_u)v, (bf16x8_u*)dst);
-            } else {
-#pragma unroll
-              for (int e = 0; e < 8; ++e)
-                if (col + e < p.N) ((__bf16*)dst)[e] = v[e];
-            }
-          }
-        }
-      }
-    }
-  } else if (stage_add) {
-    if constexpr (CAN_STAGE_F32) {
-      // C = alpha * acc + beta * C, the sum in fp32: the accumulators are parked as they are, ST row tiles at a time, and
-      // come back row-wise, eight columns a lane, beside the 16 bytes of C that they are added to.  All of C's old values
-      // are requested before the first of them is needed (up to 32 loads of a wave in flight; the fragments' registers are free).
-      // The branch below, which reads C two bytes at a time in the accumulators' layout, took 134 us at 4096^3 where the plain
-      // product takes 94; this one takes 98 (C read: 34 MB).
-      constexpr int CH4 = WTN / 4;  // 16-byte chunks per parked fp32 row
-      constexpr int NLD = WTM / RPI;
-      const int colc = lane % CH, col = map.col(colc * 8);
-      const bool whole_cols = col + 7 < p.N;
-      i32x4 old[NLD];
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // nothing of the main loop is on its way into LDS any more
-#pragma unroll
-      for (int st = 0; st < NLD; ++st) {
-        const int grow = map.row(st * RPI + lane / CH);
-        if (grow < p.M && whole_cols) old[st] = *(const i32x4_u*)(gC + ((size_t)grow * p.ldc + col) * 2);
-      }
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      const uint32_t region = lds0 + (uint32_t)wave * (ST * 16 * WTN * 4);
-#pragma unroll
-      for (int i0 = 0; i0 < TM; i0 += ST) {
-#pragma unroll
-        for (int i = i0; i < i0 + ST; ++i) {
+        for (int i = i0; i < i0 + STAGE_TM; ++i) {
           const uint32_t row = (i - i0) * 16 + row_l;
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
-            f32x4 v;
+            bf16x4 o;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = acc_get(acc[i][j][r]);
-            const uint32_t c = 4 * j + (lane >> 4);
-            *((NEOGEMM_AS3 f32x4*)(uintptr_t)(region + row * (WTN * 4) + ((c ^ (row & (CH4 - 1))) << 4))) = v;
+            for (int r = 0; r < 4; ++r) {
+              float v = acc_get(acc[i][j][r]);
+              if constexpr (decltype(scaled)::value) v *= p.alpha;
+              o[r] = (__bf16)v;
+            }
+            const uint32_t c = 2 * j + (lane >> 5);
+            const uint32_t addr = region + row * (WTN * 2) + ((c ^ (row & (CH - 1))) << 4) + (((lane >> 4) & 1) << 3);
+            *((NEOGEMM_AS3 bf16x4*)(uintptr_t)addr) = o;
           }
         }
+      };
+      if (p.alpha == 1.f) park(std::false_type{});
+      else park(std::true_type{});
+      // same wave wrote and reads: LDS operations of a wave complete in order; the compiler orders them
 #pragma unroll
-        for (int st = 0; st < ST * 16 / RPI; ++st) {
-          const uint32_t row = st * RPI + lane / CH;
-          f32x4 v[2];
+      for (int st = 0; st < STAGE_TM * 16 / RPI; ++st) {
+        const uint32_t row = st * RPI + lane / CH;
+        const uint32_t addr = region + row * (WTN * 2) + (((uint32_t)colc ^ (row & (CH - 1))) << 4);
+        const bf16x8 v = *((NEOGEMM_AS3 bf16x8*)(uintptr_t)addr);
+        const int grow = map.row(i0 * 16 + (int)row);
+        if (grow < p.M) {
+          char* dst = gC + ((size_t)grow * p.ldc + col) * 2;
+          if (col + 7 < p.N) {
+            // C is written once and not read again here: streaming stores leave the L2 to A and B
+            __builtin_nontemporal_store((bf16x8_u)v, (bf16x8_u*)dst);
+          } else {
 #pragma unroll
-          for (int h = 0; h < 2; ++h)
-            v[h] = *((NEOGEMM_AS3 f32x4*)(uintptr_t)(region + row * (WTN * 4) + (((2u * colc + h) ^ (row & (CH4 - 1))) << 4)));
-          const int grow = map.row(i0 * 16 + (int)row);
-          if (grow < p.M) {
-            char* dst = gC + ((size_t)grow * p.ldc + col) * 2;
-            if (whole_cols) {
-              const bf16x8 c = __builtin_bit_cast(bf16x8, old[i0 * 16 / RPI + st]);
-              bf16x8 o;
-#pragma unroll
-              for (int e = 0; e < 8; ++e) o[e] = (__bf16)__builtin_fmaf(p.beta, (float)c[e], v[e >> 2][e & 3] * p.alpha);
-              __builtin_nontemporal_store((bf16x8_u)o, (bf16x8_u*)dst);
-            } else {
-#pragma unroll
-              for (int e = 0; e < 8; ++e)
-                if (col + e < p.N)
-                  ((__bf16*)dst)[e] = (__bf16)__builtin_fmaf(p.beta, (float)((const __bf16*)dst)[e], v[e >> 2][e & 3] * p.alpha);
-            }
+            for (int e = 0; e < 8; ++e)
+              if (col + e < p.N) ((__bf16*)dst)[e] = v[e];
           }
         }
       }
     }
   } else if (p.ksplit == 1) {
+    // C = alpha * acc + beta * C, the sum in fp32: the accumulators are parked as they are, ST row tiles at a time, and
+    // come back row-wise, eight columns a lane, beside the 16 bytes of C that they are added to.  All of C's old values
+    // are requested before the first of them is needed (up to 32 loads of a wave in flight; the fragments' registers are free).
+    // (C read two bytes at a time in the accumulators' layout: 134 us at 4096^3 where the plain product takes 94; this way 98, C
+    // read: 34 MB.)
+    constexpr int CH4 = WTN / 4;  // 16-byte chunks per parked fp32 row
+    constexpr int NLD = WTM / RPI;
+    const int colc = lane % CH, col = map.col(colc * 8);
+    const bool whole_cols = col + 7 < p.N;
+    i32x4 old[NLD];
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // nothing of the main loop is on its way into LDS any more
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int row = map.row(i * 16 + row_l);
-      if (row >= p.M) continue;
-      char* crow = gC + (size_t)row * p.ldc * 2;
+    for (int st = 0; st < NLD; ++st) {
+      const int grow = map.row(st * RPI + lane / CH);
+      if (grow < p.M && whole_cols) old[st] = *(const i32x4_u*)(gC + ((size_t)grow * p.ldc + col) * 2);
+    }
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint32_t region = lds0 + (uint32_t)wave * (ST * 16 * WTN * 4);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int col = map.col(j * 16 + colq);
-        f32x4 v;
+    for (int i0 = 0; i0 < TM; i0 += ST) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = acc_get(acc[i][j][r]) * p.alpha;
-        if (p.beta != 0.f) {
+      for (int i = i0; i < i0 + ST; ++i) {
+        const uint32_t row = (i - i0) * 16 + row_l;
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (col + r < p.N) v[r] = __builtin_fmaf(p.beta, (float)*(const __bf16*)(crow + (size_t)(col + r) * 2), v[r]);
+        for (int j = 0; j < TN; ++j) {
+          f32x4 v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = acc_get(acc[i][j][r]);
+          const uint32_t c = 4 * j + (lane >> 4);
+          *((NEOGEMM_AS3 f32x4*)(uintptr_t)(region + row * (WTN * 4) + ((c ^ (row & (CH4 - 1))) << 4))) = v;
         }
-        const bf16x4 o = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
-        if (col + 3 < p.N) {
-          __builtin_nontemporal_store((bf16x4_u)o, (bf16x4_u*)(crow + (size_t)col * 2));
-        } else {
+      }
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (col + r < p.N) *(__bf16*)(crow + (size_t)(col + r) * 2) = o[r];
+      for (int st = 0; st < ST * 16 / RPI; ++st) {
+        const uint32_t row = st * RPI + lane / CH;
+        f32x4 v[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          v[h] = *((NEOGEMM_AS3 f32x4*)(uintptr_t)(region + row * (WTN * 4) + (((2u * colc + h) ^ (row & (CH4 - 1))) << 4)));
+        const int grow = map.row(i0 * 16 + (int)row);
+        if (grow < p.M) {
+          char* dst = gC + ((size_t)grow * p.ldc + col) * 2;
+          if (whole_cols) {
+            const bf16x8 c = __builtin_bit_cast(bf16x8, old[i0 * 16 / RPI + st]);
+            bf16x8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = (__bf16)__builtin_fmaf(p.beta, (float)c[e], v[e >> 2][e & 3] * p.alpha);
+            __builtin_nontemporal_store((bf16x8_u)o, (bf16x8_u*)dst);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (col + e < p.N)
+                ((__bf16*)dst)[e] = (__bf16)__builtin_fmaf(p.beta, (float)((const __bf16*)dst)[e], v[e >> 2][e & 3] * p.alpha);
+          }
         }
       }
     }
