@@ -1174,13 +1174,13 @@ hipError_t launch_chain(const TileArgs& a, bool bk, hipStream_t st) {
 
 // ---------------------------------------------------------------------------------------------
 // Operands at any address and with any leading dimension (an odd K or N, a view that starts in the middle of a row), which
-// gemm_generic_kernel computed at 14 TFLOP/s: 1023 x 2047 x 1535 416 us, 21 with this kernel (1024 x 2048 x 1536 by the tile
+// gemm_generic_kernel computed at 14 TFLOP/s: 1023 x 2047 x 1535 416 us, 19.5 with this kernel (1024 x 2048 x 1536 by the tile
 // kernels: 11); 512 x 1024 x 10001 767 us, 29.  The direct-to-LDS loads of the kernels above want 16-byte addresses; here a
 // chunk of eight elements is fetched into registers, which takes a two-byte address, and written to the same swizzled LDS
 // images.  The loads of tile t+3 are requested while tile t is computed (two register sets, two LDS images per operand), so that
-// a workgroup has 2.5 tiles on the way.  What bounds it is the vector memory path into the CU: 16-byte loads run at 43 B/clk
-// and CU from addresses that are a multiple of four, at 23 where every other row begins between two dwords, at 15 where all
-// do.  (Reading the dwords from the one a chunk begins in, with the fifth one by a load of its own, and shifting them together took 24 us.)
+// a workgroup has 2.5 tiles on the way.  What bounds it is the vector memory path into the CU: with nothing else going on, 16-byte
+// loads run at 60 B/clk and CU from addresses that are a multiple of four, at 34 where every other row begins between two dwords, at
+// 21 where all do.  (Reading the dwords from the one a chunk begins in, with the fifth one by a load of its own, and shifting them together took 24 us.)
 // What does not belong to the product: rows past the end of the output take the last row's place and columns past it
 // whatever lies there, in bounds, since they only reach elements that are not stored; what lies past the end of K is
 // zeroed on its way into LDS.  A chunk may reach past the end of its row, but past the end of the matrix only near its
@@ -1547,8 +1547,8 @@ hipError_t launch_shortk(TileArgs a, int run, hipStream_t st) {
 // tile of 64 rows).  What counts is the way to the first product and from the last one to C,
 // and how many CUs take part: gemm_tile_kernel takes B [K,N] in tiles of 128 columns at least, asks for three K tiles of each operand
 // before the first product, and leaves its main loop up to six K tiles before the end, to wait for every one of those with nothing
-// behind it.  704^3 with B [K,N] 10.4 -> 6.0 us, with B [N,K] 7.8 -> 5.6; 1024^3 10.3 -> 7.6 and 7.8 -> 7.0; 512^3 with B [K,N] 5.6 ->
-// 5.2; 512 x 512 x 2048 in four splits 10.4 -> 9.3; 400 x 744 x 904 12.0 -> 7.7.  Two stages are on the way while one is computed;
+// behind it.  704^3 with B [K,N] 10.4 -> 6.0 us, with B [N,K] 7.8 -> 5.6; 1024^3 10.3 -> 7.6 and 7.8 -> 6.9; 512^3 with B [K,N] 5.6 ->
+// 4.9; 512 x 512 x 2048 in four splits 10.4 -> 9.3; 400 x 744 x 904 12.0 -> 7.7.  Two stages are on the way while one is computed;
 // four or seven only make the start longer (1024^3 with B [N,K]: 7.0, 7.2 and 7.9 us).
 // R stages of 16 KiB (a 64-deep K tile of A and of B each, K-major or 64 k-rows of 64 columns, swizzled as in FragReader), one barrier
 // per stage: behind it stage t has landed and everyone is past stage t - 1, whose place takes stage t + R - 1.

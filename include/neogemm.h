@@ -96,7 +96,8 @@ extern "C" {
  *   B          [K,N] with ldb >= N (b_layout 0) or [N,K] with ldb >= K (b_layout 1)
  *   C          [M,N] row-major with ldc >= N (c_layout 0) or column-major with ldc >= M (c_layout 1)
  *   workspace  device scratch of at least neogemm_bf16_workspace_bytes(M,N,K) bytes, or NULL when
- *              that function returns 0 for the shape.  Only split-K paths use it (fp32 partials).
+ *              that function returns 0 for the shape.  Only split-K paths of operands on the 16-byte grid use it
+ *              (fp32 partials); neogemm_bf16_general also splits, and copies, operands off it.
  *
  * Unlike the reference (M,N,K % 64 == 0, nemgemmV03.cu:375) every M,N,K >= 0 is accepted; shapes or
  * pointers off the 16-byte grid (K % 8, ld % 8, alignment) run an MFMA kernel that takes any two-byte address.
@@ -135,8 +136,8 @@ size_t neogemm_bf16_batched_workspace_bytes(int64_t M, int64_t N, int64_t K, int
 /*
  * Every choice the calls above leave open in one: C = alpha * op(A) * op(B) + beta * C for `batch` problems, op(A) from
  * a_layout (lda >= K, or >= M for NEOGEMM_A_KM).  The wrappers use it for operands that are transposed views, which the
- * kernels read in place instead of a copy.  neogemm_bf16_general_workspace_bytes is what this call may use for these
- * layouts.  The reference takes both operands K-contiguous only (v01.cu:232-235).
+ * kernels read in place instead of a copy.  neogemm_bf16_general_workspace_bytes is what this call uses for operands on the
+ * 16-byte grid in these layouts (the partials of split K); for any others ask neogemm_bf16_call_workspace_bytes.  The reference takes both operands K-contiguous only (v01.cu:232-235).
  */
 int neogemm_bf16_general(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                          int64_t ldb, int64_t ldc, int a_layout, int b_layout, int c_layout, float alpha, float beta,
@@ -146,7 +147,8 @@ size_t neogemm_bf16_general_workspace_bytes(int64_t M, int64_t N, int64_t K, int
                                             int64_t batch);
 /*
  * What neogemm_bf16_general uses for exactly these operands.  Those that lie off the 16-byte grid (any pointer, leading
- * dimension, batch stride or K that is no multiple of 8 elements) run with less, or none, as well: K is then not split.
+ * dimension, batch stride or K that is no multiple of 8 elements) may be copied onto it, in at most 256 MiB at a time, beside the
+ * partials of split K; they run with less, or none, as well: in place, K not split.
  */
 size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                          int a_layout, int b_layout, int c_layout, int64_t stride_a, int64_t stride_b, int64_t batch);
