@@ -2884,9 +2884,11 @@ static bool ragged_takes(const void* A, const void* B, int64_t M, int64_t N, int
 // addresses bound it: 1023 x 2047 x 1535, 512 of them, 21 us), 0.29 alone on one (64 x 256 x 20001 in 16 splits, 14.5 us; the same
 // in 4, 26); one of the 128x128 tile, four times the work, 0.95 (1500 x 1501 x 1401: 25.3 us for 144 of them, 28.3 for 576 small
 // ones; 1023 x 2047 x 1535: 28 for 128).  A split costs the second launch and the partials (512 x 1024 x 10001 in 64x64 tiles:
-// 29 us with two, 47 unsplit).  From HBM a workgroup gains nothing by being alone on its CU unless K is in three parts or more
-// (1001 x 1024 x 4096 28 to 34 us, the estimate without this 21.6; 256 x 1024 x 8193 in four 22, 21.8), and a K tile takes 0.05 us more
-// with both operands MN-major (255 x 4096 x 4096, 256 workgroups: 35.8 us with both, 28.9 with B [N,K]).
+// 29 us with two, 47 unsplit).  From HBM a workgroup of the 64x64 tile gains nothing by being alone on its CU unless K is in three parts
+// or more (1001 x 1024 x 4096 28 to 34 us, the estimate without this 21.6; 256 x 1024 x 8193 in four 22, 21.8), and its K tile takes
+// 0.05 us more with both operands MN-major (255 x 4096 x 4096, 256 workgroups: 35.8 us with both, 28.9 with B [N,K]).  Every further
+// workgroup of the larger tiles on a CU costs its way in and out, 2 us (16231 x 672 x 69, three per CU: 21.8 us, the estimate without
+// this 9.7); those of the 64x64 tile are there at a time (3549 x 608 x 105, three per CU: 7.7 us, 5.4).
 static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, int cus, bool both_mn, int* bm, int* bn, int* split) {
   struct Tile {
     int bm, bn;
@@ -2903,7 +2905,9 @@ static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, 
       if (sp > 1) us += 5.0 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 4.0e6;
       if (us < best) {
         best = us;
-        from_hbm = us + per_cu * ceil_div(ktiles, sp) * ((per_cu > 1 || sp > 2 ? 0.0 : t.shared_us - t.alone_us) + (both_mn ? 0.05 : 0.0));
+        from_hbm = us;
+        if (t.bm * t.bn > 64 * 64) from_hbm += 2.0 * (per_cu - 1.0);
+        else if (per_cu == 1 && sp <= 2) from_hbm += ceil_div(ktiles, sp) * (t.shared_us - t.alone_us + (both_mn ? 0.05 : 0.0));
         *bm = t.bm;
         *bn = t.bn;
         *split = sp;
@@ -2997,17 +3001,17 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
       plan_model(p.rows, p.cols, K, true, c_layout, &v, &sp, p.count, b_layout, cus, bt.a_layout, &aligned_us);
       const bool row = c_layout == NEOGEMM_C_ROW;
       const double other_us =
-          in_place ? ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, !a_mk && !b_nk, &bm, &bn, &sp) + 3.0 : generic_us(M, N, K, bt.count, cus);
+          in_place ? 1.03 * ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, !a_mk && !b_nk, &bm, &bn, &sp) + 2.5 : generic_us(M, N, K, bt.count, cus);
       // a panel's copy of A is made again for each panel of columns, and a shared operand's panels for each part of the batch
       const int nb = ceil_div(bt.count, p.count), nr = ceil_div(M, p.rows), nc = ceil_div(N, p.cols);
       const double moved = (double)p.bytes_a * nr * (bt.sa ? nb : nr > 1 ? nb : 1) * (nr > 1 ? nc : 1) +
                            (double)p.bytes_b * nc * (bt.sb ? nb : nc > 1 ? nb : 1);
-      // The copy and the product that waits for it: 6.5 us and 3 MB per us; in place: 3 us over ragged_plan's estimate, which compares its
-      // own tiles only.  Both ways measured at 68 sizes with the operands in the caches and at 44 from HBM, one operand or both off the grid
+      // The copy and the product that waits for it: 6.5 us and 3 MB per us; in place: 3 % and 2.5 us over ragged_plan's estimate, which
+      // compares its own tiles only.  Both ways measured at 68 sizes with the operands in the caches and at 450 from HBM, one operand or both off the grid
       // (us, copies / in place, A [M,K] and A [K,M]): 2001 x 2000 x 504 14.5 / 17.5 and 14.1 / 17.0, 201 x 4096 x 4096 26.7 / 31.3 and 26.7 /
       // 36.9, 201 x 2048 x 8192 26.7 / 35.2 and 26.2 / 39.5, 10001 x 1024 x 512 26.0 / 38.3 and 27.2 / 34.7; below the line 777 x 784 x 776
-      // 11.6 / 11.8 and 16.9 / 11.3, 1501 x 512 x 2048 21.5 / 17.7 and 29.8 / 19.6.  The choice costs 1.7 % (1.8 % from HBM) over the better
-      // one on average, 43 % at worst (401 x 4096 x 4096, 0.4 us from the line); without the 3 us and the rates from HBM 4 % (8 %).
+      // 11.6 / 11.8 and 16.9 / 11.3, 1501 x 512 x 2048 21.5 / 17.7 and 29.8 / 19.6.  The choice costs 1.4 % (1.8 % from HBM) over the better
+      // one on average, 41 % at worst; without the 3 %, the 2.5 us and the costs from HBM 4 % (6 %).
       e.pays = (double)nb * nr * nc * (aligned_us + 6.5) + moved / 3.0e6 < other_us;
       // (the last problems, rows and columns may be fewer, and split otherwise)
       for (const int64_t c : {p.count, bt.count % p.count})

@@ -123,9 +123,9 @@ def test_copies_on_the_grid(b, M, N, K):
 # few rows of A off the grid beside a B on it: copies of A alone for the decode kernels, every number of row fragments, K whose last
 # chunk is part padding (B [K,N]; the k-rows behind K are NaN), K split
 @pytest.mark.parametrize("M,N,K,b_layout,kernel", [
-    (5, 2056, 1025, g.B_KN, "skinny"), (20, 4104, 1025, g.B_KN, "skinny"), (40, 12296, 4097, g.B_KN, "skinny"), (72, 12296, 3001, g.B_KN, "skinny"),
+    (5, 2056, 1025, g.B_KN, "skinny"), (20, 12296, 6001, g.B_KN, "skinny"), (40, 12296, 4097, g.B_KN, "skinny"), (72, 12296, 3001, g.B_KN, "skinny"),
     (96, 14344, 4097, g.B_KN, "skinny"), (40, 6152, 4097, g.B_KN, "strip"), (64, 6152, 6001, g.B_KN, "strip"), (16, 2056, 1024, g.B_NK, "skinny"),
-    (32, 2056, 1024, g.B_NK, "skinny"), (64, 2056, 1024, g.B_NK, "skinny"), (72, 12296, 3000, g.B_NK, "skinny"), (104, 4104, 3000, g.B_NK, "strip"),
+    (32, 2056, 1024, g.B_NK, "skinny"), (64, 8200, 3000, g.B_NK, "skinny"), (72, 12296, 3000, g.B_NK, "skinny"), (104, 4104, 3000, g.B_NK, "strip"),
     (128, 4104, 4096, g.B_NK, "strip"), (72, 2056, 16384, g.B_NK, "strip")])
 @pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
 def test_copies_for_the_decode_kernels(M, N, K, b_layout, kernel, c_layout):
