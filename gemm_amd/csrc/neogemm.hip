@@ -126,6 +126,9 @@ __device__ __forceinline__ i16x4 lds_read_tr16(uint32_t addr) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((NEOGEMM_AS3 i16x4*)(uintptr_t)addr);
 }
 
+// s_waitcnt's operand: at most `vm` vector loads and `lgkm` LDS operations on the way
+constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | 7 << 4 | lgkm << 8 | (vm >> 4) << 14; }
+
 template <int N, class Fn, int... I>
 __device__ __forceinline__ void static_for_impl(Fn&& fn, std::integer_sequence<int, I...>) {
   (fn(std::integral_constant<int, I>{}), ...);
@@ -1172,6 +1175,100 @@ hipError_t launch_chain(const TileArgs& a, bool bk, hipStream_t st) {
 }
 #endif
 
+// The four computing waves (2 x 2) of a workgroup whose other waves bring in the operands (gemm_roles_kernel, gemm_ragged_kernel): nst
+// stages of 64 deep through R images of a BM x 64 and a BN x 64 piece each, and the epilogue.  Barriers, in step with the other waves':
+// one when stage 0 is there; per stage t one behind which stage t + 1 is there and stage t may be overwritten; one when all is done.
+template <int BM, int BN, int R, bool AK, bool BK>
+__device__ __forceinline__ void compute_stages(const TileArgs& p, char* gC, int nst, int m0, int n0, int kz, int wave, int lane, uint32_t lds0) {
+  constexpr int WTM = BM / 2, WTN = BN / 2, TM = WTM / 16, TN = WTN / 16;
+  constexpr uint32_t A_IMG = BM * 128, STAGE = (BM + BN) * 128;
+  const int wm = wave >> 1, wn = wave & 1;
+  FragReader<BM, AK, TM> fa;
+  FragReader<BN, BK, TN> fb;
+  fa.init(lds0, wm * WTM, lane);
+  fb.init(lds0 + A_IMG, wn * WTN, lane);
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Fragments of what is being computed and of what comes behind it: stages, or slabs where two stages would not fit the registers
+  constexpr int NSL = TM * TN > 16 ? 1 : 2, NM = NSL * TM * TN;
+  bf16x8 a[2][NSL][TM], b[2][NSL][TN];
+  auto read = [&](auto set, uint32_t slot, int slab) {
+    constexpr int S = decltype(set)::value;
+#pragma unroll
+    for (int s = 0; s < NSL; ++s) {
+      const int sl = slab + s;
+      const uint32_t img = slot * STAGE;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[S][s][j] = fb.read(img + (BK ? 0 : sl * (BN * 64)), j, sl);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[S][s][i] = fa.read(img + (AK ? 0 : sl * (A_IMG / 2)), i, sl);
+    }
+  };
+  auto arrived = [] {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));  // (the builtin: the compiler then knows that the fragments have arrived)
+  };
+  auto meet = [] {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto products = [&](auto set) {
+    constexpr int S = decltype(set)::value;
+    static_for<NM>([&](auto mc) {
+      constexpr int m = decltype(mc)::value, s = m / (TM * TN), j = mfma_walk_c(TM, TN, m % (TM * TN)), i = mfma_walk_i(TM, TN, m % (TM * TN));
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[S][s][j], a[S][s][i], acc[i][j], 0, 0, 0);
+    });
+    // a read or two, a product, and so on: the reads of the four waves meet at one LDS and take longer than the products
+    constexpr int NR = (TM * (AK ? 1 : 2) + TN * (BK ? 1 : 2)) * NSL;
+    static_for<NM>([&](auto mc) {
+      constexpr int m = decltype(mc)::value, r = (m + 1) * NR / NM - m * NR / NM;
+      if constexpr (r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    });
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  read(S0{}, 0, 0);
+  if constexpr (NSL == 2) {
+    uint32_t slot = 1;  // of stage t + 1
+    auto step = [&](auto set, auto other) {
+      arrived();
+      meet();
+      read(other, slot, 0);  // (behind the last stage: a zero fill, not used)
+      slot = slot + 1 == R ? 0 : slot + 1;
+      products(set);
+    };
+    int t = 0;
+    for (; t + 1 < nst; t += 2) {
+      step(S0{}, S1{});
+      step(S1{}, S0{});
+    }
+    if (t < nst) step(S0{}, S1{});
+  } else {
+    uint32_t slot = 0;  // of stage t
+    for (int t = 0; t < nst; ++t) {
+      arrived();
+      __builtin_amdgcn_sched_barrier(0);
+      read(S1{}, slot, 1);
+      products(S0{});
+      slot = slot + 1 == R ? 0 : slot + 1;
+      arrived();
+      meet();
+      read(S0{}, slot, 0);
+      products(S1{});
+    }
+  }
+  arrived();
+  meet();
+  store_wave_tile<TM, TN, 4, R * STAGE, TM, false>(acc, p, gC, kz, lane, wave, lds0, BlockMap{m0 + wm * WTM, n0 + wn * WTN});
+}
+
 // ---------------------------------------------------------------------------------------------
 // Operands at any address and with any leading dimension (an odd K or N, a view that starts in the middle of a row), which
 // gemm_generic_kernel computed at 14 TFLOP/s: 1023 x 2047 x 1535 416 us, 19.5 with this kernel (1024 x 2048 x 1536 by the tile
@@ -1543,25 +1640,27 @@ hipError_t launch_shortk(TileArgs a, int run, hipStream_t st) {
 #endif
 
 // ---------------------------------------------------------------------------------------------
-// Small problems: a 64x64 tile, at most one of the operands MN-major (with both, and with a transposed A on the rows, the plan names no
-// tile of 64 rows).  What counts is the way to the first product and from the last one to C,
-// and how many CUs take part: gemm_tile_kernel takes B [K,N] in tiles of 128 columns at least, asks for three K tiles of each operand
-// before the first product, and leaves its main loop up to six K tiles before the end, to wait for every one of those with nothing
-// behind it.  704^3 with B [K,N] 10.4 -> 6.0 us, with B [N,K] 7.8 -> 5.6; 1024^3 10.3 -> 7.6 and 7.8 -> 6.9; 512^3 with B [K,N] 5.6 ->
-// 4.9; 512 x 512 x 2048 in four splits 10.4 -> 9.3; 400 x 744 x 904 12.0 -> 7.7.  Two stages are on the way while one is computed;
-// four or seven only make the start longer (1024^3 with B [N,K]: 7.0, 7.2 and 7.9 us).
-// R stages of 16 KiB (a 64-deep K tile of A and of B each, K-major or 64 k-rows of 64 columns, swizzled as in FragReader), one barrier
-// per stage: behind it stage t has landed and everyone is past stage t - 1, whose place takes stage t + R - 1.
+// Launches that give a CU one workgroup (two of the smallest tile): waves with roles.  In gemm_tile_kernel a wave issues its loads, its LDS
+// reads and its products in one stream, in order; a load holds it up for ~56 cycles and a read, which meets those of the other waves at one
+// LDS, for ~32, so a 64-deep stage of a 64x64 tile took 0.33 us (700 cycles, 128 of them products) however much was on the way, and one of a
+// 128x128 tile 0.45.  Here a workgroup has eight waves: four only load (one 64-deep stage of both operands after the other into a ring of R
+// images, a quarter each), four only read and compute (compute_stages), two waves to a SIMD, with one barrier per stage.  A stage of the 64x64
+// tile takes 0.21 us, of the 128x64 tile 0.30, of the 128x128 tile 0.36, of the wide ones 0.60 with operands in the caches: 1024^3 (the
+// reference's call) 7.2 -> 6.3 us, 1024 x 1024 x 4096 20.7 -> 15.3, 2048^3 20.2 -> 17.4, from HBM 25.2 -> 21.0, 768^3 6.7 -> 5.7, 256 x 4096 x 4096
+// 23.5 -> 15.1; roles_plan has the line against the other kernels.
+// Tiles 64x64 (R = 4: 64 KiB, two workgroups per CU), 128x64 (5), 128x128 (4), 256x128 and 128x256 (3), of operands in either order.  More images
+// do not help (64x64 with five and six: level in the caches, 1 to 3 % slower from HBM), nor does the ring without the roles (1024^3 7.2 us).
+// The images are laid out and swizzled as in Operand and FragReader, K-major 64 deep or two slabs of 32 k-rows.
 // ---------------------------------------------------------------------------------------------
-template <bool AK, bool BK>
-__global__ __launch_bounds__(256) void gemm_small_kernel(TileArgs p) {
-  constexpr int R = 3, BM = 64, BN = 64, NW = 4, TM = 2, TN = 2;
-  constexpr uint32_t HALF = 8192, STAGE = 2 * HALF, LDS_BYTES = R * STAGE;
+template <int BM, int BN, int R, bool AK, bool BK>
+__global__ __launch_bounds__(512, BM * BN <= 4096 ? 4 : 2) void gemm_roles_kernel(TileArgs p) {
+  constexpr uint32_t A_IMG = BM * 128, STAGE = (BM + BN) * 128;
+  constexpr int IA = BM / 32, IB = BN / 32, NL = IA + IB;  // loads of a stage per loading wave, 1 KiB each
+  static_assert((R - 1) * NL <= 63, "the wait counts must fit the counter");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(NEOGEMM_AS3 char*)smem;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
   int m0, n0, kz;
   tile_of_workgroup<BM, BN>(p, m0, n0, kz);
   const int k_begin = kz * p.ktiles_per_split * KTILE;
@@ -1569,89 +1668,84 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(TileArgs p) {
   if (k_end > p.K) k_end = p.K;
   const int klen = k_end - k_begin, nst = (klen + KTILE - 1) / KTILE;
 
-  // this wave's loads of a stage: two of 1 KiB per operand, eight rows or k-rows each (see Operand::init); `key`: depth of the chunk
-  uint32_t voa[2], vob[2];
-  int keya[2], keyb[2];
-  auto offsets = [&](auto kmaj, uint32_t (&vo)[2], int (&key)[2], long ld, int rows_left) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const uint32_t r = (wave * 2 + j) * 8 + (lane >> 3);
+  if (__builtin_amdgcn_readfirstlane(tid >> 8)) {
+    // ---- a wave that loads: which 16 bytes a lane fetches for each of its loads of a stage (see Operand::init); `key`: depth of the chunk
+    uint32_t voa[IA], vob[IB];
+    int keya[IA], keyb[IB];
+    auto offsets = [&](auto kmaj, auto rowsc, auto& vo, auto& key, long ld, int rows_left) {
       constexpr bool KM = decltype(kmaj)::value;
-      const uint32_t c = (lane & 7) ^ (KM ? swz_k(r) : swz_mn64(r & 31));
-      vo[j] = r * (uint32_t)ld * 2 + c * 16 + VOFF_BIAS - j * 1024;
-      if ((KM ? (int)r : (int)c * 8) >= rows_left) vo[j] = OOB_OFFSET;
-      key[j] = KM ? (int)c * 8 : (int)r;
-    }
-  };
-  offsets(std::integral_constant<bool, AK>{}, voa, keya, p.lda, p.M - m0);
-  offsets(std::integral_constant<bool, BK>{}, vob, keyb, p.ldb, p.N - n0);
-  const uint64_t baseA = (uint64_t)p.A + ((uint64_t)blockIdx.z * p.bsa + (AK ? (uint64_t)m0 * p.lda + k_begin : (uint64_t)k_begin * p.lda + m0)) * 2 - VOFF_BIAS;
-  const uint64_t baseB = (uint64_t)p.B + ((uint64_t)blockIdx.z * p.bsb + (BK ? (uint64_t)n0 * p.ldb + k_begin : (uint64_t)k_begin * p.ldb + n0)) * 2 - VOFF_BIAS;
-  const uint64_t advA = (AK ? (uint64_t)KTILE : (uint64_t)KTILE * p.lda) * 2, advB = (BK ? (uint64_t)KTILE : (uint64_t)KTILE * p.ldb) * 2;
-  auto issue = [&](int t, uint32_t slot) {
-    const int krem = klen - t * KTILE;
-    auto load = [&](uint64_t b, const uint32_t (&vo)[2], const int (&key)[2], uint32_t dst) {
-      const i32x4 rs = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), (int)0x80000000u, 0x00020000};
-      dma_set_m0(dst + wave * 2048);
-      static_for<2>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        dma16<j * 1024>(rs, key[j] < krem ? vo[j] : OOB_OFFSET);
-      });
+      constexpr int ROWS = decltype(rowsc)::value, I = ROWS / 32, CPR = KM ? 8 : ROWS / 8;
+#pragma unroll
+      for (int j = 0; j < I; ++j) {
+        const uint32_t r = (wave * I + j) * (64 / CPR) + lane / CPR;  // row of the tile, or k-row
+        const uint32_t c = (lane % CPR) ^ (KM ? swz_k(r) : swz_mn_rows<ROWS>(r & 31));
+        vo[j] = r * (uint32_t)ld * 2 + c * 16 + VOFF_BIAS - (j & 3) * 1024;
+        if ((KM ? (int)r : (int)c * 8) >= rows_left) vo[j] = OOB_OFFSET;
+        key[j] = KM ? (int)c * 8 : (int)r;
+      }
     };
-    load(baseA + (uint64_t)t * advA, voa, keya, lds0 + slot * STAGE);
-    load(baseB + (uint64_t)t * advB, vob, keyb, lds0 + slot * STAGE + HALF);
-  };
-  FragReader<BM, AK, TM> fa;
-  FragReader<BN, BK, TN> fb;
-  fa.init(lds0, wm * 32, lane);
-  fb.init(lds0 + HALF, wn * 32, lane);
-  f32x4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  for (int t = 0; t < R - 1 && t < nst; ++t) issue(t, t);
-  uint32_t slot = 0, slot_ld = R - 1;
-  for (int t = 0; t < nst; ++t) {
-    if (t + 1 < nst) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");  // all but the stage behind it
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of stage t - 1 have returned
+    offsets(std::integral_constant<bool, AK>{}, std::integral_constant<int, BM>{}, voa, keya, p.lda, p.M - m0);
+    offsets(std::integral_constant<bool, BK>{}, std::integral_constant<int, BN>{}, vob, keyb, p.ldb, p.N - n0);
+    const uint64_t baseA = (uint64_t)p.A + ((uint64_t)blockIdx.z * p.bsa + (AK ? (uint64_t)m0 * p.lda + k_begin : (uint64_t)k_begin * p.lda + m0)) * 2 - VOFF_BIAS;
+    const uint64_t baseB = (uint64_t)p.B + ((uint64_t)blockIdx.z * p.bsb + (BK ? (uint64_t)n0 * p.ldb + k_begin : (uint64_t)k_begin * p.ldb + n0)) * 2 - VOFF_BIAS;
+    const uint64_t advA = (AK ? (uint64_t)KTILE : (uint64_t)KTILE * p.lda) * 2, advB = (BK ? (uint64_t)KTILE : (uint64_t)KTILE * p.ldb) * 2;
+    // all loads of stage t into its slot; past the end of K as zero fills (resource size 0): the counts of loads in flight hold for any K
+    auto issue = [&](int t, uint32_t slot) {
+      const int krem = klen - t * KTILE;
+      auto part = [&](auto& vo, auto& key, uint64_t b, uint32_t dst, auto count) {
+        const i32x4 rs = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), t < nst ? (int)0x80000000u : 0, 0x00020000};
+        static_for<decltype(count)::value>([&](auto jc) {
+          constexpr int j = decltype(jc)::value;
+          if constexpr (j % 4 == 0) dma_set_m0(dst + j * 1024);
+          dma16<(j & 3) * 1024>(rs, key[j] < krem ? vo[j] : OOB_OFFSET);
+        });
+      };
+      part(voa, keya, baseA + (uint64_t)t * advA, lds0 + slot * STAGE + wave * IA * 1024, std::integral_constant<int, IA>{});
+      part(vob, keyb, baseB + (uint64_t)t * advB, lds0 + slot * STAGE + A_IMG + wave * IB * 1024, std::integral_constant<int, IB>{});
+    };
+    for (int t = 0; t < R; ++t) issue(t, t);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * NL) : "memory");
     __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (t + R - 1 < nst) issue(t + R - 1, slot_ld);
-    const uint32_t img = slot * STAGE;
-    bf16x8 a[2][TM], b[2][TN];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) a[s][i] = fa.read(img + (AK ? 0 : s * 4096), i, s);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) b[s][j] = fb.read(img + (BK ? 0 : s * 4096), j, s);
+    uint32_t slot = 0;
+    for (int t = 0; t < nst; ++t) {
+      // stage t + 1 has landed (this wave's part of it); behind the barrier everyone's, and stage t is in the other waves' registers
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * NL) : "memory");
+      __builtin_amdgcn_s_barrier();
+      issue(t + R, slot);
+      slot = slot + 1 == R ? 0 : slot + 1;
     }
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][j], a[s][i], acc[i][j], 0, 0, 0);
-    slot = slot + 1 == R ? 0 : slot + 1;
-    slot_ld = slot_ld + 1 == R ? 0 : slot_ld + 1;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the zero fills are done before the epilogue takes the LDS
+    __builtin_amdgcn_s_barrier();
+    return;
   }
-  store_wave_tile<TM, TN, NW, LDS_BYTES, TM, false>(acc, p, p.C + (size_t)blockIdx.z * p.bsc * 2, kz, lane, wave, lds0, BlockMap{m0 + wm * 32, n0 + wn * 32});
+
+  // ---- a wave that computes
+  compute_stages<BM, BN, R, AK, BK>(p, p.C + (size_t)blockIdx.z * p.bsc * 2, nst, m0, n0, kz, wave, lane, lds0);
 }
 
-hipError_t launch_small(const TileArgs& a, bool ak, bool bk, hipStream_t st);
+// bm x bn: 64x64, 128x64 or 128x128
+hipError_t launch_roles(const TileArgs& a, int bm, int bn, bool ak, bool bk, hipStream_t st);
 #if NEOGEMM_HAS_PART(9)
-hipError_t launch_small(const TileArgs& a, bool ak, bool bk, hipStream_t st) {
-  const size_t lds = 3 * 16384;
-  dim3 grid(a.ntm * a.ntn * a.ksplit, 1, a.batch), block(256);
-  auto go = [&](auto kern) -> hipError_t {
-    kern<<<grid, block, lds, st>>>(a);
-    return hipGetLastError();
+hipError_t launch_roles(const TileArgs& a, int bm, int bn, bool ak, bool bk, hipStream_t st) {
+  dim3 grid(a.ntm * a.ntn * a.ksplit, 1, a.batch), block(512);
+  auto pick = [&](auto mc, auto nc, auto rc) -> hipError_t {
+    constexpr int BM = decltype(mc)::value, BN = decltype(nc)::value, R = decltype(rc)::value;
+    auto go = [&](auto kern) -> hipError_t {
+      const size_t lds = (size_t)R * (BM + BN) * 128;
+      if (lds > 65536)
+        if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
+      kern<<<grid, block, lds, st>>>(a);
+      return hipGetLastError();
+    };
+    if (ak) return bk ? go(gemm_roles_kernel<BM, BN, R, true, true>) : go(gemm_roles_kernel<BM, BN, R, true, false>);
+    return bk ? go(gemm_roles_kernel<BM, BN, R, false, true>) : go(gemm_roles_kernel<BM, BN, R, false, false>);
   };
-  if (ak) return bk ? go(gemm_small_kernel<true, true>) : go(gemm_small_kernel<true, false>);
-  return bk ? go(gemm_small_kernel<false, true>) : hipErrorInvalidValue;
+  using std::integral_constant;
+  if (bm == 64 && bn == 64) return pick(integral_constant<int, 64>{}, integral_constant<int, 64>{}, integral_constant<int, 4>{});
+  if (bm == 128 && bn == 64) return pick(integral_constant<int, 128>{}, integral_constant<int, 64>{}, integral_constant<int, 5>{});
+  if (bm == 128 && bn == 128) return pick(integral_constant<int, 128>{}, integral_constant<int, 128>{}, integral_constant<int, 4>{});
+  if (bm == 256) return pick(integral_constant<int, 256>{}, integral_constant<int, 128>{}, integral_constant<int, 3>{});
+  return pick(integral_constant<int, 128>{}, integral_constant<int, 256>{}, integral_constant<int, 3>{});
 }
 #endif
 
@@ -2687,15 +2781,17 @@ static const std::vector<PlanEntry>& plan_table() {
   }();
   return table;
 }
-static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
-                          int64_t batch, int b_layout, int ncus, int a_layout);
+static bool plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
+                          int64_t batch, int b_layout, int ncus, int a_layout, double* estimate_us);
 // The cost model walks every (tile, split) candidate: a few microseconds on the host, as long as a small GEMM takes
 // on the GPU.  A caller in a loop repeats a handful of shapes, so each thread remembers its last few answers.
+// estimate_us: the model's, or 0 where a table of the user's names the kernel.
 static void plan(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
-                 int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int a_layout = NEOGEMM_A_MK) {
+                 int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int a_layout = NEOGEMM_A_MK, double* estimate_us = nullptr) {
   struct Memo {
     int64_t M = -1, N = -1, K = -1, batch = -1;
     int a_layout = -1, b_layout = -1, c_layout = -1, aligned = -1, ncus = -1, variant = 0, split_k = 0;
+    double estimate_us = 0;
   };
   static thread_local Memo memo[32];  // the workspace query alone asks for four layouts of a shape
   static thread_local unsigned next = 0;
@@ -2705,10 +2801,14 @@ static void plan(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, in
         m.aligned == (int)aligned && m.ncus == ncus && m.a_layout == a_layout) {
       *variant = m.variant;
       *split_k = m.split_k;
+      if (estimate_us) *estimate_us = m.estimate_us;
       return;
     }
-  plan_uncached(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout);
+  double us = 0;
+  if (plan_uncached(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout, &us)) us = 0;
+  if (estimate_us) *estimate_us = us;
   Memo& m = memo[next++ & 31];
+  m.estimate_us = us;
   m.M = M, m.N = N, m.K = K, m.batch = batch, m.b_layout = b_layout, m.c_layout = c_layout, m.aligned = (int)aligned;
   m.ncus = ncus, m.a_layout = a_layout;
   m.variant = *variant, m.split_k = *split_k;
@@ -2721,8 +2821,10 @@ static const int kDefaultPlanCus = 256;
 static const PlanEntry kDefaultPlan[] = {
 #include "neogemm_default_plan.inc"
 };
-static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
-                          int64_t batch, int b_layout, int ncus, int a_layout) {
+// true: the choice of the user's table
+static bool plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
+                          int64_t batch, int b_layout, int ncus, int a_layout, double* estimate_us) {
+  plan_model(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout, estimate_us);
   if (aligned && K > 0 && batch == 1 && a_layout == NEOGEMM_A_MK) {
     auto match = [&](const PlanEntry& e) {
       return e.M == M && e.N == N && e.K == K && e.c_layout == c_layout && e.b_layout == b_layout;
@@ -2731,17 +2833,104 @@ static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_l
       if (match(e)) {
         *variant = e.variant;
         *split_k = e.variant == NEOGEMM_VARIANT_GENERIC ? 1 : e.split_k;
-        return;
+        return true;
       }
     if (ncus == kDefaultPlanCus)
       for (const PlanEntry& e : kDefaultPlan)
         if (match(e)) {
           *variant = e.variant;
           *split_k = e.split_k;
-          return;
+          break;
         }
   }
-  plan_model(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout);
+  return false;
+}
+
+// Whether gemm_roles_kernel takes a call that the plan gives to kernel v with split_max splits of K, estimated at plan_us; in the kernel's
+// terms: `rows` x `cols` of C as it lies in memory, ak / bk: the row / column operand has K-contiguous rows, lda / ldb their leading dimensions.
+// Fitted to 3300 timings of 600 problems with these tiles (64 to 6000 rows and columns, 128 to 65000 deep, both layouts of each operand,
+// batches; the operands in the caches and from HBM, the mean of both), rms 8 %: a launch, a way in and out per round of workgroups, per 64
+// deep what a stage takes, more where rows of an operand are no whole cache lines apart (a piece of 128 bytes then lies in two lines, and
+// is requested twice), and the reduction.  A CU holds two workgroups of the 64x64 tile, which then take 1.8 times as long, and one of the others.
+// The best of these by estimate is 0.8 % behind the best measured on average.  It is taken where it beats the plan's estimate times a factor
+// by planned tile (64x128 and 128x128 tiles take 1.35 and 1.2 times their estimates, and in one round of 128 rows and more the roles were at most
+// 2 % behind): 485 of 790 problems, 9 % faster on average over all of them (2048^3 from HBM 23.2 -> 20.8 us, 512 x 4096 x 4096 31.4 -> 26.7,
+// 1024 x 1024 x 2048 14.3 -> 11.8), 10 of them more than 3 % slower.  Short K and several rounds of planned workgroups count for less: the way in
+// and out of a workgroup is longer here, and a CU holds one (18 x 576 x 576 x 96 8.6 us in 128x128 tiles of gemm_tile_kernel, of which a CU holds two,
+// 11.8 here; 10001 x 1024 x 512 with a transposed A 17.5 and 21; 4096^3 in one-round tiles 91 and 124).  Not where the plan names strips (124 x
+// 5248 x 20608 from HBM 57.7 -> 60.9), 256x256 tiles or 192x256 ones with K split (304 x 1864 x 50048 80 -> 95).
+// No more splits than planned: what a caller's workspace holds, or whether one is needed, does not change.
+struct RolesPlan {
+  int bm = 0, bn = 0, split = 1;  // bm == 0: not taken
+};
+static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, int64_t cols, int64_t K, int64_t batch, bool ak, bool bk,
+                            int64_t lda, int64_t ldb) {
+  double against = 0;
+  switch (v) {
+    case NEOGEMM_VARIANT_T64x128_W4:
+    case NEOGEMM_VARIANT_T64x64_W4: against = 1.4; break;
+    case NEOGEMM_VARIANT_T96x128_W4: against = 1.8; break;
+    case NEOGEMM_VARIANT_T128x128_W4: against = 2.0; break;
+    case NEOGEMM_VARIANT_T256x128_W4:
+    case NEOGEMM_VARIANT_T128x256_W4: against = 1.4; break;
+    case NEOGEMM_VARIANT_T192x256_W4: against = split_max == 1 ? 1.0 : 0.0; break;
+    default: break;
+  }
+  if (against == 0) return RolesPlan();
+  const int cus = planning_cus();
+  if (K <= 256 && against > 1.2) against = 1.2;
+  if ((double)ceil_div(rows, kVariants[v].bm) * (double)ceil_div(cols, kVariants[v].bn) * split_max * (double)batch > 2.0 * cus && against > 1.0) against = 1.0;
+  const bool a_whole = (lda & 63) == 0, b_whole = (ldb & 63) == 0;
+  struct Memo {
+    int64_t rows = -1, cols = -1, K = -1, batch = -1;
+    int v = -1, split_max = -1, cus = -1, what = -1;
+    double plan_us = -1;
+    RolesPlan plan;
+  };
+  const int what = (int)ak | (int)bk << 1 | (int)a_whole << 2 | (int)b_whole << 3;
+  static thread_local Memo memo[32];
+  static thread_local unsigned next = 0;
+  for (const Memo& m : memo)
+    if (m.rows == rows && m.cols == cols && m.K == K && m.batch == batch && m.v == v && m.split_max == split_max && m.cus == cus && m.what == what &&
+        m.plan_us == plan_us)
+      return m.plan;
+  struct Tile {
+    int bm, bn, per_cu;
+    double fixed_us, stage_us, full_us;  // per workgroup; per stage on an empty chip, and how much more on a full one
+  };
+  static const Tile kTiles[] = {{64, 64, 2, 1.07, 0.188, 0.022}, {128, 64, 1, 1.36, 0.274, 0.056}, {128, 128, 1, 2.14, 0.355, 0.086},
+                                {256, 128, 1, 3.77, 0.576, 0.036}, {128, 256, 1, 4.70, 0.583, 0.029}};
+  const int64_t ktiles = ceil_div(K, KTILE);
+  const double floor_us = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch / 6.0e6;
+  double best = against * plan_us;
+  RolesPlan p;
+  for (const Tile& t : kTiles) {
+    // further lines a piece of an operand's row touches: one in two for 128 bytes along K, 64 columns of an MN-major operand likewise
+    auto more = [](bool kmaj, bool whole, int w) { return whole ? 0.0 : kmaj ? 1.0 : 64.0 / w; };
+    const double lines = (t.bm * more(ak, a_whole, t.bm) + t.bn * more(bk, b_whole, t.bn)) / (t.bm + t.bn);
+    for (int sp : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+      if (sp > split_max || (sp > 1 && ktiles / sp < 4)) break;
+      const double per = (double)ceil_div(ktiles, sp), wgs = (double)ceil_div(rows, t.bm) * (double)ceil_div(cols, t.bn) * sp * (double)batch;
+      if (wgs > 2.0 * cus) break;
+      const double one = t.stage_us * (1.0 + 0.46 * lines), full = t.fixed_us + per * (one + t.full_us);
+      double us = 2.9;
+      if (wgs <= cus) us += t.fixed_us + per * (one + t.full_us * wgs / cus);
+      else if (t.per_cu == 2) us += t.fixed_us + per * (one + t.full_us) * 1.8;
+      else us += full + t.fixed_us + per * (one + t.full_us * (wgs - cus) / cus);
+      if (us < floor_us) us = floor_us + 0.01 * us;
+      if (sp > 1) us += 2.0 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 2.65e6;
+      if (us < best) {
+        best = us;
+        p.bm = t.bm;
+        p.bn = t.bn;
+        p.split = sp;
+      }
+    }
+  }
+  Memo& m = memo[next++ & 31];
+  m.rows = rows, m.cols = cols, m.K = K, m.batch = batch, m.v = v, m.split_max = split_max, m.cus = cus, m.what = what, m.plan_us = plan_us;
+  m.plan = p;
+  return p;
 }
 
 // The largest split-K factor plan() returns for this shape over the four (b_layout, c_layout) combinations a call can
@@ -3163,10 +3352,11 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                                               NEOGEMM_VARIANT_GENERIC, 1, 0, nullptr, alpha, beta, bt);
   };
   int v = variant, s = split_k;
+  double plan_us = 0;
   if (v == NEOGEMM_VARIANT_AUTO) {
     if (!aligned) return unaligned();
     int pv, ps;
-    plan(M, N, K, aligned, c_layout, &pv, &ps, bt.count, b_layout, bt.a_layout);
+    plan(M, N, K, aligned, c_layout, &pv, &ps, bt.count, b_layout, bt.a_layout, &plan_us);
     v = pv;
     if (s == 0) s = ps;
     // a C that is not on 8-byte addresses (bt.sc: any problem of a batch) needs no workspace: such calls always ran, unsplit, without one
@@ -3200,8 +3390,16 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
 
   if (!aligned) return NEOGEMM_ERR_UNSUPPORTED;
 
-  if (v == NEOGEMM_VARIANT_SKINNY16 || v == NEOGEMM_VARIANT_SKINNY32 || v == NEOGEMM_VARIANT_SKINNY64 ||
-      v == NEOGEMM_VARIANT_SKINNY128 || v == NEOGEMM_VARIANT_STRIP) {
+  // gemm_roles_kernel takes any rows and columns of a K-major operand, whole chunks of an MN-major one
+  RolesPlan roles;
+  {
+    const bool row = c_layout == NEOGEMM_C_ROW, b_nk = b_layout == NEOGEMM_B_NK, rk = row ? a_mk : b_nk, ck = row ? b_nk : a_mk;
+    const int64_t rows = row ? M : N, cols = row ? N : M;
+    if (plan_us > 0 && split_k == 0 && (rk || (rows & 7) == 0 || bt.padded) && (ck || (cols & 7) == 0 || bt.padded))
+      roles = roles_plan(v, s, plan_us, rows, cols, K, bt.count, rk, ck, row ? lda : ldb, row ? ldb : lda);
+  }
+  if (!roles.bm && (v == NEOGEMM_VARIANT_SKINNY16 || v == NEOGEMM_VARIANT_SKINNY32 || v == NEOGEMM_VARIANT_SKINNY64 ||
+                    v == NEOGEMM_VARIANT_SKINNY128 || v == NEOGEMM_VARIANT_STRIP)) {
     // what the skinny kernel assumes: M within its rows, whole 16-byte chunks of B [K,N] inside the matrix,
     // one problem.  If M is too large but N fits and B is [N,K], it runs the transposed problem
     // C^T = B * A^T: its small operand is B then, its wide one A, and the layout of C flips.
@@ -3308,10 +3506,11 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   // (the chained 256x256 kernel takes its rows from a K-major operand only, K in whole periods of 128 and no split)
   const bool fits = (ak || mn_ok(vi.bm, a.M)) && (bk || mn_ok(vi.bn, a.N)) &&
                     (v != NEOGEMM_VARIANT_C256x256_W4 || (ak && K % (2 * KTILE) == 0 && s <= 1));
-  // Where the plan says 64 rows per tile, gemm_small_kernel takes over, with B [K,N] on the rows too (a column-major C; that went to the
-  // 128x128 tile), as long as the 64x64 tiles fit the CUs one and a half times (B [N,K]: 1152^3, 324 of them, 10.6 -> 9.0 us, 1280^3, 400, level, 1024 x 2048 x 1536, 512, 11.8 and 12.4) or twice
-  // (B [K,N]: 13.7 and 12.5 for that last one).  Few workgroups with whole trips of the tile kernel's main loop stay there: 256 x 1024 x
-  // 1024, 64 of them, 5.9 us and 6.7 with B [N,K], 7.1 and 7.3 with B [K,N]; 200 x 1000 x 1000 with B [K,N] 9.3 and 7.6.
+  // Where the plan says 64 rows per tile and roles_plan does not take the call, 64x64 tiles of gemm_roles_kernel do, with B [K,N] on the rows
+  // too (a column-major C; that went to the 128x128 tile), as long as they fit the CUs one and a half times (B [N,K]: 1152^3, 324 of them, 10.6 us
+  // in tiles of gemm_tile_kernel and 9.0, 1280^3, 400, level, 1024 x 2048 x 1536, 512, 11.8 and 12.4) or twice (B [K,N]: 13.7 and 12.5 for that last
+  // one).  Few workgroups with whole trips of the tile kernel's main loop stay there: 256 x 1024 x 1024, 64 of them, 5.9 us and 6.7 with B [N,K],
+  // 7.1 and 7.3 with B [K,N]; 200 x 1000 x 1000 with B [K,N] 9.3 and 7.6.
   bool small = false;
   if (variant == NEOGEMM_VARIANT_AUTO && (v == NEOGEMM_VARIANT_T64x64_W4 || v == NEOGEMM_VARIANT_T64x128_W4) &&
       (ak || bk) && (ak || (a.M & 7) == 0 || bt.padded) && (bk || (a.N & 7) == 0 || bt.padded)) {
@@ -3320,7 +3519,11 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     if (ak && bk) small = 2 * wgs <= 3 * cus && !(wgs <= 64 && s == 1 && kt >= 8 && kt % 4 == 0);
     else small = wgs <= 2 * cus && !(fits && wgs <= 64 && s == 1 && K >= 1024 && K % 256 == 0);
   }
-  if (!fits && !small) {
+  if (small && !roles.bm) {
+    roles.bm = roles.bn = 64;
+    roles.split = s;
+  }
+  if (!fits && !roles.bm) {
     if (variant != NEOGEMM_VARIANT_AUTO) return NEOGEMM_ERR_UNSUPPORTED;
     // the planned tile is too wide for an MN-major operand: the 128x128 tile needs the least
     if (v == NEOGEMM_VARIANT_T128x128_W4) return unaligned();
@@ -3328,10 +3531,11 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                       NEOGEMM_VARIANT_T128x128_W4, s, 0, nullptr, alpha, beta, bt);
     return r == NEOGEMM_ERR_UNSUPPORTED ? unaligned() : r;
   }
-  a.ntm = ceil_div(a.M, small ? 64 : vi.bm);
-  a.ntn = ceil_div(a.N, small ? 64 : vi.bn);
+  if (roles.bm) s = roles.split;
+  a.ntm = ceil_div(a.M, roles.bm ? roles.bm : vi.bm);
+  a.ntn = ceil_div(a.N, roles.bm ? roles.bn : vi.bn);
   // (the few 64x64 tiles: an XCD's share of eight lies closer to a square, 512 x 512 x 1024 7.5 -> 5.9 us, 1024 x 200 x 1024 8.1 -> 6.4)
-  a.group_m = group_m > 0 ? group_m : v == NEOGEMM_VARIANT_T64x64_W4 && (int64_t)a.ntm * a.ntn * s <= 64 ? 2 : 8;
+  a.group_m = group_m > 0 ? group_m : (roles.bm || v == NEOGEMM_VARIANT_T64x64_W4) && (int64_t)a.ntm * a.ntn * s <= 64 ? 2 : 8;
   const int ktiles = ceil_div(K, KTILE);
   if (s > ktiles) s = ktiles;
   a.ktiles_per_split = ceil_div(ktiles, s);
@@ -3365,7 +3569,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
 
   if (bt.only_name) return *bt.only_name = small ? Kernel::kSmall : v == NEOGEMM_VARIANT_C256x256_W4 ? Kernel::kChain : Kernel::kTile, NEOGEMM_OK;
   hipError_t e;
-  if (small) e = launch_small(a, ak, bk, st);
+  if (roles.bm) e = launch_roles(a, roles.bm, roles.bn, ak, bk, st);
   else switch (v) {
     case NEOGEMM_VARIANT_T256x256_W4: e = launch_tile<256, 256, 2, 2>(a, ak, bk, st); break;
     case NEOGEMM_VARIANT_T128x128_W4: e = launch_tile<128, 128, 2, 2>(a, ak, bk, st); break;

@@ -154,7 +154,7 @@ size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M
                                          int a_layout, int b_layout, int c_layout, int64_t stride_a, int64_t stride_b, int64_t batch);
 /*
  * Which kernel neogemm_bf16_general runs for exactly these operands, given that many bytes of workspace: "tile", "chain" (the 256x256
- * tile that accumulates twice in a row), "small", "short K", "skinny", "strip", each with "copy+" in front where operands are first
+ * tile that accumulates twice in a row), "small" (few 64x64 tiles planned), "short K", "skinny", "strip", each with "copy+" in front where operands are first
  * copied onto the 16-byte grid; "ragged" (operands at any address), "generic", "none" (an empty problem); NULL for a call that is
  * refused.  Host only, for tests and tuning: the pointers are not read, their low bits are what counts.
  */
@@ -203,8 +203,9 @@ int neogemm_bf16_variant(const void* A, const void* B, void* C, int64_t M, int64
 /*
  * What neogemm_bf16 would pick for this call: writes the variant id and split-K factor.  Host only.
  * `aligned` is nonzero when pointers and leading dimensions satisfy the MFMA path (16-byte / 8-element); without it the answer is
- * NEOGEMM_VARIANT_GENERIC, which stands for every kernel outside the plan (operands at any address among them).  Where the answer has
- * 64 rows per tile, or K is at most 128, a call may run a kernel of its own for small problems or short K instead, in the same order of sums.
+ * NEOGEMM_VARIANT_GENERIC, which stands for every kernel outside the plan (operands at any address among them).  Where the answer is a
+ * tile of 192x256 or less, a call may run a kernel with waves of their own for the loads instead, in another tile and with fewer splits of K
+ * (so in another order of sums than neogemm_bf16_variant with the planned variant); where K is at most 128, one for short K.
  * The choice comes from a cost model over the tile variants; if the environment variable
  * NEOGEMM_PLAN_TABLE names a JSON file of tuned choices (an array of objects with the integer fields
  * "M","N","K","b_layout","c_layout","variant","split_k"; the layouts default to 0; gemm_amd/tune.py writes one), an

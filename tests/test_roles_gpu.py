@@ -1,0 +1,79 @@
+"""gemm_roles_kernel (four waves that load, four that compute): small integers, so that every order of summation gives the same bits."""
+import pytest
+import torch
+
+import gemm_amd as g
+from gemm_amd import _abi
+
+pytestmark = pytest.mark.gpu
+
+
+def ints(gen, *shape, top=2):
+    return torch.randint(-top, top + 1, shape, generator=gen, device="cuda").to(torch.bfloat16)
+
+
+# The tile that the rule chooses at 256 CUs: 64x64 | 128x64 with a transposed A, 64x64 else | 128x128, then one more row and column than whole
+# chunks (of K-major operands), five and six stages (more than the ring holds) with 8 and 64 of them filled | 256x128 | 128x256 and, with a
+# column-major C, 256x128 | the same the other way round | 128x128 in four splits | 256x128 and 128x256 in three | 64x64, 128x64 and 128x128 in 4 to 12
+@pytest.mark.parametrize("M,N,K", [(520, 1544, 1032), (1000, 2048, 1000), (1800, 1928, 392), (1801, 1929, 392), (1928, 1800, 264), (2056, 1928, 320),
+                                   (2600, 2576, 584), (1800, 4104, 1096), (4104, 1800, 1096), (904, 904, 4104), (2056, 1032, 8200),
+                                   (136, 1032, 8200), (1032, 136, 8200)])
+@pytest.mark.parametrize("a_layout", [g.A_MK, g.A_KM])
+@pytest.mark.parametrize("b_layout", [g.B_KN, g.B_NK])
+@pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
+def test_roles(M, N, K, a_layout, b_layout, c_layout):
+    if (M % 8 and a_layout == g.A_KM) or (N % 8 and b_layout == g.B_KN):
+        pytest.skip("whole chunks only of an MN-major operand")
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+
+    def operand(rows, cols, pad):   # NaN between the rows
+        m = torch.full((rows, cols + pad), float("nan"), dtype=torch.bfloat16, device="cuda")
+        m[:, :cols] = ints(gen, rows, cols)
+        return m[:, :cols]
+
+    A, B = operand(*((M, K) if a_layout == g.A_MK else (K, M)), 8), operand(*((K, N) if b_layout == g.B_KN else (N, K)), 16)
+    want = (A if a_layout == g.A_MK else A.t()).float() @ (B if b_layout == g.B_KN else B.t()).float()
+    C = torch.full((M, N) if c_layout == g.C_ROW else (N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
+    got = C if c_layout == g.C_ROW else C.t()
+    assert _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout,
+                            a_layout) in ("tile", "small")
+    g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout)
+    assert torch.equal(got, want.to(torch.bfloat16))
+    old = got.clone()
+    g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout, alpha=0.5, beta=-1.0)
+    assert torch.equal(got, (0.5 * want - old.float()).to(torch.bfloat16))
+
+
+# 64x64, 128x128, 128x256: the problems of a batch, the second operand shared or not
+@pytest.mark.parametrize("batch,M,N,K", [(4, 1024, 128, 1024), (32, 1024, 128, 1024), (20, 1024, 136, 1000)])
+def test_roles_batched(batch, M, N, K):
+    import neoGEMM
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    A, B = ints(gen, batch, M, K), ints(gen, batch, K, N)
+    for b in (B, B[0]):
+        want = torch.stack([A[i].float() @ (b[i] if b.dim() == 3 else b).float() for i in range(batch)])
+        assert torch.equal(neoGEMM.bmm(A, b), want.to(torch.bfloat16))
+
+
+def test_roles_first_call_under_capture():
+    """A kernel instance whose LDS limit is raised at its first launch, captured without a call before it in this process."""
+    import subprocess
+    import sys
+    code = """
+import torch, neoGEMM
+A = torch.randint(-2, 3, (1800, 392), device="cuda").to(torch.bfloat16)
+B = torch.randint(-2, 3, (392, 1928), device="cuda").to(torch.bfloat16)
+neoGEMM.gemm(A[:64, :64].contiguous(), B[:64, :64].contiguous())
+torch.cuda.synchronize()
+graph = torch.cuda.CUDAGraph()
+with torch.cuda.graph(graph):
+    C = neoGEMM.gemm(A, B)
+for _ in range(3):
+    C.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(C, (A.float() @ B.float()).to(torch.bfloat16))
+print("ok")
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "ok" in r.stdout, r.stdout + r.stderr
