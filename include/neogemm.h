@@ -148,7 +148,7 @@ size_t neogemm_bf16_general_workspace_bytes(int64_t M, int64_t N, int64_t K, int
 /*
  * What neogemm_bf16_general uses for exactly these operands.  Those that lie off the 16-byte grid (any pointer, leading
  * dimension, batch stride or K that is no multiple of 8 elements) may be copied onto it, in at most 256 MiB at a time, beside the
- * partials of split K; they run with less, or none, as well: in place, K not split.
+ * partials of split K; they run with less, or none, as well: in place, K split less or not at all.
  */
 size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                          int a_layout, int b_layout, int c_layout, int64_t stride_a, int64_t stride_b, int64_t batch);
