@@ -2883,23 +2883,25 @@ static bool plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_l
 
 // Whether gemm_roles_kernel takes a call that the plan gives to kernel v with split_max splits of K, estimated at plan_us; in the kernel's
 // terms: `rows` x `cols` of C as it lies in memory, ak / bk: the row / column operand has K-contiguous rows, lda / ldb their leading dimensions.
-// Fitted to 3300 timings of 600 problems with these tiles (64 to 6000 rows and columns, 128 to 65000 deep, both layouts of each operand,
-// batches; the operands in the caches and from HBM, the mean of both), rms 8 %: a launch, a way in and out per round of workgroups, per 64
-// deep what a stage takes, more where rows of an operand are no whole cache lines apart (a piece of 128 bytes then lies in two lines, and
-// is requested twice), and the reduction.  A CU holds two workgroups of the 64x64 tile, which then take 1.8 times as long, and one of the others.
-// The best of these by estimate is 0.8 % behind the best measured on average.  It is taken where it beats the plan's estimate times a factor
-// by planned tile (64x128 and 128x128 tiles take 1.35 and 1.2 times their estimates, and in one round of 128 rows and more the roles were at most
-// 2 % behind): 485 of 790 problems, 9 % faster on average over all of them (2048^3 from HBM 23.2 -> 20.8 us, 512 x 4096 x 4096 31.4 -> 26.7,
-// 1024 x 1024 x 2048 14.3 -> 11.8), 10 of them more than 3 % slower.  Short K and several rounds of planned workgroups count for less: the way in
-// and out of a workgroup is longer here, and a CU holds one (18 x 576 x 576 x 96 8.6 us in 128x128 tiles of gemm_tile_kernel, of which a CU holds two,
-// 11.8 here; 10001 x 1024 x 512 with a transposed A 17.5 and 21; 4096^3 in one-round tiles 91 and 124).  Not where the plan names strips (124 x
-// 5248 x 20608 from HBM 57.7 -> 60.9), 256x256 tiles or 192x256 ones with K split (304 x 1864 x 50048 80 -> 95).
+// Fitted to 9900 timings of 1010 problems with these tiles (1 to 20000 rows and columns, 32 to 65000 deep, both layouts of each operand, batches),
+// up to 48 MB to the mean of operands in the caches and from HBM, above to operands from HBM, rms 9 and 10 %: a launch, a way in and out per
+// round of workgroups, per 64 deep what a stage takes, more where rows of an operand are no whole cache lines apart (a piece of 128 bytes then lies
+// in two lines, and is requested twice), and the reduction.  A CU holds two workgroups of the 64x64 tile, which then take 1.75 times as long, and one
+// of the others.  The best of these by estimate is 0.8 % behind the best measured on average.  It is taken where it beats the plan's estimate times a
+// factor by planned tile (64x128 and 128x128 tiles take 1.35 and 1.2 times their estimates, and in one round of 128 rows and more the roles
+// were at most 2 % behind): 620 of 1010 problems, 9 % faster on average over all of them (2048^3 from HBM 23.2 -> 20.8 us, 512 x 4096 x 4096
+// 31.4 -> 26.7, 1024 x 1024 x 2048 14.3 -> 11.8), 9 of them more than 3 % slower.  Short K and more planned workgroups than CUs count for less: the way
+// in and out of a workgroup is longer here, and a CU holds one (18 x 576 x 576 x 96 8.6 us in 128x128 tiles of gemm_tile_kernel, of which a CU holds
+// two, 11.8 here; 10001 x 1024 x 512 with a transposed A 17.5 and 21; 1856 x 3392 x 472 11.4 and 13.0).  Not where the plan names strips (124 x 5248 x
+// 20608 from HBM 57.7 -> 60.9), 256x256 tiles, or 192x256 ones with K split or from HBM (304 x 1864 x 50048 80 -> 95, 449 x 20352 x 5120 103 -> 129).
 // No more splits than planned: what a caller's workspace holds, or whether one is needed, does not change.
 struct RolesPlan {
   int bm = 0, bn = 0, split = 1;  // bm == 0: not taken
 };
 static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, int64_t cols, int64_t K, int64_t batch, bool ak, bool bk,
                             int64_t lda, int64_t ldb) {
+  const double bytes = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch;
+  const bool hbm = bytes > 48e6;
   double against = 0;
   switch (v) {
     case NEOGEMM_VARIANT_T64x128_W4:
@@ -2908,13 +2910,14 @@ static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, 
     case NEOGEMM_VARIANT_T128x128_W4: against = 2.0; break;
     case NEOGEMM_VARIANT_T256x128_W4:
     case NEOGEMM_VARIANT_T128x256_W4: against = 1.4; break;
-    case NEOGEMM_VARIANT_T192x256_W4: against = split_max == 1 ? 1.0 : 0.0; break;
+    case NEOGEMM_VARIANT_T192x256_W4: against = split_max == 1 && !hbm ? 1.0 : 0.0; break;
     default: break;
   }
   if (against == 0) return RolesPlan();
   const int cus = planning_cus();
   if (K <= 256 && against > 1.2) against = 1.2;
-  if ((double)ceil_div(rows, kVariants[v].bm) * (double)ceil_div(cols, kVariants[v].bn) * split_max * (double)batch > 2.0 * cus && against > 1.0) against = 1.0;
+  const double planned = (double)ceil_div(rows, kVariants[v].bm) * (double)ceil_div(cols, kVariants[v].bn) * split_max * (double)batch;
+  if (against > 1.0 && planned > (v == NEOGEMM_VARIANT_T256x128_W4 || v == NEOGEMM_VARIANT_T128x256_W4 || v == NEOGEMM_VARIANT_T96x128_W4 ? 2.0 : 1.0) * cus) against = 1.0;
   const bool a_whole = (lda & 63) == 0, b_whole = (ldb & 63) == 0;
   struct Memo {
     int64_t rows = -1, cols = -1, K = -1, batch = -1;
@@ -2933,13 +2936,15 @@ static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, 
     int bm, bn, per_cu;
     double fixed_us, stage_us, full_us;  // per workgroup; per stage on an empty chip, and how much more on a full one
   };
-  static const Tile kTiles[] = {{64, 64, 2, 1.07, 0.188, 0.022}, {128, 64, 1, 1.36, 0.274, 0.056}, {128, 128, 1, 2.14, 0.355, 0.086},
-                                {256, 128, 1, 3.77, 0.576, 0.036}, {128, 256, 1, 4.70, 0.583, 0.029}};
+  static const Tile kTiles[2][5] = {{{64, 64, 2, 1.10, 0.177, 0.029}, {128, 64, 1, 1.37, 0.253, 0.071}, {128, 128, 1, 2.16, 0.337, 0.082},
+                                     {256, 128, 1, 4.21, 0.562, -0.095}, {128, 256, 1, 4.91, 0.573, -0.104}},
+                                    {{64, 64, 2, 3.11, 0.223, 0.030}, {128, 64, 1, 0.93, 0.329, 0.053}, {128, 128, 1, 2.46, 0.433, 0.077},
+                                     {256, 128, 1, 2.17, 0.618, 0.066}, {128, 256, 1, 4.54, 0.686, 0.009}}};
   const int64_t ktiles = ceil_div(K, KTILE);
-  const double floor_us = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch / 6.0e6;
+  const double floor_us = hbm ? bytes / 6.0e6 : 0.0;
   double best = against * plan_us;
   RolesPlan p;
-  for (const Tile& t : kTiles) {
+  for (const Tile& t : kTiles[hbm]) {
     // further lines a piece of an operand's row touches: one in two for 128 bytes along K, 64 columns of an MN-major operand likewise
     auto more = [](bool kmaj, bool whole, int w) { return whole ? 0.0 : kmaj ? 1.0 : 64.0 / w; };
     const double lines = (t.bm * more(ak, a_whole, t.bm) + t.bn * more(bk, b_whole, t.bn)) / (t.bm + t.bn);
@@ -2947,13 +2952,13 @@ static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, 
       if (sp > split_max || (sp > 1 && ktiles / sp < 4)) break;
       const double per = (double)ceil_div(ktiles, sp), wgs = (double)ceil_div(rows, t.bm) * (double)ceil_div(cols, t.bn) * sp * (double)batch;
       if (wgs > 2.0 * cus) break;
-      const double one = t.stage_us * (1.0 + 0.46 * lines), full = t.fixed_us + per * (one + t.full_us);
-      double us = 2.9;
+      const double one = t.stage_us * (1.0 + (hbm ? 0.61 : 0.46) * lines), full = t.fixed_us + per * (one + t.full_us);
+      double us = hbm ? 2.9 : 3.2;
       if (wgs <= cus) us += t.fixed_us + per * (one + t.full_us * wgs / cus);
-      else if (t.per_cu == 2) us += t.fixed_us + per * (one + t.full_us) * 1.8;
+      else if (t.per_cu == 2) us += t.fixed_us + per * (one + t.full_us) * (hbm ? 1.71 : 1.77);
       else us += full + t.fixed_us + per * (one + t.full_us * (wgs - cus) / cus);
       if (us < floor_us) us = floor_us + 0.01 * us;
-      if (sp > 1) us += 2.0 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 2.65e6;
+      if (sp > 1) us += (hbm ? 0.3 : 1.6) + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / (hbm ? 1.82e6 : 2.38e6);
       if (us < best) {
         best = us;
         p.bm = t.bm;
