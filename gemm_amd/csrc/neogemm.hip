@@ -167,7 +167,27 @@ struct TileArgs {
   long bsa, bsb, bsc;            // batch strides in elements; blockIdx.z is the batch index
   int early_stores;              // gemm_chain_kernel: stage the epilogue a quarter wave tile at a time (see launch_chain)
   int batch;
+  int stagger;                   // gemm_roles_kernel: the tiles of C start at so many different stages of K (0: all at the first)
+  // what the kernels divide by: tiles of C, tiles of a group, tile-rows of a whole group and of the last one, stagger (set_order)
+  uint32_t inv_tiles, inv_group, inv_rows, inv_last, inv_stagger;
+
+  // after ntm, ntn, group_m and stagger
+  void set_order() {
+    auto inv = [](uint64_t d) { return d == 0 || d > 0xffffffffu ? 0u : 0xffffffffu / (uint32_t)d; };
+    inv_tiles = inv((uint64_t)ntm * ntn);
+    inv_group = inv((uint64_t)group_m * ntn);
+    inv_rows = inv(group_m);
+    inv_last = inv(ntm % group_m);
+    inv_stagger = inv(stagger);
+  }
 };
+
+// n / d for inv = (2^32 - 1) / d, any n and d < 2^31: the product's upper half is the quotient or one less.  (The compiler's own division is 25
+// instructions in a chain, and a workgroup's first loads wait for three of them.)
+__device__ __forceinline__ int div_by(int n, int d, uint32_t inv) {
+  const uint32_t q = __umulhi((uint32_t)n, inv);
+  return (int)((uint32_t)n - q * (uint32_t)d >= (uint32_t)d ? q + 1 : q);
+}
 
 // Workgroup id -> (K split, output tile).  Consecutive ids land on different XCDs (round-robin over the 8
 // dies, each with its own L2), so id%8 selects a contiguous slice of the work order, and the work
@@ -181,15 +201,17 @@ __device__ __forceinline__ void tile_of_workgroup(const TileArgs& p, int& m0, in
   const int pid = blockIdx.x;
   const int q = work >> 3, r = work & 7, x = pid & 7;
   const int w = x * q + (x < r ? x : r) + (pid >> 3);
-  kz = w / total;
+  kz = div_by(w, total, p.inv_tiles);
   const int lin = w - kz * total;
   const int per_group = p.group_m * p.ntn;
-  const int g = lin / per_group;
+  const int g = div_by(lin, per_group, p.inv_group);
   const int first = g * p.group_m;
-  const int gsz = (p.ntm - first) < p.group_m ? (p.ntm - first) : p.group_m;
+  const bool last = p.ntm - first < p.group_m;
+  const int gsz = last ? p.ntm - first : p.group_m;
   const int rem = lin - g * per_group;
-  m0 = (first + rem % gsz) * BM;
-  n0 = (rem / gsz) * BN;
+  const int col = div_by(rem, gsz, last ? p.inv_last : p.inv_rows);
+  m0 = (first + rem - col * gsz) * BM;
+  n0 = col * BN;
 }
 
 // Global -> LDS side of one operand: which 16 bytes each lane fetches for each of this wave's
@@ -1686,6 +1708,13 @@ hipError_t launch_shortk(TileArgs a, int run, hipStream_t st) {
 // Tiles 64x64 (R = 4: 64 KiB, two workgroups per CU), 128x64 (5), 128x128 (4), 256x128 and 128x256 (3), of operands in either order.  More images
 // do not help (64x64 with five and six: level in the caches, 1 to 3 % slower from HBM), nor does the ring without the roles (1024^3 7.2 us).
 // The images are laid out and swizzled as in Operand and FragReader, K-major 64 deep or two slabs of 32 k-rows.
+// `stagger`: workgroups that start together and keep step ask for the same 128 bytes of every row at the same time, and rows a round number of
+// KiB apart lie in a few of the memory's channels.  So the tile in row i and column j of C starts at stage (i + j) mod `stagger` and comes round
+// to the stages before it at the end; fp32 sums in another order, of the same products.  From HBM 1024^3 7.9 -> 7.1 us, 1536^3 18.4 -> 16.3,
+// 792 x 2888 x 3008 28.0 -> 24.6, 400 x 8192 x 3072 31.4 -> 25.9; in the caches level.  (A spread over 4 or 8 stages gives a part of it; by rows
+// only nothing; by a hash of the tile's number, without the neighbours close to each other in K, up to 60 % slower.)  launch_roles has the line.
+// The way in costs: with the stages' wrap-around in it and three divisions the first loads left 0.2 us later (512^3 4.27 us, now 4.2), hence
+// set_order's reciprocals, no wrap-around among the first R stages, and all arguments asked for at once.
 // ---------------------------------------------------------------------------------------------
 template <int BM, int BN, int R, bool AK, bool BK>
 __global__ __launch_bounds__(512, BM * BN <= 4096 ? 4 : 2) void gemm_roles_kernel(TileArgs p) {
@@ -1694,6 +1723,9 @@ __global__ __launch_bounds__(512, BM * BN <= 4096 ? 4 : 2) void gemm_roles_kerne
   static_assert((R - 1) * NL <= 63, "the wait counts must fit the counter");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(NEOGEMM_AS3 char*)smem;
+  // the arguments in one round trip to memory: left to themselves, the later ones are asked for where they are needed
+  asm volatile("" ::"s"(p.A), "s"(p.B), "s"(p.C), "s"(p.M), "s"(p.K), "s"(p.lda), "s"(p.ldb), "s"(p.ntm), "s"(p.ksplit), "s"(p.bsa), "s"(p.bsb),
+               "s"(p.stagger), "s"(p.inv_tiles), "s"(p.inv_last));
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
   int m0, n0, kz;
@@ -1724,21 +1756,34 @@ __global__ __launch_bounds__(512, BM * BN <= 4096 ? 4 : 2) void gemm_roles_kerne
     const uint64_t baseA = (uint64_t)p.A + ((uint64_t)blockIdx.z * p.bsa + (AK ? (uint64_t)m0 * p.lda + k_begin : (uint64_t)k_begin * p.lda + m0)) * 2 - VOFF_BIAS;
     const uint64_t baseB = (uint64_t)p.B + ((uint64_t)blockIdx.z * p.bsb + (BK ? (uint64_t)n0 * p.ldb + k_begin : (uint64_t)k_begin * p.ldb + n0)) * 2 - VOFF_BIAS;
     const uint64_t advA = (AK ? (uint64_t)KTILE : (uint64_t)KTILE * p.lda) * 2, advB = (BK ? (uint64_t)KTILE : (uint64_t)KTILE * p.ldb) * 2;
-    // all loads of stage t into its slot; past the end of K as zero fills (resource size 0): the counts of loads in flight hold for any K
-    auto issue = [&](int t, uint32_t slot) {
-      const int krem = klen - t * KTILE;
+    // the stage to fetch next: where it begins in both operands, how deep what is left of K from there
+    uint64_t curA = baseA, curB = baseB;
+    int krem = klen;
+    if (p.stagger) {
+      const int d = m0 / BM + n0 / BN;
+      int first = d - div_by(d, p.stagger, p.inv_stagger) * p.stagger;
+      if (first + R > nst) first = 0;  // (a last split of K with fewer stages)
+      curA += (uint64_t)first * advA, curB += (uint64_t)first * advB;
+      krem -= first * KTILE;
+    }
+    // all its loads into a slot; i, how many were fetched before it: behind the last as zero fills (resource size 0), so that the counts of loads
+    // in flight hold for any K
+    auto issue = [&](int i, uint32_t slot, bool wrap) {
       auto part = [&](auto& vo, auto& key, uint64_t b, uint32_t dst, auto count) {
-        const i32x4 rs = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), t < nst ? (int)0x80000000u : 0, 0x00020000};
+        const i32x4 rs = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), i < nst ? (int)0x80000000u : 0, 0x00020000};
         static_for<decltype(count)::value>([&](auto jc) {
           constexpr int j = decltype(jc)::value;
           if constexpr (j % 4 == 0) dma_set_m0(dst + j * 1024);
           dma16<(j & 3) * 1024>(rs, key[j] < krem ? vo[j] : OOB_OFFSET);
         });
       };
-      part(voa, keya, baseA + (uint64_t)t * advA, lds0 + slot * STAGE + wave * IA * 1024, std::integral_constant<int, IA>{});
-      part(vob, keyb, baseB + (uint64_t)t * advB, lds0 + slot * STAGE + A_IMG + wave * IB * 1024, std::integral_constant<int, IB>{});
+      part(voa, keya, curA, lds0 + slot * STAGE + wave * IA * 1024, std::integral_constant<int, IA>{});
+      part(vob, keyb, curB, lds0 + slot * STAGE + A_IMG + wave * IB * 1024, std::integral_constant<int, IB>{});
+      curA += advA, curB += advB;
+      krem -= KTILE;
+      if (wrap && krem <= 0) curA = baseA, curB = baseB, krem = klen;
     };
-    for (int t = 0; t < R; ++t) issue(t, t);
+    for (int t = 0; t < R; ++t) issue(t, t, t == R - 1);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * NL) : "memory");
     __builtin_amdgcn_s_barrier();
     uint32_t slot = 0;
@@ -1746,7 +1791,7 @@ __global__ __launch_bounds__(512, BM * BN <= 4096 ? 4 : 2) void gemm_roles_kerne
       // stage t + 1 has landed (this wave's part of it); behind the barrier everyone's, and stage t is in the other waves' registers
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * NL) : "memory");
       __builtin_amdgcn_s_barrier();
-      issue(t + R, slot);
+      issue(t + R, slot, true);
       slot = slot + 1 == R ? 0 : slot + 1;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the zero fills are done before the epilogue takes the LDS
@@ -1758,10 +1803,20 @@ __global__ __launch_bounds__(512, BM * BN <= 4096 ? 4 : 2) void gemm_roles_kerne
   compute_stages<BM, BN, R, AK, BK>(p, p.C + (size_t)blockIdx.z * p.bsc * 2, nst, m0, n0, kz, wave, lane, lds0);
 }
 
-// bm x bn: 64x64, 128x64 or 128x128
-hipError_t launch_roles(const TileArgs& a, int bm, int bn, bool ak, bool bk, hipStream_t st);
+// bm x bn: 64x64, 128x64, 128x128, 256x128 or 128x256.
+// Staggered: of 223 problems of all sizes and layouts that these tiles take the 108 of 13 to 64 stages with tiles up to 128 wide, not batched, and
+// from HBM with K whole: 5.3 % faster from HBM (75 by more than 2 %, 2 slower by that, the worst 2.6 %), 0.6 % in the caches.  The others gain nothing
+// on average and lose singly: fewer stages (3400 x 640 x 512 7.7 -> 8.0 us), more (484 x 7304 x 4744 54 -> 56), 256 wide (2272 x 2752 x 1024 17.8 ->
+// 18.5), batches (32 x 1024 x 128 x 1024 23.0 -> 24.0), and K split over operands from HBM, where tiles side by side best read the parts of a row of an
+// MN-major one at the same time (134 x 10816 x 13312 66.2 -> 71.5).
+hipError_t launch_roles(TileArgs a, int bm, int bn, bool ak, bool bk, hipStream_t st);
 #if NEOGEMM_HAS_PART(9)
-hipError_t launch_roles(const TileArgs& a, int bm, int bn, bool ak, bool bk, hipStream_t st) {
+hipError_t launch_roles(TileArgs a, int bm, int bn, bool ak, bool bk, hipStream_t st) {
+  const double bytes = 2.0 * ((double)a.M * a.K + (double)a.K * a.N + (double)a.M * a.N) * a.batch;
+  if (a.batch == 1 && bm <= 128 && bn <= 128 && a.ktiles_per_split >= 13 && a.ktiles_per_split <= 64 && (a.ksplit == 1 || bytes <= 48e6)) {
+    a.stagger = a.ktiles_per_split - (bm == 128 && bn == 64 ? 5 : 4) + 1;  // a tile's first R stages in a row
+    a.set_order();
+  }
   dim3 grid(a.ntm * a.ntn * a.ksplit, 1, a.batch), block(512);
   auto pick = [&](auto mc, auto nc, auto rc) -> hipError_t {
     constexpr int BM = decltype(mc)::value, BN = decltype(nc)::value, R = decltype(rc)::value;
@@ -2892,7 +2947,9 @@ static bool plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_l
 // were at most 2 % behind): 620 of 1010 problems, 9 % faster on average over all of them (2048^3 from HBM 23.2 -> 20.8 us, 512 x 4096 x 4096
 // 31.4 -> 26.7, 1024 x 1024 x 2048 14.3 -> 11.8), 9 of them more than 3 % slower.  Short K and more planned workgroups than CUs count for less: the way
 // in and out of a workgroup is longer here, and a CU holds one (18 x 576 x 576 x 96 8.6 us in 128x128 tiles of gemm_tile_kernel, of which a CU holds
-// two, 11.8 here; 10001 x 1024 x 512 with a transposed A 17.5 and 21; 1856 x 3392 x 472 11.4 and 13.0).  Not where the plan names strips (124 x 5248 x
+// two, 11.8 here; 10001 x 1024 x 512 with a transposed A 17.5 and 21; 1856 x 3392 x 472 11.4 and 13.0), as do 96x128 tiles of two K-major operands
+// a multiple of 256 deep (3000 x 760 x 1024 9.9 and 11.3, 1344 x 1792 x 768 7.7 and 7.9; 1600 deep and from HBM the roles are ahead again, 672 x
+// 3840 x 1536 17.6 and 15.0; in the caches 1536^3 is the worst, 10.9 and 12.9).  Not where the plan names strips (124 x 5248 x
 // 20608 from HBM 57.7 -> 60.9), 256x256 tiles, or 192x256 ones with K split or from HBM (304 x 1864 x 50048 80 -> 95, 449 x 20352 x 5120 103 -> 129).
 // No more splits than planned: what a caller's workspace holds, or whether one is needed, does not change.
 struct RolesPlan {
@@ -2906,7 +2963,7 @@ static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, 
   switch (v) {
     case NEOGEMM_VARIANT_T64x128_W4:
     case NEOGEMM_VARIANT_T64x64_W4: against = 1.4; break;
-    case NEOGEMM_VARIANT_T96x128_W4: against = 1.8; break;
+    case NEOGEMM_VARIANT_T96x128_W4: against = ak && bk && K % 256 == 0 && K <= 1024 ? 1.0 : 1.8; break;
     case NEOGEMM_VARIANT_T128x128_W4: against = 2.0; break;
     case NEOGEMM_VARIANT_T256x128_W4:
     case NEOGEMM_VARIANT_T128x256_W4: against = 1.4; break;
@@ -3388,6 +3445,7 @@ static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, in
   const int ktiles = ceil_div(K, KTILE);
   a.ktiles_per_split = ceil_div(ktiles, split);
   a.ksplit = ceil_div(ktiles, a.ktiles_per_split);  // no empty split
+  a.set_order();
   if ((int64_t)a.ntm * a.ntn * a.ksplit > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;
   a.ws = (float*)ws;
   if (bt.only_name) return *bt.only_name = Kernel::kRagged, NEOGEMM_OK;
@@ -3630,6 +3688,8 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   if (s > ktiles) s = ktiles;
   a.ktiles_per_split = ceil_div(ktiles, s);
   a.ksplit = ceil_div(ktiles, a.ktiles_per_split);  // no empty split
+  a.stagger = 0;
+  a.set_order();
   if ((int64_t)a.ntm * a.ntn * a.ksplit > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;  // grid.x counts (split, tile) pairs
   a.ws = nullptr;
   a.prof = prof;

@@ -15,6 +15,8 @@ def ints(gen, *shape, top=2):
 # The tile that the rule chooses at 256 CUs: 64x64 | 128x64 with a transposed A, 64x64 else | 128x128, then one more row and column than whole
 # chunks (of K-major operands), five and six stages (more than the ring holds) with 8 and 64 of them filled | 256x128 | 128x256 and, with a
 # column-major C, 256x128 | the same the other way round | 128x128 in four splits | 256x128 and 128x256 in three | 64x64, 128x64 and 128x128 in 4 to 12
+# (13 to 64 stages of the tiles up to 128x128 are staggered: 520 x 1544 x 1032 has more tiles in a row and column than stages; 1000, 1032, 1096,
+# 4104 and 8200 end in a part of a stage that is not the last to be fetched; 904 x 904 x 4104 has three splits of 17 stages and one of 14)
 @pytest.mark.parametrize("M,N,K", [(520, 1544, 1032), (1000, 2048, 1000), (1800, 1928, 392), (1801, 1929, 392), (1928, 1800, 264), (2056, 1928, 320),
                                    (2600, 2576, 584), (1800, 4104, 1096), (4104, 1800, 1096), (904, 904, 4104), (2056, 1032, 8200),
                                    (136, 1032, 8200), (1032, 136, 8200)])
