@@ -1808,12 +1808,14 @@ __global__ __launch_bounds__(512, BM * BN <= 4096 ? 4 : 2) void gemm_roles_kerne
 // from HBM with K whole: 5.3 % faster from HBM (75 by more than 2 %, 2 slower by that, the worst 2.6 %), 0.6 % in the caches.  The others gain nothing
 // on average and lose singly: fewer stages (3400 x 640 x 512 7.7 -> 8.0 us), more (484 x 7304 x 4744 54 -> 56), 256 wide (2272 x 2752 x 1024 17.8 ->
 // 18.5), batches (32 x 1024 x 128 x 1024 23.0 -> 24.0), and K split over operands from HBM, where tiles side by side best read the parts of a row of an
-// MN-major one at the same time (134 x 10816 x 13312 66.2 -> 71.5).
+// MN-major one at the same time (134 x 10816 x 13312 66.2 -> 71.5); nor does one that only one row of tiles reads, K whole (112 x 14336 x 4096 with
+// B [K,N] 36.7 -> 37.7, 100 x 28672 x 4096 48.0 -> 50.7).
 hipError_t launch_roles(TileArgs a, int bm, int bn, bool ak, bool bk, hipStream_t st);
 #if NEOGEMM_HAS_PART(9)
 hipError_t launch_roles(TileArgs a, int bm, int bn, bool ak, bool bk, hipStream_t st) {
   const double bytes = 2.0 * ((double)a.M * a.K + (double)a.K * a.N + (double)a.M * a.N) * a.batch;
-  if (a.batch == 1 && bm <= 128 && bn <= 128 && a.ktiles_per_split >= 13 && a.ktiles_per_split <= 64 && (a.ksplit == 1 || bytes <= 48e6)) {
+  const bool once = (a.ntm == 1 && !bk) || (a.ntn == 1 && !ak);
+  if (a.batch == 1 && bm <= 128 && bn <= 128 && a.ktiles_per_split >= 13 && a.ktiles_per_split <= 64 && !once && (a.ksplit == 1 || bytes <= 48e6)) {
     a.stagger = a.ktiles_per_split - (bm == 128 && bn == 64 ? 5 : 4) + 1;  // a tile's first R stages in a row
     a.set_order();
   }
