@@ -3681,12 +3681,20 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                       NEOGEMM_VARIANT_T128x128_W4, s, 0, nullptr, alpha, beta, bt);
     return r == NEOGEMM_ERR_UNSUPPORTED ? unaligned() : r;
   }
+  const int ktiles = ceil_div(K, KTILE);
+  if (roles.bm && roles.split < s) {
+    // the workspace a call must bring is the plan's, whatever the kernel makes of it: whether a call runs does not hang on roles_plan's timings
+    const int planned = ceil_div(ktiles, ceil_div(ktiles, s < ktiles ? s : ktiles));
+    if (planned > 1) {
+      if (!workspace || workspace_bytes < (size_t)planned * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count) return NEOGEMM_ERR_WORKSPACE;
+      if (((uintptr_t)workspace & 15) != 0) return NEOGEMM_ERR_BAD_ARG;
+    }
+  }
   if (roles.bm) s = roles.split;
   a.ntm = ceil_div(a.M, roles.bm ? roles.bm : vi.bm);
   a.ntn = ceil_div(a.N, roles.bm ? roles.bn : vi.bn);
   // (the few 64x64 tiles: an XCD's share of eight lies closer to a square, 512 x 512 x 1024 7.5 -> 5.9 us, 1024 x 200 x 1024 8.1 -> 6.4)
   a.group_m = group_m > 0 ? group_m : (roles.bm || v == NEOGEMM_VARIANT_T64x64_W4) && (int64_t)a.ntm * a.ntn * s <= 64 ? 2 : 8;
-  const int ktiles = ceil_div(K, KTILE);
   if (s > ktiles) s = ktiles;
   a.ktiles_per_split = ceil_div(ktiles, s);
   a.ksplit = ceil_div(ktiles, a.ktiles_per_split);  // no empty split

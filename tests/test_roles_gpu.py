@@ -79,3 +79,25 @@ print("ok")
 """
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "ok" in r.stdout, r.stdout + r.stderr
+
+
+# planned with K split, run here without: the call is refused without the planned workspace all the same, and says so when asked
+@pytest.mark.parametrize("M,N,K,a_layout,b_layout,c_layout", [(624, 2464, 3448, g.A_KM, g.B_KN, g.C_COL), (1184, 504, 2616, g.A_MK, g.B_NK, g.C_COL)])
+def test_roles_with_fewer_splits_want_the_planned_workspace(M, N, K, a_layout, b_layout, c_layout):
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    A, B = ints(gen, *((M, K) if a_layout == g.A_MK else (K, M))), ints(gen, *((K, N) if b_layout == g.B_KN else (N, K)))
+    C = torch.zeros(N, M, dtype=torch.bfloat16, device="cuda")
+    need = _abi.call_workspace_bytes(A.data_ptr(), B.data_ptr(), M, N, K, A.stride(0), B.stride(0), b_layout, c_layout, a_layout)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+
+    def call(bytes_):
+        return _abi.load().neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), M, a_layout, b_layout,
+                                                c_layout, 1.0, 0.0, 0, 0, 0, 1, ws.data_ptr() if bytes_ else None, bytes_, None)
+
+    assert call(0) == _abi.ERR_WORKSPACE and call(M * N * 4) == _abi.ERR_WORKSPACE
+    assert _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), M, b_layout, c_layout, a_layout, ws_bytes=0) is None
+    torch.cuda.synchronize()
+    assert call(need) == 0
+    torch.cuda.synchronize()
+    want = (A if a_layout == g.A_MK else A.t()).float() @ (B if b_layout == g.B_KN else B.t()).float()
+    assert torch.equal(C.t(), want.to(torch.bfloat16))
