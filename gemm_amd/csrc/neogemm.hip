@@ -3141,7 +3141,7 @@ static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream
 }
 
 // The kernels that a call may end on, without the copies ahead of them and the reduction behind them.
-enum class Kernel { kNone, kGeneric, kRagged, kTile, kChain, kSkinny, kStrip, kSmall, kShortK };
+enum class Kernel { kNone, kGeneric, kRagged, kTile, kChain, kSkinny, kStrip, kShortK, kRoles64x64, kRoles128x64, kRoles128x128, kRoles256x128, kRoles128x256 };
 // A batch of `count` problems of one shape; strides in elements between consecutive problems (0: shared operand); and how
 // A is laid out, which only the general entry point lets a caller choose.
 struct BatchArgs {
@@ -3727,7 +3727,13 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     a.ws = (float*)workspace;
   }
 
-  if (bt.only_name) return *bt.only_name = small ? Kernel::kSmall : v == NEOGEMM_VARIANT_C256x256_W4 ? Kernel::kChain : Kernel::kTile, NEOGEMM_OK;
+  if (bt.only_name) {
+    if (!roles.bm) *bt.only_name = v == NEOGEMM_VARIANT_C256x256_W4 ? Kernel::kChain : Kernel::kTile;
+    else if (roles.bm == 64) *bt.only_name = Kernel::kRoles64x64;
+    else if (roles.bm == 256) *bt.only_name = Kernel::kRoles256x128;
+    else *bt.only_name = roles.bn == 64 ? Kernel::kRoles128x64 : roles.bn == 128 ? Kernel::kRoles128x128 : Kernel::kRoles128x256;
+    return NEOGEMM_OK;
+  }
   hipError_t e;
   if (roles.bm) e = launch_roles(a, roles.bm, roles.bn, ak, bk, st);
   else switch (v) {
@@ -3882,7 +3888,9 @@ const char* neogemm_bf16_call_kernel(const void* A, const void* B, const void* C
                                      int64_t stride_c, int64_t batch, size_t workspace_bytes) {
   static const char* const kNames[][2] = {{"none", "none"},         {"generic", "copy+generic"}, {"ragged", "copy+ragged"},
                                           {"tile", "copy+tile"}, {"chain", "copy+chain"},    {"skinny", "copy+skinny"},
-                                          {"strip", "copy+strip"}, {"small", "copy+small"}, {"short K", "copy+short K"}};
+                                          {"strip", "copy+strip"}, {"short K", "copy+short K"}, {"roles 64x64", "copy+roles 64x64"},
+                                          {"roles 128x64", "copy+roles 128x64"}, {"roles 128x128", "copy+roles 128x128"},
+                                          {"roles 256x128", "copy+roles 256x128"}, {"roles 128x256", "copy+roles 128x256"}};
   neogemm::BatchArgs bt;
   bt.count = batch;
   bt.sa = stride_a;

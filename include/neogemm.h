@@ -154,8 +154,8 @@ size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M
                                          int a_layout, int b_layout, int c_layout, int64_t stride_a, int64_t stride_b, int64_t batch);
 /*
  * Which kernel neogemm_bf16_general runs for exactly these operands, given that many bytes of workspace: "tile", "chain" (the 256x256
- * tile that accumulates twice in a row), "small" (few 64x64 tiles planned), "short K", "skinny", "strip", each with "copy+" in front where operands are first
- * copied onto the 16-byte grid; "ragged" (operands at any address), "generic", "none" (an empty problem); NULL for a call that is
+ * tile that accumulates twice in a row), "roles 64x64" and 128x64, 128x128, 256x128, 128x256 (waves that load and waves that compute, and the
+ * tile of C as it lies in memory), "short K", "skinny", "strip", each with "copy+" in front where operands are first copied onto the 16-byte grid; "ragged" (operands at any address), "generic", "none" (an empty problem); NULL for a call that is
  * refused.  Host only, for tests and tuning: the pointers are not read, their low bits are what counts.
  */
 const char* neogemm_bf16_call_kernel(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,

@@ -112,7 +112,7 @@ def test_copies_on_the_grid(b, M, N, K):
                 for size in (need, 0):   # with the copies, and by the kernel that reads in place
                     kernel = _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, C.stride(1), b_layout, c_layout, a_layout, 1.0,
                                               sa, 0, M * N, b, size)
-                    assert kernel == ("copy+tile" if size else "ragged")
+                    assert kernel.startswith("copy+") if size else kernel == "ragged"
                     C.copy_(old)
                     assert lib.neogemm_bf16_general(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, lda, ldb, C.stride(1), a_layout, b_layout, c_layout,
                                                     1.0, 1.0, sa, 0, M * N, b, ws.data_ptr(), size, st) == _abi.OK

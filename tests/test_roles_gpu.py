@@ -37,8 +37,10 @@ def test_roles(M, N, K, a_layout, b_layout, c_layout):
     want = (A if a_layout == g.A_MK else A.t()).float() @ (B if b_layout == g.B_KN else B.t()).float()
     C = torch.full((M, N) if c_layout == g.C_ROW else (N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
     got = C if c_layout == g.C_ROW else C.t()
-    assert _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout,
-                            a_layout) in ("tile", "small")
+    # (the plan's 128x128 tiles are kept for two rounds of workgroups, and for one where both operands are K-major)
+    kept = (M, N, K) in ((2056, 1928, 320), (2600, 2576, 584)) or ((M, N, K) == (1000, 2048, 1000) and (a_layout, b_layout) == (g.A_MK, g.B_NK))
+    name = _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout)
+    assert name == "tile" if kept else name.startswith("roles "), name
     g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout)
     assert torch.equal(got, want.to(torch.bfloat16))
     old = got.clone()

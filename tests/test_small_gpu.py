@@ -1,4 +1,4 @@
-"""Small problems (gemm_small_kernel): small integers, so that every order of summation gives the same bits."""
+"""Small problems (64x64 tiles of gemm_roles_kernel): small integers, so that every order of summation gives the same bits."""
 import pytest
 import torch
 
@@ -25,14 +25,17 @@ def test_small(M, N, K, a_layout, b_layout, c_layout):
 
     A, B = ints(*((M, K) if a_layout == g.A_MK else (K, M)), 8), ints(*((K, N) if b_layout == g.B_KN else (N, K)), 16)
     want = (A if a_layout == g.A_MK else A.t()).float() @ (B if b_layout == g.B_KN else B.t()).float()
-    # with B [N,K] at most one and a half 64x64 tiles per CU; few tiles and whole trips of the tile kernel's main loop; a transposed A only
-    # where it supplies the columns of a product whose rows are K-major
-    stays = {(1024, 2048, 264): b_layout == g.B_NK, (256, 1024, 1024): (b_layout, c_layout) != (g.B_KN, g.C_COL)}.get((M, N, K), False)
-    here = not stays if a_layout == g.A_MK else (b_layout, c_layout) == (g.B_NK, g.C_COL) and (M, N, K) != (256, 1024, 1024)
+    # more than one and a half 64x64 tiles per CU of two K-major operands stay in 128x128 tiles; a transposed A (but for its columns beside
+    # K-major rows) is planned in 128x128 tiles, which are weighed against 128x64 tiles too and, K at most 256 deep, kept
+    kernel = "roles 64x64"
+    if a_layout == g.A_KM and (b_layout, c_layout) != (g.B_NK, g.C_COL):
+        kernel = "tile" if K <= 256 else "roles 128x64" if M * N > 1024 * 1024 else kernel
+    elif (M, N, K) == (1024, 2048, 264) and a_layout == g.A_MK and b_layout == g.B_NK:
+        kernel = "tile"
     C = torch.full((M, N) if c_layout == g.C_ROW else (N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
     got = C if c_layout == g.C_ROW else C.t()
     assert _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout,
-                            a_layout) == ("small" if here else "tile")
+                            a_layout) == kernel
     g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout)
     assert torch.equal(got, want.to(torch.bfloat16))
     old = got.clone()
