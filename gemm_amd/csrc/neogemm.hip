@@ -2589,6 +2589,51 @@ static int planning_cus() {
   }
   return cus;
 }
+// The estimate of one tile kernel with K in sp parts; rows x cols of C as it lies in memory, both_k: both operands K-major.
+static double tile_estimate(const PlanCand& c, int sp, int64_t rows, int64_t cols, int64_t K, int64_t batch, bool both_k, double cus) {
+  const int64_t ktiles = ceil_div(K, KTILE);
+  const double bytes = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch;
+  const double stream_us = bytes / 5.0e6, lat_us = bytes > 32e6 ? 0.7 : 0.3;
+  const double tiles = (double)ceil_div(rows, kVariants[c.variant].bm) * (double)ceil_div(cols, kVariants[c.variant].bn);
+  const double ktps = (double)ceil_div(ktiles, sp), wgs = tiles * sp * (double)batch;
+  // a partial round runs on an emptier chip (more power and bandwidth per CU): measured at 0.7 of a round
+  // when nearly empty, rising to 1 when full
+  auto rounds_of = [](double x) {
+    const double full = __builtin_floor(x), frac = x - full;
+    return full + (frac > 0.0 ? 0.7 + 0.3 * frac : 0.0);
+  };
+  const double per_cu_wgs = rounds_of(wgs / cus);
+  const double rounds = rounds_of(wgs / (cus * c.per_cu));
+  double t = per_cu_wgs * ktps * c.ktile_us;
+  // both operands K-major: the tall tile runs a little ahead of the wide one (2560^3: 33.8 against 35.0 us)
+  if (c.variant == NEOGEMM_VARIANT_T128x256_W4 && both_k) t *= 1.02;
+  // latency knows no discount, and two latency-bound workgroups on one CU were measured to take turns
+  // (with both operands K-major the 128x128 tile has three tiles of each in flight when it streams: 256 x 14336 x 4096
+  // unsplit, 224 workgroups, runs its 64 K tiles in 32.3 us; with far fewer workgroups than CUs a K tile takes longer,
+  // and with more than CUs the second workgroup of a CU goes at the pace of the first: 128 x 5120 x 27648 with split 6,
+  // 240 workgroups, 69 us; split 8, 320 of them, 98; split 12, 480, 76)
+  const double lat_v =
+      c.variant == NEOGEMM_VARIANT_T128x128_W4 && bytes > 32e6 && both_k && wgs >= 0.6 * cus && wgs <= cus ? 0.46 : lat_us;
+  const double lat_floor = __builtin_ceil(wgs / cus) * ktps * lat_v;
+  if (t < lat_floor) t = lat_floor;
+  t += rounds * (c.fixed_us + (sp > 1 ? c.split_fixed_us : 0.0));
+  // fewer workgroups than CUs pull less from HBM: 112 of them 4.0 TB/s, 224 and more 5 and above (64x11008x14336
+  // with split 3, 129 workgroups: 87 us; split 4, 172: 73; 128x28672x14336 unsplit, 112: 230; split 2: 173)
+  const double fill = wgs < cus ? wgs / cus : 1.0;
+  const double floor_us = stream_us / (0.55 + 0.45 * fill);
+  if (t < floor_us) t = floor_us;
+  // Few rows against weights that stream from HBM: every further tile along the short side requests the weights again,
+  // from the L2s, which is not free when the launch lives on its loads: 50 ns per MB (512 x 7168 x 7168 with B [N,K]:
+  // four row tiles of 128, 72 us; two of 256, 62).  Fitted to the candidate timings of 16 to 512 rows with cold weights,
+  // where it takes the plan's mean loss against the best candidate from 6.0 % to 3.6 %.
+  if (bytes > 32e6 && (rows <= 512 || cols <= 512)) {
+    const double again = cols >= rows ? (double)(ceil_div(rows, kVariants[c.variant].bm) - 1) * (double)cols
+                                      : (double)(ceil_div(cols, kVariants[c.variant].bn) - 1) * (double)rows;
+    t += again * (double)K * 2.0 * (double)batch * 5.0e-8;
+  }
+  if (sp > 1) t += 4.0 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 5.0e6;
+  return t;
+}
 static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
                        int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int ncus = 256, int a_layout = NEOGEMM_A_MK,
                        double* estimate_us = nullptr) {
@@ -2604,7 +2649,7 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
   const int64_t ktiles = ceil_div(K, KTILE);
   const double cus = (double)ncus;
   const double bytes = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch;
-  const double stream_us = bytes / 5.0e6, lat_us = bytes > 32e6 ? 0.7 : 0.3;
+  const double stream_us = bytes / 5.0e6;
   static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   double best = 1e300;
   int bv = NEOGEMM_VARIANT_T128x128_W4, bs = 1;
@@ -2617,46 +2662,9 @@ static void plan_model(int64_t M, int64_t N, int64_t K, bool aligned, int c_layo
     // the small tiles have too little in flight to stream from HBM; 64x64 takes K-major operands only
     if ((c.variant == NEOGEMM_VARIANT_T96x128_W4 || c.variant == NEOGEMM_VARIANT_T64x64_W4) && bytes > 32e6) continue;
     if (c.variant == NEOGEMM_VARIANT_T64x64_W4 && !both_k) continue;
-    const double tiles = (double)ceil_div(rows, kVariants[c.variant].bm) * (double)ceil_div(cols, kVariants[c.variant].bn);
     for (int sp : kSplits) {
       if (sp > 1 && ktiles / sp < 2) break;  // at least 128 deep per split
-      const double ktps = (double)ceil_div(ktiles, sp), wgs = tiles * sp * (double)batch;
-      // a partial round runs on an emptier chip (more power and bandwidth per CU): measured at 0.7 of a round
-      // when nearly empty, rising to 1 when full
-      auto rounds_of = [](double x) {
-        const double full = __builtin_floor(x), frac = x - full;
-        return full + (frac > 0.0 ? 0.7 + 0.3 * frac : 0.0);
-      };
-      const double per_cu_wgs = rounds_of(wgs / cus);
-      const double rounds = rounds_of(wgs / (cus * c.per_cu));
-      double t = per_cu_wgs * ktps * c.ktile_us;
-      // both operands K-major: the tall tile runs a little ahead of the wide one (2560^3: 33.8 against 35.0 us)
-      if (c.variant == NEOGEMM_VARIANT_T128x256_W4 && both_k) t *= 1.02;
-      // latency knows no discount, and two latency-bound workgroups on one CU were measured to take turns
-      // (with both operands K-major the 128x128 tile has three tiles of each in flight when it streams: 256 x 14336 x 4096
-      // unsplit, 224 workgroups, runs its 64 K tiles in 32.3 us; with far fewer workgroups than CUs a K tile takes longer,
-      // and with more than CUs the second workgroup of a CU goes at the pace of the first: 128 x 5120 x 27648 with split 6,
-      // 240 workgroups, 69 us; split 8, 320 of them, 98; split 12, 480, 76)
-      const double lat_v =
-          c.variant == NEOGEMM_VARIANT_T128x128_W4 && bytes > 32e6 && both_k && wgs >= 0.6 * cus && wgs <= cus ? 0.46 : lat_us;
-      const double lat_floor = __builtin_ceil(wgs / cus) * ktps * lat_v;
-      if (t < lat_floor) t = lat_floor;
-      t += rounds * (c.fixed_us + (sp > 1 ? c.split_fixed_us : 0.0));
-      // fewer workgroups than CUs pull less from HBM: 112 of them 4.0 TB/s, 224 and more 5 and above (64x11008x14336
-      // with split 3, 129 workgroups: 87 us; split 4, 172: 73; 128x28672x14336 unsplit, 112: 230; split 2: 173)
-      const double fill = wgs < cus ? wgs / cus : 1.0;
-      const double floor_us = stream_us / (0.55 + 0.45 * fill);
-      if (t < floor_us) t = floor_us;
-      // Few rows against weights that stream from HBM: every further tile along the short side requests the weights again,
-      // from the L2s, which is not free when the launch lives on its loads: 50 ns per MB (512 x 7168 x 7168 with B [N,K]:
-      // four row tiles of 128, 72 us; two of 256, 62).  Fitted to the candidate timings of 16 to 512 rows with cold weights,
-      // where it takes the plan's mean loss against the best candidate from 6.0 % to 3.6 %.
-      if (bytes > 32e6 && (rows <= 512 || cols <= 512)) {
-        const double again = cols >= rows ? (double)(ceil_div(rows, kVariants[c.variant].bm) - 1) * (double)cols
-                                          : (double)(ceil_div(cols, kVariants[c.variant].bn) - 1) * (double)rows;
-        t += again * (double)K * 2.0 * (double)batch * 5.0e-8;
-      }
-      if (sp > 1) t += 4.0 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 5.0e6;
+      const double t = tile_estimate(c, sp, rows, cols, K, batch, both_k, cus);
       if (t < best) {
         best = t;
         bv = c.variant;
@@ -3515,6 +3523,11 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
         (!workspace || ((uintptr_t)workspace & 15) != 0 || workspace_bytes < (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count)) {
       v = NEOGEMM_VARIANT_T128x128_W4;
       s = 1;
+      if (plan_us > 0) {  // (of the split plan; roles_plan compares with what runs)
+        const bool row = c_layout == NEOGEMM_C_ROW;
+        for (const PlanCand& c : kPlanCands)
+          if (c.variant == v) plan_us = tile_estimate(c, 1, row ? M : N, row ? N : M, K, bt.count, a_mk && b_layout == NEOGEMM_B_NK, (double)planning_cus());
+      }
     }
   }
   if (s == 0) s = 1;

@@ -202,6 +202,14 @@ def test_call_kernel_names_without_a_gpu():
     assert _abi.call_kernel(p, q, c, 1024, 1024, 32768, 32768, 1024, 1024, 0, 0, ws_bytes=0) is None
 
 
+def test_roles_are_weighed_against_the_kernel_that_would_run():
+    """A C off 8-byte addresses without a workspace runs unsplit 128x128 tiles where the plan splits K: it is their time that counts then."""
+    p, q, c = 1 << 20, 1 << 40, (1 << 44) + 2
+    for (M, N, K, b, want) in ((2776, 48, 8696, 0, "roles 64x64"), (904, 5008, 13376, 1, "roles 256x128"), (840, 16, 7248, 1, "roles 64x64")):
+        assert _abi.plan(M, N, K, b, 0)[1] > 1
+        assert _abi.call_kernel(p, q, c, M, N, K, K, N if b == 0 else K, N, b, 0, ws_bytes=0) == want
+
+
 def test_copies_are_made_where_they_pay():
     """Shapes measured both ways, A one element off the grid ([M,K]) or with odd rows ([K,M]): us with copies / in place beside each."""
     for (M, N, K), better in (((2001, 2000, 504), "copy"),     # 14.1 / 17.0, transposed A 13.9 / 16.7
