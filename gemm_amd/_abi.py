@@ -24,10 +24,12 @@ VARIANT_T96x128_W4, VARIANT_T64x64_W4 = 13, 14
 VARIANT_C256x256_W4 = 15
 VARIANT_SKINNY128 = 16
 VARIANT_STRIP = 17
-VARIANT_COUNT = 18
+VARIANT_R64x64, VARIANT_R128x64, VARIANT_R128x128, VARIANT_R256x128, VARIANT_R128x256 = 18, 19, 20, 21, 22
+VARIANT_COUNT = 23
 VARIANT_NAMES = {0: "auto", 1: "generic", 2: "retired", 3: "256x256_w4", 4: "128x128_w4", 5: "256x128_w4",
                  6: "128x256_w4", 7: "64x128_w4", 8: "retired", 9: "skinny16", 10: "skinny32", 11: "skinny64", 12: "192x256_w4", 13: "96x128_w4", 14: "64x64_w4",
-                 15: "256x256_w4_chain", 16: "skinny128", 17: "strip"}
+                 15: "256x256_w4_chain", 16: "skinny128", 17: "strip", 18: "64x64_roles", 19: "128x64_roles",
+                 20: "128x128_roles", 21: "256x128_roles", 22: "128x256_roles"}
 
 # every symbol include/neogemm.h declares, with its prototype
 _i64, _int, _vp, _sz = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t
@@ -45,6 +47,8 @@ PROTOTYPES = {
     "neogemm_bf16_call_workspace_bytes": (_sz, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _i64, _i64, _i64]),
     "neogemm_bf16_call_kernel": (ctypes.c_char_p, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, ctypes.c_float,
                                                    _i64, _i64, _i64, _i64, _sz]),
+    "neogemm_bf16_call_plan": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, ctypes.c_float, _i64, _i64, _i64, _i64,
+                                      _sz, ctypes.POINTER(_int), ctypes.POINTER(_int)]),
     "neogemm_bf16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "neogemm_bf16_variant": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _sz, _vp,
                                     _int, _int, _int]),
@@ -108,6 +112,17 @@ def call_kernel(A_ptr, B_ptr, C_ptr, M, N, K, lda, ldb, ldc, b_layout, c_layout,
     name = load().neogemm_bf16_call_kernel(A_ptr, B_ptr, C_ptr, M, N, K, lda, ldb, ldc, a_layout, b_layout, c_layout, beta, stride_a, stride_b,
                                            stride_c, batch, ws_bytes)
     return name.decode() if name else None
+
+
+def call_plan(A_ptr, B_ptr, C_ptr, M, N, K, lda, ldb, ldc, b_layout, c_layout, a_layout=A_MK, beta=0.0, stride_a=0, stride_b=0,
+              stride_c=0, batch=1, ws_bytes=None):
+    """(variant, split of K) that neogemm_bf16_general would run, with the workspace its query asks for or with ws_bytes; None: refused."""
+    if ws_bytes is None:
+        ws_bytes = call_workspace_bytes(A_ptr, B_ptr, M, N, K, lda, ldb, b_layout, c_layout, a_layout, stride_a, stride_b, batch)
+    v, s = _int(0), _int(0)
+    st = load().neogemm_bf16_call_plan(A_ptr, B_ptr, C_ptr, M, N, K, lda, ldb, ldc, a_layout, b_layout, c_layout, beta, stride_a, stride_b,
+                                       stride_c, batch, ws_bytes, ctypes.byref(v), ctypes.byref(s))
+    return (v.value, s.value) if st == OK else None
 
 
 def plan(M, N, K, b_layout=B_KN, c_layout=C_ROW, aligned=True):

@@ -2541,8 +2541,9 @@ struct VariantInfo {
 static const VariantInfo kVariants[NEOGEMM_VARIANT_COUNT] = {
     {0, 0, 0}, {16, 16, 4}, {0, 0, 0}, {256, 256, 4}, {128, 128, 4}, {256, 128, 4}, {128, 256, 4}, {64, 128, 4}, {0, 0, 0},
     {16, 64, 4}, {32, 64, 4}, {64, 64, 4}, {192, 256, 4}, {96, 128, 4}, {64, 64, 4}, {256, 256, 4}, {128, 64, 4},
-    {128, 64, 4},
+    {128, 64, 4}, {64, 64, 8}, {128, 64, 8}, {128, 128, 8}, {256, 128, 8}, {128, 256, 8},
 };
+static bool variant_roles(int v) { return v >= NEOGEMM_VARIANT_R64x64 && v <= NEOGEMM_VARIANT_R128x256; }
 // Two identifiers of earlier builds (a 256x256 tile with eight waves, a 128x128 tile with a 1x4 wave grid) never won
 // a shape against the kernels above in any sweep; their numbers stay reserved and a call that names one is refused.
 static bool variant_retired(int v) { return v == NEOGEMM_VARIANT_RETIRED_2 || v == NEOGEMM_VARIANT_RETIRED_8; }
@@ -3150,6 +3151,18 @@ static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream
 
 // The kernels that a call may end on, without the copies ahead of them and the reduction behind them.
 enum class Kernel { kNone, kGeneric, kRagged, kTile, kChain, kSkinny, kStrip, kShortK, kRoles64x64, kRoles128x64, kRoles128x128, kRoles256x128, kRoles128x256 };
+// What a call ends on: kernel, variant number (0: it has none) and split of K of the product, and whether copies on the 16-byte grid come first.
+struct Choice {
+  Kernel kernel = Kernel::kNone;
+  int variant = NEOGEMM_VARIANT_AUTO, split = 1;
+  bool copies = false;
+  int set(Kernel k, int v, int s) {
+    kernel = k;
+    variant = v;
+    split = s;
+    return NEOGEMM_OK;
+  }
+};
 // A batch of `count` problems of one shape; strides in elements between consecutive problems (0: shared operand); and how
 // A is laid out, which only the general entry point lets a caller choose.
 struct BatchArgs {
@@ -3157,8 +3170,7 @@ struct BatchArgs {
   int a_layout = NEOGEMM_A_MK;
   bool scratch_unaligned = false;  // operands off the 16-byte grid may use the workspace (see neogemm_bf16_call_workspace_bytes)
   bool padded = false;             // rows of both operands end on whole chunks in memory, zeros behind K (pack_kernel)
-  Kernel* only_name = nullptr;     // nothing is launched; what would be is written here (neogemm_bf16_call_kernel) ...
-  bool* copies = nullptr;          // ... and here whether copies on the 16-byte grid come first
+  Choice* only = nullptr;          // nothing is launched; what would be is written here (neogemm_bf16_call_kernel, neogemm_bf16_call_plan)
 };
 
 // ld limits keep every in-tile byte offset below 2^31 (the buffer range check uses 32-bit offsets)
@@ -3402,8 +3414,8 @@ static int launch_packed(const PackPlan& p, const void* A, const void* B, void* 
         in_a = a;
         in_b = b;
         const bool one = (!pa.blocks || pa.bs == 0) && (!pb.blocks || pb.bs == 0);  // nothing that differs between the problems is copied
-        if (bt.only_name) {
-          *bt.copies = true;
+        if (bt.only) {
+          bt.only->copies = true;
         } else if (pa.blocks + pb.blocks) {
           pack_kernel<<<dim3(pa.blocks + pb.blocks, 1, one ? 1u : (unsigned)count), 256, 0, st>>>(pa, pb);
           if (hipError_t e = hipGetLastError(); e != hipSuccess) {
@@ -3418,7 +3430,7 @@ static int launch_packed(const PackPlan& p, const void* A, const void* B, void* 
         if (p.b) to.sb = pb.bs ? (int64_t)pb.rows * pb.cpr * 8 : 0;
         const int r = run(p.a ? at_a : a, p.b ? at_b : b, c, rows, cols, K, p.a ? (int64_t)pa.cpr * 8 : lda, p.b ? (int64_t)pb.cpr * 8 : ldb, ldc,
                           b_layout, c_layout, ws, p.partials, (void*)st, NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, alpha, beta, to);
-        if (r != NEOGEMM_OK || bt.only_name) return r;
+        if (r != NEOGEMM_OK || bt.only) return r;
       }
   return NEOGEMM_OK;
 }
@@ -3458,7 +3470,7 @@ static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, in
   a.set_order();
   if ((int64_t)a.ntm * a.ntn * a.ksplit > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;
   a.ws = (float*)ws;
-  if (bt.only_name) return *bt.only_name = Kernel::kRagged, NEOGEMM_OK;
+  if (bt.only) return bt.only->set(Kernel::kRagged, NEOGEMM_VARIANT_AUTO, a.ksplit);
   if (hipError_t e = launch_ragged(a, ak, bk, bm, bn, st); e != hipSuccess) {
     fprintf(stderr, "neogemm: ragged kernel launch failed: %s\n", hipGetErrorString(e));
     return NEOGEMM_ERR_LAUNCH;
@@ -3538,7 +3550,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     const long scm = c_layout == NEOGEMM_C_ROW ? ldc : 1, scn = c_layout == NEOGEMM_C_ROW ? 1 : ldc;
     const int64_t nbx = ceil_div(N, 16), nblocks = nbx * ceil_div(M, 16);
     if (nblocks > 0x7fffffff) return NEOGEMM_ERR_UNSUPPORTED;
-    if (bt.only_name) return *bt.only_name = Kernel::kGeneric, NEOGEMM_OK;
+    if (bt.only) return bt.only->set(Kernel::kGeneric, NEOGEMM_VARIANT_GENERIC, 1);
     dim3 grid((unsigned)nblocks, 1, (unsigned)bt.count);
     gemm_generic_kernel<<<grid, 256, 0, st>>>((const __bf16*)A, (const __bf16*)B, (__bf16*)C, (int)M, (int)N, (int)K,
                                               sam, sak, sbk, sbn, scm, scn, alpha, beta, bt.sa, bt.sb, bt.sc,
@@ -3558,8 +3570,10 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   {
     const bool row = c_layout == NEOGEMM_C_ROW, b_nk = b_layout == NEOGEMM_B_NK, rk = row ? a_mk : b_nk, ck = row ? b_nk : a_mk;
     const int64_t rows = row ? M : N, cols = row ? N : M;
-    if (plan_us > 0 && split_k == 0 && (rk || (rows & 7) == 0 || bt.padded) && (ck || (cols & 7) == 0 || bt.padded))
-      roles = roles_plan(v, s, plan_us, rows, cols, K, bt.count, rk, ck, row ? lda : ldb, row ? ldb : lda);
+    if ((rk || (rows & 7) == 0 || bt.padded) && (ck || (cols & 7) == 0 || bt.padded)) {
+      if (variant_roles(v)) roles = RolesPlan{kVariants[v].bm, kVariants[v].bn, s};
+      else if (plan_us > 0 && split_k == 0) roles = roles_plan(v, s, plan_us, rows, cols, K, bt.count, rk, ck, row ? lda : ldb, row ? ldb : lda);
+    }
   }
   if (!roles.bm && (v == NEOGEMM_VARIANT_SKINNY16 || v == NEOGEMM_VARIANT_SKINNY32 || v == NEOGEMM_VARIANT_SKINNY64 ||
                     v == NEOGEMM_VARIANT_SKINNY128 || v == NEOGEMM_VARIANT_STRIP)) {
@@ -3577,7 +3591,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                     NEOGEMM_VARIANT_T128x128_W4, 1, 0, nullptr, alpha, beta, bt);
       return st2 == NEOGEMM_ERR_UNSUPPORTED ? unaligned() : st2;
     }
-    if (bt.only_name) return *bt.only_name = v == NEOGEMM_VARIANT_STRIP ? Kernel::kStrip : Kernel::kSkinny, NEOGEMM_OK;
+    if (bt.only) return bt.only->set(v == NEOGEMM_VARIANT_STRIP ? Kernel::kStrip : Kernel::kSkinny, v, s);
     SkinnyArgs sa{(const char*)A, (const char*)B, (char*)C, (int)M, (int)N, (int)K, (long)lda, (long)ldb, (long)ldc, alpha, beta, 0, 64};
     bool bkm = b_layout == NEOGEMM_B_NK, ccol = c_layout == NEOGEMM_C_COL;
     if (swap) {
@@ -3667,7 +3681,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   // matrix edge).
   auto mn_ok = [&](int tile, int rows) { return tile >= 128 && (tile & (tile - 1)) == 0 && ((rows & 7) == 0 || bt.padded); };
   // (the chained 256x256 kernel takes its rows from a K-major operand only, K in whole periods of 128 and no split)
-  const bool fits = (ak || mn_ok(vi.bm, a.M)) && (bk || mn_ok(vi.bn, a.N)) &&
+  const bool fits = !variant_roles(v) && (ak || mn_ok(vi.bm, a.M)) && (bk || mn_ok(vi.bn, a.N)) &&
                     (v != NEOGEMM_VARIANT_C256x256_W4 || (ak && K % (2 * KTILE) == 0 && s <= 1));
   // Where the plan says 64 rows per tile and roles_plan does not take the call, 64x64 tiles of gemm_roles_kernel do, with B [K,N] on the rows
   // too (a column-major C; that went to the 128x128 tile), as long as they fit the CUs one and a half times (B [N,K]: 1152^3, 324 of them, 10.6 us
@@ -3688,7 +3702,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   }
   if (!fits && !roles.bm) {
     if (variant != NEOGEMM_VARIANT_AUTO) return NEOGEMM_ERR_UNSUPPORTED;
-    // the planned tile is too wide for an MN-major operand: the 128x128 tile needs the least
+    // the planned tile is too wide for an MN-major operand (or takes whole chunks of it only): the 128x128 tile needs the least
     if (v == NEOGEMM_VARIANT_T128x128_W4) return unaligned();
     const int r = run(A, B, C, M, N, K, lda, ldb, ldc, b_layout, c_layout, workspace, workspace_bytes, hip_stream,
                       NEOGEMM_VARIANT_T128x128_W4, s, 0, nullptr, alpha, beta, bt);
@@ -3723,7 +3737,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     // at least two column tiles for each of two workgroups per CU (16 x 512 x 512 x 96, one each: level with the tile kernels)
     const int64_t tiles = (int64_t)ceil_div(a.M, 128) * ceil_div(a.N, 64) * bt.count, slots = 2 * (int64_t)planning_cus();
     if (tiles >= 2 * slots) {
-      if (bt.only_name) return *bt.only_name = Kernel::kShortK, NEOGEMM_OK;
+      if (bt.only) return bt.only->set(Kernel::kShortK, NEOGEMM_VARIANT_AUTO, 1);
       const int64_t per_row = ceil_div(slots, (int64_t)ceil_div(a.M, 128) * bt.count);  // workgroups that share a block of rows
       const hipError_t e = launch_shortk(a, ceil_div(ceil_div(a.N, 64), per_row), st);
       if (e == hipSuccess) return NEOGEMM_OK;
@@ -3740,12 +3754,11 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     a.ws = (float*)workspace;
   }
 
-  if (bt.only_name) {
-    if (!roles.bm) *bt.only_name = v == NEOGEMM_VARIANT_C256x256_W4 ? Kernel::kChain : Kernel::kTile;
-    else if (roles.bm == 64) *bt.only_name = Kernel::kRoles64x64;
-    else if (roles.bm == 256) *bt.only_name = Kernel::kRoles256x128;
-    else *bt.only_name = roles.bn == 64 ? Kernel::kRoles128x64 : roles.bn == 128 ? Kernel::kRoles128x128 : Kernel::kRoles128x256;
-    return NEOGEMM_OK;
+  if (bt.only) {
+    if (!roles.bm) return bt.only->set(v == NEOGEMM_VARIANT_C256x256_W4 ? Kernel::kChain : Kernel::kTile, v, a.ksplit);
+    int i = 0;  // the tile's place among the variants and the names
+    while (kVariants[NEOGEMM_VARIANT_R64x64 + i].bm != roles.bm || kVariants[NEOGEMM_VARIANT_R64x64 + i].bn != roles.bn) ++i;
+    return bt.only->set((Kernel)((int)Kernel::kRoles64x64 + i), NEOGEMM_VARIANT_R64x64 + i, a.ksplit);
   }
   hipError_t e;
   if (roles.bm) e = launch_roles(a, roles.bm, roles.bn, ak, bk, st);
@@ -3801,6 +3814,23 @@ static int scratch_on_current_device(void** out) {
   }
   *out = ptrs[dev];
   return NEOGEMM_OK;
+}
+
+// What neogemm_bf16_general runs for these operands with so much workspace, without launching it.
+static int ask(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int a_layout,
+               int b_layout, int c_layout, float beta, int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t batch, size_t workspace_bytes,
+               Choice* c) {
+  BatchArgs bt;
+  bt.count = batch;
+  bt.sa = stride_a;
+  bt.sb = stride_b;
+  bt.sc = stride_c;
+  bt.a_layout = a_layout;
+  bt.scratch_unaligned = true;
+  bt.only = c;
+  void* ws = workspace_bytes ? (void*)256 : nullptr;  // never read
+  return run(A, B, const_cast<void*>(C), M, N, K, lda, ldb, ldc, b_layout, c_layout, ws, workspace_bytes, nullptr, NEOGEMM_VARIANT_AUTO, 0, 0, nullptr, 1.f,
+             beta, bt);
 }
 
 }  // namespace neogemm
@@ -3904,22 +3934,21 @@ const char* neogemm_bf16_call_kernel(const void* A, const void* B, const void* C
                                           {"strip", "copy+strip"}, {"short K", "copy+short K"}, {"roles 64x64", "copy+roles 64x64"},
                                           {"roles 128x64", "copy+roles 128x64"}, {"roles 128x128", "copy+roles 128x128"},
                                           {"roles 256x128", "copy+roles 256x128"}, {"roles 128x256", "copy+roles 128x256"}};
-  neogemm::BatchArgs bt;
-  bt.count = batch;
-  bt.sa = stride_a;
-  bt.sb = stride_b;
-  bt.sc = stride_c;
-  bt.a_layout = a_layout;
-  bt.scratch_unaligned = true;
-  neogemm::Kernel kernel = neogemm::Kernel::kNone;
-  bool copies = false;
-  bt.only_name = &kernel;
-  bt.copies = &copies;
-  void* ws = workspace_bytes ? (void*)256 : nullptr;  // never read: nothing is launched
-  if (neogemm::run(A, B, const_cast<void*>(C), M, N, K, lda, ldb, ldc, b_layout, c_layout, ws, workspace_bytes, nullptr, NEOGEMM_VARIANT_AUTO, 0, 0,
-                   nullptr, 1.f, beta, bt) != NEOGEMM_OK)
+  neogemm::Choice c;
+  if (neogemm::ask(A, B, C, M, N, K, lda, ldb, ldc, a_layout, b_layout, c_layout, beta, stride_a, stride_b, stride_c, batch, workspace_bytes, &c) != NEOGEMM_OK)
     return nullptr;
-  return kNames[(int)kernel][copies ? 1 : 0];
+  return kNames[(int)c.kernel][c.copies ? 1 : 0];
+}
+
+int neogemm_bf16_call_plan(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
+                           int a_layout, int b_layout, int c_layout, float beta, int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t batch,
+                           size_t workspace_bytes, int* variant, int* split_k) {
+  if (!variant || !split_k) return NEOGEMM_ERR_BAD_ARG;
+  neogemm::Choice c;
+  const int st = neogemm::ask(A, B, C, M, N, K, lda, ldb, ldc, a_layout, b_layout, c_layout, beta, stride_a, stride_b, stride_c, batch, workspace_bytes, &c);
+  *variant = c.variant;
+  *split_k = c.split;
+  return st;
 }
 
 size_t neogemm_bf16_batched_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t batch) {

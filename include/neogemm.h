@@ -84,7 +84,14 @@ extern "C" {
    argument of neogemm_bf16_variant carries the ring depths, 16 * stages of A + stages of B (0: the defaults); rings that
    do not fit the 160 KiB of LDS are refused. */
 #define NEOGEMM_VARIANT_STRIP 17
-#define NEOGEMM_VARIANT_COUNT 18
+/* Eight wave64: four only load, a 64-deep stage of both operands after the other into a ring of LDS images, four only compute (2x2); for
+   launches of about one workgroup per CU.  Operands in either order (of an MN-major one whole chunks of eight); K in split_k parts. */
+#define NEOGEMM_VARIANT_R64x64 18
+#define NEOGEMM_VARIANT_R128x64 19
+#define NEOGEMM_VARIANT_R128x128 20
+#define NEOGEMM_VARIANT_R256x128 21
+#define NEOGEMM_VARIANT_R128x256 22
+#define NEOGEMM_VARIANT_COUNT 23
 
 /*
  * C = A * op(B), bf16 in, fp32 accumulate, bf16 out.
@@ -161,6 +168,13 @@ size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M
 const char* neogemm_bf16_call_kernel(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                      int64_t ldc, int a_layout, int b_layout, int c_layout, float beta, int64_t stride_a, int64_t stride_b,
                                      int64_t stride_c, int64_t batch, size_t workspace_bytes);
+/*
+ * The same as numbers: the variant that runs (the roles' tiles among them; 0 for the kernels without a number, "ragged", "short K" and "none") and
+ * its split of K, of the product on the copies where there are copies.  The status is the call's own.
+ */
+int neogemm_bf16_call_plan(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
+                           int a_layout, int b_layout, int c_layout, float beta, int64_t stride_a, int64_t stride_b, int64_t stride_c,
+                           int64_t batch, size_t workspace_bytes, int* variant, int* split_k);
 
 /*
  * neogemm_bf16 for callers that cannot allocate device memory (code under HIP graph capture, tight serving
@@ -205,7 +219,8 @@ int neogemm_bf16_variant(const void* A, const void* B, void* C, int64_t M, int64
  * `aligned` is nonzero when pointers and leading dimensions satisfy the MFMA path (16-byte / 8-element); without it the answer is
  * NEOGEMM_VARIANT_GENERIC, which stands for every kernel outside the plan (operands at any address among them).  Where the answer is a
  * tile of 192x256 or less, a call may run a kernel with waves of their own for the loads instead, in another tile and with fewer splits of K
- * (so in another order of sums than neogemm_bf16_variant with the planned variant); where K is at most 128, one for short K.
+ * (so in another order of sums than neogemm_bf16_variant with the planned variant; neogemm_bf16_call_plan tells); where K is at most 128, one for
+ * short K.
  * The choice comes from a cost model over the tile variants; if the environment variable
  * NEOGEMM_PLAN_TABLE names a JSON file of tuned choices (an array of objects with the integer fields
  * "M","N","K","b_layout","c_layout","variant","split_k"; the layouts default to 0; gemm_amd/tune.py writes one), an

@@ -202,6 +202,22 @@ def test_call_kernel_names_without_a_gpu():
     assert _abi.call_kernel(p, q, c, 1024, 1024, 32768, 32768, 1024, 1024, 0, 0, ws_bytes=0) is None
 
 
+def test_call_plan_tells_tile_and_split():
+    """neogemm_bf16_call_plan: the numbers of what neogemm_bf16_call_kernel names, as the forced variant takes them."""
+    p, q, c = 1 << 20, 1 << 40, 1 << 44
+    assert _abi.call_plan(p, q, c, 1024, 1024, 1024, 1024, 1024, 1024, _abi.B_NK, _abi.C_COL) == (_abi.VARIANT_R64x64, 1)
+    assert _abi.call_plan(p, q, c, 1024, 1024, 32768, 32768, 1024, 1024, 0, 0) == (_abi.VARIANT_R256x128, 8)
+    assert _abi.call_plan(p, q, c, 1024, 1024, 32768, 32768, 1024, 1024, 0, 0, ws_bytes=0) is None
+    assert _abi.call_plan(p, q, c, 8192, 8192, 8192, 8192, 8192, 8192, 0, 0) == _abi.plan(8192, 8192, 8192)
+    assert _abi.call_plan(p, q, c, 16, 14336, 4096, 4096, 14336, 14336, 0, 0) == _abi.plan(16, 14336, 4096)
+    assert _abi.call_plan(p, q, c, 128, 8192, 8192, 8192, 8192, 8192, 1, 0) == (_abi.VARIANT_STRIP, 2)
+    assert _abi.call_plan(p, q, c, 100, 100, 101, 101, 100, 100, 0, 0) == (0, 1)          # operands at any address
+    assert _abi.call_plan(p, q, c, 4001, 4001, 4001, 4001, 4001, 4001, 0, 0)[0] == _abi.plan(4001, 4001, 4001)[0]   # the product on the copies
+    assert _abi.call_plan(p, q, c, 8, 8, 0, 1, 8, 8, 0, 0) == (_abi.VARIANT_GENERIC, 1) and _abi.call_plan(0, 0, 0, 0, 8, 8, 8, 8, 8, 0, 0) == (0, 1)
+    for v in range(_abi.VARIANT_COUNT):
+        assert v in _abi.VARIANT_NAMES
+
+
 def test_roles_are_weighed_against_the_kernel_that_would_run():
     """A C off 8-byte addresses without a workspace runs unsplit 128x128 tiles where the plan splits K: it is their time that counts then."""
     p, q, c = 1 << 20, 1 << 40, (1 << 44) + 2

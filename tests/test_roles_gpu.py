@@ -48,6 +48,38 @@ def test_roles(M, N, K, a_layout, b_layout, c_layout):
     assert torch.equal(got, (0.5 * want - old.float()).to(torch.bfloat16))
 
 
+TILES = {g.VARIANT_R64x64: (64, 64, 4), g.VARIANT_R128x64: (128, 64, 5), g.VARIANT_R128x128: (128, 128, 4), g.VARIANT_R256x128: (256, 128, 3),
+         g.VARIANT_R128x256: (128, 256, 3)}   # rows, columns, images in the ring
+
+
+# Every tile by its number.  Stages: one, the ring less one, whole and one more, each with 8 and with 64 of the last one filled (a K that is no
+# multiple of 64 ends every wrap-around in the middle of the tile's stages); 13 and 40 are staggered (tiles of up to 128, over fewer stages than there are
+# tiles in a row and column of C with 13), 65 are not; in two and three splits, the last one shorter.  C on the 8-byte grid and off it.
+@pytest.mark.parametrize("variant", TILES)
+@pytest.mark.parametrize("b_layout,c_layout", [(g.B_KN, g.C_ROW), (g.B_NK, g.C_ROW), (g.B_KN, g.C_COL), (g.B_NK, g.C_COL)])
+def test_every_tile(variant, b_layout, c_layout):
+    bm, bn, ring = TILES[variant]
+    gen = torch.Generator(device="cuda").manual_seed(variant)
+    for stages, split in [(s, 1) for s in (1, ring - 1, ring, ring + 1, 13, 40, 65)] + [(ring + 1, 2), (29, 2), (47, 3)]:
+        for last in (8, 64):
+            K = 64 * (stages - 1) + last
+            if split > 1 and last == 64:
+                continue
+            # tiles in a row and column of C as it lies in memory, then less than one tile
+            for rows, cols in ((3 * bm + 8, (10 if stages == 13 else 2) * bn - 24), (8, 16)):
+                M, N = (rows, cols) if c_layout == g.C_ROW else (cols, rows)
+                A = torch.full((M, K + 8), float("nan"), dtype=torch.bfloat16, device="cuda")[:, :K]
+                B = torch.full((K, N + 16) if b_layout == g.B_KN else (N, K + 16), float("nan"), dtype=torch.bfloat16, device="cuda")[:, :-16]
+                A.copy_(ints(gen, M, K)), B.copy_(ints(gen, *B.shape))
+                want = (A.float() @ (B if b_layout == g.B_KN else B.t()).float()).to(torch.bfloat16)
+                for off in (0, 1):
+                    buf = torch.full((rows * cols + 1,), float("nan"), dtype=torch.bfloat16, device="cuda")
+                    C = buf[off:off + rows * cols].view(rows, cols)
+                    g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), cols, b_layout, c_layout, variant, split)
+                    assert torch.equal(C if c_layout == g.C_ROW else C.t(), want), (stages, split, K, rows, cols, off)
+                    assert bool(torch.isnan(buf[rows * cols if off == 0 else 0]))
+
+
 # 64x64, 128x128, 128x256: the problems of a batch, the second operand shared or not
 @pytest.mark.parametrize("batch,M,N,K", [(4, 1024, 128, 1024), (32, 1024, 128, 1024), (20, 1024, 136, 1000)])
 def test_roles_batched(batch, M, N, K):
