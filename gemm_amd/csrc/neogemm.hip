@@ -2882,11 +2882,11 @@ static const std::vector<PlanEntry>& plan_table() {
   }();
   return table;
 }
-static bool plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
+static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
                           int64_t batch, int b_layout, int ncus, int a_layout, double* estimate_us);
 // The cost model walks every (tile, split) candidate: a few microseconds on the host, as long as a small GEMM takes
 // on the GPU.  A caller in a loop repeats a handful of shapes, so each thread remembers its last few answers.
-// estimate_us: the model's, or 0 where a table of the user's names the kernel.
+// estimate_us: the model's, or 0 where a table names the kernel.
 static void plan(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
                  int64_t batch = 1, int b_layout = NEOGEMM_B_KN, int a_layout = NEOGEMM_A_MK, double* estimate_us = nullptr) {
   struct Memo {
@@ -2906,7 +2906,7 @@ static void plan(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, in
       return;
     }
   double us = 0;
-  if (plan_uncached(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout, &us)) us = 0;
+  plan_uncached(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout, &us);
   if (estimate_us) *estimate_us = us;
   Memo& m = memo[next++ & 31];
   m.estimate_us = us;
@@ -2922,10 +2922,12 @@ static const int kDefaultPlanCus = 256;
 static const PlanEntry kDefaultPlan[] = {
 #include "neogemm_default_plan.inc"
 };
-// true: the choice of the user's table
-static bool plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
+// A table's entry, the user's or the library's, names the kernel that runs (the roles' tiles by their numbers) and was measured as such: nothing
+// is weighed against it.  (The shipped entries were for a time, by the estimate of the model's own choice: 64 x 28672 x 8192 ran 118 us in 64x64
+// tiles of the roles where the entry's 256-wide tiles take 93 and the roles' 128x128, which it names now, 89; of 300 entries 82 lost more than 2 %.)
+static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_layout, int* variant, int* split_k,
                           int64_t batch, int b_layout, int ncus, int a_layout, double* estimate_us) {
-  plan_model(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout, estimate_us);
+  *estimate_us = 0;
   if (aligned && K > 0 && batch == 1 && a_layout == NEOGEMM_A_MK) {
     auto match = [&](const PlanEntry& e) {
       return e.M == M && e.N == N && e.K == K && e.c_layout == c_layout && e.b_layout == b_layout;
@@ -2934,17 +2936,17 @@ static bool plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_l
       if (match(e)) {
         *variant = e.variant;
         *split_k = e.variant == NEOGEMM_VARIANT_GENERIC ? 1 : e.split_k;
-        return true;
+        return;
       }
     if (ncus == kDefaultPlanCus)
       for (const PlanEntry& e : kDefaultPlan)
         if (match(e)) {
           *variant = e.variant;
           *split_k = e.split_k;
-          break;
+          return;
         }
   }
-  return false;
+  plan_model(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout, estimate_us);
 }
 
 // Whether gemm_roles_kernel takes a call that the plan gives to kernel v with split_max splits of K, estimated at plan_us; in the kernel's
@@ -3687,9 +3689,9 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   // too (a column-major C; that went to the 128x128 tile), as long as they fit the CUs one and a half times (B [N,K]: 1152^3, 324 of them, 10.6 us
   // in tiles of gemm_tile_kernel and 9.0, 1280^3, 400, level, 1024 x 2048 x 1536, 512, 11.8 and 12.4) or twice (B [K,N]: 13.7 and 12.5 for that last
   // one).  Few workgroups with whole trips of the tile kernel's main loop stay there: 256 x 1024 x 1024, 64 of them, 5.9 us and 6.7 with B [N,K],
-  // 7.1 and 7.3 with B [K,N]; 200 x 1000 x 1000 with B [K,N] 9.3 and 7.6.
+  // 7.1 and 7.3 with B [K,N]; 200 x 1000 x 1000 with B [K,N] 9.3 and 7.6.  (plan_us: the model's choice, not a table's.)
   bool small = false;
-  if (variant == NEOGEMM_VARIANT_AUTO && (v == NEOGEMM_VARIANT_T64x64_W4 || v == NEOGEMM_VARIANT_T64x128_W4) &&
+  if (plan_us > 0 && (v == NEOGEMM_VARIANT_T64x64_W4 || v == NEOGEMM_VARIANT_T64x128_W4) &&
       (ak || bk) && (ak || (a.M & 7) == 0 || bt.padded) && (bk || (a.N & 7) == 0 || bt.padded)) {
     const int64_t cus = planning_cus(), wgs = (int64_t)ceil_div(a.M, 64) * ceil_div(a.N, 64) * s * bt.count;
     const int kt = ceil_div(K, KTILE);
@@ -3733,7 +3735,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   a.alpha = alpha;
   a.early_stores = 0;
   a.beta = beta;
-  if (variant == NEOGEMM_VARIANT_AUTO && ak && bk && K <= 2 * KTILE && beta == 0.f && a.ksplit == 1) {
+  if (plan_us > 0 && ak && bk && K <= 2 * KTILE && beta == 0.f && a.ksplit == 1) {
     // at least two column tiles for each of two workgroups per CU (16 x 512 x 512 x 96, one each: level with the tile kernels)
     const int64_t tiles = (int64_t)ceil_div(a.M, 128) * ceil_div(a.N, 64) * bt.count, slots = 2 * (int64_t)planning_cus();
     if (tiles >= 2 * slots) {

@@ -217,14 +217,15 @@ int neogemm_bf16_variant(const void* A, const void* B, void* C, int64_t M, int64
 /*
  * What neogemm_bf16 would pick for this call: writes the variant id and split-K factor.  Host only.
  * `aligned` is nonzero when pointers and leading dimensions satisfy the MFMA path (16-byte / 8-element); without it the answer is
- * NEOGEMM_VARIANT_GENERIC, which stands for every kernel outside the plan (operands at any address among them).  Where the answer is a
- * tile of 192x256 or less, a call may run a kernel with waves of their own for the loads instead, in another tile and with fewer splits of K
+ * NEOGEMM_VARIANT_GENERIC, which stands for every kernel outside the plan (operands at any address among them).  Where the answer is the
+ * model's and a tile of 192x256 or less, a call may run a kernel with waves of their own for the loads instead, in another tile and with fewer splits of K
  * (so in another order of sums than neogemm_bf16_variant with the planned variant; neogemm_bf16_call_plan tells); where K is at most 128, one for
  * short K.
  * The choice comes from a cost model over the tile variants; if the environment variable
  * NEOGEMM_PLAN_TABLE names a JSON file of tuned choices (an array of objects with the integer fields
  * "M","N","K","b_layout","c_layout","variant","split_k"; the layouts default to 0; gemm_amd/tune.py writes one), an
- * entry for the exact shape and layouts wins.  The file is read once per process.
+ * entry for the exact shape and layouts wins and is what runs; so does one of the table that the library ships.  The file is read once per
+ * process.
  */
 int neogemm_bf16_plan(int64_t M, int64_t N, int64_t K, int b_layout, int c_layout, int aligned,
                       int* variant, int* split_k);

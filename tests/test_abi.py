@@ -309,6 +309,10 @@ def test_plan_table_overrides_the_model(tmp_path):
         {"M": 8192, "N": 8192, "K": 8192, "c_layout": 0, "variant": 99, "split_k": 1},           # unknown variant
         {"M": 1024, "N": 1024, "K": 1024, "c_layout": 0, "variant": _abi.VARIANT_T128x128_W4, "split_k": 0},  # bad split
         {"M": 2048, "N": 2048, "K": 2048, "b_layout": 1, "c_layout": 1, "variant": _abi.VARIANT_T128x256_W4, "split_k": 1},
+        {"M": 640, "N": 640, "K": 640, "b_layout": 1, "variant": _abi.VARIANT_T64x64_W4, "split_k": 1},
+        {"M": 1024, "N": 1024, "K": 1024, "b_layout": 1, "variant": _abi.VARIANT_R128x64, "split_k": 2},
+        {"M": 2048, "N": 2048, "K": 128, "b_layout": 1, "variant": _abi.VARIANT_T256x256_W4, "split_k": 1},
+        {"M": 100, "N": 1028, "K": 1024, "variant": _abi.VARIANT_R64x64, "split_k": 1},          # no whole chunks of B [K,N]
     ]))
     code = ("from gemm_amd import _abi\n"
             "print(_abi.plan(512, 512, 512), _abi.plan(4096, 4096, 4096), _abi.plan(8192, 8192, 8192), "
@@ -322,6 +326,14 @@ def test_plan_table_overrides_the_model(tmp_path):
             # an entry is keyed on both layouts: B [N,K] calls of a shape tuned with B [K,N] keep the model's choice
             _abi.plan(512, 512, 512, b_layout=1), (_abi.VARIANT_T128x256_W4, 1), _abi.plan(2048, 2048, 2048, 0, 1))
     assert out.strip() == " ".join(str(w) for w in want)
+    # an entry names the kernel that runs: no other one for small problems, for short K or with waves of its own for the loads
+    code = ("from gemm_amd import _abi\n"
+            "print([_abi.call_plan(1 << 20, 1 << 40, 1 << 44, M, N, K, K, ldb, N, b, 0) for M, N, K, ldb, b in "
+            "((512, 512, 512, 512, 0), (640, 640, 640, 640, 1), (1024, 1024, 1024, 1024, 1), (2048, 2048, 128, 128, 1))], "
+            "_abi.call_kernel(1 << 20, 1 << 40, 1 << 44, 100, 1028, 1024, 1024, 1032, 1028, 0, 0))")
+    out = subprocess.run([sys.executable, "-c", code], env=env, cwd=ROOT, capture_output=True, text=True, check=True).stdout
+    want = [(_abi.VARIANT_T128x128_W4, 2), (_abi.VARIANT_T64x64_W4, 1), (_abi.VARIANT_R128x64, 2), (_abi.VARIANT_T256x256_W4, 1)]
+    assert out.strip() == str(want) + " ragged"
     # an unreadable file changes nothing
     env = dict(os.environ, NEOGEMM_PLAN_TABLE=str(tmp_path / "missing.json"))
     out = subprocess.run([sys.executable, "-c", "from gemm_amd import _abi\nprint(_abi.plan(512, 512, 512))"], env=env,
@@ -340,7 +352,8 @@ def test_shipped_plan_table():
     rows = [r for r in rows if r[0] > 0]
     assert len(rows) >= 10
     assert len({r[:5] for r in rows}) == len(rows)                       # one entry per shape and layout pair
-    tile_variants = (_abi.VARIANT_T256x256_W4, _abi.VARIANT_T128x128_W4, _abi.VARIANT_T256x128_W4, _abi.VARIANT_T128x256_W4,
+    tile_variants = (_abi.VARIANT_R64x64, _abi.VARIANT_R128x64, _abi.VARIANT_R128x128, _abi.VARIANT_R256x128, _abi.VARIANT_R128x256,
+                     _abi.VARIANT_T256x256_W4, _abi.VARIANT_T128x128_W4, _abi.VARIANT_T256x128_W4, _abi.VARIANT_T128x256_W4,
                      _abi.VARIANT_T64x128_W4, _abi.VARIANT_T192x256_W4, _abi.VARIANT_T96x128_W4, _abi.VARIANT_T64x64_W4,
                      _abi.VARIANT_C256x256_W4)
     for (M, N, K, b, c, v, s) in rows:
@@ -350,5 +363,6 @@ def test_shipped_plan_table():
         if v in (_abi.VARIANT_C256x256_W4, _abi.VARIANT_SKINNY128) or v >= _abi.VARIANT_SKINNY16 and v <= _abi.VARIANT_SKINNY64:
             assert s == 1      # (the strip kernel is the one streaming kernel that splits K)
         assert _abi.plan(M, N, K, b, c) == (v, s), (M, N, K, b, c)
+        assert _abi.call_plan(1 << 20, 1 << 40, 1 << 44, M, N, K, K, N if b == _abi.B_KN else K, N if c == _abi.C_ROW else M, b, c) == (v, s), (M, N, K, b, c)
         assert _abi.workspace_bytes(M, N, K) >= (s * M * N * 4 if s > 1 else 0)
         assert _abi.plan(M, N, K, b, c, aligned=False) == (_abi.VARIANT_GENERIC, 1)   # the table is for the MFMA path only
