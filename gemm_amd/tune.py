@@ -7,8 +7,8 @@
 The table is the JSON array libneogemm.so looks up before its cost model (neogemm_bf16_plan): objects
 {"M","N","K","b_layout","c_layout","variant","split_k"}; an entry applies to exactly its shape and layouts
 (--b-layout 1 tunes B [N,K], --c-layout 1 a column-major C: --b-layout 1 --c-layout 1 is the reference's call,
-nemgemmV03.cu:343-391).  Only shapes whose best measured candidate beats the model's
-choice by more than --margin are written.  The reference has nothing of the kind: its tile and stage
+nemgemmV03.cu:343-391).  Only shapes whose best measured candidate beats what the library runs by
+itself by more than --margin are written (the model's choice too, where a call runs the kernel with roles instead of it).  The reference has nothing of the kind: its tile and stage
 counts are template arguments (v01.cu:275-278, 304-311).
 """
 import argparse
@@ -24,7 +24,8 @@ from ._abi import B_KN, B_NK, C_COL, C_ROW, ERR_UNSUPPORTED, NeoGemmError
 CANDIDATE_VARIANTS = (_abi.VARIANT_T256x256_W4, _abi.VARIANT_C256x256_W4, _abi.VARIANT_T128x256_W4,
                       _abi.VARIANT_T256x128_W4, _abi.VARIANT_T128x128_W4, _abi.VARIANT_T64x128_W4,
                       _abi.VARIANT_T192x256_W4, _abi.VARIANT_T96x128_W4, _abi.VARIANT_T64x64_W4, _abi.VARIANT_SKINNY16, _abi.VARIANT_SKINNY32, _abi.VARIANT_SKINNY64,
-                      _abi.VARIANT_SKINNY128, _abi.VARIANT_STRIP)
+                      _abi.VARIANT_SKINNY128, _abi.VARIANT_STRIP, _abi.VARIANT_R64x64, _abi.VARIANT_R128x64, _abi.VARIANT_R128x128,
+                      _abi.VARIANT_R256x128, _abi.VARIANT_R128x256)
 CANDIDATE_SPLITS = (1, 2, 3, 4, 6, 8, 12, 16, 24, 32)
 
 
@@ -53,7 +54,8 @@ def time_us(fn, warmup=5, iters=30, preheat_ms=0.0):
 
 
 def tune_shape(M, N, K, nbuf=1, log=sys.stderr, b_layout=B_KN, c_layout=C_ROW, dump=None):
-    """Returns (model choice, its time, best choice, its time) for A [M,K], B in `b_layout`, C in `c_layout`."""
+    """Returns (model choice, time of the call without a choice, best choice, its time) for A [M,K], B in `b_layout`, C in `c_layout`.  The two
+    times are equal, and the best choice is what runs (the model's if that has no number), where no candidate beats it."""
     gen = torch.Generator().manual_seed(0)
     A = (torch.randn(M, K, generator=gen) / math.sqrt(K)).to(torch.bfloat16).cuda()
     b_shape = (K, N) if b_layout == B_KN else (N, K)
@@ -66,9 +68,17 @@ def tune_shape(M, N, K, nbuf=1, log=sys.stderr, b_layout=B_KN, c_layout=C_ROW, d
         gemm_into(A, Bs[turn[0] % nbuf], C, M, N, K, K, b_shape[1], C.shape[1], b_layout, c_layout, variant, split, 0)
 
     model = plan(M, N, K, b_layout, c_layout)
+    runs = _abi.call_plan(A.data_ptr(), Bs[0].data_ptr(), C.data_ptr(), M, N, K, K, b_shape[1], C.shape[1], b_layout, c_layout)
+    if runs is not None and runs[0] == _abi.VARIANT_AUTO:
+        runs = None   # a kernel without a number: none of the candidates is what runs
+    ktiles = -(-K // 64)
+
+    def is_what_runs(c):   # (splits that would be empty are left out)
+        return runs is not None and c[0] == runs[0] and runs[1] in (c[1], -(-ktiles // -(-ktiles // c[1])))
+
     heat = 150.0 if 2.0 * M * N * K > 5e10 else 0.0   # GEMMs of tens of microseconds and more run into the power limit
     t_model = time_us(lambda: call(None, 0), preheat_ms=heat)
-    best, t_best = model, t_model
+    best, t_best = runs or model, t_model
     for v in CANDIDATE_VARIANTS:
         for s in CANDIDATE_SPLITS:
             if s > 1 and K // (64 * s) < 2:
@@ -92,9 +102,9 @@ def tune_shape(M, N, K, nbuf=1, log=sys.stderr, b_layout=B_KN, c_layout=C_ROW, d
             if t < t_best:
                 best, t_best = (v, s), t
     t_model = min(t_model, time_us(lambda: call(None, 0), preheat_ms=heat))   # the first measurement ran on a cold clock
-    if best == model or t_model <= t_best:
-        best, t_best = model, t_model
-    print(f"{M}x{N}x{K} b{b_layout} c{c_layout}: model {model} {t_model:.2f} us, best {best} {t_best:.2f} us", file=log)
+    if is_what_runs(best) or t_model <= t_best:
+        best, t_best = runs or model, t_model
+    print(f"{M}x{N}x{K} b{b_layout} c{c_layout}: model {model}, runs {runs or 'another kernel'} {t_model:.2f} us, best {best} {t_best:.2f} us", file=log)
     return model, t_model, best, t_best
 
 
@@ -124,7 +134,7 @@ def main():
     ap.add_argument("--out")
     ap.add_argument("--merge", nargs="+", metavar="TABLE.json", help="merge these tables instead of measuring (no GPU needed)")
     ap.add_argument("--inc", help="with --merge: write the merged table as the library's default-plan include file")
-    ap.add_argument("--margin", type=float, default=0.03, help="minimum relative gain over the model's choice")
+    ap.add_argument("--margin", type=float, default=0.03, help="minimum relative gain over what the library runs by itself")
     ap.add_argument("--nbuf", type=int, default=1, help="rotate this many B buffers (streaming shapes)")
     ap.add_argument("--cold-weights-mb", type=float, default=0.0,
                     help="rotate as many B buffers as it takes to exceed this many MB (more than the last-level cache: every "
@@ -159,7 +169,7 @@ def main():
             with open(args.dump, "a") as f:
                 for d in dump:
                     f.write(json.dumps(d) + "\n")
-        if best != model and t_best < t_model * (1.0 - args.margin):
+        if t_best < t_model * (1.0 - args.margin):
             table.append({"M": M, "N": N, "K": K, "b_layout": args.b_layout, "c_layout": args.c_layout,
                           "variant": best[0], "split_k": best[1]})
         # the table so far after every shape: a sweep that is cut short keeps what it has measured

@@ -135,3 +135,31 @@ def test_roles_with_fewer_splits_want_the_planned_workspace(M, N, K, a_layout, b
     torch.cuda.synchronize()
     want = (A if a_layout == g.A_MK else A.t()).float() @ (B if b_layout == g.B_KN else B.t()).float()
     assert torch.equal(C.t(), want.to(torch.bfloat16))
+
+
+def test_tuner_compares_with_what_runs(monkeypatch):
+    """gemm_amd.tune: the planned kernel, where a call runs the roles instead of it and it is the faster one, is an entry; what runs anyway is none."""
+    import io
+
+    from gemm_amd import tune
+    M, N, K = 1800, 1928, 392
+    planned = g.plan(M, N, K)
+    runs = _abi.call_plan(1 << 20, 1 << 40, 1 << 44, M, N, K, K, N, N, g.B_KN, g.C_ROW)
+    assert runs == (g.VARIANT_R128x128, 1) and planned[0] != runs[0]
+    last, times = [None], {}
+
+    def timed(fn, **kw):
+        fn()
+        return times.get(last[0], 50.0)
+
+    def note(*args):
+        last[0] = args[-3:-1]
+
+    monkeypatch.setattr(tune, "gemm_into", note)
+    monkeypatch.setattr(tune, "time_us", timed)
+    times.update({(None, 0): 12.0, planned: 10.0, runs: 11.0})
+    assert tune.tune_shape(M, N, K, log=io.StringIO()) == (planned, 12.0, planned, 10.0)
+    times.update({(None, 0): 12.0, planned: 13.0, runs: 11.0})
+    assert tune.tune_shape(M, N, K, log=io.StringIO()) == (planned, 12.0, runs, 12.0)
+    times.update({(None, 0): 9.0, planned: 10.0, (g.VARIANT_R64x64, 1): 8.0})
+    assert tune.tune_shape(M, N, K, log=io.StringIO()) == (planned, 9.0, (g.VARIANT_R64x64, 1), 8.0)
