@@ -2949,45 +2949,40 @@ static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_l
   plan_model(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout, estimate_us);
 }
 
-// Whether gemm_roles_kernel takes a call that the plan gives to kernel v with split_max splits of K, estimated at plan_us; in the kernel's
+// Whether gemm_roles_kernel takes a call that the model gives to kernel v with split_max splits of K, estimated at plan_us; in the kernel's
 // terms: `rows` x `cols` of C as it lies in memory, ak / bk: the row / column operand has K-contiguous rows, lda / ldb their leading dimensions.
-// Fitted to 9900 timings of 1010 problems with these tiles (1 to 20000 rows and columns, 32 to 65000 deep, both layouts of each operand, batches),
-// up to 48 MB to the mean of operands in the caches and from HBM, above to operands from HBM, rms 9 and 10 %: a launch, a way in and out per
-// round of workgroups, per 64 deep what a stage takes, more where rows of an operand are no whole cache lines apart (a piece of 128 bytes then lies
-// in two lines, and is requested twice), and the reduction.  A CU holds two workgroups of the 64x64 tile, which then take 1.75 times as long, and one
-// of the others.  The best of these by estimate is 0.8 % behind the best measured on average.  It is taken where it beats the plan's estimate times a
-// factor by planned tile (64x128 and 128x128 tiles take 1.35 and 1.2 times their estimates, and in one round of 128 rows and more the roles
-// were at most 2 % behind): 620 of 1010 problems, 9 % faster on average over all of them (2048^3 from HBM 23.2 -> 20.8 us, 512 x 4096 x 4096
-// 31.4 -> 26.7, 1024 x 1024 x 2048 14.3 -> 11.8), 9 of them more than 3 % slower.  Short K and more planned workgroups than CUs count for less: the way
-// in and out of a workgroup is longer here, and a CU holds one (18 x 576 x 576 x 96 8.6 us in 128x128 tiles of gemm_tile_kernel, of which a CU holds
-// two, 11.8 here; 10001 x 1024 x 512 with a transposed A 17.5 and 21; 1856 x 3392 x 472 11.4 and 13.0), as do 96x128 tiles of two K-major operands
-// a multiple of 256 deep (3000 x 760 x 1024 9.9 and 11.3, 1344 x 1792 x 768 7.7 and 7.9; 1600 deep and from HBM the roles are ahead again, 672 x
-// 3840 x 1536 17.6 and 15.0; in the caches 1536^3 is the worst, 10.9 and 12.9).  Not where the plan names strips (124 x 5248 x
-// 20608 from HBM 57.7 -> 60.9), 256x256 tiles, or 192x256 ones with K split or from HBM (304 x 1864 x 50048 80 -> 95, 449 x 20352 x 5120 103 -> 129).
+// Fitted to 42000 timings of 4700 problems with these tiles (1 to 20000 rows and columns, 32 to 65000 deep, both layouts of each operand, batches),
+// to the mean of operands in the caches and from HBM up to 32 MB, from HBM alone from 64 MB on and in between to what lies between, rms 8.2 %: a
+// launch, a way in and out per round of workgroups, per 64 deep what a stage takes (longer from HBM) and how much more on a full chip, and the
+// reduction.  A stage takes more where rows of an operand are no whole cache lines apart (a piece of 128 bytes then lies in two lines, and is
+// requested twice), where an MN-major operand from HBM is read in pieces of 64 columns, and in the 64-wide tiles beyond the 64 stages of the
+// stagger; less where the tile reaches past the matrix.  A CU holds two workgroups of the 64x64 tile, which then take 1.66 times as long, and one of
+// the others.  The best of these by estimate is 1 % behind the best measured on average.
+// It is taken where it beats the plan's estimate times what the planned kernels take of theirs.  Tiles of up to 128x128 take 1.1 to 2.4 times it, most
+// with a short K (1272 x 1160 x 208 with a transposed A 7.9 us, 6.2 here), and in one round of workgroups were seldom ahead (64 and 96 rows by 2 % in
+// 9 of 1059 problems); but of more rounds a CU holds two of theirs and one of these (3072 x 3264 x 304 with a transposed A 15.6 us, 16.2 and more here;
+// 63 x 276 x 276 x 96 11.7 and 17.6).  Not where the plan names strips (124 x 5248 x 20608 from HBM 57.7 -> 60.9) or 256x256 tiles.  Against the rule
+// before (constants of two sizes of problems that met at 48 MB, factors with exceptions by K and workgroups): 4500 problems 1.5 % faster on average; of
+// the 3400 above 8 us 650 by more than 3 %, 150 slower by that (most from HBM with fewer than 64 rows, where these tiles' times scatter).
 // No more splits than planned: what a caller's workspace holds, or whether one is needed, does not change.
 struct RolesPlan {
   int bm = 0, bn = 0, split = 1;  // bm == 0: not taken
 };
 static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, int64_t cols, int64_t K, int64_t batch, bool ak, bool bk,
                             int64_t lda, int64_t ldb) {
-  const double bytes = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch;
-  const bool hbm = bytes > 48e6;
+  const int cus = planning_cus();
+  const double planned = (double)ceil_div(rows, kVariants[v].bm) * (double)ceil_div(cols, kVariants[v].bn) * split_max * (double)batch;
   double against = 0;
   switch (v) {
     case NEOGEMM_VARIANT_T64x128_W4:
-    case NEOGEMM_VARIANT_T64x64_W4: against = 1.4; break;
-    case NEOGEMM_VARIANT_T96x128_W4: against = ak && bk && K % 256 == 0 && K <= 1024 ? 1.0 : 1.8; break;
-    case NEOGEMM_VARIANT_T128x128_W4: against = 2.0; break;
+    case NEOGEMM_VARIANT_T64x64_W4:
+    case NEOGEMM_VARIANT_T96x128_W4:
+    case NEOGEMM_VARIANT_T128x128_W4: against = planned <= cus ? 3.0 : 1.0; break;
     case NEOGEMM_VARIANT_T256x128_W4:
     case NEOGEMM_VARIANT_T128x256_W4: against = 1.4; break;
-    case NEOGEMM_VARIANT_T192x256_W4: against = split_max == 1 && !hbm ? 1.0 : 0.0; break;
-    default: break;
+    case NEOGEMM_VARIANT_T192x256_W4: against = 1.0; break;
+    default: return RolesPlan();
   }
-  if (against == 0) return RolesPlan();
-  const int cus = planning_cus();
-  if (K <= 256 && against > 1.2) against = 1.2;
-  const double planned = (double)ceil_div(rows, kVariants[v].bm) * (double)ceil_div(cols, kVariants[v].bn) * split_max * (double)batch;
-  if (against > 1.0 && planned > (v == NEOGEMM_VARIANT_T256x128_W4 || v == NEOGEMM_VARIANT_T128x256_W4 || v == NEOGEMM_VARIANT_T96x128_W4 ? 2.0 : 1.0) * cus) against = 1.0;
   const bool a_whole = (lda & 63) == 0, b_whole = (ldb & 63) == 0;
   struct Memo {
     int64_t rows = -1, cols = -1, K = -1, batch = -1;
@@ -3003,32 +2998,40 @@ static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, 
         m.plan_us == plan_us)
       return m.plan;
   struct Tile {
-    int bm, bn, per_cu;
-    double fixed_us, stage_us, full_us;  // per workgroup; per stage on an empty chip, and how much more on a full one
+    int bm, bn;
+    double fixed_us, cached_us, hbm_us, full_us;  // per workgroup; per stage on an empty chip, from the caches and from HBM; how much more on a full one
   };
-  static const Tile kTiles[2][5] = {{{64, 64, 2, 1.10, 0.177, 0.029}, {128, 64, 1, 1.37, 0.253, 0.071}, {128, 128, 1, 2.16, 0.337, 0.082},
-                                     {256, 128, 1, 4.21, 0.562, -0.095}, {128, 256, 1, 4.91, 0.573, -0.104}},
-                                    {{64, 64, 2, 3.11, 0.223, 0.030}, {128, 64, 1, 0.93, 0.329, 0.053}, {128, 128, 1, 2.46, 0.433, 0.077},
-                                     {256, 128, 1, 2.17, 0.618, 0.066}, {128, 256, 1, 4.54, 0.686, 0.009}}};
+  static const Tile kTiles[] = {{64, 64, 1.37, 0.143, 0.223, 0.057},
+                                {128, 64, 1.85, 0.225, 0.305, 0.073},
+                                {128, 128, 2.65, 0.330, 0.470, 0.063},
+                                {256, 128, 4.21, 0.589, 0.692, 0.056},
+                                {128, 256, 5.31, 0.560, 0.713, 0.032}};
   const int64_t ktiles = ceil_div(K, KTILE);
-  const double floor_us = hbm ? bytes / 6.0e6 : 0.0;
+  const double bytes = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch;
+  const double hbm = bytes <= 32e6 ? 0.0 : bytes >= 64e6 ? 1.0 : __builtin_log2(bytes / 32e6);  // how much of the operands comes from there
   double best = against * plan_us;
   RolesPlan p;
-  for (const Tile& t : kTiles[hbm]) {
-    // further lines a piece of an operand's row touches: one in two for 128 bytes along K, 64 columns of an MN-major operand likewise
+  for (const Tile& t : kTiles) {
+    // shares of a stage's lines: with a neighbour that is requested too (one for 128 bytes along K, one in two for 128 columns of an MN-major
+    // operand); in pieces of 64 columns; past the matrix
     auto more = [](bool kmaj, bool whole, int w) { return whole ? 0.0 : kmaj ? 1.0 : 64.0 / w; };
-    const double lines = (t.bm * more(ak, a_whole, t.bm) + t.bn * more(bk, b_whole, t.bn)) / (t.bm + t.bn);
+    auto past = [](int w, int64_t n) { return n < w ? w - (double)n : 0.0; };
+    const double all = t.bm + t.bn, lines = (t.bm * more(ak, a_whole, t.bm) + t.bn * more(bk, b_whole, t.bn)) / all;
+    const double narrow = ((!ak && t.bm == 64 ? t.bm : 0) + (!bk && t.bn == 64 ? t.bn : 0)) / all, waste = (past(t.bm, rows) + past(t.bn, cols)) / all;
+    const double one = (t.cached_us + (t.hbm_us - t.cached_us) * hbm) * (1.0 + 0.428 * lines + 0.333 * hbm * narrow) * (1.0 - 0.383 * waste);
     for (int sp : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
       if (sp > split_max || (sp > 1 && ktiles / sp < 4)) break;
       const double per = (double)ceil_div(ktiles, sp), wgs = (double)ceil_div(rows, t.bm) * (double)ceil_div(cols, t.bn) * sp * (double)batch;
       if (wgs > 2.0 * cus) break;
-      const double one = t.stage_us * (1.0 + (hbm ? 0.61 : 0.46) * lines), full = t.fixed_us + per * (one + t.full_us);
-      double us = hbm ? 2.9 : 3.2;
-      if (wgs <= cus) us += t.fixed_us + per * (one + t.full_us * wgs / cus);
-      else if (t.per_cu == 2) us += t.fixed_us + per * (one + t.full_us) * (hbm ? 1.71 : 1.77);
-      else us += full + t.fixed_us + per * (one + t.full_us * (wgs - cus) / cus);
+      const double stage = t.bn == 64 && per > 64.0 ? one * (1.0 + 0.266 * (1.0 - hbm)) : one;  // (no stagger)
+      const double full = t.fixed_us + per * (stage + t.full_us);
+      double us = 2.67;
+      if (wgs <= cus) us += t.fixed_us + per * (stage + t.full_us * wgs / cus);
+      else if (t.bn == 64 && t.bm == 64) us += 1.656 * full;
+      else us += full + t.fixed_us + per * (stage + t.full_us * (wgs - cus) / cus);
+      const double floor_us = hbm * bytes / 5.41e6;
       if (us < floor_us) us = floor_us + 0.01 * us;
-      if (sp > 1) us += (hbm ? 0.3 : 1.6) + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / (hbm ? 1.82e6 : 2.38e6);
+      if (sp > 1) us += 1.97 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 2.74e6;
       if (us < best) {
         best = us;
         p.bm = t.bm;
@@ -3685,23 +3688,6 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   // (the chained 256x256 kernel takes its rows from a K-major operand only, K in whole periods of 128 and no split)
   const bool fits = !variant_roles(v) && (ak || mn_ok(vi.bm, a.M)) && (bk || mn_ok(vi.bn, a.N)) &&
                     (v != NEOGEMM_VARIANT_C256x256_W4 || (ak && K % (2 * KTILE) == 0 && s <= 1));
-  // Where the plan says 64 rows per tile and roles_plan does not take the call, 64x64 tiles of gemm_roles_kernel do, with B [K,N] on the rows
-  // too (a column-major C; that went to the 128x128 tile), as long as they fit the CUs one and a half times (B [N,K]: 1152^3, 324 of them, 10.6 us
-  // in tiles of gemm_tile_kernel and 9.0, 1280^3, 400, level, 1024 x 2048 x 1536, 512, 11.8 and 12.4) or twice (B [K,N]: 13.7 and 12.5 for that last
-  // one).  Few workgroups with whole trips of the tile kernel's main loop stay there: 256 x 1024 x 1024, 64 of them, 5.9 us and 6.7 with B [N,K],
-  // 7.1 and 7.3 with B [K,N]; 200 x 1000 x 1000 with B [K,N] 9.3 and 7.6.  (plan_us: the model's choice, not a table's.)
-  bool small = false;
-  if (plan_us > 0 && (v == NEOGEMM_VARIANT_T64x64_W4 || v == NEOGEMM_VARIANT_T64x128_W4) &&
-      (ak || bk) && (ak || (a.M & 7) == 0 || bt.padded) && (bk || (a.N & 7) == 0 || bt.padded)) {
-    const int64_t cus = planning_cus(), wgs = (int64_t)ceil_div(a.M, 64) * ceil_div(a.N, 64) * s * bt.count;
-    const int kt = ceil_div(K, KTILE);
-    if (ak && bk) small = 2 * wgs <= 3 * cus && !(wgs <= 64 && s == 1 && kt >= 8 && kt % 4 == 0);
-    else small = wgs <= 2 * cus && !(fits && wgs <= 64 && s == 1 && K >= 1024 && K % 256 == 0);
-  }
-  if (small && !roles.bm) {
-    roles.bm = roles.bn = 64;
-    roles.split = s;
-  }
   if (!fits && !roles.bm) {
     if (variant != NEOGEMM_VARIANT_AUTO) return NEOGEMM_ERR_UNSUPPORTED;
     // the planned tile is too wide for an MN-major operand (or takes whole chunks of it only): the 128x128 tile needs the least

@@ -226,6 +226,23 @@ def test_roles_are_weighed_against_the_kernel_that_would_run():
         assert _abi.call_kernel(p, q, c, M, N, K, K, N if b == 0 else K, N, b, 0, ws_bytes=0) == want
 
 
+def test_roles_without_a_step():
+    """The tile and split that a call runs do not hang on a few bytes, nor on more than the rule names: sizes to either side of 48 MB of operands, and
+    problems planned in 64 rows per tile, in 128x128 tiles with a short K and in two rounds of them."""
+    p, q, c = 1 << 20, 1 << 40, 1 << 44
+
+    def runs(M, N, K, a=_abi.A_MK, b=_abi.B_KN):
+        return _abi.call_plan(p, q, c, M, N, K, K if a == _abi.A_MK else M, N if b == _abi.B_KN else K, N, b, _abi.C_ROW, a)
+
+    for M, N in ((2048, 2048), (1024, 4096), (1000, 3000), (512, 8192), (700, 4000), (1500, 2500)):
+        K = int((48e6 / 2 - M * N) / (M + N)) // 64 * 64
+        got = [runs(M, N, k, b=b) for b in (_abi.B_KN, _abi.B_NK) for k in (K - 64, K, K + 64, K + 128)]
+        assert len(set(got[:4])) == 1 and len(set(got[4:])) == 1, (M, N, K, got)
+    assert runs(256, 1024, 1024, b=_abi.B_NK)[0] == _abi.VARIANT_R64x64           # (whole trips of the tile kernel's main loop)
+    assert runs(1272, 1160, 208, a=_abi.A_KM)[0] == _abi.VARIANT_R128x64           # 7.9 us in the planned tiles, 6.2
+    assert runs(3072, 3264, 304, a=_abi.A_KM)[0] == _abi.VARIANT_T128x128_W4       # 15.6, 16.2
+
+
 def test_copies_are_made_where_they_pay():
     """Shapes measured both ways, A one element off the grid ([M,K]) or with odd rows ([K,M]): us with copies / in place beside each."""
     for (M, N, K), better in (((2001, 2000, 504), "copy"),     # 14.1 / 17.0, transposed A 13.9 / 16.7

@@ -12,18 +12,23 @@ def ints(gen, *shape, top=2):
     return torch.randint(-top, top + 1, shape, generator=gen, device="cuda").to(torch.bfloat16)
 
 
-# The tile that the rule chooses at 256 CUs: 64x64 | 128x64 with a transposed A, 64x64 else | 128x128, then one more row and column than whole
-# chunks (of K-major operands), five and six stages (more than the ring holds) with 8 and 64 of them filled | 256x128 | 128x256 and, with a
-# column-major C, 256x128 | the same the other way round | 128x128 in four splits | 256x128 and 128x256 in three | 64x64, 128x64 and 128x128 in 4 to 12
-# (13 to 64 stages of the tiles up to 128x128 are staggered: 520 x 1544 x 1032 has more tiles in a row and column than stages; 1000, 1032, 1096,
-# 4104 and 8200 end in a part of a stage that is not the last to be fetched; 904 x 904 x 4104 has three splits of 17 stages and one of 14)
-@pytest.mark.parametrize("M,N,K", [(520, 1544, 1032), (1000, 2048, 1000), (1800, 1928, 392), (1801, 1929, 392), (1928, 1800, 264), (2056, 1928, 320),
-                                   (2600, 2576, 584), (1800, 4104, 1096), (4104, 1800, 1096), (904, 904, 4104), (2056, 1032, 8200),
-                                   (136, 1032, 8200), (1032, 136, 8200)])
+# Tile and split that the rule chooses at 256 CUs, by the order of C where they differ (a column-major C exchanges rows and columns), and by the order of
+# A, B and C for the last two.  13 to 64 stages of the tiles up to 128x128 are staggered: 520 x 1544 x 1032 has more tiles in a row and column than
+# stages; 1000, 1032, 4104 and 8200 end in a part of a stage that is not the last to be fetched; 904 x 904 x 4104 has three splits of 17 stages and one of 14.
+R64, R12864, R128, R256128, R128256 = g.VARIANT_R64x64, g.VARIANT_R128x64, g.VARIANT_R128x128, g.VARIANT_R256x128, g.VARIANT_R128x256
+TALL = {(0, 0, 1): (R12864, 8), (0, 1, 1): (R12864, 8), (1, 0, 0): (R128, 12), (1, 0, 1): (R12864, 8), (1, 1, 1): (R12864, 8)}
+WIDE = {(0, 0, 0): (R12864, 8), (0, 1, 0): (R12864, 8), (1, 0, 0): (R12864, 8), (1, 0, 1): (R128, 12), (1, 1, 0): (R12864, 8)}
+
+
+@pytest.mark.parametrize("M,N,K,chosen", [
+    (520, 1544, 1032, (R64, 1)), (1000, 2048, 1000, (R12864, 1)), (1800, 1928, 392, (R128, 1)), (1801, 1929, 392, (R128, 1)), (1928, 1800, 264, (R128, 1)),
+    (2040, 1928, 320, (R128, 1)), (1800, 4104, 1096, [(R128256, 1), (R256128, 1)]), (4104, 1800, 1096, [(R256128, 1), (R128256, 1)]),
+    (904, 904, 4104, (R128, 4)), (2056, 1032, 8200, {(0, 0, 0): (R128256, 3), (1, 1, 1): (R128256, 3), None: (R256128, 3)}),
+    (136, 1032, 8200, {**TALL, None: (R64, 4)}), (1032, 136, 8200, {**WIDE, None: (R64, 4)})])
 @pytest.mark.parametrize("a_layout", [g.A_MK, g.A_KM])
 @pytest.mark.parametrize("b_layout", [g.B_KN, g.B_NK])
 @pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
-def test_roles(M, N, K, a_layout, b_layout, c_layout):
+def test_roles(M, N, K, chosen, a_layout, b_layout, c_layout):
     if (M % 8 and a_layout == g.A_KM) or (N % 8 and b_layout == g.B_KN):
         pytest.skip("whole chunks only of an MN-major operand")
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
@@ -37,10 +42,11 @@ def test_roles(M, N, K, a_layout, b_layout, c_layout):
     want = (A if a_layout == g.A_MK else A.t()).float() @ (B if b_layout == g.B_KN else B.t()).float()
     C = torch.full((M, N) if c_layout == g.C_ROW else (N, M), float("nan"), dtype=torch.bfloat16, device="cuda")
     got = C if c_layout == g.C_ROW else C.t()
-    # (the plan's 128x128 tiles are kept for two rounds of workgroups, and for one where both operands are K-major)
-    kept = (M, N, K) in ((2056, 1928, 320), (2600, 2576, 584)) or ((M, N, K) == (1000, 2048, 1000) and (a_layout, b_layout) == (g.A_MK, g.B_NK))
-    name = _abi.call_kernel(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout)
-    assert name == "tile" if kept else name.startswith("roles "), name
+    if isinstance(chosen, dict):
+        chosen = chosen.get((a_layout, b_layout, c_layout), chosen[None])
+    elif isinstance(chosen, list):
+        chosen = chosen[c_layout]
+    assert _abi.call_plan(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout) == chosen
     g.gemm_into(A, B, C, M, N, K, A.stride(0), B.stride(0), C.stride(0), b_layout, c_layout, a_layout=a_layout)
     assert torch.equal(got, want.to(torch.bfloat16))
     old = got.clone()
