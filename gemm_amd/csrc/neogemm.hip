@@ -2949,6 +2949,9 @@ static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_l
   plan_model(M, N, K, aligned, c_layout, variant, split_k, batch, b_layout, ncus, a_layout, estimate_us);
 }
 
+// How much of its operands a problem of so many bytes is taken to have in HBM, more than the mean of that and of the caches.
+static double hbm_share(double bytes) { return bytes <= 32e6 ? 0.0 : bytes >= 64e6 ? 1.0 : __builtin_log2(bytes / 32e6); }
+
 // Whether gemm_roles_kernel takes a call that the model gives to kernel v with split_max splits of K, estimated at plan_us; in the kernel's
 // terms: `rows` x `cols` of C as it lies in memory, ak / bk: the row / column operand has K-contiguous rows, lda / ldb their leading dimensions.
 // Fitted to 42000 timings of 4700 problems with these tiles (1 to 20000 rows and columns, 32 to 65000 deep, both layouts of each operand, batches),
@@ -2967,6 +2970,7 @@ static void plan_uncached(int64_t M, int64_t N, int64_t K, bool aligned, int c_l
 // No more splits than planned: what a caller's workspace holds, or whether one is needed, does not change.
 struct RolesPlan {
   int bm = 0, bn = 0, split = 1;  // bm == 0: not taken
+  double us = 0;
 };
 static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, int64_t cols, int64_t K, int64_t batch, bool ak, bool bk,
                             int64_t lda, int64_t ldb) {
@@ -3008,7 +3012,7 @@ static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, 
                                 {128, 256, 5.31, 0.560, 0.713, 0.032}};
   const int64_t ktiles = ceil_div(K, KTILE);
   const double bytes = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch;
-  const double hbm = bytes <= 32e6 ? 0.0 : bytes >= 64e6 ? 1.0 : __builtin_log2(bytes / 32e6);  // how much of the operands comes from there
+  const double hbm = hbm_share(bytes);
   double best = against * plan_us;
   RolesPlan p;
   for (const Tile& t : kTiles) {
@@ -3034,9 +3038,7 @@ static RolesPlan roles_plan(int v, int split_max, double plan_us, int64_t rows, 
       if (sp > 1) us += 1.97 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 2.74e6;
       if (us < best) {
         best = us;
-        p.bm = t.bm;
-        p.bn = t.bn;
-        p.split = sp;
+        p = RolesPlan{t.bm, t.bn, sp, us};
       }
     }
   }
@@ -3192,24 +3194,17 @@ static bool ragged_takes(const void* A, const void* B, int64_t M, int64_t N, int
   const int64_t ext_b = b_layout == NEOGEMM_B_KN ? (K - 1) * ldb + N : (N - 1) * ldb + K;
   return K > 0 && ext_a >= 8 && ext_b >= 8 && lda < (1 << 21) && ldb < (1 << 21) && (((uintptr_t)A | (uintptr_t)B) & 1) == 0;
 }
-// Tile (bm x bn of the output as it lies in memory, rows x cols) and split of K of gemm_ragged_kernel, by the time of its K tiles;
-// returns the estimate for operands that come from HBM.  A workgroup of the 64x64 tile takes 0.40 us per K tile where several share a CU (the loads at two-byte
-// addresses bound it: 1023 x 2047 x 1535, 512 of them, 21 us), 0.29 alone on one (64 x 256 x 20001 in 16 splits, 14.5 us; the same
-// in 4, 26); one of the 128x128 tile, four times the work, 0.95 (1500 x 1501 x 1401: 25.3 us for 144 of them, 28.3 for 576 small
-// ones; 1023 x 2047 x 1535: 28 for 128).  A split costs the second launch and the partials (512 x 1024 x 10001 in 64x64 tiles:
-// 29 us with two, 47 unsplit).  From HBM a workgroup of the 64x64 tile gains nothing by being alone on its CU unless K is in three parts
-// or more (1001 x 1024 x 4096 28 to 34 us, the estimate without this 21.6; 256 x 1024 x 8193 in four 22, 21.8), and its K tile takes
-// 0.05 us more with both operands MN-major (255 x 4096 x 4096, 256 workgroups: 35.8 us with both, 28.9 with B [N,K]).  Every further
-// workgroup of the larger tiles on a CU costs its way in and out, 2 us (16231 x 672 x 69, three per CU: 21.8 us, the estimate without
-// this 9.7); those of the 64x64 tile are there at a time (3549 x 608 x 105, three per CU: 7.7 us, 5.4).
-static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, int cus, bool both_mn, int* bm, int* bn, int* split) {
+// The most splits of K that gemm_ragged_kernel may take for rows x cols of C as it lies in memory: what a workspace is sized for.  By the time of K
+// tiles of that kernel before it had waves with roles (so that what a caller's workspace holds stays as it was; ragged_choice has today's times).
+static int ragged_splits(int64_t rows, int64_t cols, int64_t K, int64_t batch, int cus) {
   struct Tile {
     int bm, bn;
     double alone_us, shared_us, fixed_us;  // per K tile of a workgroup that has its CU to itself / shares it
   };
   static const Tile kTiles[] = {{64, 64, 0.29, 0.40, 3.0}, {128, 64, 0.56, 0.56, 3.5}, {128, 128, 0.95, 0.95, 4.0}};
   const int64_t ktiles = ceil_div(K, KTILE);
-  double best = 1e300, from_hbm = 0;
+  double best = 1e300;
+  int split = 1;
   for (const Tile& t : kTiles)
     for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
       if (sp > 1 && ktiles / sp < 4) break;
@@ -3218,65 +3213,70 @@ static double ragged_plan(int64_t rows, int64_t cols, int64_t K, int64_t batch, 
       if (sp > 1) us += 5.0 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 4.0e6;
       if (us < best) {
         best = us;
-        from_hbm = us;
-        if (t.bm * t.bn > 64 * 64) from_hbm += 2.0 * (per_cu - 1.0);
-        else if (per_cu == 1 && sp <= 2) from_hbm += ceil_div(ktiles, sp) * (t.shared_us - t.alone_us + (both_mn ? 0.05 : 0.0));
-        *bm = t.bm;
-        *bn = t.bn;
-        *split = sp;
+        split = sp;
       }
     }
-  return from_hbm;
+  return split;
 }
-// Tile and split of K that gemm_ragged_kernel is launched with, at most the split of ragged_plan (what a workspace is sized for) and split_max.  Fitted to
-// 2600 timings of 220 problems (odd sizes from 65 to 20001; the operands in the caches and from HBM, the mean of both), rms 7 %, 1.1 % behind the
-// best of them on average.  A CU holds two workgroups, which take 1.7 times as long each (128x128: twice).
+// Tile and split of K that gemm_ragged_kernel is launched with, at most the split of ragged_splits and split_max, and its time.  Fitted to 29700
+// timings of 4600 problems (odd sizes from 1 to 80000 rows and columns and views, the mean of operands in the caches and from HBM as for roles_plan), rms
+// 9 %, 1.7 % behind the best of them on average: a launch and the writing of C (5 MB per us), per workgroup a way in and out and its stages (more of both
+// on a full chip).  More workgroups than CUs: two of the smaller tiles share a CU, two of the 128x128 tile come after each other, and a pair takes
+// `two` times as long as one; from the second pair on `again` more.
 struct RaggedChoice {
   int bm, bn, split;
+  double us;
 };
-static RaggedChoice ragged_choice(int64_t rows, int64_t cols, int64_t K, int64_t batch, bool ak, bool bk, int split_max) {
+static RaggedChoice ragged_choice(int64_t rows, int64_t cols, int64_t K, int64_t batch, int split_max) {
   struct Memo {
     int64_t rows = -1, cols = -1, K = -1, batch = -1;
-    int what = -1, cus = -1;
+    int split_max = -1, cus = -1;
     RaggedChoice c;
   };
-  const int cus = planning_cus(), what = split_max << 2 | (int)ak << 1 | (int)bk;
+  const int cus = planning_cus();
   static thread_local Memo memo[32];
   static thread_local unsigned next = 0;
   for (const Memo& m : memo)
-    if (m.rows == rows && m.cols == cols && m.K == K && m.batch == batch && m.what == what && m.cus == cus) return m.c;
+    if (m.rows == rows && m.cols == cols && m.K == K && m.batch == batch && m.split_max == split_max && m.cus == cus) return m.c;
   struct Tile {
     int bm, bn;
-    double fixed_us, stage_us, full_us, two;
+    double fixed_us, stage_us, full_us, two, again;
   };
-  static const Tile kTiles[] = {{64, 64, 2.06, 0.301, 0.037, 1.69}, {128, 64, 2.50, 0.466, 0.063, 1.68}, {128, 128, 3.40, 0.638, 0.125, 2.05}};
-  RaggedChoice c{128, 128, 1};
-  int most = 1;
-  ragged_plan(rows, cols, K, batch, cus, false, &c.bm, &c.bn, &most);
-  if (most > split_max) most = split_max;
+  static const Tile kTiles[] = {{64, 64, 0.13, 0.309, 0.036, 1.64, 0.48}, {128, 64, 0.54, 0.462, 0.042, 1.57, 1.07}, {128, 128, 1.63, 0.615, 0.027, 1.92, 1.07}};
+  RaggedChoice c{128, 128, 1, 0.0};
+  const int most = std::min(ragged_splits(rows, cols, K, batch, cus), split_max);
   const int64_t ktiles = ceil_div(K, KTILE);
+  const double bytes = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch, hbm = hbm_share(bytes);
+  const double out = 2.0 * (double)rows * (double)cols * (double)batch;
   double best = 1e300;
   for (const Tile& t : kTiles)
     for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
       if (sp > most) break;
       const double per = (double)ceil_div(ktiles, sp), wgs = (double)ceil_div(rows, t.bm) * (double)ceil_div(cols, t.bn) * sp * (double)batch;
-      const double one = t.stage_us * (1.0 - 0.06 * (2 - (int)ak - (int)bk)), full = t.fixed_us + per * (one + t.full_us);
-      const double rounds = __builtin_floor(wgs / (2.0 * cus)), left = wgs - rounds * 2.0 * cus;  // of two workgroups per CU, and what they leave
-      double us = 2.66 + rounds * full * t.two;
+      const double one = t.stage_us * (1.0 + 0.138 * hbm), full = t.fixed_us + per * (one + t.full_us);
+      const double pairs = wgs / (2.0 * cus), whole = __builtin_floor(pairs), left = wgs - whole * 2.0 * cus;
+      double us = whole * full * t.two + out / 5.06e6;
       if (left > cus) us += full * t.two;
       else if (left > 0) us += t.fixed_us + per * (one + t.full_us * left / cus);
-      const double floor_us = 2.0 * ((double)rows * K + (double)K * cols + (double)rows * cols) * (double)batch / 5.0e6;
+      if (pairs > 1.0) us += t.again * (pairs - 1.0);
+      const double floor_us = bytes / 4.72e6;
       if (us < floor_us) us = floor_us + 0.01 * us;
-      if (sp > 1) us += 2.06 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 2.46e6;
+      us += 3.89;
+      if (sp > 1) us += 2.12 + (4.0 * sp + 2.0) * (double)rows * (double)cols * (double)batch / 2.5e6;
       if (us < best) {
         best = us;
-        c = RaggedChoice{t.bm, t.bn, sp};
+        c = RaggedChoice{t.bm, t.bn, sp, us};
       }
     }
   Memo& m = memo[next++ & 31];
-  m.rows = rows, m.cols = cols, m.K = K, m.batch = batch, m.what = what, m.cus = cus;
+  m.rows = rows, m.cols = cols, m.K = K, m.batch = batch, m.split_max = split_max, m.cus = cus;
   m.c = c;
   return c;
+}
+// K of at most two stages, both operands K-major, K whole (k_major): gemm_shortk_kernel, with at least two column tiles for each of two workgroups per
+// CU (16 x 512 x 512 x 96, one each: level with the tile kernels)
+static bool shortk_takes(int64_t rows, int64_t cols, int64_t K, int64_t batch, bool k_major) {
+  return k_major && K <= 2 * KTILE && (int64_t)ceil_div(rows, 128) * ceil_div(cols, 64) * batch >= 4 * (int64_t)planning_cus();
 }
 // What gemm_generic_kernel takes, which runs where nothing else does (a leading dimension of 2^21 or more): a round trip per 16 deep,
 // and 0.125 us for each 16x16 block of a CU (129 x 64 x 4096 118 us, 1024^3 148, 2048 x 2048 x 1024 527, 20000 x 64 x 128 24.8).
@@ -3359,23 +3359,33 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
     p.b = b;
     m = &e;
     if (pack_passes(M, N, K, a_mk, b_nk, bt, p)) {
-      int v, bm, bn, sp;
-      double aligned_us = 0;
-      plan_model(p.rows, p.cols, K, true, c_layout, &v, &sp, p.count, b_layout, cus, bt.a_layout, &aligned_us);
-      const bool row = c_layout == NEOGEMM_C_ROW;
-      const double other_us =
-          in_place ? 1.03 * ragged_plan(row ? M : N, row ? N : M, K, bt.count, cus, !a_mk && !b_nk, &bm, &bn, &sp) + 2.5 : generic_us(M, N, K, bt.count, cus);
+      // the product on the copies, by the kernel that would run: for short K it writes C at 1.3 MB per us, 3 where its rows are whole pieces of 64 bytes;
+      // the tile kernels take what writing C costs more than their estimates, the strips 1.07 times them
+      int v, sp;
+      double product_us = 0;
+      plan_model(p.rows, p.cols, K, true, c_layout, &v, &sp, p.count, b_layout, cus, bt.a_layout, &product_us);
+      const bool row = c_layout == NEOGEMM_C_ROW, rk = row ? a_mk : b_nk, ck = row ? b_nk : a_mk;
+      const int64_t rows = row ? p.rows : p.cols, cols = row ? p.cols : p.rows;
+      const int64_t la = a ? chunked(a_mk ? K : p.rows) : lda, lb = b ? chunked(b_nk ? K : p.cols) : ldb;
+      const RolesPlan roles = roles_plan(v, sp, product_us, rows, cols, K, p.count, rk, ck, row ? la : lb, row ? lb : la);
+      const bool strips = v == NEOGEMM_VARIANT_STRIP || v == NEOGEMM_VARIANT_SKINNY128 || (v >= NEOGEMM_VARIANT_SKINNY16 && v <= NEOGEMM_VARIANT_SKINNY64);
+      const double out = 2.0 * (double)rows * (double)cols * (double)p.count;
+      if (shortk_takes(rows, cols, K, p.count, rk && ck && sp == 1)) product_us = out / (cols % 32 == 0 ? 3.0e6 : 1.3e6);
+      else if (roles.bm) product_us = roles.us;
+      else product_us = strips ? 1.07 * product_us : 1.03 * product_us + out / 12.4e6;
+      const double in_place_us = in_place ? ragged_choice(row ? M : N, row ? N : M, K, bt.count, 64).us : generic_us(M, N, K, bt.count, cus);
       // a panel's copy of A is made again for each panel of columns, and a shared operand's panels for each part of the batch
       const int nb = ceil_div(bt.count, p.count), nr = ceil_div(M, p.rows), nc = ceil_div(N, p.cols);
       const double moved = (double)p.bytes_a * nr * (bt.sa ? nb : nr > 1 ? nb : 1) * (nr > 1 ? nc : 1) +
                            (double)p.bytes_b * nc * (bt.sb ? nb : nc > 1 ? nb : 1);
-      // The copy and the product that waits for it: 6.5 us and 3 MB per us; in place: 3 % and 2.5 us over ragged_plan's estimate, which
-      // compares its own tiles only.  Both ways measured at 68 sizes with the operands in the caches and at 450 from HBM, one operand or both off the grid
-      // (us, copies / in place, A [M,K] and A [K,M]): 2001 x 2000 x 504 14.5 / 17.5 and 14.1 / 17.0, 201 x 4096 x 4096 26.7 / 31.3 and 26.7 /
-      // 36.9, 201 x 2048 x 8192 26.7 / 35.2 and 26.2 / 39.5, 10001 x 1024 x 512 26.0 / 38.3 and 27.2 / 34.7; below the line 777 x 784 x 776
-      // 11.6 / 11.8 and 16.9 / 11.3, 1501 x 512 x 2048 21.5 / 17.7 and 29.8 / 19.6.  The choice costs 1.4 % (1.8 % from HBM) over the better
-      // one on average, 41 % at worst; without the 3 %, the 2.5 us and the costs from HBM 4 % (6 %).
-      e.pays = (double)nb * nr * nc * (aligned_us + 6.5) + moved / 3.0e6 < other_us;
+      // the copies are in the caches when the product reads them, which its estimate does not know
+      const double bytes = 2.0 * ((double)p.rows * K + (double)K * p.cols + (double)p.rows * p.cols) * (double)p.count;
+      product_us *= 1.0 - 0.325 * hbm_share(bytes) * std::min(1.0, (double)(p.bytes_a + p.bytes_b) / bytes);
+      // The copy and the product that waits for it: 2.7 us and 1.84 MB per us.  Both ways measured at 4200 sizes with the operands in the caches and from
+      // HBM, one operand or both off the grid (us from HBM, copies / in place: 1511 x 1189 x 1909 29.7 / 24.3, 2704 x 432 x 3424 37.8 / 29.4,
+      // 917 x 1289 x 885 15.4 / 13.3; 114 x 6576 x 5207 30.1 / 39.7, 2209 x 1504 x 5171 56.1 / 70.9): the choice costs 0.7 % over the better one on
+      // average.  With the times of gemm_ragged_kernel before it had waves with roles it cost 3 %, and those first three were copied.
+      e.pays = (double)nb * nr * nc * (product_us + 2.7) + moved / 1.84e6 < 0.98 * in_place_us;
       // (the last problems, rows and columns may be fewer, and split otherwise)
       for (const int64_t c : {p.count, bt.count % p.count})
         for (const int64_t r : {p.rows, M % p.rows})
@@ -3464,7 +3474,7 @@ static int launch_unaligned(const void* A, const void* B, void* C, int64_t M, in
   a.alpha = alpha; a.beta = beta;
   const size_t partial = (size_t)M * (size_t)N * sizeof(float) * (size_t)bt.count;
   const int most = !bt.scratch_unaligned || !ws || ((uintptr_t)ws & 15) != 0 ? 1 : (int)std::min<size_t>(ws_bytes / partial, 64);
-  const RaggedChoice rc = ragged_choice(a.M, a.N, K, bt.count, ak, bk, most < 2 ? 1 : most);
+  const RaggedChoice rc = ragged_choice(a.M, a.N, K, bt.count, most < 2 ? 1 : most);
   const int bm = rc.bm, bn = rc.bn, split = rc.split;
   a.ntm = ceil_div(a.M, bm);
   a.ntn = ceil_div(a.N, bn);
@@ -3576,7 +3586,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     const bool row = c_layout == NEOGEMM_C_ROW, b_nk = b_layout == NEOGEMM_B_NK, rk = row ? a_mk : b_nk, ck = row ? b_nk : a_mk;
     const int64_t rows = row ? M : N, cols = row ? N : M;
     if ((rk || (rows & 7) == 0 || bt.padded) && (ck || (cols & 7) == 0 || bt.padded)) {
-      if (variant_roles(v)) roles = RolesPlan{kVariants[v].bm, kVariants[v].bn, s};
+      if (variant_roles(v)) roles = RolesPlan{kVariants[v].bm, kVariants[v].bn, s, 0.0};
       else if (plan_us > 0 && split_k == 0) roles = roles_plan(v, s, plan_us, rows, cols, K, bt.count, rk, ck, row ? lda : ldb, row ? ldb : lda);
     }
   }
@@ -3722,9 +3732,8 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
   a.early_stores = 0;
   a.beta = beta;
   if (plan_us > 0 && ak && bk && K <= 2 * KTILE && beta == 0.f && a.ksplit == 1) {
-    // at least two column tiles for each of two workgroups per CU (16 x 512 x 512 x 96, one each: level with the tile kernels)
-    const int64_t tiles = (int64_t)ceil_div(a.M, 128) * ceil_div(a.N, 64) * bt.count, slots = 2 * (int64_t)planning_cus();
-    if (tiles >= 2 * slots) {
+    if (shortk_takes(a.M, a.N, K, bt.count, true)) {
+      const int64_t slots = 2 * (int64_t)planning_cus();
       if (bt.only) return bt.only->set(Kernel::kShortK, NEOGEMM_VARIANT_AUTO, 1);
       const int64_t per_row = ceil_div(slots, (int64_t)ceil_div(a.M, 128) * bt.count);  // workgroups that share a block of rows
       const hipError_t e = launch_shortk(a, ceil_div(ceil_div(a.N, 64), per_row), st);
@@ -3901,7 +3910,7 @@ size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M
   bt.sa = stride_a;
   bt.sb = stride_b;
   bt.a_layout = a_layout;
-  int v, w, s = 1;
+  int v, s = 1;
   const bool row = c_layout == NEOGEMM_C_ROW;
   neogemm::PackPlan pp;
   // (an MN-major operand whose rows do not end on a chunk goes the same way as one off the 16-byte grid)
@@ -3910,7 +3919,7 @@ size_t neogemm_bf16_call_workspace_bytes(const void* A, const void* B, int64_t M
   else if (neogemm::pack_plan(A, B, M, N, K, lda, ldb, b_layout, c_layout, bt, &pp))
     return pp.total();
   else if (neogemm::ragged_takes(A, B, M, N, K, lda, ldb, b_layout, bt))
-    neogemm::ragged_plan(row ? M : N, row ? N : M, K, batch, neogemm::planning_cus(), false, &v, &w, &s);
+    s = neogemm::ragged_splits(row ? M : N, row ? N : M, K, batch, neogemm::planning_cus());
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) * (size_t)batch : 0;
 }
 

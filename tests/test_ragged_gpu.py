@@ -92,7 +92,7 @@ def test_batches_of_views(b, M, N, K):
 
 # large enough that copies on the 16-byte grid pay: K a part of a chunk past a tile, MN-major rows that end inside a chunk, one operand
 # on the grid already, K split, a batch with a shared and with a strided operand
-@pytest.mark.parametrize("b,M,N,K", [(1, 1501, 1503, 1505), (1, 512, 1024, 10001), (1, 2049, 1032, 1001), (1, 2501, 1001, 1000), (3, 1001, 1003, 1005)])
+@pytest.mark.parametrize("b,M,N,K", [(1, 2501, 2503, 2505), (1, 603, 1584, 15177), (1, 4097, 3080, 3001), (1, 3501, 2001, 2000), (3, 2001, 2003, 2005)])
 def test_copies_on_the_grid(b, M, N, K):
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
     lib = _abi.load()
@@ -123,12 +123,14 @@ def test_copies_on_the_grid(b, M, N, K):
 # few rows of A off the grid beside a B on it: copies of A alone for the decode kernels, every number of row fragments, K whose last
 # chunk is part padding (B [K,N]; the k-rows behind K are NaN), K split
 @pytest.mark.parametrize("M,N,K,b_layout,kernel", [
-    (5, 2056, 1025, g.B_KN, "skinny"), (20, 12296, 6001, g.B_KN, "skinny"), (40, 12296, 4097, g.B_KN, "skinny"), (72, 12296, 3001, g.B_KN, "skinny"),
-    (96, 14344, 4097, g.B_KN, "skinny"), (40, 6152, 4097, g.B_KN, "strip"), (64, 6152, 6001, g.B_KN, "strip"), (16, 2056, 1024, g.B_NK, "skinny"),
-    (32, 2056, 1024, g.B_NK, "skinny"), (64, 8200, 3000, g.B_NK, "skinny"), (72, 12296, 3000, g.B_NK, "skinny"), (104, 4104, 3000, g.B_NK, "strip"),
-    (128, 4104, 4096, g.B_NK, "strip"), (72, 2056, 16384, g.B_NK, "strip")])
+    (5, 4104, 1025, g.B_KN, "skinny"), (16, 12296, 6001, g.B_KN, "skinny"), (20, 6152, 2001, g.B_KN, "skinny"), (33, 13144, 20789, g.B_KN, "skinny"),
+    (70, 13872, 4142, g.B_KN, "skinny"), (92, 15272, 5205, g.B_KN, "skinny"), (36, 5464, 16310, g.B_KN, "strip"), (63, 5552, 13379, g.B_KN, "strip"),
+    (16, 2056, 1024, g.B_NK, "skinny"), (32, 1032, 1024, g.B_NK, "skinny"), (33, 13376, 14376, g.B_NK, "skinny"), (72, 14344, 7840, g.B_NK, "skinny"),
+    (96, 14344, 4096, g.B_NK, "skinny"), (104, 4104, 4096, g.B_NK, "strip"), (128, 4104, 4096, g.B_NK, "strip"), (72, 6648, 8896, g.B_NK, "strip")])
 @pytest.mark.parametrize("c_layout", [g.C_ROW, g.C_COL])
 def test_copies_for_the_decode_kernels(M, N, K, b_layout, kernel, c_layout):
+    if c_layout == g.C_COL and (M, N) in ((33, 13144), (36, 5464), (63, 5552)):
+        pytest.skip("read in place")
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
     A, B = between_nans(gen, M, K, 0, 1), between_nans(gen, *((K, N) if b_layout == g.B_KN else (N, K)), 8, 8)
     want = A.float() @ (B if b_layout == g.B_KN else B.t()).float()
@@ -145,9 +147,9 @@ def test_copies_for_the_decode_kernels(M, N, K, b_layout, kernel, c_layout):
 # copies of more than 256 MiB in panels: of the rows, of the columns, of both (a panel of A copied for each panel of columns), of the
 # problems of a batch; a last panel of one row, split otherwise than the others; rows of A [K,M] 2^21 elements apart and more
 @pytest.mark.parametrize("b,M,N,K,a_layout,b_layout,c_layout", [
-    (1, 70001, 520, 2049, g.A_MK, g.B_KN, g.C_ROW), (1, 70001, 520, 2048, g.A_KM, g.B_KN, g.C_COL), (1, 513, 70003, 2049, g.A_MK, g.B_NK, g.C_ROW),
-    (1, 4001, 4001, 40001, g.A_MK, g.B_KN, g.C_COL), (1, 4001, 4003, 40001, g.A_KM, g.B_NK, g.C_ROW), (1, 257, 2056, 600001, g.A_MK, g.B_KN, g.C_ROW),
-    (41, 1001, 1003, 1801, g.A_MK, g.B_KN, g.C_ROW), (1, 2097167, 264, 16, g.A_KM, g.B_KN, g.C_ROW)])
+    (1, 70001, 2056, 2049, g.A_MK, g.B_KN, g.C_ROW), (1, 70001, 2056, 2048, g.A_KM, g.B_KN, g.C_COL), (1, 513, 70003, 2049, g.A_MK, g.B_NK, g.C_ROW),
+    (1, 4001, 4001, 40001, g.A_MK, g.B_KN, g.C_COL), (1, 4001, 4003, 40001, g.A_KM, g.B_NK, g.C_ROW), (1, 1001, 2056, 300001, g.A_MK, g.B_KN, g.C_ROW),
+    (41, 1501, 1503, 1801, g.A_MK, g.B_KN, g.C_ROW), (1, 2097167, 264, 16, g.A_KM, g.B_KN, g.C_ROW)])
 def test_copies_in_panels(b, M, N, K, a_layout, b_layout, c_layout):
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
 
