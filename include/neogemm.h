@@ -109,6 +109,10 @@ extern "C" {
  * Unlike the reference (M,N,K % 64 == 0, nemgemmV03.cu:375) every M,N,K >= 0 is accepted; shapes or
  * pointers off the 16-byte grid (K % 8, ld % 8, alignment) run an MFMA kernel that takes any two-byte address.
  * M == 0 or N == 0 is a no-op; K == 0 writes zeros.
+ *
+ * The same call gives the same bits every time.  The order of the fp32 sums depends on the kernel, and with NEOGEMM_VARIANT_R64x64, R128x64 and
+ * R128x128 (13 to 64 stages of 64 of K per split), NEOGEMM_VARIANT_STRIP and the skinny variants also on the tile or strip that an element lies in: equal
+ * rows of A need not give equal rows of C bit for bit there (they differ by the rounding of another order of the same sum).
  */
 int neogemm_bf16(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                  int64_t ldb, int64_t ldc, int b_layout, int c_layout, void* workspace,

@@ -86,6 +86,38 @@ def test_every_tile(variant, b_layout, c_layout):
                     assert bool(torch.isnan(buf[rows * cols if off == 0 else 0]))
 
 
+# 64x64 tiles, 128x128 tiles; B [N,K] with a column-major C is the reference's call
+@pytest.mark.parametrize("n,b_layout,c_layout", [(1024, g.B_NK, g.C_COL), (1024, g.B_KN, g.C_ROW), (1536, g.B_NK, g.C_ROW)])
+def test_stagger_changes_the_order_of_sums_and_no_more(n, b_layout, c_layout):
+    """Tiles start at different stages of K, so a row of A in another tile gives a row of C that differs by the order of its sums: each within half a bf16
+    ulp and 4 sqrt(K) 2^-24 sum |a||b| of the exact product (the oracle's bound), few of them by a rounding; the same bits in every row of a tile, on every
+    call and for scaled operands."""
+    from oracle import gemm_oracle as o
+
+    def run(A, B, K=n):
+        C = torch.empty((n, n), dtype=torch.bfloat16, device="cuda")
+        g.gemm_into(A, B, C, n, n, K, A.stride(0), B.stride(0), n, b_layout, c_layout)
+        return C if c_layout == g.C_ROW else C.t()
+
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn(n, n, generator=gen, device="cuda").to(torch.bfloat16)
+    B = (torch.randn(n, n, generator=gen, device="cuda") * n ** -0.5).to(torch.bfloat16)
+    variant, split = _abi.call_plan(A.data_ptr(), B.data_ptr(), A.data_ptr(), n, n, n, n, n, n, b_layout, c_layout)
+    assert variant in (g.VARIANT_R64x64, g.VARIANT_R128x128) and split == 1
+    tile = TILES[variant][0]
+    C, moved = run(A, B), run(A.roll(tile, 0), B).roll(-tile, 0)   # every row one tile further down
+    differ = C != moved
+    assert 0 < int(differ.sum()) < 1e-3 * n * n   # (that they differ is not promised; if they no longer do, this test has nothing to hold)
+    rows = differ.any(1).nonzero()[:64, 0].cpu()
+    for got in (C, moved):
+        o.assert_parity(got.cpu()[rows], A.cpu()[rows], B.cpu(), b_layout="kn" if b_layout == g.B_KN else "nk", what=f"{n}^3, rows that differ")
+    assert torch.equal(C, run(A, B)) and torch.equal(run((A.float() * 4).bfloat16(), B), (C.float() * 4).bfloat16())
+    perm = torch.arange(n, device="cuda").view(-1, tile).flip(1).reshape(-1)   # within the tiles
+    assert torch.equal(run(A[perm], B), C[perm])
+    # fewer stages than the stagger takes (K = 768 is twelve)
+    assert torch.equal(run(A.roll(tile, 0), B, 768), run(A, B, 768).roll(tile, 0))
+
+
 # 64x64, 128x128, 128x256: the problems of a batch, the second operand shared or not
 @pytest.mark.parametrize("batch,M,N,K", [(4, 1024, 128, 1024), (32, 1024, 128, 1024), (20, 1024, 136, 1000)])
 def test_roles_batched(batch, M, N, K):
