@@ -3062,13 +3062,28 @@ static int max_planned_split(int64_t M, int64_t N, int64_t K, int64_t batch) {
   return best;
 }
 
+// The kernels that a call may end on, without the copies ahead of them and the reduction behind them.
+enum class Kernel { kNone, kGeneric, kRagged, kTile, kChain, kSkinny, kStrip, kShortK, kRoles64x64, kRoles128x64, kRoles128x128, kRoles256x128, kRoles128x256 };
+// What a call ends on: kernel, variant number (0: it has none) and split of K of the product, and whether copies on the 16-byte grid come first.
+struct Choice {
+  Kernel kernel = Kernel::kNone;
+  int variant = NEOGEMM_VARIANT_AUTO, split = 1;
+  bool copies = false;
+  int set(Kernel k, int v, int s) {
+    kernel = k;
+    variant = v;
+    split = s;
+    return NEOGEMM_OK;
+  }
+};
 // Launch of gemm_strip_kernel (65 to 128 rows).  `rings` = 16 * RA + RB forces the ring depths (0: the defaults below).
 // split_k > 1: that many workgroups per strip, each with a run of 128-deep stages; `ws` takes the partial sums and the
-// reduction kernel follows.
-static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream_t st, int split_k = 1, void* ws = nullptr,
-                        size_t ws_bytes = 0) {
+// reduction kernel follows.  only: the checks without the launch.
+static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream_t st, int split_k, void* ws, size_t ws_bytes, Choice* only) {
   int cus = 0;
-  if (hipError_t e = current_device_cus(&cus); e != hipSuccess) {
+  if (only) {
+    cus = planning_cus();
+  } else if (hipError_t e = current_device_cus(&cus); e != hipSuccess) {
     fprintf(stderr, "neogemm: device query failed: %s\n", hipGetErrorString(e));
     return NEOGEMM_ERR_LAUNCH;
   }
@@ -3120,6 +3135,7 @@ static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream
   // rings that fit the LDS
   if (sa.ra < 2 || sa.rb < 2 || sa.ra > 9 || sa.rb > 9 || (sa.ra - 2) * tmf > 63 || (sa.rb - 2) * 4 > 63 || lds > 160 * 1024)
     return NEOGEMM_ERR_UNSUPPORTED;
+  if (only) return only->set(Kernel::kStrip, NEOGEMM_VARIANT_STRIP, sa.ksplit);
   auto go = [&](auto kern) -> hipError_t {
     if (hipError_t e = allow_lds(kern, lds); e != hipSuccess) return e;
     kern<<<dim3(ceil_div(sa.N, sa.strip) * sa.ksplit), 512, lds, st>>>(sa);
@@ -3156,20 +3172,6 @@ static int launch_strip(SkinnyArgs sa, bool bkm, bool ccol, int rings, hipStream
   return NEOGEMM_OK;
 }
 
-// The kernels that a call may end on, without the copies ahead of them and the reduction behind them.
-enum class Kernel { kNone, kGeneric, kRagged, kTile, kChain, kSkinny, kStrip, kShortK, kRoles64x64, kRoles128x64, kRoles128x128, kRoles256x128, kRoles128x256 };
-// What a call ends on: kernel, variant number (0: it has none) and split of K of the product, and whether copies on the 16-byte grid come first.
-struct Choice {
-  Kernel kernel = Kernel::kNone;
-  int variant = NEOGEMM_VARIANT_AUTO, split = 1;
-  bool copies = false;
-  int set(Kernel k, int v, int s) {
-    kernel = k;
-    variant = v;
-    split = s;
-    return NEOGEMM_OK;
-  }
-};
 // A batch of `count` problems of one shape; strides in elements between consecutive problems (0: shared operand); and how
 // A is laid out, which only the general entry point lets a caller choose.
 struct BatchArgs {
@@ -3606,7 +3608,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
                     NEOGEMM_VARIANT_T128x128_W4, 1, 0, nullptr, alpha, beta, bt);
       return st2 == NEOGEMM_ERR_UNSUPPORTED ? unaligned() : st2;
     }
-    if (bt.only) return bt.only->set(v == NEOGEMM_VARIANT_STRIP ? Kernel::kStrip : Kernel::kSkinny, v, s);
+    if (bt.only && v != NEOGEMM_VARIANT_STRIP) return bt.only->set(Kernel::kSkinny, v, 1);
     SkinnyArgs sa{(const char*)A, (const char*)B, (char*)C, (int)M, (int)N, (int)K, (long)lda, (long)ldb, (long)ldc, alpha, beta, 0, 64};
     bool bkm = b_layout == NEOGEMM_B_NK, ccol = c_layout == NEOGEMM_C_COL;
     if (swap) {
@@ -3616,7 +3618,7 @@ static int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     }
     const bool wide = v == NEOGEMM_VARIANT_SKINNY128;
     sa.rot = bkm && sa.ldb % 8192 == 0;  // rows of the wide operand a multiple of 16 KiB apart
-    if (v == NEOGEMM_VARIANT_STRIP) return launch_strip(sa, bkm, ccol, group_m, st, s, workspace, workspace_bytes);
+    if (v == NEOGEMM_VARIANT_STRIP) return launch_strip(sa, bkm, ccol, group_m, st, s, workspace, workspace_bytes, bt.only);
     if (bkm) {
       // A strip of a K-major B may start at any row of it and be of any width that is a multiple of 8: the width is
       // chosen so that whole rounds of strips fill the CUs (N = 14336: 256 strips of 56 columns instead of 224 of 64,

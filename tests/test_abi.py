@@ -200,6 +200,15 @@ def test_call_kernel_names_without_a_gpu():
     assert _abi.call_kernel(p, q, c, 1800, 4104, 1096, 1096, 4104, 4104, 0, 0) == "roles 128x256"
     assert _abi.call_kernel(p, q, c, 4096, 4096, 4104, 4104, 4096, 4096, 0, 0) == "tile"
     assert _abi.call_kernel(p, q, c, 1024, 1024, 32768, 32768, 1024, 1024, 0, 0, ws_bytes=0) is None
+    # so is one of the strip kernel
+    for M, N, K, b in ((128, 8192, 8192, nk), (64, 4096, 12288, _abi.B_KN)):
+        ldb = K if b == nk else N
+        split = _abi.plan(M, N, K, b)[1]
+        need = split * M * N * 4
+        assert _abi.call_kernel(p, q, c, M, N, K, K, ldb, N, b, 0) == "strip" and split > 1
+        assert _abi.call_plan(p, q, c, M, N, K, K, ldb, N, b, 0, ws_bytes=need) == (_abi.VARIANT_STRIP, split)
+        assert _abi.call_kernel(p, q, c, M, N, K, K, ldb, N, b, 0, ws_bytes=need - 1) is None
+        assert _abi.call_kernel(p, q, c, M, N, K, K, ldb, N, b, 0, ws_bytes=0) is None
 
 
 def test_call_plan_tells_tile_and_split():
