@@ -148,7 +148,7 @@ def test_copies_for_the_decode_kernels(M, N, K, b_layout, kernel, c_layout):
 # problems of a batch; a last panel of one row, split otherwise than the others; rows of A [K,M] 2^21 elements apart and more
 @pytest.mark.parametrize("b,M,N,K,a_layout,b_layout,c_layout", [
     (1, 70001, 2056, 2049, g.A_MK, g.B_KN, g.C_ROW), (1, 70001, 2056, 2048, g.A_KM, g.B_KN, g.C_COL), (1, 513, 70003, 2049, g.A_MK, g.B_NK, g.C_ROW),
-    (1, 4001, 4001, 40001, g.A_MK, g.B_KN, g.C_COL), (1, 4001, 4003, 40001, g.A_KM, g.B_NK, g.C_ROW), (1, 1001, 2056, 300001, g.A_MK, g.B_KN, g.C_ROW),
+    (1, 4001, 4001, 40001, g.A_MK, g.B_KN, g.C_COL), (1, 4001, 4003, 40001, g.A_KM, g.B_NK, g.C_ROW), (1, 513, 4104, 300001, g.A_MK, g.B_KN, g.C_ROW),
     (41, 1501, 1503, 1801, g.A_MK, g.B_KN, g.C_ROW), (1, 2097167, 264, 16, g.A_KM, g.B_KN, g.C_ROW)])
 def test_copies_in_panels(b, M, N, K, a_layout, b_layout, c_layout):
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
