@@ -3385,9 +3385,11 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
       product_us *= 1.0 - 0.325 * hbm_share(bytes) * std::min(1.0, (double)(p.bytes_a + p.bytes_b) / bytes);
       // The copy and the product that waits for it: 2.7 us and 1.84 MB per us.  Both ways measured at 4200 sizes with the operands in the caches and from
       // HBM, one operand or both off the grid (us from HBM, copies / in place: 1511 x 1189 x 1909 29.7 / 24.3, 2704 x 432 x 3424 37.8 / 29.4,
-      // 917 x 1289 x 885 15.4 / 13.3; 114 x 6576 x 5207 30.1 / 39.7, 2209 x 1504 x 5171 56.1 / 70.9): the choice costs 0.7 % over the better one on
+      // 917 x 1289 x 885 15.4 / 13.3; 114 x 6576 x 5207 30.1 / 39.7, 2209 x 1504 x 5171 56.1 / 70.9): the choice costs 0.5 % over the better one on
       // average.  With the times of gemm_ragged_kernel before it had waves with roles it cost 3 %, and those first three were copied.
-      e.pays = (double)nb * nr * nc * (product_us + 2.7) + moved / 1.84e6 < 0.98 * in_place_us;
+      // Beyond the caches the estimates are a few percent high for copies and low in place, hence the factor.
+      const double whole = 2.0 * ((double)M * K + (double)K * N + (double)M * N) * (double)bt.count;
+      e.pays = (double)nb * nr * nc * (product_us + 2.7) + moved / 1.84e6 < (0.96 + 0.12 * hbm_share(whole)) * in_place_us;
       // (the last problems, rows and columns may be fewer, and split otherwise)
       for (const int64_t c : {p.count, bt.count % p.count})
         for (const int64_t r : {p.rows, M % p.rows})
