@@ -3387,9 +3387,11 @@ static bool pack_plan(const void* A, const void* B, int64_t M, int64_t N, int64_
       // HBM, one operand or both off the grid (us from HBM, copies / in place: 1511 x 1189 x 1909 29.7 / 24.3, 2704 x 432 x 3424 37.8 / 29.4,
       // 917 x 1289 x 885 15.4 / 13.3; 114 x 6576 x 5207 30.1 / 39.7, 2209 x 1504 x 5171 56.1 / 70.9): the choice costs 0.5 % over the better one on
       // average.  With the times of gemm_ragged_kernel before it had waves with roles it cost 3 %, and those first three were copied.
-      // Beyond the caches the estimates are a few percent high for copies and low in place, hence the factor.
+      // Beyond the caches the estimates are a few percent high for copies and low in place, hence the factor.  Up to 32 MB 0.96 and 0.98 choose alike on
+      // average (202 sizes within 20 % of the line: 1.97 and 1.96 % over the better one), but a product added to C costs more in place (the weight
+      // gradient 10001 x 1024 x 512: 28.6 / 31.2 added, 25.7 / 25.2 written, which this rule does not see): 0.98 0.6 % over the better one for those, 0.96 0.75.
       const double whole = 2.0 * ((double)M * K + (double)K * N + (double)M * N) * (double)bt.count;
-      e.pays = (double)nb * nr * nc * (product_us + 2.7) + moved / 1.84e6 < (0.96 + 0.12 * hbm_share(whole)) * in_place_us;
+      e.pays = (double)nb * nr * nc * (product_us + 2.7) + moved / 1.84e6 < (0.98 + 0.10 * hbm_share(whole)) * in_place_us;
       // (the last problems, rows and columns may be fewer, and split otherwise)
       for (const int64_t c : {p.count, bt.count % p.count})
         for (const int64_t r : {p.rows, M % p.rows})

@@ -271,6 +271,7 @@ def test_copies_are_made_where_they_pay():
     for (M, N, K), want in (((20001, 2048, 128), "copy"),    # 30.2 / 43.5
                             ((30001, 1024, 256), "copy"),    # 37.2 / 46.9
                             ((5951, 1920, 207), "copy"),     # 16.7 / 19.6
+                            ((10001, 1024, 512), "copy"),    # 28.6 / 31.2 added to C
                             ((989, 1088, 959), "ragged"),    # 12.9 / 11.0
                             ((3549, 608, 105), "ragged")):   # 9.3 / 5.7
         got = _abi.call_kernel(1 << 20, 1 << 40, 1 << 44, M, N, K, M, N, N, _abi.B_KN, _abi.C_ROW, _abi.A_KM)
